@@ -13,7 +13,7 @@
 #include <vector>
 
 #include "rt_internal.hpp"
-#include "traverse.hpp"
+#include "team.hpp"
 
 namespace rtgpu {
 namespace {
@@ -110,6 +110,42 @@ __device__ __forceinline__ void store_refined(const SceneView &sc, const Trav &t
     }
     store_hit_nt(hits, i, h);
     if (counts) reinterpret_cast<uint2 *>(counts)[i] = make_uint2(t.nbox, t.ntri);
+}
+
+// One team of T lanes per ray, one wave per block, every ray at once: no work counter, no refill.
+template <int T, bool ANY, bool REFINE> __global__ __launch_bounds__(64) void k_trace_team(TraceArgs a, uint32_t limit) {
+    __shared__ uint2 stacks[64 / T * team_stack(T)];
+    const uint32_t i = blockIdx.x * (64u / T) + threadIdx.x / T;
+    const bool live = i < a.n;
+    v3 o{0.0f, 0.0f, 0.0f}, d{0.0f, 0.0f, 0.0f};
+    float tmin = 0.0f, tmax = 0.0f;
+    if (live) load_ray(a.rays, i, o, tmin, d, tmax);
+    const TeamHit h = team_trace<T, ANY>(live, o, d, tmin, tmax, a.sc.wide, a.sc.nwide, a.sc.rec, stacks, limit);
+    if (!live) return;
+    if (h.owner || (h.slot == kEmpty && threadIdx.x % T == 0)) {
+        Trav t;
+        t.o = o;
+        t.d = d;
+        t.bt = h.t;
+        t.bslot = h.slot;
+        t.bu = h.u;
+        t.bv = h.v;
+        if constexpr (REFINE) store_refined(a.sc, t, a.hits, nullptr, i);
+        else store_hit(a.sc, t, a.hits, nullptr, i);
+    }
+}
+
+template <int T> void *team_kernel_t(bool any, bool refine) {
+    if (any) return refine ? (void *)k_trace_team<T, true, true> : (void *)k_trace_team<T, true, false>;
+    return refine ? (void *)k_trace_team<T, false, true> : (void *)k_trace_team<T, false, false>;
+}
+void *team_kernel(uint32_t t, bool any, bool refine) {
+    switch (t) {
+        case 8: return team_kernel_t<8>(any, refine);
+        case 16: return team_kernel_t<16>(any, refine);
+        case 32: return team_kernel_t<32>(any, refine);
+        default: return team_kernel_t<64>(any, refine);
+    }
 }
 
 // REFINE: store each hit with t, u, v refined in double (store_refined) instead of the fp32 values.
@@ -401,6 +437,24 @@ LaunchCfg resolve_cfg(const rt_context *ctx, const Scene &sc, const rt_launch_co
     return c;
 }
 
+// Lanes per ray of a plain launch of n rays; 0: one lane per ray.  The lines lie where the times
+// cross (us; 256 CUs; closest hit, 1 M triangles unless stated):
+//   24 rays per CU     a wave per ray, every wave resident: 4,096 rays 21.4 with 64 lanes, 22.6 with 32
+//   128 rays per CU    16,384 rays 33.0 with 32 lanes, 42.5 with 16; 65,536 rays 80.1 and 75.0
+//   1,024 rays per CU  131,072 rays 114.8 with 16 lanes, 126.7 with 8; 524,288 rays 359 and 347
+//   3,072 rays per CU  524,288 rays 347 with 8 lanes, 472 with one; 1,000,000 rays 632 and 604
+//                      (4 M triangles 426 and 579, 768 and 715; 1,024 triangles 113 and 230, 202 and 323)
+// Four lanes per ray were slower than eight at every size.  A launch that counts tests per ray keeps
+// one lane per ray (its counts are those of the ordered traversal), as do the widths 2 and 8, a
+// caller's one-lane-per-ray configuration, and a tree too deep for the team's stack.
+static uint32_t team_size(const rt_context *ctx, const Scene &sc, uint32_t n, const LaunchCfg &c, bool count) {
+    if (sc.width != 4 || count || !c.persistent) return 0;
+    const uint64_t cus = (uint64_t)ctx->num_cus;
+    if (n > 3072u * cus) return 0;
+    const uint32_t t = n <= 24u * cus ? 64u : n <= 128u * cus ? 32u : n <= 1024u * cus ? 16u : 8u;
+    return team_limit(t, sc.stack_bound) ? t : 0u;
+}
+
 void launch_trace(rt_context *ctx, const Scene &sc, const rt_ray *rays, uint32_t n, rt_hit *hits, uint32_t *counts,
                   uint32_t flags, const LaunchCfg &c, hipStream_t stream) {
     if (n == 0) return;
@@ -414,6 +468,13 @@ void launch_trace(rt_context *ctx, const Scene &sc, const rt_ray *rays, uint32_t
     const bool refine_in_kernel = refine && !any && c.persistent;
     TraceArgs a{view_of(sc), rays, hits, counts, n, c.refill, nullptr, c.leaf_weight, nullptr};
     const size_t lds = stack_lds_bytes(c.lds_stack, c.block);
+    if (const uint32_t team = team_size(ctx, sc, n, c, counts != nullptr)) {
+        uint32_t limit = team_limit(team, sc.stack_bound);
+        void *args[] = {&a, &limit};
+        RT_HIP(hipLaunchKernel(team_kernel(team, any, refine), dim3((n + 64u / team - 1) / (64u / team)), dim3(64), args, 0, stream));
+        RT_HIP(hipGetLastError());
+        return;
+    }
     if (!c.persistent) {
         void *k = pick_kernel(sc.width, c.lds_stack, 0, any, counts != nullptr);
         const uint32_t grid = (uint32_t)(((uint64_t)n + c.block - 1) / c.block);
