@@ -165,8 +165,9 @@ typedef struct rt_launch_config {
 
 /* Closest-hit / any-hit ray query (the hitBVH/sceneHit semantics of raytraceBVH.comp:195-274
  * with per-ray [tmin, tmax]).  A launch of few rays over a width-4 tree without counts traces each ray with
- * several lanes (cfg then only chooses between persistent and one lane per ray).  rays, hits: device.  counts (device, may be NULL): per ray
- * uint32 {AABB tests, primitive tests}.  cfg may be NULL (defaults / autotuned). */
+ * several lanes (cfg then only chooses between persistent and one lane per ray).  rays, hits: device.
+ * counts (device, may be NULL): per ray uint32 {AABB tests, primitive tests}.  cfg may be NULL (defaults /
+ * autotuned). */
 int rt_trace(rt_context *ctx, uint32_t scene_id, const rt_ray *rays, uint32_t n, rt_hit *hits,
              uint32_t *counts, uint32_t flags, const rt_launch_config *cfg, void *stream);
 

@@ -203,7 +203,7 @@ int rt_render_batch(rt_context *ctx, const rt_render_job *jobs, uint32_t njobs, 
         if (njobs == 0) return;
         const LaunchCfg c = resolve_cfg(ctx, ctx->scene(jobs[0].scene_id), cfg, false);
         hipStream_t st = static_cast<hipStream_t>(stream);
-        std::map<uint32_t, std::vector<RenderJob>> by_width;
+        std::map<uint32_t, std::vector<RenderJob>> by_layout;
         std::vector<std::pair<const Scene *, RenderJob>> waves;  // images rendered bounce by bounce, as rt_render would
         std::vector<std::pair<uintptr_t, uintptr_t>> ranges;
         std::vector<std::pair<RenderJob *, uint32_t>> split;  // (job, samples per item)
@@ -217,12 +217,12 @@ int rt_render_batch(rt_context *ctx, const rt_render_job *jobs, uint32_t njobs, 
             const uintptr_t b = reinterpret_cast<uintptr_t>(j.accum);
             ranges.emplace_back(b, b + 16ull * j.width * j.height);
             if (j.spp && wave_schedule(j.width, j.height, j.spp, j.flags)) waves.emplace_back(&s, rj);
-            else by_width[s.width].push_back(rj);
+            else by_layout[rj.layout].push_back(rj);
         }
         std::sort(ranges.begin(), ranges.end());
         for (size_t i = 1; i < ranges.size(); ++i)
             RT_REQUIRE(ranges[i].first >= ranges[i - 1].second, "rt_render_batch: accumulation images overlap");
-        for (auto &kv : by_width)
+        for (auto &kv : by_layout)
             for (RenderJob &rj : kv.second)
                 if (const uint32_t g = split_group(ctx, rj.width, rj.height, rj.spp, rj.flags)) {
                     split.emplace_back(&rj, g);
@@ -236,7 +236,7 @@ int rt_render_batch(rt_context *ctx, const rt_render_job *jobs, uint32_t njobs, 
             make_split(*rj, reinterpret_cast<float4 *>(scratch + off), g);
             off += 16ull * rj->width * rj->height * rj->spp;
         }
-        for (auto &kv : by_width) launch_render_jobs(ctx, kv.second, kv.first, segments, c, st);
+        for (auto &kv : by_layout) launch_render_jobs(ctx, kv.second, kv.first, segments, c, st);
         for (auto &[s, rj] : waves) launch_render_wave(ctx, *s, rj, segments, c, st, nullptr, 0);
         const int used = ctx->record_use(st);
         for (uint32_t i = 0; i < njobs; ++i) ctx->scene(jobs[i].scene_id).note_use(st, used);

@@ -9,7 +9,9 @@
 // leaf slot (LeafRecord).  The reference's single-workgroup reduction and sort
 // are replaced by device-wide kernels.
 #include <algorithm>
+#include <cmath>
 #include <cstring>
+#include <limits>
 #include <vector>
 
 #include "rt_internal.hpp"
@@ -637,6 +639,111 @@ __global__ void k_collapse_emit(CollapseArgs a, const uint32_t *queue, uint32_t 
     }
 }
 
+// One axis of a compressed node (rt_device.hpp): lo, hi are the planes of its nc children.  False when a
+// plane is not finite or too large, or a box is inverted: its exact tests do not order the two planes.
+__device__ inline bool compress_axis(const float *lo, const float *hi, const uint32_t *child, float &org, float &scale,
+                                     uint32_t &qlo, uint32_t &qhi) {
+    float mn = 0x1p24f, mx = -0x1p24f;
+    bool ok = true;
+    for (int k = 0; k < 4; ++k)
+        if (child[k] != kEmpty) {
+            ok = ok && fabsf(lo[k]) < 0x1p24f && fabsf(hi[k]) < 0x1p24f && lo[k] <= hi[k];
+            mn = fminf(mn, lo[k]);
+            mx = fmaxf(mx, hi[k]);
+        }
+    qlo = qhi = 0u;
+    // 248 steps over the extent; a step is no finer than the origin's rounding, at most a quarter of it
+    scale = fmaxf(fmaxf((mx - mn) * (1.0f / 248.0f), 0x1p-22f * fmaxf(fabsf(mn), fabsf(mx))), 0x1p-100f);
+    org = (float)((double)mn - 1026.0 * (double)scale);
+    const double s = 1.0 / (double)scale;
+    for (int k = 0; k < 4; ++k) {
+        double l = 255.0, h = 0.0;
+        if (child[k] != kEmpty) {
+            l = floor(((double)lo[k] - (double)org) * s - (1024.0 + kPlaneMargin));
+            h = ceil(((double)hi[k] - (double)org) * s - (1024.0 - kPlaneMargin));
+            ok = ok && l >= 0.0 && h <= 255.0;
+        }
+        qlo |= ((uint32_t)l & 255u) << (8 * k);
+        qhi |= ((uint32_t)h & 255u) << (8 * k);
+    }
+    return ok;
+}
+
+// A caller's node buffer may hold any boxes; compressed nodes need every box to hold what is below it.
+// *bad = 1 when one does not (one store per wave).
+__global__ void k_check_boxes(const rt_bvh_node *nodes, uint32_t n, const rt_triangle *tris, const rt_sphere *sph,
+                              const uint32_t *slot_prim, uint32_t *bad) {
+    const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
+    if (i >= 2u * n - 1u) return;
+    const rt_bvh_node nd = nodes[i];
+    const float lo[3] = {nd.minX, nd.minY, nd.minZ}, hi[3] = {nd.maxX, nd.maxY, nd.maxZ};
+    bool ok = true;
+    if (i < n - 1u) {
+        for (uint32_t c : {nd.left, nd.right}) {
+            const rt_bvh_node b = nodes[c];
+            ok = ok && lo[0] <= b.minX && b.maxX <= hi[0] && lo[1] <= b.minY && b.maxY <= hi[1] && lo[2] <= b.minZ &&
+                 b.maxZ <= hi[2];
+        }
+    } else {
+        const uint32_t p = slot_prim[i - (n - 1u)];
+        for (int a = 0; a < 3; ++a) {
+            if (p & RT_SPHERE_BIT) {
+                const rt_sphere &s = sph[p & ~RT_SPHERE_BIT];
+                const float r = fabsf(s.radius);
+                ok = ok && lo[a] <= s.center[a] - r && s.center[a] + r <= hi[a];
+            } else {
+                const rt_triangle &t = tris[p];
+                ok = ok && lo[a] <= t.v0[a] && lo[a] <= t.v1[a] && lo[a] <= t.v2[a] && t.v0[a] <= hi[a] &&
+                     t.v1[a] <= hi[a] && t.v2[a] <= hi[a];
+            }
+        }
+    }
+    const unsigned long long fail = __ballot(!ok);
+    if (fail != 0ull && __lane_id() == (uint32_t)__ffsll((long long)fail) - 1u) *bad = 1u;
+}
+
+// Compressed copies of the width-4 nodes, and the node and child that hold each leaf slot.  info[0] = 1 when
+// some node cannot be compressed (one store per wave); info[1], info[2]: the scene's largest coordinate in
+// magnitude and its largest extent (the root's planes).
+__global__ void k_compress(const uint32_t *wide, uint32_t nwide, uint32_t *qwide, uint32_t *slot_ref, uint32_t *info) {
+    const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
+    if (i >= nwide) return;
+    const uint32_t *nd = wide + (size_t)i * 32u;
+    const float *f = reinterpret_cast<const float *>(nd);
+    const uint4 ch = reinterpret_cast<const uint4 *>(nd)[6];
+    const uint32_t child[4] = {ch.x, ch.y, ch.z, ch.w};
+    float org[3], scale[3];
+    uint32_t lo[3], hi[3];
+    bool ok = true;
+    for (int a = 0; a < 3; ++a)
+        ok = compress_axis(f + 8 * a, f + 8 * a + 4, child, org[a], scale[a], lo[a], hi[a]) && ok;
+    uint4 *q = reinterpret_cast<uint4 *>(qwide) + (size_t)i * 4u;
+    q[0] = make_uint4(__float_as_uint(org[0]), __float_as_uint(org[1]), __float_as_uint(org[2]), __float_as_uint(scale[0]));
+    q[1] = make_uint4(child[0], lo[0], child[1], hi[0]);
+    q[2] = make_uint4(child[2], lo[1], child[3], hi[1]);
+    q[3] = make_uint4(lo[2], hi[2], __float_as_uint(scale[1]), __float_as_uint(scale[2]));
+    for (uint32_t k = 0; k < 4; ++k)
+        if (child[k] != kEmpty && (child[k] & kLeafBit))
+            for (uint32_t s = leaf_first(child[k]), e = s + leaf_count(child[k]); s < e; ++s) slot_ref[s] = 4u * i + k;
+    const unsigned long long fail = __ballot(!ok);
+    if (fail != 0ull && __lane_id() == (uint32_t)__ffsll((long long)fail) - 1u) info[0] = 1u;
+    if (i == 0) {
+        float far = 0.0f, ext = 0.0f;
+        for (int a = 0; a < 3; ++a) {
+            float mn = f[8 * a], mx = f[8 * a + 4];
+            for (int k = 1; k < 4; ++k)
+                if (child[k] != kEmpty) {
+                    mn = fminf(mn, f[8 * a + k]);
+                    mx = fmaxf(mx, f[8 * a + 4 + k]);
+                }
+            far = fmaxf(far, fmaxf(fabsf(mn), fabsf(mx)));
+            ext = fmaxf(ext, mx - mn);
+        }
+        info[1] = __float_as_uint(far);
+        info[2] = __float_as_uint(ext);
+    }
+}
+
 template <class T> void upload(DevBuf &b, const T *src, size_t count) {
     b.alloc(sizeof(T) * count);
     if (count) RT_HIP(hipMemcpy(b.p, src, sizeof(T) * count, hipMemcpyHostToDevice));
@@ -746,11 +853,15 @@ void build_scene(rt_context *ctx, Scene &sc, const rt_triangle *tris, uint32_t n
     }
     // centre-based u, v of every sphere (raytraceBVH.comp:172-173), from its world-space centre
     DevBuf duv;
+    float min_radius = std::numeric_limits<float>::max();
     if (nsph) {
         std::vector<rt_sphere> world(sph, sph + nsph);
         if (models) RT_HIP(hipMemcpy(world.data(), dsph.p, sizeof(rt_sphere) * nsph, hipMemcpyDeviceToHost));
         std::vector<float2> uv(nsph);
-        for (uint32_t i = 0; i < nsph; ++i) sphere_uv(world[i].center, uv[i].x, uv[i].y);
+        for (uint32_t i = 0; i < nsph; ++i) {
+            sphere_uv(world[i].center, uv[i].x, uv[i].y);
+            min_radius = std::fmin(min_radius, std::fabs(world[i].radius));
+        }
         upload(duv, uv.data(), nsph);
     }
     sc.slot_prim.alloc(sizeof(uint32_t) * n);
@@ -812,7 +923,7 @@ void build_scene(rt_context *ctx, Scene &sc, const rt_triangle *tris, uint32_t n
     uint32_t *wide_tmp = tmp.take<uint32_t>(8ull * W * max_nodes);
     uint32_t *qa = tmp.take<uint32_t>(max_nodes), *qb = tmp.take<uint32_t>(max_nodes);
     uint32_t *newcount = tmp.take<uint32_t>(max_nodes), *child_base = tmp.take<uint32_t>(max_nodes);
-    uint32_t *d_total = tmp.take<uint32_t>(1);
+    uint32_t *d_total = tmp.take<uint32_t>(3);
     k_fill_u32<<<1, 64, 0, st>>>(qa, 0u, 1u);  // the root
     uint32_t qn = 1, level_base = 0, depth = 0;
     uint32_t *qcur = qa, *qnext = qb;
@@ -840,6 +951,26 @@ void build_scene(rt_context *ctx, Scene &sc, const rt_triangle *tris, uint32_t n
     sc.nwide = level_base;
     sc.wide.alloc((size_t)sc.nwide * 32u * W);
     RT_HIP(hipMemcpy(sc.wide.p, wide_tmp, (size_t)sc.nwide * 32u * W, hipMemcpyDeviceToDevice));
+    if (W == 4) {
+        sc.qwide.alloc((size_t)sc.nwide * 64u);
+        sc.slot_ref.alloc(sizeof(uint32_t) * n);
+        k_fill_u32<<<1, 64, 0, st>>>(d_total, 0u, 1u);
+        if (nodes)
+            k_check_boxes<<<grid_for(2ull * n - 1), kB, 0, st>>>(binary, n, dtris.as<rt_triangle>(), dsph.as<rt_sphere>(),
+                                                                 sc.slot_prim.as<uint32_t>(), d_total);
+        k_compress<<<grid_for(sc.nwide), kB, 0, st>>>(sc.wide.as<uint32_t>(), sc.nwide, sc.qwide.as<uint32_t>(),
+                                                      sc.slot_ref.as<uint32_t>(), d_total);
+        RT_HIP(hipGetLastError());
+        struct { uint32_t bad; float far, extent; } info{};
+        RT_HIP(hipMemcpy(&info, d_total, sizeof info, hipMemcpyDeviceToHost));
+        // see Scene::far_limit: origins may lie this far outside the scene's coordinates
+        const float reach = std::min(1000.0f * info.extent, 512.0f * min_radius);
+        sc.far_limit = info.far + reach;
+        if (info.bad || !(reach >= 1.8f * info.extent)) {  // also where a sphere is too small to be seen across the scene
+            sc.qwide.release();
+            sc.slot_ref.release();
+        }
+    }
     sc.wide_depth = depth;
     sc.leaf_size = L;
     sc.stack_bound = (W - 1u) * depth + 1u;

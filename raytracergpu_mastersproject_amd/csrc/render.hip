@@ -90,7 +90,7 @@ struct PixelState {
     uint32_t pc_slot;  // cached first segment
     float pc_t;
     bool pc_valid;
-    const uint32_t *wide;  // the job's BVH (multi-image launches)
+    const uint32_t *nodes;  // the job's BVH (multi-image launches)
     const LeafRecord *rec;
 };
 
@@ -104,9 +104,9 @@ template <bool MULTI> __device__ __forceinline__ const LeafRecord *rec_of(const 
     else return a.job0.rec;
 }
 
-template <bool MULTI> __device__ __forceinline__ const uint32_t *wide_of(const RenderArgs &a, const PixelState &ps) {
-    if constexpr (MULTI) return ps.wide;
-    else return a.job0.wide;
+template <bool MULTI> __device__ __forceinline__ const uint32_t *nodes_of(const RenderArgs &a, const PixelState &ps) {
+    if constexpr (MULTI) return ps.nodes;
+    else return a.job0.nodes;
 }
 
 __device__ __forceinline__ void primary(const RenderJob &J, uint32_t x, uint32_t y, v3 &o, v3 &d) {
@@ -117,7 +117,7 @@ __device__ __forceinline__ void primary(const RenderJob &J, uint32_t x, uint32_t
     d = normalize(normalize(ps - org));  // getRay normalises; rayColor normalises again
 }
 
-template <bool MULTI>
+template <int W, bool MULTI>
 __device__ __forceinline__ void begin_segment(const RenderArgs &a, PixelState &ps, Trav &t, uint32_t &segs) {
     if (ps.bounce == 0 && ps.pc_valid) {
         ps.hslot = ps.pc_slot;
@@ -125,12 +125,12 @@ __device__ __forceinline__ void begin_segment(const RenderArgs &a, PixelState &p
         ps.phase = kResolved;
         return;
     }
-    trav_init(t, ps.o, ps.d, 0.001f, 10000000.0f, job_of<MULTI>(a, ps).nwide);
+    trav_init<W>(t, ps.o, ps.d, 0.001f, 10000000.0f, job_of<MULTI>(a, ps).nwide);
     ps.phase = kTracing;
     segs++;
 }
 
-template <bool MULTI>
+template <int W, bool MULTI>
 __device__ __forceinline__ void begin_sample(const RenderArgs &a, PixelState &ps, Trav &t, uint32_t &segs) {
     const RenderJob &J = job_of<MULTI>(a, ps);
     ps.st = ps.seed0 + f2u_sat(ps.acc[3] * 4294967294.0f);  // the literal is 2^32 in fp32
@@ -144,11 +144,11 @@ __device__ __forceinline__ void begin_sample(const RenderArgs &a, PixelState &ps
         ps.phase = kResolved;
         return;
     }
-    begin_segment<MULTI>(a, ps, t, segs);
+    begin_segment<W, MULTI>(a, ps, t, segs);
 }
 
 // returns false when the pixel is finished
-template <bool MULTI>
+template <int W, bool MULTI>
 __device__ __forceinline__ bool end_sample(const RenderArgs &a, PixelState &ps, Trav &t, uint32_t &segs) {
     const RenderJob &J = job_of<MULTI>(a, ps);
     if (J.group) {  // split job: hand the sample to the in-order sum, then the item's next one
@@ -157,7 +157,7 @@ __device__ __forceinline__ bool end_sample(const RenderArgs &a, PixelState &ps, 
         ps.sample++;
         if (ps.sample < J.spp && ps.sample % J.group != 0) {
             ps.acc[3] = ps.next;
-            begin_sample<MULTI>(a, ps, t, segs);
+            begin_sample<W, MULTI>(a, ps, t, segs);
             return true;
         }
         ps.phase = kIdle;
@@ -169,7 +169,7 @@ __device__ __forceinline__ bool end_sample(const RenderArgs &a, PixelState &ps, 
     ps.acc[3] = ps.next;
     ps.sample++;
     if (ps.sample < J.spp) {
-        begin_sample<MULTI>(a, ps, t, segs);
+        begin_sample<W, MULTI>(a, ps, t, segs);
         return true;
     }
     reinterpret_cast<float4 *>(J.accum)[ps.pix] = make_float4(ps.acc[0], ps.acc[1], ps.acc[2], ps.acc[3]);
@@ -273,7 +273,7 @@ __device__ __forceinline__ bool shade_segment(const RenderJob &J, const LeafReco
 }
 
 // a resolved segment of a persistent-kernel path
-template <bool MULTI>
+template <int W, bool MULTI>
 __device__ __forceinline__ void shade(const RenderArgs &a, PixelState &ps, Trav &t, uint32_t &segs) {
     const RenderJob &J = job_of<MULTI>(a, ps);
     if (ps.bounce == 0 && !ps.pc_valid && !(J.flags & RT_RENDER_NO_PRIMARY_CACHE)) {
@@ -282,15 +282,15 @@ __device__ __forceinline__ void shade(const RenderArgs &a, PixelState &ps, Trav 
         ps.pc_valid = true;
     }
     if (!shade_segment(J, rec_of<MULTI>(a, ps), ps.hslot, ps.ht, ps.o, ps.d, ps.st, ps.color, ps.atten)) {
-        end_sample<MULTI>(a, ps, t, segs);
+        end_sample<W, MULTI>(a, ps, t, segs);
         return;
     }
     ps.bounce++;
     if (ps.bounce >= J.depth) {
-        end_sample<MULTI>(a, ps, t, segs);
+        end_sample<W, MULTI>(a, ps, t, segs);
         return;
     }
-    begin_segment<MULTI>(a, ps, t, segs);
+    begin_segment<W, MULTI>(a, ps, t, segs);
 }
 
 // `local` is the item index within its job.  Pixel jobs: 64 items per 8x8 tile.  Split
@@ -337,6 +337,12 @@ __device__ __forceinline__ uint32_t find_job(const RenderJob *jobs, uint32_t njo
     return lo;
 }
 
+// exact leaf boxes of a job's scene
+struct JobBoxes {
+    const RenderJob &j;
+    __device__ LeafBoxes operator()() const { return LeafBoxes{j.wide, j.slot_ref}; }
+};
+
 template <int W, int S, bool MULTI>
 __global__ __launch_bounds__(256) void k_render(RenderArgs a) {
     extern __shared__ uint32_t lds[];
@@ -380,7 +386,7 @@ __global__ __launch_bounds__(256) void k_render(RenderArgs a) {
                 uint32_t x, y, sample;
                 if (item_to_pixel(J, item - J.first_item, x, y, sample)) {
                     if constexpr (MULTI) {
-                        ps.wide = J.wide;
+                        ps.nodes = J.nodes;
                         ps.rec = J.rec;
                     }
                     ps.x = x;
@@ -393,7 +399,7 @@ __global__ __launch_bounds__(256) void k_render(RenderArgs a) {
                     if (J.group) ps.acc[3] = carry_at(ps.seed0, acc.w, sample);  // this item's samples only
                     ps.pc_valid = false;
                     if (J.spp == 0) ps.phase = kIdle;
-                    else begin_sample<MULTI>(a, ps, t, segs);
+                    else begin_sample<W, MULTI>(a, ps, t, segs);
                 }
             }
         }
@@ -402,15 +408,16 @@ __global__ __launch_bounds__(256) void k_render(RenderArgs a) {
         const unsigned long long mres = __ballot(ps.phase == kResolved), mtr = __ballot(ps.phase == kTracing);
         if (shade_now(mres, mtr, a.shade_min)) {
             // resolved segments may chain (cached primary hit, depth reached): bounded by spp*depth
-            while (ps.phase == kResolved) shade<MULTI>(a, ps, t, segs);
+            while (ps.phase == kResolved) shade<W, MULTI>(a, ps, t, segs);
         } else {
             const bool tracing = ps.phase == kTracing;
             const bool on_node = tracing && at_node(t), on_leaf = tracing && at_leaf(t);
             if (choose_leaf_phase(on_node, on_leaf, a.leaf_weight)) {
-                if (on_leaf) leaf_step<S, false, false>(t, m, rec_of<MULTI>(a, ps));
+                if (on_leaf) leaf_step<W, S, false, false>(t, m, rec_of<MULTI>(a, ps), JobBoxes{job_of<MULTI>(a, ps)});
             } else {
-                if (on_node) node_step<W, S, false, false>(t, m, wide_of<MULTI>(a, ps));
+                if (on_node) walk_node<W, S, false, false>(t, m, nodes_of<MULTI>(a, ps));
             }
+            if (tracing) walk_pop<W, S, false>(t, m);
             if (tracing && trav_done(t)) {
                 ps.hslot = t.bslot;
                 ps.ht = t.bt;
@@ -744,7 +751,7 @@ template <int W, int S> __global__ __launch_bounds__(256) void k_wave_finish(Fin
                     atten = v3{at.x, at.y, at.z};
                     st = __float_as_uint(at.w);
                     bounce = a.bounce;
-                    trav_init(t, v3{r0.x, r0.y, r0.z}, v3{r1.x, r1.y, r1.z}, r0.w, r1.w, J.nwide);
+                    trav_init<W>(t, v3{r0.x, r0.y, r0.z}, v3{r1.x, r1.y, r1.z}, r0.w, r1.w, J.nwide);
                     phase = kTracing;
                 }
                 q_next += take;
@@ -757,7 +764,7 @@ template <int W, int S> __global__ __launch_bounds__(256) void k_wave_finish(Fin
                 v3 o = t.o, d = t.d;
                 if (shade_segment(J, J.rec, hslot, ht, o, d, st, color, atten) && bounce + 1 < J.depth) {
                     bounce++;
-                    trav_init(t, o, d, 0.001f, 10000000.0f, J.nwide);
+                    trav_init<W>(t, o, d, 0.001f, 10000000.0f, J.nwide);
                     phase = kTracing;
                     segs++;
                 } else {
@@ -769,10 +776,11 @@ template <int W, int S> __global__ __launch_bounds__(256) void k_wave_finish(Fin
             const bool tracing = phase == kTracing;
             const bool on_node = tracing && at_node(t), on_leaf = tracing && at_leaf(t);
             if (choose_leaf_phase(on_node, on_leaf, f.leaf_weight)) {
-                if (on_leaf) leaf_step<S, false, false>(t, m, J.rec);
+                if (on_leaf) leaf_step<W, S, false, false>(t, m, J.rec, JobBoxes{J});
             } else {
-                if (on_node) node_step<W, S, false, false>(t, m, J.wide);
+                if (on_node) walk_node<W, S, false, false>(t, m, J.nodes);
             }
+            if (tracing) walk_pop<W, S, false>(t, m);
             if (tracing && trav_done(t)) {
                 hslot = t.bslot;
                 ht = t.bt;
@@ -791,8 +799,9 @@ template <int W> void *pick_finish_s(uint32_t s) {
     return s == 4 ? (void *)k_wave_finish<W, 4> : s == 16 ? (void *)k_wave_finish<W, 16> : (void *)k_wave_finish<W, 8>;
 }
 
-void *pick_finish(uint32_t width, uint32_t s) {
-    switch (width) {
+void *pick_finish(uint32_t layout, uint32_t s) {
+    switch (layout) {
+        case kQ4: return pick_finish_s<kQ4>(s);
         case 2: return pick_finish_s<2>(s);
         case 8: return pick_finish_s<8>(s);
         default: return pick_finish_s<4>(s);
@@ -830,15 +839,16 @@ template <int W, bool MULTI> void *pick_render_s(uint32_t s) {
     return s == 4 ? (void *)k_render<W, 4, MULTI> : s == 16 ? (void *)k_render<W, 16, MULTI> : (void *)k_render<W, 8, MULTI>;
 }
 
-void *pick_render(uint32_t width, uint32_t s, bool multi) {
-    switch (width) {
+void *pick_render(uint32_t layout, uint32_t s, bool multi) {
+    switch (layout) {
+        case kQ4: return multi ? pick_render_s<kQ4, true>(s) : pick_render_s<kQ4, false>(s);
         case 2: return multi ? pick_render_s<2, true>(s) : pick_render_s<2, false>(s);
         case 8: return multi ? pick_render_s<8, true>(s) : pick_render_s<8, false>(s);
         default: return multi ? pick_render_s<4, true>(s) : pick_render_s<4, false>(s);
     }
 }
 
-void launch_render_kernel(rt_context *ctx, RenderArgs &a, uint32_t bvh_width, bool multi, const LaunchCfg &c,
+void launch_render_kernel(rt_context *ctx, RenderArgs &a, uint32_t layout, bool multi, const LaunchCfg &c,
                           hipStream_t stream) {
     a.refill = c.refill;
     a.leaf_weight = c.leaf_weight;
@@ -846,7 +856,7 @@ void launch_render_kernel(rt_context *ctx, RenderArgs &a, uint32_t bvh_width, bo
     a.work = ctx->counter_slot();
     k_zero<<<1, 64, 0, stream>>>(a.work);
     const size_t lds = stack_lds_bytes(c.lds_stack, c.block);
-    void *k = pick_render(bvh_width, c.lds_stack, multi);
+    void *k = pick_render(layout, c.lds_stack, multi);
     int per_cu = 0;
     RT_HIP(hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, k, (int)c.block, lds));
     const uint64_t waves_needed = (a.nitems + kRenderChunk - 1) / kRenderChunk;  // no more waves than chunks
@@ -924,7 +934,12 @@ RenderJob make_render_job(const Scene &sc, const rt_params &p, uint32_t width, u
     RT_REQUIRE(width > 0 && height > 0, "image size must be positive");
     RT_REQUIRE((uint64_t)width * height < (1ull << 31), "image too large");
     RenderJob j{};
+    const float far = std::max(std::max(std::fabs(p.camPos[0]), std::fabs(p.camPos[1])), std::fabs(p.camPos[2]));
+    const bool exact = sc.qwide.p && !(far <= sc.far_limit);
+    j.layout = exact ? sc.width : sc.layout();
+    j.nodes = exact ? sc.wide.as<uint32_t>() : sc.nodes();
     j.wide = sc.wide.as<uint32_t>();
+    j.slot_ref = sc.slot_ref.as<uint32_t>();
     j.rec = sc.records.as<LeafRecord>();
     j.slot_mat = sc.slot_mat.as<uint32_t>();
     j.mats = sc.materials.as<rt_material>();
@@ -1097,7 +1112,7 @@ void launch_render_wave(rt_context *ctx, const Scene &sc, const RenderJob &j, un
                                   yield ? yield->flag : nullptr, yield ? yield->yield_at : 0u};
                 k_zero<<<1, 64, 0, stream>>>(w.fa.work);
                 w.lds = stack_lds_bytes(tc.lds_stack, tc.block);
-                w.kernel = pick_finish(sc.width, tc.lds_stack);
+                w.kernel = pick_finish(j.layout, tc.lds_stack);
                 int per_cu = 0;
                 RT_HIP(hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, w.kernel, (int)tc.block, w.lds));
                 w.grid = (uint32_t)std::max(1, per_cu) * (uint32_t)ctx->num_cus;
@@ -1180,11 +1195,11 @@ void launch_render(rt_context *ctx, const Scene &sc, const rt_params &p, uint32_
     a.njobs = 1;
     a.nitems = j.nitems;
     a.segments = segments;
-    launch_render_kernel(ctx, a, sc.width, false, c, stream);
+    launch_render_kernel(ctx, a, j.layout, false, c, stream);
     if (split) launch_sum_samples(a, false, width * height, stream);
 }
 
-uint64_t launch_render_jobs(rt_context *ctx, std::vector<RenderJob> &jobs, uint32_t bvh_width,
+uint64_t launch_render_jobs(rt_context *ctx, std::vector<RenderJob> &jobs, uint32_t layout,
                             unsigned long long *segments, const LaunchCfg &c, hipStream_t stream) {
     uint64_t total = 0;
     uint32_t max_split_pix = 0;
@@ -1203,7 +1218,7 @@ uint64_t launch_render_jobs(rt_context *ctx, std::vector<RenderJob> &jobs, uint3
     a.njobs = (uint32_t)jobs.size();
     a.nitems = (uint32_t)total;
     a.segments = segments;
-    launch_render_kernel(ctx, a, bvh_width, true, c, stream);
+    launch_render_kernel(ctx, a, layout, true, c, stream);
     launch_sum_samples(a, true, max_split_pix, stream);
     ctx->tables.commit(slot, stream);
     return total;

@@ -289,6 +289,16 @@ __host__ __device__ inline bool refine_sphere(d3 c, double radius, d3 o, d3 d, f
 // child: kEmpty, a wide node index (bit 31 clear), or a leaf
 //   kLeafBit | (count-1) << 27 | first_slot.
 // ---------------------------------------------------------------------------
+//
+// Width-4 trees also have compressed nodes, 64 bytes each and numbered as the wide ones, in four
+// 16-byte rows:
+//   {origin.x, origin.y, origin.z, scale.x}  {child 0, lo.x, child 1, hi.x}
+//   {child 2, lo.y, child 3, hi.y}           {lo.z, hi.z, scale.y, scale.z}
+// A plane word holds one byte q per child: the plane lies at origin + (1024 + q) * scale, outside the
+// child's box (below a low plane, above a high one) by at least kPlaneMargin of a step.  1024 + q is the
+// half-precision number with the bits 0x6400 | q, which an FMA takes as it is.  An empty child's box is
+// inverted (lo 255, hi 0).
+constexpr double kPlaneMargin = 0.002;
 constexpr uint32_t kEmpty = 0xFFFFFFFFu;
 constexpr uint32_t kLeafBit = 0x80000000u;
 constexpr uint32_t kSlotMask = 0x07FFFFFFu;

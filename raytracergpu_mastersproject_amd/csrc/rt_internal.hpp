@@ -82,6 +82,8 @@ struct Scene {
     uint32_t nwide = 0, wide_depth = 0, stack_bound = 0;
     float build_ms = 0.0f;
     DevBuf wide;       // nwide * 32*width bytes
+    DevBuf qwide;      // width 4: nwide * 64 bytes, compressed nodes; empty when the scene needs the exact ones
+    DevBuf slot_ref;   // with qwide: nprim * u32, leaf slot -> 4 * node + child that holds it
     DevBuf records;    // nprim * LeafRecord
     DevBuf slot_prim;  // nprim * u32: leaf slot -> primitive id (RT_SPHERE_BIT for spheres)
     DevBuf slot_mat;   // nprim * u32: leaf slot -> material index
@@ -103,11 +105,20 @@ struct Scene {
     Scene(const Scene &) = delete;
     Scene &operator=(const Scene &) = delete;
 
+    // Rays whose origin has a coordinate beyond this are traced in the exact nodes' order (with qwide).
+    // fp32 intersection at great distances gives a hit a t outside its own box by more than the slab test
+    // allows for; which of two such hits a traversal keeps depends on its order.  Rays from up to 1,000 scene extents
+    // away, spheres from up to 512 radii: no hit differed between orders below 19,000 extents (12 M rays).
+    float far_limit = 0.0f;
+    // the node layout that the traversal kernels read: the width, or 44 (kQ4) for compressed width-4 nodes
+    uint32_t layout() const { return qwide.p ? 44u : width; }
+    const uint32_t *nodes() const { return qwide.p ? qwide.as<uint32_t>() : wide.as<uint32_t>(); }
+
     // After an entry point's launches that read the scene on `stream`, with the result of
     // rt_context::record_use for that stream.
     void note_use(hipStream_t stream, int recorded);
     uint64_t device_bytes() const {
-        return wide.bytes + records.bytes + slot_prim.bytes + slot_mat.bytes + materials.bytes + binary.bytes +
+        return wide.bytes + qwide.bytes + slot_ref.bytes + records.bytes + slot_prim.bytes + slot_mat.bytes + materials.bytes + binary.bytes +
                tris.bytes + spheres.bytes;
     }
 };
@@ -117,7 +128,8 @@ struct Scene {
 // pixels in 8x8 tiles; each job's items start at a multiple of kRenderChunk so a
 // wave's chunk of items never spans two jobs.
 struct RenderJob {
-    const uint32_t *wide;
+    const uint32_t *nodes;     // of the launch's layout
+    const uint32_t *wide, *slot_ref;  // exact leaf boxes of compressed layouts
     const LeafRecord *rec;
     const uint32_t *slot_mat;
     const rt_material *mats;
@@ -125,7 +137,8 @@ struct RenderJob {
     float4 *samples;   // split jobs: per (pixel, sample) {colour, next carry}, [sample][pixel]
     uint32_t nwide, width, height, spp;
     uint32_t depth, random_state, flags, tiles_x;
-    uint32_t first_item, nitems, group, _pad;  // group: samples per split item (0 = whole pixels)
+    uint32_t first_item, nitems, group;
+    uint32_t layout;  // of `nodes` (Scene::layout, or the width from a camera beyond Scene::far_limit); group: samples per split item (0 = whole pixels)
     float cam[12];  // pixel00, deltaU, deltaV, origin
 };
 // Split jobs give every (pixel, group of `group` consecutive samples) its own work item; the
@@ -490,8 +503,8 @@ void *noalloc_scratch_address();
 uint64_t noalloc_scratch_bytes();
 RenderJob make_render_job(const Scene &sc, const rt_params &p, uint32_t width, uint32_t height, uint32_t spp,
                           uint32_t flags, float *accum);
-// One launch over all jobs (all scenes must have BVH width `bvh_width`); returns the work items launched.
-uint64_t launch_render_jobs(rt_context *ctx, std::vector<RenderJob> &jobs, uint32_t bvh_width,
+// One launch over all jobs (all scenes must have node layout `layout`); returns the work items launched.
+uint64_t launch_render_jobs(rt_context *ctx, std::vector<RenderJob> &jobs, uint32_t layout,
                             unsigned long long *segments, const LaunchCfg &cfg, hipStream_t stream);
 // With `gate` (a yieldable pass's counters, WaveResume::counters), nothing is written unless that pass is complete.
 void launch_resolve(const float *accum, uint32_t npix, uint32_t spp, float *out, hipStream_t stream,

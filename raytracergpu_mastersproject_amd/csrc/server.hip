@@ -429,7 +429,7 @@ bool enqueue_step(rt_server *s, bool big_lane) {
     RT_HIP(hipEventRecord(step.start, stream));
     const uint32_t group = (uint32_t)std::max<uint64_t>(1, total / (32ull * device_lanes(s)));
     char *storage = static_cast<char *>(s->arena_mem.p) + s->scratch_base + scratch_off;
-    std::map<uint32_t, std::vector<RenderJob>> by_width;
+    std::map<uint32_t, std::vector<RenderJob>> by_layout;
     LaunchCfg rc;
     bool rc_set = false;
     for (auto &[r, q] : plan) {
@@ -458,7 +458,7 @@ bool enqueue_step(rt_server *s, bool big_lane) {
             RenderJob j = make_render_job(*r->scene, r->req.params, r->req.width, r->req.height, q, kflags, accum);
             make_split(j, reinterpret_cast<float4 *>(storage), std::min(group, q));
             storage += 16ull * npix * q;
-            by_width[r->scene->width].push_back(j);
+            by_layout[j.layout].push_back(j);
         }
         r->remaining -= q;
         r->done_units += q;
@@ -466,7 +466,7 @@ bool enqueue_step(rt_server *s, bool big_lane) {
         step.samples += npix * q;
         step.members.push_back(r);
     }
-    for (auto &kv : by_width)
+    for (auto &kv : by_layout)
         launch_render_jobs(s->ctx, kv.second, kv.first, s->segments.as<unsigned long long>(), rc, stream);
     if (!queries.empty()) {
         const double rshare = s->ray_rate * s->cfg.step_us / (double)queries.size();

@@ -8,7 +8,7 @@
 //   Closest hit: the nearest quad's children on top, each quad's nearest first.  More nodes are
 //   visited than one after the other would (a hit culls only what has not been started), but every
 //   box that the ordered traversal enters is entered, and the closest hit is the smallest
-//   (t, leaf slot) of all hits whatever the order.
+//   (t, leaf slot) of all hits whatever the order (Scene::far_limit says for which rays that holds).
 //   Any hit: the stack keeps depth-first child order, first entry on top, and lanes follow it.  A
 //   hit discards everything later in that order and the search goes on with what is earlier, so the
 //   result is the hit that the depth-first traversal finds first.

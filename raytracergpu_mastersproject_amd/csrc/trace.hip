@@ -19,13 +19,15 @@ namespace rtgpu {
 namespace {
 
 struct SceneView {
-    const uint32_t *wide;
+    const uint32_t *nodes;  // of the launch's layout
+    const uint32_t *wide, *slot_ref;
     const LeafRecord *rec;
     const uint32_t *slot_prim;
     const rt_triangle *tris;  // world-space primitives, for the refined results
     const rt_sphere *sph;
     uint32_t nwide;
-    uint32_t _pad;
+    float far_limit;
+    __device__ LeafBoxes operator()() const { return LeafBoxes{wide, slot_ref}; }
 };
 
 struct TraceArgs {
@@ -81,8 +83,8 @@ __global__ __launch_bounds__(256) void k_trace_direct(TraceArgs a) {
     float tmin, tmax;
     load_ray(a.rays, i, o, tmin, d, tmax);
     Trav t;
-    trav_init(t, o, d, tmin, tmax, a.sc.nwide);
-    trav_run<W, S, ANY, COUNT>(t, m, a.sc.wide, a.sc.rec, a.leaf_weight);
+    walk_init<W, S, ANY>(t, m, o, d, tmin, tmax, a.sc.nwide, a.sc.far_limit, a.sc.rec, a.sc, a.leaf_weight);
+    trav_run<W, S, ANY, COUNT>(t, m, a.sc.nodes, a.sc.rec, a.sc, a.leaf_weight);
     store_hit(a.sc, t, a.hits, a.counts, i);
 }
 
@@ -116,10 +118,22 @@ __device__ __forceinline__ void store_refined(const SceneView &sc, const Trav &t
 template <int T, bool ANY, bool REFINE> __global__ __launch_bounds__(64) void k_trace_team(TraceArgs a, uint32_t limit) {
     __shared__ uint2 stacks[64 / T * team_stack(T)];
     const uint32_t i = blockIdx.x * (64u / T) + threadIdx.x / T;
-    const bool live = i < a.n;
+    bool live = i < a.n;
     v3 o{0.0f, 0.0f, 0.0f}, d{0.0f, 0.0f, 0.0f};
     float tmin = 0.0f, tmax = 0.0f;
     if (live) load_ray(a.rays, i, o, tmin, d, tmax);
+    const bool ordered = live && needs_exact_nodes(o, d, a.sc.far_limit);
+    if (__ballot(ordered) != 0ull) {  // rare: a team's first lane runs such a ray alone, in the stacks' memory
+        uint2 spill[kSpillCap];
+        if (ordered && threadIdx.x % T == 0) {
+            Trav t;
+            trav_init<4>(t, o, d, tmin, tmax, a.sc.nwide);
+            trav_run<4, 16, ANY, false>(t, stack_mem<16>(stacks, spill), a.sc.wide, a.sc.rec, a.sc, a.leaf_weight);
+            if constexpr (REFINE) store_refined(a.sc, t, a.hits, nullptr, i);
+            else store_hit(a.sc, t, a.hits, nullptr, i);
+        }
+        live = live && !ordered;
+    }
     const TeamHit h = team_trace<T, ANY>(live, o, d, tmin, tmax, a.sc.wide, a.sc.nwide, a.sc.rec, stacks, limit);
     if (!live) return;
     if (h.owner || (h.slot == kEmpty && threadIdx.x % T == 0)) {
@@ -197,7 +211,7 @@ __global__ __launch_bounds__(256) void k_trace_persistent(TraceArgs a) {
                     v3 o, d;
                     float tmin, tmax;
                     load_ray(a.rays, (uint32_t)rid, o, tmin, d, tmax);
-                    trav_init(t, o, d, tmin, tmax, a.sc.nwide);
+                    walk_init<W, S, ANY>(t, m, o, d, tmin, tmax, a.sc.nwide, a.sc.far_limit, a.sc.rec, a.sc, a.leaf_weight);
                 }
                 q_next += take;
             }
@@ -205,10 +219,11 @@ __global__ __launch_bounds__(256) void k_trace_persistent(TraceArgs a) {
         if (__ballot(rid >= 0) == 0ull) break;  // every lane idle and the queue is drained
         const bool on_node = rid >= 0 && at_node(t), on_leaf = rid >= 0 && at_leaf(t);
         if (choose_leaf_phase(on_node, on_leaf, a.leaf_weight)) {
-            if (on_leaf) leaf_step<S, ANY, COUNT>(t, m, a.sc.rec);
+            if (on_leaf) leaf_step<W, S, ANY, COUNT>(t, m, a.sc.rec, a.sc);
         } else {
-            if (on_node) node_step<W, S, ANY, COUNT>(t, m, a.sc.wide);
+            if (on_node) walk_node<W, S, ANY, COUNT>(t, m, a.sc.nodes);
         }
+        walk_pop<W, S, ANY>(t, m);
         if (rid >= 0 && trav_done(t)) {
             if constexpr (REFINE) done = rid;
             else store((uint32_t)rid);
@@ -299,7 +314,7 @@ __global__ __launch_bounds__(256) void k_trace_batch(BatchArgs a) {
     uint32_t c_lo = 0, c_hi = 1;     // the items the chunk's rays belong to: [c_lo, c_hi)
     // the lane's scene, kept in registers: a table load per traversal step would add its
     // latency to every step
-    const uint32_t *wide = nullptr;
+    const uint32_t *nodes = nullptr;
     const LeafRecord *rec = nullptr;
     const ChunkSchedule<uint64_t> sched(a.total, gridDim.x * (blockDim.x / 64u), false);
     Trav t;
@@ -337,22 +352,23 @@ __global__ __launch_bounds__(256) void k_trace_batch(BatchArgs a) {
             if (!active && r < take) {
                 item = find_item(a.items, c_lo, c_hi, g);
                 local = (uint32_t)(g - a.items[item].first);
-                wide = a.items[item].sc.wide;
+                nodes = a.items[item].sc.nodes;
                 rec = a.items[item].sc.rec;
                 v3 o, d;
                 float tmin, tmax;
                 load_ray(a.items[item].rays, local, o, tmin, d, tmax);
-                trav_init(t, o, d, tmin, tmax, a.items[item].sc.nwide);
+                walk_init<W, S, ANY>(t, m, o, d, tmin, tmax, a.items[item].sc.nwide, a.items[item].sc.far_limit, rec, a.items[item].sc, a.leaf_weight);
                 active = true;
             }
         }
         if (__ballot(active) == 0ull) break;
         const bool on_node = active && at_node(t), on_leaf = active && at_leaf(t);
         if (choose_leaf_phase(on_node, on_leaf, a.leaf_weight)) {
-            if (on_leaf) leaf_step<S, ANY, false>(t, m, rec);
+            if (on_leaf) leaf_step<W, S, ANY, false>(t, m, rec, a.items[item].sc);
         } else {
-            if (on_node) node_step<W, S, ANY, false>(t, m, wide);
+            if (on_node) walk_node<W, S, ANY, false>(t, m, nodes);
         }
+        walk_pop<W, S, ANY>(t, m);
         if (active && trav_done(t)) {
             if constexpr (REFINE) pending = true;
             else store();
@@ -367,16 +383,18 @@ __global__ void k_zero_counter(unsigned int *c) {
 }
 
 SceneView view_of(const Scene &sc) {
-    return SceneView{sc.wide.as<uint32_t>(), sc.records.as<LeafRecord>(), sc.slot_prim.as<uint32_t>(),
-                     sc.tris.as<rt_triangle>(), sc.spheres.as<rt_sphere>(), sc.nwide, 0u};
+    return SceneView{sc.nodes(), sc.wide.as<uint32_t>(), sc.slot_ref.as<uint32_t>(), sc.records.as<LeafRecord>(), sc.slot_prim.as<uint32_t>(),
+                     sc.tris.as<rt_triangle>(), sc.spheres.as<rt_sphere>(), sc.nwide, sc.far_limit};
 }
 
 template <int W, int S> struct Kernels {
     template <bool ANY> static void *direct(bool count) {
-        return count ? (void *)k_trace_direct<W, S, ANY, true> : (void *)k_trace_direct<W, S, ANY, false>;
+        if constexpr (W == kQ4) return (void *)k_trace_direct<W, S, ANY, false>;
+        else return count ? (void *)k_trace_direct<W, S, ANY, true> : (void *)k_trace_direct<W, S, ANY, false>;
     }
     template <bool ANY, bool REFINE> static void *persistent(bool count) {
-        return count ? (void *)k_trace_persistent<W, S, ANY, true, REFINE>
+        if constexpr (W == kQ4) return (void *)k_trace_persistent<W, S, ANY, false, REFINE>;
+        else return count ? (void *)k_trace_persistent<W, S, ANY, true, REFINE>
                      : (void *)k_trace_persistent<W, S, ANY, false, REFINE>;
     }
     static void *get(int which, bool any, bool count) {
@@ -396,10 +414,11 @@ template <int W> void *pick(uint32_t s, int which, bool any, bool count) {
     }
 }
 
-// which: 0 one lane per ray, 1 persistent, 2 persistent over many scenes (never counts), 3 persistent
+// layout: Scene::layout (compressed nodes never count); which: 0 one lane per ray, 1 persistent, 2 persistent over many scenes (never counts), 3 persistent
 // storing refined hits, 4 persistent over many scenes storing refined hits
-void *pick_kernel(uint32_t width, uint32_t s, int which, bool any, bool count) {
-    switch (width) {
+void *pick_kernel(uint32_t layout, uint32_t s, int which, bool any, bool count) {
+    switch (layout) {
+        case kQ4: return pick<kQ4>(s, which, any, count);
         case 2: return pick<2>(s, which, any, count);
         case 8: return pick<8>(s, which, any, count);
         default: return pick<4>(s, which, any, count);
@@ -448,7 +467,7 @@ LaunchCfg resolve_cfg(const rt_context *ctx, const Scene &sc, const rt_launch_co
 // one lane per ray (its counts are those of the ordered traversal), as do the widths 2 and 8, a
 // caller's one-lane-per-ray configuration, and a tree too deep for the team's stack.
 static uint32_t team_size(const rt_context *ctx, const Scene &sc, uint32_t n, const LaunchCfg &c, bool count) {
-    if (sc.width != 4 || count || !c.persistent) return 0;
+    if (sc.layout() != kQ4 || count || !c.persistent) return 0;
     const uint64_t cus = (uint64_t)ctx->num_cus;
     if (n > 3072u * cus) return 0;
     const uint32_t t = n <= 24u * cus ? 64u : n <= 128u * cus ? 32u : n <= 1024u * cus ? 16u : 8u;
@@ -467,6 +486,11 @@ void launch_trace(rt_context *ctx, const Scene &sc, const rt_ray *rays, uint32_t
     // against 3,410 Mrays/s, so they keep the separate pass.
     const bool refine_in_kernel = refine && !any && c.persistent;
     TraceArgs a{view_of(sc), rays, hits, counts, n, c.refill, nullptr, c.leaf_weight, nullptr};
+    uint32_t layout = sc.layout();
+    if (counts) {  // the counts are those of the exact boxes
+        layout = sc.width;
+        a.sc.nodes = a.sc.wide;
+    }
     const size_t lds = stack_lds_bytes(c.lds_stack, c.block);
     if (const uint32_t team = team_size(ctx, sc, n, c, counts != nullptr)) {
         uint32_t limit = team_limit(team, sc.stack_bound);
@@ -476,14 +500,14 @@ void launch_trace(rt_context *ctx, const Scene &sc, const rt_ray *rays, uint32_t
         return;
     }
     if (!c.persistent) {
-        void *k = pick_kernel(sc.width, c.lds_stack, 0, any, counts != nullptr);
+        void *k = pick_kernel(layout, c.lds_stack, 0, any, counts != nullptr);
         const uint32_t grid = (uint32_t)(((uint64_t)n + c.block - 1) / c.block);
         void *args[] = {&a};
         RT_HIP(hipLaunchKernel(k, dim3(grid), dim3(c.block), args, lds, stream));
     } else {
         a.work = ctx->counter_slot();
         k_zero_counter<<<1, 64, 0, stream>>>(a.work);
-        void *k = pick_kernel(sc.width, c.lds_stack, refine_in_kernel ? 3 : 1, any, counts != nullptr);
+        void *k = pick_kernel(layout, c.lds_stack, refine_in_kernel ? 3 : 1, any, counts != nullptr);
         // no more lanes than rays: a small batch would otherwise launch the whole device's worth of
         // waves, nearly all of which find no chunk and exit
         const uint32_t grid = (uint32_t)std::min<uint64_t>(persistent_grid(ctx, k, c.block, lds),
@@ -509,14 +533,14 @@ void launch_trace_queue(rt_context *ctx, const Scene &sc, const rt_ray *rays, ui
         // pixels, and about two thirds of them leave the scene at once.  One thread per ray lets
         // such waves retire and new ones start (0.45 vs 0.69 ms for the 1080p frame's primaries);
         // refilling lanes in a persistent wave mixes rays at different depths instead.
-        void *k = pick_kernel(sc.width, c.lds_stack, 0, false, false);
+        void *k = pick_kernel(sc.layout(), c.lds_stack, 0, false, false);
         void *args[] = {&a};
         RT_HIP(hipLaunchKernel(k, dim3((uint32_t)(((uint64_t)n_max + c.block - 1) / c.block)), dim3(c.block), args, lds, stream));
         RT_HIP(hipGetLastError());
         return;
     }
     k_zero_counter<<<1, 64, 0, stream>>>(a.work);
-    void *k = pick_kernel(sc.width, c.lds_stack, 1, false, false);
+    void *k = pick_kernel(sc.layout(), c.lds_stack, 1, false, false);
     const uint32_t grid = persistent_grid(ctx, k, c.block, lds);
     void *args[] = {&a};
     RT_HIP(hipLaunchKernel(k, dim3(grid), dim3(c.block), args, lds, stream));
@@ -525,12 +549,12 @@ void launch_trace_queue(rt_context *ctx, const Scene &sc, const rt_ray *rays, ui
 
 void launch_trace_items(rt_context *ctx, const std::vector<TraceItem> &items, uint32_t flags, const LaunchCfg &c,
                         hipStream_t stream) {
-    // one launch per BVH width present, each over that width's items in order
-    for (uint32_t width : {2u, 4u, 8u}) {
+    // one launch per node layout present, each over that layout's items in order
+    for (uint32_t layout : {2u, 4u, 8u, (uint32_t)kQ4}) {
         std::vector<BatchItemDev> hv;
         uint64_t total = 0;
         for (const TraceItem &it : items) {
-            if (it.sc->width != width) continue;
+            if (it.sc->layout() != layout) continue;
             RT_REQUIRE(it.n == 0 || (it.rays && it.hits), "batch item with NULL rays/hits");
             check_stack(*it.sc, c);
             hv.push_back(BatchItemDev{view_of(*it.sc), it.rays, it.hits, total});
@@ -545,7 +569,7 @@ void launch_trace_items(rt_context *ctx, const std::vector<TraceItem> &items, ui
                     c.leaf_weight};
         const bool any = (flags & RT_TRACE_ANY) != 0;
         const size_t lds = stack_lds_bytes(c.lds_stack, c.block);
-        void *k = pick_kernel(width, c.lds_stack, (flags & RT_TRACE_FP32) ? 2 : 4, any, false);
+        void *k = pick_kernel(layout, c.lds_stack, (flags & RT_TRACE_FP32) ? 2 : 4, any, false);
         const uint64_t chunks = (total + kChunk - 1) / kChunk, wpb = c.block / 64u;
         const uint32_t grid = (uint32_t)std::max<uint64_t>(
             1, std::min<uint64_t>(persistent_grid(ctx, k, c.block, lds), (chunks + wpb - 1) / wpb));

@@ -123,13 +123,15 @@ constexpr uint32_t kOrdLowest = 0x00800000u;  // ord_key(-FLT_MAX): never culled
 // per-lane traversal state
 struct Trav {
     v3 o, d, idir;
-    v3 nlo, nhi;        // per-axis slab offsets of the low and high planes (see slab_axis)
+    v3 nlo, nhi;        // per-axis slab offsets of the low and high planes (see slab_axis); of the planes a
+                        // ray enters and leaves through on compressed nodes
     float tmin, bt;     // ray start; best t so far (initially tmax)
     uint32_t bslot;     // leaf slot of the best hit (kEmpty = none)
     float bu, bv;       // barycentrics of the best hit
     uint32_t cur;       // current entry (node index or leaf entry)
-    float cur_tn;       // its entry distance
     bool have;          // cur is valid
+    float cur_tn;       // its entry distance (not beside cur: a compressed node step stores both from one
+                        // 64-bit key, which the compiler would then do through scratch memory)
     uint32_t top, nspill;
     uint32_t nbox, ntri;
 };
@@ -211,12 +213,36 @@ __device__ __forceinline__ void slab_axis(float d, float o, float &idir, float &
     nhi = n + e;
 }
 
-__device__ __forceinline__ void trav_init(Trav &t, v3 o, v3 d, float tmin, float tmax, uint32_t nwide) {
+constexpr int kQ4 = 44;  // layout code of width 4 with compressed nodes (see node_step_q); 2, 4, 8: exact nodes
+
+// slab_axis for compressed nodes: offsets of the planes the ray enters and leaves through
+__device__ __forceinline__ void slab_axis_q(float d, float o, float &idir, float &near, float &far) {
+    float lo, hi;
+    slab_axis(d, o, idir, lo, hi);
+    near = idir < 0.0f ? hi : lo;
+    far = idir < 0.0f ? lo : hi;
+}
+
+// A ray that compressed nodes are not made for: a direction component so small, and not zero, that plane
+// distances overflow, or an origin beyond the scene's limit (Scene::far_limit).  It is traced over the exact
+// nodes at once when its lane takes it up.
+__device__ __forceinline__ bool needs_exact_nodes(v3 o, v3 d, float far_limit) {
+    return fmaxf(fmaxf(fabsf(o.x), fabsf(o.y)), fabsf(o.z)) > far_limit || (d.x != 0.0f && fabsf(d.x) < 0x1p-90f) || (d.y != 0.0f && fabsf(d.y) < 0x1p-90f) ||
+           (d.z != 0.0f && fabsf(d.z) < 0x1p-90f);
+}
+
+template <int W> __device__ __forceinline__ void trav_init(Trav &t, v3 o, v3 d, float tmin, float tmax, uint32_t nwide) {
     t.o = o;
     t.d = d;
-    slab_axis(d.x, o.x, t.idir.x, t.nlo.x, t.nhi.x);
-    slab_axis(d.y, o.y, t.idir.y, t.nlo.y, t.nhi.y);
-    slab_axis(d.z, o.z, t.idir.z, t.nlo.z, t.nhi.z);
+    if constexpr (W == kQ4) {
+        slab_axis_q(d.x, o.x, t.idir.x, t.nlo.x, t.nhi.x);
+        slab_axis_q(d.y, o.y, t.idir.y, t.nlo.y, t.nhi.y);
+        slab_axis_q(d.z, o.z, t.idir.z, t.nlo.z, t.nhi.z);
+    } else {
+        slab_axis(d.x, o.x, t.idir.x, t.nlo.x, t.nhi.x);
+        slab_axis(d.y, o.y, t.idir.y, t.nlo.y, t.nhi.y);
+        slab_axis(d.z, o.z, t.idir.z, t.nlo.z, t.nhi.z);
+    }
     t.tmin = tmin;
     t.bt = tmax;
     t.bslot = kEmpty;
@@ -300,9 +326,185 @@ __device__ __forceinline__ void node_step(Trav &t, const StackMem &m, const uint
     if (!t.have && t.top > 0) pop<S>(t, m);
 }
 
+// ---------------------------------------------------------------------------
+// Compressed width-4 nodes (layout code kQ4; rt_device.hpp describes them).
+//
+// What bounds the per-lane traversal is the L1's address pipe: a 16-byte load takes one tag lookup per
+// lane, and a 128-byte node takes seven of them (measured on the 16.8 M-ray / 4.2 M-triangle query: 2.58e9
+// lookups, address unit busy 95 % of the launch).  A 64-byte node takes four, and moves half the bytes.
+// Decoding costs less than it seems: the planes of four children lie in one word, so the near and far
+// planes of a ray are chosen per axis and not per child; a pair of children's planes becomes two half
+// floats with one byte permute, which a mixed-precision FMA reads directly.  Children are sorted as
+// doubles {distance, child} by v_min_f64 / v_max_f64, two instructions per comparator.
+//
+// The boxes are only ever larger than the exact ones, so every box that the exact test enters is
+// entered: with N the ray's plane offset and A = 1/d, the exact distance is fl(P*A + N) and this one
+// fl((1024+q)*fl(scale*A) + fl(origin*A + N)); the plane lies kPlaneMargin steps outside and the
+// roundings are below 4e-4 steps plus 1u of the distance, for which kSlackQ leaves room (4u more than
+// kRobust; applied to |tf|, so that it widens negative distances too).  A hit in a leaf that only the larger
+// boxes reach must not count, or results would depend on the node format: a hit is taken only if the ray enters
+// the leaf's exact box (leaf_entered, evaluated once per hit).
+//
+// Measured, exact -> compressed: 16.8 M rays / 4.2 M triangles 5.65 -> 3.68 ms (lookups 1.56e9, VALU
+// issue now 0.9 of the launch, HBM 19.2 GB = 5.2 TB/s, the rate of a large copy); 1080p x 16 spp frame 6.12 ->
+// 5.31 ms; 1.0 M any-hit rays / 1 M triangles 612 -> 556 us.
+// ---------------------------------------------------------------------------
+constexpr float kSlackQ = 0x1.4p-21f;  // 10 * 2^-24
+
+// where a leaf's exact box is found
+struct LeafBoxes {
+    const uint32_t *wide;      // the exact width-4 nodes
+    const uint32_t *slot_ref;  // leaf slot -> 4 * node + child
+};
+
+// Entry and exit distances of one axis of a box lo <= hi, as slab_axis and node_step compute them.
+__device__ __forceinline__ void axis_span(float lo, float hi, float idir, float near, float far, float &tn, float &tf) {
+    tn = fmaf(idir < 0.0f ? hi : lo, idir, near);
+    tf = fmaf(idir < 0.0f ? lo : hi, idir, far);
+}
+
+// the exact slab test of the leaf that holds `slot`, as node_step makes it
+__device__ __forceinline__ bool leaf_entered(const LeafBoxes &b, const Trav &t, uint32_t slot) {
+    const uint32_t ref = b.slot_ref[slot];
+    const float *p = reinterpret_cast<const float *>(b.wide) + (size_t)(ref >> 2) * 32u + (ref & 3u);
+    float nx, fx, ny, fy, nz, fz;
+    axis_span(p[0], p[4], t.idir.x, t.nlo.x, t.nhi.x, nx, fx);
+    axis_span(p[8], p[12], t.idir.y, t.nlo.y, t.nhi.y, ny, fy);
+    axis_span(p[16], p[20], t.idir.z, t.nlo.z, t.nhi.z, nz, fz);
+    return fmaxf(fmaxf(nx, ny), fmaxf(nz, t.tmin)) <= fminf(fminf(fx, fy), fminf(fz, t.bt)) * kRobust;
+}
+
+// True when the ray enters the primitive's own box, from its record and drawn in by the record's
+// rounding, so that it lies inside the leaf's box: then the leaf is entered too.  Nearly every hit
+// passes; the others (a hit near the box's corner, a triangle in an axis plane) look the leaf's box up.
+__device__ __forceinline__ bool primitive_entered(const LeafRecord &r, const Trav &t) {
+    const bool sphere = is_sphere_record(r);
+    const auto axis = [&](float v0, float a, float b, float idir, float near, float far, float &tn,
+                          float &tf) __attribute__((always_inline)) {
+        const float v1 = sphere ? v0 - r.r0.w : v0 + a, v2 = sphere ? v0 + r.r0.w : v0 + b;
+        const float lo = fminf(fminf(v0, v1), v2), hi = fmaxf(fmaxf(v0, v1), v2);
+        const float in = 0x1p-21f * fmaxf(fabsf(lo), fabsf(hi));
+        axis_span(lo + in, hi - in, idir, near, far, tn, tf);
+    };
+    float nx, fx, ny, fy, nz, fz;
+    axis(r.r0.x, r.r1.x, r.r2.x, t.idir.x, t.nlo.x, t.nhi.x, nx, fx);
+    axis(r.r0.y, r.r1.y, r.r2.y, t.idir.y, t.nlo.y, t.nhi.y, ny, fy);
+    axis(r.r0.z, r.r1.z, r.r2.z, t.idir.z, t.nlo.z, t.nhi.z, nz, fz);
+    return fmaxf(fmaxf(nx, ny), fmaxf(nz, t.tmin)) <= fminf(fminf(fx, fy), fminf(fz, t.bt)) * kRobust;
+}
+
+__device__ __forceinline__ double sort_min(double a, double b) {  // no canonicalisation: the bits are a key
+    double r;
+    asm("v_min_f64 %0, %1, %2" : "=v"(r) : "v"(a), "v"(b));
+    return r;
+}
+__device__ __forceinline__ double sort_max(double a, double b) {
+    double r;
+    asm("v_max_f64 %0, %1, %2" : "=v"(r) : "v"(a), "v"(b));
+    return r;
+}
+__device__ __forceinline__ void cswap(double *k, int i, int j) {
+    const double a = k[i], b = k[j];
+    k[i] = sort_min(a, b);
+    k[j] = sort_max(a, b);
+}
+
+typedef _Float16 half2_t __attribute__((ext_vector_type(2)));
+// the planes 1024 + q of children 0 and 1 (PAIR 0) or 2 and 3 (PAIR 1) of a plane word
+template <int PAIR> __device__ __forceinline__ half2_t plane_pair(uint32_t w) {
+    return __builtin_bit_cast(half2_t, __builtin_amdgcn_perm(0x64646464u, w, PAIR ? 0x07030602u : 0x05010400u));
+}
+
+constexpr uint32_t kMissKey = 0x7FE00000u;  // high word of a missed child's key: above every distance, a finite double
+
+template <int S, bool ANY>
+__device__ __forceinline__ void node_step_q(Trav &t, const StackMem &m, const uint32_t *__restrict__ nodes) {
+    const uint4 *p = reinterpret_cast<const uint4 *>(nodes) + (size_t)t.cur * 4u;
+    const uint4 r0 = p[0], r1 = p[1], r2 = p[2], r3 = p[3];
+    const v3 org{__uint_as_float(r0.x), __uint_as_float(r0.y), __uint_as_float(r0.z)};
+    const float sx = __uint_as_float(r0.w) * t.idir.x, sy = __uint_as_float(r3.z) * t.idir.y,
+                sz = __uint_as_float(r3.w) * t.idir.z;
+    const float nx = fmaf(org.x, t.idir.x, t.nlo.x), fx = fmaf(org.x, t.idir.x, t.nhi.x);
+    const float ny = fmaf(org.y, t.idir.y, t.nlo.y), fy = fmaf(org.y, t.idir.y, t.nhi.y);
+    const float nz = fmaf(org.z, t.idir.z, t.nlo.z), fz = fmaf(org.z, t.idir.z, t.nhi.z);
+    const bool gx = t.idir.x < 0.0f, gy = t.idir.y < 0.0f, gz = t.idir.z < 0.0f;
+    const uint32_t wnx = gx ? r1.w : r1.y, wfx = gx ? r1.y : r1.w;
+    const uint32_t wny = gy ? r2.w : r2.y, wfy = gy ? r2.y : r2.w;
+    const uint32_t wnz = gz ? r3.y : r3.x, wfz = gz ? r3.x : r3.y;
+    double key[4];
+    const auto child = [&](int c, uint32_t e, _Float16 hnx, _Float16 hny, _Float16 hnz, _Float16 hfx, _Float16 hfy,
+                           _Float16 hfz) __attribute__((always_inline)) {
+        const float tn = fmaxf(fmaxf(fmaxf(fmaf((float)hnx, sx, nx), fmaf((float)hny, sy, ny)),
+                                     fmaf((float)hnz, sz, nz)), t.tmin);
+        const float tf = fminf(fminf(fminf(fmaf((float)hfx, sx, fx), fmaf((float)hfy, sy, fy)),
+                                     fmaf((float)hfz, sz, fz)), t.bt);
+        const bool hit = tn <= fmaf(fabsf(tf), kSlackQ, tf);
+        key[c] = __hiloint2double((int)(hit ? (ANY ? (uint32_t)c : __float_as_uint(tn)) : kMissKey), (int)e);
+    };
+    {
+        const half2_t a = plane_pair<0>(wnx), b = plane_pair<0>(wny), c = plane_pair<0>(wnz);
+        const half2_t d = plane_pair<0>(wfx), e = plane_pair<0>(wfy), f = plane_pair<0>(wfz);
+        child(0, r1.x, a.x, b.x, c.x, d.x, e.x, f.x);
+        child(1, r1.z, a.y, b.y, c.y, d.y, e.y, f.y);
+    }
+    {
+        const half2_t a = plane_pair<1>(wnx), b = plane_pair<1>(wny), c = plane_pair<1>(wnz);
+        const half2_t d = plane_pair<1>(wfx), e = plane_pair<1>(wfy), f = plane_pair<1>(wfz);
+        child(2, r2.x, a.x, b.x, c.x, d.x, e.x, f.x);
+        child(3, r2.z, a.y, b.y, c.y, d.y, e.y, f.y);
+    }
+    cswap(key, 0, 1); cswap(key, 2, 3);
+    cswap(key, 0, 2); cswap(key, 1, 3);
+    cswap(key, 1, 2);
+    t.have = __double2hiint(key[0]) < (int)kMissKey;
+    if (t.have) {
+        while (t.top + 3u - t.nspill > (uint32_t)S) {  // room for three in the LDS part: move its oldest entries out
+            const uint32_t o = (t.nspill & (S - 1)) * m.stride;
+            if (t.nspill < kSpillCap) m.spill[t.nspill] = make_uint2(m.ent[o], (uint32_t)m.key[o] << 16);
+            t.nspill++;
+        }
+#pragma unroll
+        for (int k = 3; k >= 1; --k) {
+            const uint32_t hi = (uint32_t)__double2hiint(key[k]);
+            if ((int)hi < (int)kMissKey) {
+                const uint32_t o = (t.top & (S - 1)) * m.stride;
+                m.ent[o] = (uint32_t)__double2loint(key[k]);
+                m.key[o] = (uint16_t)(hi >> 16);
+                t.top++;
+            }
+        }
+        t.cur = (uint32_t)__double2loint(key[0]);
+    }
+}
+
+// Takes the next entry of a lane that has none, unless the best hit culls it: one entry per wave step (a
+// loop until an entry holds runs for the whole wave: 3.86 against 3.70 ms for the 16.8 M-ray query).  An
+// entry's distance is its upper 16 bits, no larger than the true one if that is positive; one that is not
+// positive is never culled.
+template <int S, bool ANY> __device__ __forceinline__ void pop_q(Trav &t, const StackMem &m) {
+    if (t.have || t.top == 0) return;
+    t.top--;
+    uint32_t e;
+    float tn;
+    if (t.top >= t.nspill) {
+        const uint32_t o = (t.top & (S - 1)) * m.stride;
+        e = m.ent[o];
+        asm("" : "+v"(e));  // else this load and the other become one through a generic pointer
+        tn = __uint_as_float((uint32_t)m.key[o] << 16);
+    } else {
+        t.nspill--;
+        const uint2 v = m.spill[min(t.nspill, kSpillCap - 1u)];
+        e = v.x;
+        tn = __uint_as_float(v.y);
+    }
+    t.cur = e;
+    t.have = ANY || !(tn > fmaxf(t.bt * kRobust, 0.0f));
+}
+
 // Test the primitives of one leaf entry; true when an any-hit query has found its hit.
-template <bool ANY, bool COUNT>
-__device__ __forceinline__ bool test_leaf(Trav &t, uint32_t entry, const LeafRecord *__restrict__ rec) {
+// boxes(): the LeafBoxes of compressed layouts (W == kQ4), not called for the others.
+template <int W, bool ANY, bool COUNT, class B>
+__device__ __forceinline__ bool test_leaf(Trav &t, uint32_t entry, const LeafRecord *__restrict__ rec, const B &boxes) {
     const uint32_t first = leaf_first(entry), cnt = leaf_count(entry);
     for (uint32_t s = first; s < first + cnt; ++s) {
         if constexpr (COUNT) t.ntri++;
@@ -317,6 +519,9 @@ __device__ __forceinline__ bool test_leaf(Trav &t, uint32_t entry, const LeafRec
             hit = triangle_test(r, t.o, t.d, t.tmin, t.bt, th, a, b);
         }
         if (hit && (th < t.bt || (th == t.bt && s < t.bslot))) {
+            if constexpr (W == kQ4) {
+                if (!primitive_entered(r, t) && !leaf_entered(boxes(), t, s)) continue;
+            }
             t.bt = th;
             t.bslot = s;
             t.bu = a;
@@ -329,14 +534,19 @@ __device__ __forceinline__ bool test_leaf(Trav &t, uint32_t entry, const LeafRec
 
 // Test the primitives of the current leaf, unless a closer hit found since it was pushed culls it.
 // Precondition: at_leaf(t).
-template <int S, bool ANY, bool COUNT = true>
-__device__ __forceinline__ void leaf_step(Trav &t, const StackMem &m, const LeafRecord *__restrict__ rec) {
-    if (t.cur_tn <= t.bt * kRobust && test_leaf<ANY, COUNT>(t, t.cur, rec)) {
-        t.top = 0;  // any hit: done
-        t.nspill = 0;
+template <int W, int S, bool ANY, bool COUNT = true, class B>
+__device__ __forceinline__ void leaf_step(Trav &t, const StackMem &m, const LeafRecord *__restrict__ rec, const B &boxes) {
+    if constexpr (W == kQ4) {  // culled when popped; an empty child's inverted box can be entered from very far away
+        if (t.cur != kEmpty && test_leaf<W, ANY, COUNT>(t, t.cur, rec, boxes)) t.top = t.nspill = 0;
+        t.have = false;
+    } else {
+        if (t.cur_tn <= t.bt * kRobust && test_leaf<W, ANY, COUNT>(t, t.cur, rec, boxes)) {
+            t.top = 0;  // any hit: done
+            t.nspill = 0;
+        }
+        t.have = false;
+        if (t.top > 0) pop<S>(t, m);
     }
-    t.have = false;
-    if (t.top > 0) pop<S>(t, m);
 }
 
 // Wave-level choice of which lanes advance this iteration: leaves when enough lanes
@@ -348,17 +558,45 @@ __device__ __forceinline__ bool choose_leaf_phase(bool on_node, bool on_leaf, ui
     return (uint32_t)__popcll(ml) * leaf_weight >= (uint32_t)__popcll(mn);
 }
 
+// One step of a lane whose ray is on a node.
+template <int W, int S, bool ANY, bool COUNT>
+__device__ __forceinline__ void walk_node(Trav &t, const StackMem &m, const uint32_t *nodes) {
+    if constexpr (W == kQ4) node_step_q<S, ANY>(t, m, nodes);
+    else node_step<W, S, ANY, COUNT>(t, m, nodes);
+}
+
+// After the wave's step, whatever its phase.
+template <int W, int S, bool ANY> __device__ __forceinline__ void walk_pop(Trav &t, const StackMem &m) {
+    if constexpr (W == kQ4) pop_q<S, ANY>(t, m);
+}
+
 // Run one ray to completion (used where lanes are not refilled).
-template <int W, int S, bool ANY, bool COUNT = true>
-__device__ __forceinline__ void trav_run(Trav &t, const StackMem &m, const uint32_t *wide, const LeafRecord *rec,
-                                         uint32_t leaf_weight) {
+template <int W, int S, bool ANY, bool COUNT, class B>
+__device__ __forceinline__ void trav_run(Trav &t, const StackMem &m, const uint32_t *nodes, const LeafRecord *rec,
+                                         const B &boxes, uint32_t leaf_weight) {
     for (;;) {
         const bool on_node = at_node(t), on_leaf = at_leaf(t);
-        if (__ballot(on_node || on_leaf) == 0ull) break;
+        if (__ballot(!trav_done(t)) == 0ull) break;
         if (choose_leaf_phase(on_node, on_leaf, leaf_weight)) {
-            if (on_leaf) leaf_step<S, ANY, COUNT>(t, m, rec);
+            if (on_leaf) leaf_step<W, S, ANY, COUNT>(t, m, rec, boxes);
         } else {
-            if (on_node) node_step<W, S, ANY, COUNT>(t, m, wide);
+            if (on_node) walk_node<W, S, ANY, COUNT>(t, m, nodes);
+        }
+        walk_pop<W, S, ANY>(t, m);
+    }
+}
+
+// Starts a ray; on compressed nodes a ray that needs the exact ones is run to its end here (rare: the other
+// lanes of its wave wait).
+template <int W, int S, bool ANY, class B>
+__device__ __forceinline__ void walk_init(Trav &t, const StackMem &m, v3 o, v3 d, float tmin, float tmax,
+                                          uint32_t nwide, float far_limit, const LeafRecord *rec, const B &boxes,
+                                          uint32_t leaf_weight) {
+    trav_init<W>(t, o, d, tmin, tmax, nwide);
+    if constexpr (W == kQ4) {
+        if (needs_exact_nodes(o, d, far_limit)) {
+            trav_init<4>(t, o, d, tmin, tmax, nwide);
+            trav_run<4, S, ANY, false>(t, m, boxes().wide, rec, boxes, leaf_weight);
         }
     }
 }
