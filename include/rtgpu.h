@@ -181,11 +181,11 @@ int rt_trace(rt_context *ctx, uint32_t scene_id, const rt_ray *rays, uint32_t n,
  * image is the same either way. */
 #define RT_RENDER_SPLIT_SAMPLES 4u       /* always one lane per (pixel, sample) */
 #define RT_RENDER_NO_SPLIT 8u            /* always one lane per pixel */
-/* How paths are scheduled.  An image of at least 2^22 pixel-samples is rendered bounce by
- * bounce by default: the primary segments are traced once per pixel, a shading kernel runs
- * every sample's first bounce and queues the paths that scatter, and one persistent launch
- * carries every queued path to its end.  Smaller images carry every path to its end inside
- * one persistent launch from the start.  The image is the same either way.
+/* How paths are scheduled.  By default rt_render renders bounce by bounce over width-4 trees with compressed nodes:
+ * the primary segments are traced once per pixel, a shading kernel runs every sample's first bounce and queues
+ * the paths that scatter, and one persistent launch carries every queued path to its end, with several lanes per path
+ * for small images.  Over other trees, and in rt_render_batch, an image of fewer than 2^22 pixel-samples
+ * instead carries every path to its end inside one persistent launch from the start.  The image is the same either way.
  * RT_RENDER_SPLIT_SAMPLES and RT_RENDER_NO_SPLIT describe the persistent launch and select it. */
 #define RT_RENDER_WAVEFRONT 16u          /* always bounce by bounce */
 #define RT_RENDER_PERSISTENT_PATHS 32u   /* always one persistent launch */
@@ -215,9 +215,8 @@ typedef struct rt_render_job {
     rt_params params;   /* this image's UBO */
 } rt_render_job;
 
-/* Renders every job's image: the ones rt_render would run in one persistent launch share
- * one launch per BVH width present; the ones it would render bounce by bounce (see
- * RT_RENDER_WAVEFRONT) follow, each on its own (no such call exists in the reference, whose
+/* Renders every job's image: the ones of fewer than 2^22 pixel-samples share one persistent
+ * launch per node layout present; the others (and RT_RENDER_WAVEFRONT) follow bounce by bounce, each on its own (no such call exists in the reference, whose
  * S2 renders one image: RaytracerBVH.cpp:1000-1078).  Each image is bit-identical to
  * rt_render of its job alone.  jobs: host array; the accum images must not overlap.
  * segments (device, may be NULL) as for rt_render. */
@@ -229,8 +228,9 @@ int rt_render_batch(rt_context *ctx, const rt_render_job *jobs, uint32_t njobs, 
  * image is bit-identical to rt_render's with the same arguments.  Every scratch buffer (per-sample
  * storage, bounce-by-bounce path state and queues) comes from one static device array of
  * RT_NOALLOC_SCRATCH_BYTES per GPU, held until the process ends, instead of the context's cache:
- * bounce-by-bounce images run in as many passes as the array needs, and images that would keep
- * per-sample storage keep whole pixels per lane when it does not fit.  RT_ERR_BUDGET when one
+ * bounce-by-bounce images run in as many passes as the array needs (an image of fewer than 2^22 pixel-samples
+ * of which one sample does not fit runs in one persistent launch), and images that would keep per-sample storage
+ * keep whole pixels per lane when it does not fit.  RT_ERR_BUDGET when one
  * sample of a bounce-by-bounce image (120 B per pixel) or a forced RT_RENDER_SPLIT_SAMPLES image
  * (16 B per pixel-sample) exceeds the array.  Calls on one GPU share its array: calls that
  * overlap on one GPU (other streams, other contexts of the process) race. */

@@ -5,16 +5,17 @@
 // chain through the image's alpha channel (the RNG carry).  Two schedules reproduce it bit
 // for bit; every path performs the same operations in the same order under both.
 //
-// Bounce by bounce (images of 2^22+ pixel-samples, and RT_RENDER_WAVEFRONT): a pass holds
+// Bounce by bounce (rt_render on compressed nodes, images of 2^22+ pixel-samples elsewhere, and
+// RT_RENDER_WAVEFRONT): a pass holds
 // whole samples of every pixel.  Primary rays have no jitter (raytraceBVH.comp:338), so one
 // primary ray per pixel is traced, one thread per ray; k_wave_first then runs each pixel's
 // samples in order (carry, RNG state, first shading off the pixel's primary surface) and
 // queues the paths that scatter, those off dielectrics in a queue of their own;
 // k_wave_finish carries every queued path to its end in one persistent launch, the
-// dielectric queue first (those paths enter closed meshes and bounce longest); the samples
-// are added to the image in order.  Path state lives in HBM between launches.
+// dielectric queue first (those paths enter closed meshes and bounce longest), or k_path_team with several
+// lanes per path when the pass holds few; the samples are added to the image in order.  Path state lives in HBM between launches.
 //
-// One persistent launch (smaller images, RT_RENDER_PERSISTENT_PATHS and the layout flags):
+// One persistent launch (fused small images, RT_RENDER_PERSISTENT_PATHS and the layout flags):
 // lanes take work items from 8x8 pixel tiles and run their samples to completion, advancing
 // every active lane by one traversal step per iteration.  A pixel job keeps the accumulator
 // in registers and traces the shared first segment once per pixel.  A split job gives each
@@ -31,7 +32,7 @@
 #include <cstdlib>
 
 #include "rt_internal.hpp"
-#include "traverse.hpp"
+#include "team.hpp"
 
 namespace rtgpu {
 
@@ -795,6 +796,81 @@ template <int W, int S> __global__ __launch_bounds__(256) void k_wave_finish(Fin
     }
 }
 
+// Runs the paths of a queue to their ends with a team of T lanes per path: the finish kernel's place in passes
+// of few paths, which would otherwise last as long as their longest path's segments traced one lane each.
+// The teams of a wave trace their segments together (team_trace), then every lane of a team shades: the
+// lanes of a team hold the same path.  A team whose path has ended takes the next entry before the wave
+// traces again.  Lanes per path: path_team_size.
+struct TeamPathArgs {
+    WaveArgs w;
+    unsigned int *work;
+    uint32_t limit;  // team_trace's
+};
+
+template <int T> __global__ __launch_bounds__(64) void k_path_team(TeamPathArgs f) {
+    __shared__ uint2 stacks[64 / T * team_stack(T)];
+    const WaveArgs &a = f.w;
+    const RenderJob &J = a.J;
+    const uint32_t n2 = a.n_in2 ? *a.n_in2 : 0u;  // the second queue's entries come first
+    const uint32_t n = *a.n_in + n2;
+    const uint32_t lane = threadIdx.x, first_lane = lane & ~(uint32_t)(T - 1);
+    bool live = false, more = true;
+    uint32_t p = 0, bounce = 0, st = 0, segs = 0;
+    float next = 0.0f;
+    v3 color{0.0f, 0.0f, 0.0f}, atten{1.0f, 1.0f, 1.0f}, o{0.0f, 0.0f, 0.0f}, d{0.0f, 0.0f, 0.0f};
+    for (;;) {
+        const unsigned long long idle = __ballot(!live);
+        if (more && idle != 0ull) {
+            const uint32_t want = (uint32_t)__popcll(idle) / T;
+            uint32_t base = 0;
+            if (lane == 0) base = atomicAdd(f.work, want);
+            base = (uint32_t)__builtin_amdgcn_readfirstlane((int)base);
+            const uint32_t i = base + (uint32_t)__popcll(idle & ((1ull << first_lane) - 1ull)) / T;
+            more = base + want < n;
+            if (!live && i < n) {
+                const bool second = i < n2;
+                const uint32_t qi = second ? i : i - n2;
+                p = (second ? a.ids_in2 : a.ids_in)[qi];
+                const float4 *q = reinterpret_cast<const float4 *>((second ? a.rays_in2 : a.rays_in) + qi);
+                const float4 r0 = q[0], r1 = q[1];
+                const float4 c = a.col[p], at = a.att[p];
+                o = v3{r0.x, r0.y, r0.z};
+                d = v3{r1.x, r1.y, r1.z};
+                color = v3{c.x, c.y, c.z};
+                next = c.w;
+                atten = v3{at.x, at.y, at.z};
+                st = __float_as_uint(at.w);
+                bounce = a.bounce;
+                live = true;
+            }
+        }
+        if (__ballot(live) == 0ull) break;
+        const TeamHit h = team_trace<T, false>(live, o, d, 0.001f, 10000000.0f, J.wide, J.nwide, J.rec, stacks, f.limit);
+        if (live) {
+            if (shade_segment(J, J.rec, h.slot, h.t, o, d, st, color, atten) && bounce + 1 < J.depth) {
+                bounce++;
+                segs++;
+            } else {
+                if (lane == first_lane) a.col[p] = make_float4(color.x, color.y, color.z, next);
+                live = false;
+            }
+        }
+    }
+    if (a.segments) {
+        unsigned long long sg = lane == first_lane ? segs : 0u;
+        for (int off = 32; off > 0; off >>= 1) sg += __shfl_xor(sg, off);
+        if (lane == 0 && sg) atomicAdd(a.segments, sg);
+    }
+}
+
+void *pick_path_team(uint32_t t) {
+    switch (t) {
+        case 8: return (void *)k_path_team<8>;
+        case 16: return (void *)k_path_team<16>;
+        default: return (void *)k_path_team<32>;
+    }
+}
+
 template <int W> void *pick_finish_s(uint32_t s) {
     return s == 4 ? (void *)k_wave_finish<W, 4> : s == 16 ? (void *)k_wave_finish<W, 16> : (void *)k_wave_finish<W, 8>;
 }
@@ -986,6 +1062,22 @@ uint32_t wave_finish_bounce() {
 }
 }  // namespace
 
+namespace {
+// Lanes per path of a pass of `paths` paths, at most a quarter of which usually queue after the first
+// bounce; 0: the finish kernel's one lane per path.  Whole frames (us; 256 CUs; 200 k triangles unless stated),
+// one lane -> 32 / 16 / 8 lanes per path:
+//   4,096 paths    900 -> 164 / 171 / 184  (1,024 triangles 238 -> 79 / 80 / 83)
+//   65,536 paths   1,054 -> 350 / 353 / 371 (1,024 triangles 260 -> 243 / 230 / 225, 1 M 1,244 -> 391 / 389 / 401)
+//   262,144 paths  1,181 -> -- / 764 / 641  (1,024 triangles 297 -> -- / 511 / 349, 1 M 1,256 -> -- / 905 / 749)
+//   1,048,576      1,343 -> -- / 2,055 / 1,327 (1,024 triangles 411 -> -- / 1,575 / 900)
+uint32_t path_team_size(const rt_context *ctx, uint32_t layout, uint32_t stack_bound, uint64_t paths) {
+    const uint64_t cus = (uint64_t)ctx->num_cus;
+    if (layout != kQ4 || paths > 1024u * cus) return 0;
+    const uint32_t t = paths <= 32u * cus ? 32u : paths <= 128u * cus ? 16u : 8u;
+    return team_limit(t, stack_bound) ? t : 0u;
+}
+}  // namespace
+
 // A yieldable pass: its finish launch and gated sum, launched again until the pass is complete.
 struct WaveResume {
     FinishArgs fa;
@@ -1107,6 +1199,20 @@ void launch_render_wave(rt_context *ctx, const Scene &sc, const RenderJob &j, un
                 a.rays_in = rays[cur];
                 a.ids_in = ids[cur];
                 a.n_in = count + cur;
+                if (const uint32_t team = yield ? 0u : path_team_size(ctx, j.layout, sc.stack_bound, paths)) {
+                    TeamPathArgs ta{a, count + 2, team_limit(team, sc.stack_bound)};
+                    k_zero<<<1, 64, 0, stream>>>(ta.work);
+                    void *k = pick_path_team(team);
+                    int per_cu = 0;
+                    RT_HIP(hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, k, 64, 0));
+                    const uint64_t per_wave = 64u / team;  // no more waves than the pass can have queued
+                    const uint32_t g = (uint32_t)std::min<uint64_t>((uint64_t)std::max(1, per_cu) * (uint32_t)ctx->num_cus,
+                                                                    (paths + per_wave - 1) / per_wave);
+                    void *args[] = {&ta};
+                    RT_HIP(hipLaunchKernel(k, dim3(g), dim3(64), args, 0, stream));
+                    RT_HIP(hipGetLastError());
+                    break;
+                }
                 WaveResume w{};
                 w.fa = FinishArgs{a, count + 2, tc.refill, tc.leaf_weight, tc.shade_min,
                                   yield ? yield->flag : nullptr, yield ? yield->yield_at : 0u};
@@ -1158,14 +1264,27 @@ bool wave_schedule(uint32_t width, uint32_t height, uint32_t spp, uint32_t flags
     return (flags & RT_RENDER_WAVEFRONT) || (!layout && (uint64_t)width * height * spp >= kWaveMinSamples);
 }
 
+// rt_render's own choice.  One image is faster bounce by bounce at every size on compressed nodes: from
+// 1,024 paths per CU with one lane per path (2 M samples on 200 k triangles 1,905 us in one persistent
+// launch, 1,475 bounce by bounce; 1 M samples on 1,024 triangles 638 and 411), below with a team
+// per path (path_team_size).  Other layouts keep wave_schedule's line.
+static bool bounce_by_bounce(rt_context *ctx, const Scene &sc, const RenderJob &j, uint32_t flags) {
+    const bool layout_flags = (flags & (RT_RENDER_SPLIT_SAMPLES | RT_RENDER_NO_SPLIT | RT_RENDER_PERSISTENT_PATHS)) != 0;
+    if (wave_schedule(j.width, j.height, j.spp, flags)) return true;
+    const uint64_t samples = (uint64_t)j.width * j.height * j.spp;
+    return !layout_flags && j.layout == kQ4 &&
+           (samples > 1024u * (uint64_t)ctx->num_cus || path_team_size(ctx, j.layout, sc.stack_bound, samples));
+}
+
 void launch_render(rt_context *ctx, const Scene &sc, const rt_params &p, uint32_t width, uint32_t height, uint32_t spp,
                    uint32_t flags, float *accum, unsigned long long *segments, const LaunchCfg &c,
                    hipStream_t stream, char *scratch, uint64_t scratch_bytes) {
     RenderJob j = make_render_job(sc, p, width, height, spp, flags, accum);
     if (spp == 0) return;
     check_stack(sc, c);
-    if (wave_schedule(width, height, spp, flags)) {
-        if (scratch && scratch_bytes < wave_scratch_bytes((uint64_t)width * height))
+    const bool fits = !scratch || scratch_bytes >= wave_scratch_bytes((uint64_t)width * height);
+    if (bounce_by_bounce(ctx, sc, j, flags) && (fits || wave_schedule(width, height, spp, flags))) {
+        if (!fits)
             throw Error(RT_ERR_BUDGET, "one sample of a " + std::to_string(width) + "x" + std::to_string(height) +
                                            " image needs " + std::to_string(wave_scratch_bytes((uint64_t)width * height)) +
                                            " bytes of path storage; the scratch holds " + std::to_string(scratch_bytes));
