@@ -10,6 +10,7 @@
 // are replaced by device-wide kernels.
 #include <algorithm>
 #include <cmath>
+#include <cstddef>
 #include <cstring>
 #include <limits>
 #include <vector>
@@ -32,11 +33,6 @@ __device__ inline float fkey_dec(uint32_t k) {
 inline uint32_t grid_for(uint64_t n, int block = kB) {
     uint64_t g = (n + block - 1) / block;
     return (uint32_t)std::max<uint64_t>(1, std::min<uint64_t>(g, 1u << 30));
-}
-
-__global__ void k_fill_u32(uint32_t *p, uint32_t v, uint64_t n) {
-    for (uint64_t i = blockIdx.x * (uint64_t)blockDim.x + threadIdx.x; i < n; i += (uint64_t)gridDim.x * blockDim.x)
-        p[i] = v;
 }
 
 // ModelSpaceToWorldSpace.comp:32-48: v' = M * vec4(v, 1) evaluated left to right
@@ -76,15 +72,37 @@ __device__ inline v3 centroid(const rt_triangle *tris, uint32_t ntri, const rt_s
     return v3{s.center[0], s.center[1], s.center[2]};
 }
 
-__global__ void k_bounds_init(uint32_t *keys) {
-    if (threadIdx.x < 3) keys[threadIdx.x] = fkey(1000000000.0f);
-    else if (threadIdx.x < 6) keys[threadIdx.x] = fkey(-1000000000.0f);
+// Centroid bounds (GetEnclosingAABB.comp): min and max in a total order (-0 < +0), so the result does not depend
+// on the order.  One partial result per block; the Morton kernel's blocks reduce the few partials
+// themselves.  Atomics on six shared words from every block took 272 us of 1 M triangles' build, this takes 20.
+constexpr uint32_t kBoundsBlocks = 256;
+
+__device__ inline void bounds_reduce(uint32_t (&mn)[3], uint32_t (&mx)[3]) {  // block-wide, valid in every thread
+    __shared__ uint32_t red[6][kB / 64];
+    for (int a = 0; a < 3; ++a) {
+        for (int off = 32; off > 0; off >>= 1) {
+            mn[a] = min(mn[a], (uint32_t)__shfl_xor((int)mn[a], off));
+            mx[a] = max(mx[a], (uint32_t)__shfl_xor((int)mx[a], off));
+        }
+    }
+    const int wave = threadIdx.x / 64, lane = threadIdx.x % 64;
+    if (lane == 0)
+        for (int a = 0; a < 3; ++a) { red[a][wave] = mn[a]; red[3 + a][wave] = mx[a]; }
+    __syncthreads();
+    for (int w = 0; w < kB / 64; ++w)
+        for (int a = 0; a < 3; ++a) {
+            mn[a] = min(mn[a], red[a][w]);
+            mx[a] = max(mx[a], red[3 + a][w]);
+        }
 }
 
-// device-wide min/max of centroids in a total order (-0 < +0): order-independent result
-__global__ void k_centroid_bounds(const rt_triangle *tris, uint32_t ntri, const rt_sphere *sph, uint32_t n,
-                                  uint32_t *keys) {
-    uint32_t mn[3] = {0xFFFFFFFFu, 0xFFFFFFFFu, 0xFFFFFFFFu}, mx[3] = {0u, 0u, 0u};
+__global__ __launch_bounds__(kB) void k_centroid_bounds(const rt_triangle *tris, uint32_t ntri, const rt_sphere *sph,
+                                                        uint32_t n, uint32_t *partial) {
+    uint32_t mn[3], mx[3];
+    for (int a = 0; a < 3; ++a) {  // GetEnclosingAABB.comp starts from +-1e9
+        mn[a] = fkey(1000000000.0f);
+        mx[a] = fkey(-1000000000.0f);
+    }
     for (uint32_t i = blockIdx.x * blockDim.x + threadIdx.x; i < n; i += gridDim.x * blockDim.x) {
         v3 c = centroid(tris, ntri, sph, i);
         uint32_t k[3] = {fkey(c.x), fkey(c.y), fkey(c.z)};
@@ -93,41 +111,12 @@ __global__ void k_centroid_bounds(const rt_triangle *tris, uint32_t ntri, const 
             mx[a] = max(mx[a], k[a]);
         }
     }
-    __shared__ uint32_t red[6][kB / 64];
-    for (int a = 0; a < 3; ++a) {
-        for (int off = 32; off > 0; off >>= 1) {
-            mn[a] = min(mn[a], (uint32_t)__shfl_xor((int)mn[a], off));
-            mx[a] = max(mx[a], (uint32_t)__shfl_xor((int)mx[a], off));
-        }
-    }
-    int wave = threadIdx.x / 64, lane = threadIdx.x % 64;
-    if (lane == 0)
-        for (int a = 0; a < 3; ++a) { red[a][wave] = mn[a]; red[3 + a][wave] = mx[a]; }
-    __syncthreads();
-    if (threadIdx.x == 0) {
-        for (int w = 1; w < (int)(blockDim.x / 64); ++w)
-            for (int a = 0; a < 3; ++a) {
-                red[a][0] = min(red[a][0], red[a][w]);
-                red[3 + a][0] = max(red[3 + a][0], red[3 + a][w]);
-            }
+    bounds_reduce(mn, mx);
+    if (threadIdx.x == 0)
         for (int a = 0; a < 3; ++a) {
-            atomicMin(&keys[a], red[a][0]);
-            atomicMax(&keys[3 + a], red[3 + a][0]);
+            partial[6u * blockIdx.x + a] = mn[a];
+            partial[6u * blockIdx.x + 3 + a] = mx[a];
         }
-    }
-}
-
-// padAABB (GetEnclosingAABB.comp:33-46); out: emin[3], emax[3], span[3]
-__global__ void k_bounds_finalize(const uint32_t *keys, float *bounds) {
-    if (threadIdx.x != 0) return;
-    const float delta = 0.001f, pad = 0.001f / 2.0f;
-    for (int a = 0; a < 3; ++a) {
-        float mn = fkey_dec(keys[a]), mx = fkey_dec(keys[3 + a]);
-        if (mx - mn < delta) { mn -= pad; mx += pad; }
-        bounds[a] = mn;
-        bounds[3 + a] = mx;
-        bounds[6 + a] = mx - mn;
-    }
 }
 
 __device__ inline uint32_t sep3(uint32_t v) {  // GenerateMortonCodesOfPrimitives.comp:20-28
@@ -139,15 +128,30 @@ __device__ inline uint32_t sep3(uint32_t v) {  // GenerateMortonCodesOfPrimitive
     return v;
 }
 
-__global__ void k_morton(const rt_triangle *tris, uint32_t ntri, const rt_sphere *sph, uint32_t n,
-                         const float *bounds, uint32_t ref_morton, uint32_t *keys, uint32_t *vals) {
+__global__ __launch_bounds__(kB) void k_morton(const rt_triangle *tris, uint32_t ntri, const rt_sphere *sph, uint32_t n,
+                                               const uint32_t *partial, uint32_t nparts, uint32_t ref_morton,
+                                               uint32_t *keys, uint32_t *vals) {
+    uint32_t mn[3], mx[3];
+    for (int a = 0; a < 3; ++a) {  // nparts <= kB
+        mn[a] = threadIdx.x < nparts ? partial[6u * threadIdx.x + a] : 0xFFFFFFFFu;
+        mx[a] = threadIdx.x < nparts ? partial[6u * threadIdx.x + 3 + a] : 0u;
+    }
+    bounds_reduce(mn, mx);
     uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
     if (i >= n) return;
+    float lo[3], span[3];
+    const float delta = 0.001f, pad = 0.001f / 2.0f;
+    for (int a = 0; a < 3; ++a) {  // padAABB (GetEnclosingAABB.comp:33-46)
+        float l = fkey_dec(mn[a]), h = fkey_dec(mx[a]);
+        if (h - l < delta) { l -= pad; h += pad; }
+        lo[a] = l;
+        span[a] = h - l;
+    }
     v3 c = centroid(tris, ntri, sph, i);
     float cc[3] = {c.x, c.y, c.z};
     uint32_t q[3];
     for (int a = 0; a < 3; ++a) {
-        float off = ref_morton ? cc[a] / bounds[6 + a] : (cc[a] - bounds[a]) / bounds[6 + a];
+        float off = ref_morton ? cc[a] / span[a] : (cc[a] - lo[a]) / span[a];
         q[a] = f2u_sat(off * 1024.0f);
     }
     keys[i] = (sep3(q[2]) << 2) | (sep3(q[1]) << 1) | sep3(q[0]);
@@ -155,7 +159,7 @@ __global__ void k_morton(const rt_triangle *tris, uint32_t ntri, const rt_sphere
 }
 
 // ---------------------------------------------------------------------------
-// Exclusive scan of u32 (device-wide, recursive over 2048-element blocks)
+// Exclusive scan of u32 (one block, or device-wide and recursive over 2048-element blocks)
 // ---------------------------------------------------------------------------
 constexpr int kScanItems = 8;
 constexpr int kScanTile = kB * kScanItems;
@@ -193,7 +197,38 @@ __global__ void k_scan_block(const uint32_t *in, uint32_t *out, uint32_t n, uint
         if (base + k < n) out[base + k] = pre;
         pre += v[k];
     }
-    if (threadIdx.x == 0 && block_sums) block_sums[blockIdx.x] = tot;
+    if (threadIdx.x == 0) block_sums[blockIdx.x] = tot;
+}
+// one block over up to kScanOne elements, in tiles of 8,192
+constexpr uint32_t kScanOne = 1u << 17;
+__global__ __launch_bounds__(1024) void k_scan_one(const uint32_t *in, uint32_t *out, uint32_t n) {
+    __shared__ uint32_t wsum[2][16];
+    const uint32_t lane = threadIdx.x % 64u, wave = threadIdx.x / 64u;
+    uint32_t run = 0;
+    for (uint32_t t0 = 0, phase = 0; t0 < n; t0 += 8192u, phase ^= 1u) {
+        const uint32_t base = t0 + threadIdx.x * 8u;
+        uint32_t v[8], s = 0;
+        for (int k = 0; k < 8; ++k) {
+            v[k] = base + k < n ? in[base + k] : 0u;
+            s += v[k];
+        }
+        uint32_t x = s;
+        for (int off = 1; off < 64; off <<= 1) {
+            const uint32_t y = (uint32_t)__shfl_up((int)x, off);
+            if (lane >= (uint32_t)off) x += y;
+        }
+        if (lane == 63u) wsum[phase][wave] = x;
+        __syncthreads();  // the other phase's sums are read before the next tile's barrier, so two sets suffice
+        uint32_t pre = run + x - s;
+        for (uint32_t w = 0; w < 16u; ++w) {
+            if (w < wave) pre += wsum[phase][w];
+            run += wsum[phase][w];
+        }
+        for (int k = 0; k < 8; ++k) {
+            if (base + k < n) out[base + k] = pre;
+            pre += v[k];
+        }
+    }
 }
 __global__ void k_scan_add(uint32_t *out, uint32_t n, const uint32_t *block_offsets) {
     uint64_t i = (uint64_t)blockIdx.x * kScanTile + threadIdx.x;
@@ -201,10 +236,6 @@ __global__ void k_scan_add(uint32_t *out, uint32_t n, const uint32_t *block_offs
     for (int k = 0; k < kScanItems; ++k, i += kB)
         if (i < n) out[i] += add;
 }
-__global__ void k_scan_total(const uint32_t *in, const uint32_t *out, uint32_t n, uint32_t *total) {
-    if (threadIdx.x == 0) *total = n ? out[n - 1] + in[n - 1] : 0u;
-}
-
 // Temporaries of one build, carved from one block of the context's scratch cache.  Every
 // launch of a build is on one stream, so a range can be handed out again as soon as the
 // launches using it have been enqueued (mark / release); the block itself returns to the
@@ -232,22 +263,21 @@ uint64_t round256(uint64_t b) { return (b + 255u) & ~uint64_t(255); }
 // bytes exclusive_scan takes from Temps for n elements
 uint64_t scan_temp_bytes(uint64_t n) {
     const uint64_t nb = (n + kScanTile - 1) / kScanTile;
-    return nb <= 1 ? 0 : 2 * round256(4 * nb) + scan_temp_bytes(nb);
+    return n <= kScanOne ? 0 : 2 * round256(4 * nb) + scan_temp_bytes(nb);
 }
 
-void exclusive_scan(const uint32_t *in, uint32_t *out, uint32_t n, uint32_t *d_total, hipStream_t st, Temps &tmp) {
-    uint32_t nb = (n + kScanTile - 1) / kScanTile;
-    if (nb <= 1) {
-        k_scan_block<<<1, kB, 0, st>>>(in, out, n, nullptr);
-    } else {
-        const uint64_t m = tmp.mark();
-        uint32_t *sums = tmp.take<uint32_t>(nb), *sums_scan = tmp.take<uint32_t>(nb);
-        k_scan_block<<<nb, kB, 0, st>>>(in, out, n, sums);
-        exclusive_scan(sums, sums_scan, nb, nullptr, st, tmp);
-        k_scan_add<<<nb, kB, 0, st>>>(out, n, sums_scan);
-        tmp.release(m);
+void exclusive_scan(const uint32_t *in, uint32_t *out, uint32_t n, hipStream_t st, Temps &tmp) {
+    if (n <= kScanOne) {
+        k_scan_one<<<1, 1024, 0, st>>>(in, out, n);
+        return;
     }
-    if (d_total) k_scan_total<<<1, 64, 0, st>>>(in, out, n, d_total);
+    const uint32_t nb = (n + kScanTile - 1) / kScanTile;
+    const uint64_t m = tmp.mark();
+    uint32_t *sums = tmp.take<uint32_t>(nb), *sums_scan = tmp.take<uint32_t>(nb);
+    k_scan_block<<<nb, kB, 0, st>>>(in, out, n, sums);
+    exclusive_scan(sums, sums_scan, nb, st, tmp);
+    k_scan_add<<<nb, kB, 0, st>>>(out, n, sums_scan);
+    tmp.release(m);
 }
 
 // ---------------------------------------------------------------------------
@@ -315,8 +345,43 @@ uint64_t radix_temp_bytes(uint64_t n) {
     return 2 * round256(4 * n) + 2 * round256(4 * 256 * nblocks) + scan_temp_bytes(256 * nblocks);
 }
 
+// The whole sort of few keys in one block: a bitonic network over (key, value) pairs in LDS.  The values are
+// the keys' original places, so equal keys keep their order and the result is the stable sort's.  4,096
+// keys in one launch, against twelve or more of the multi-block passes.
+constexpr uint32_t kSmallSort = 4096;
+
+__global__ __launch_bounds__(1024) void k_sort_small(uint32_t *keys, uint32_t *vals, uint32_t n, uint32_t padded) {
+    __shared__ uint64_t k[kSmallSort];
+    for (uint32_t i = threadIdx.x; i < padded; i += blockDim.x)
+        k[i] = i < n ? ((uint64_t)keys[i] << 32) | vals[i] : ~0ull;
+    for (uint32_t size = 2; size <= padded; size <<= 1)
+        for (uint32_t stride = size >> 1; stride > 0; stride >>= 1) {
+            __syncthreads();
+            for (uint32_t t = threadIdx.x; t < padded / 2; t += blockDim.x) {
+                const uint32_t i = 2u * t - (t & (stride - 1u)), j = i + stride;
+                const uint64_t a = k[i], b = k[j];
+                if ((a > b) == ((i & size) == 0u)) {
+                    k[i] = b;
+                    k[j] = a;
+                }
+            }
+        }
+    __syncthreads();
+    for (uint32_t i = threadIdx.x; i < n; i += blockDim.x) {
+        keys[i] = (uint32_t)(k[i] >> 32);
+        vals[i] = (uint32_t)k[i];
+    }
+}
+
+// vals: 0..n-1 in order
 void radix_sort(uint32_t *keys, uint32_t *vals, uint32_t n, hipStream_t st, Temps &tmp) {
     if (n <= 1) return;
+    if (n <= kSmallSort) {
+        uint32_t padded = 2;
+        while (padded < n) padded <<= 1;
+        k_sort_small<<<1, std::min(1024u, std::max(64u, padded / 2)), 0, st>>>(keys, vals, n, padded);
+        return;
+    }
     uint32_t nblocks = (n + kSortTile - 1) / kSortTile;
     const uint64_t m = tmp.mark();
     uint32_t *k2 = tmp.take<uint32_t>(n), *v2 = tmp.take<uint32_t>(n);
@@ -325,7 +390,7 @@ void radix_sort(uint32_t *keys, uint32_t *vals, uint32_t n, hipStream_t st, Temp
     for (int pass = 0; pass < 4; ++pass) {  // an even number of passes: the result is back in keys/vals
         uint32_t shift = 8u * pass;
         k_radix_hist<<<nblocks, kB, 0, st>>>(ka, n, shift, hist, nblocks);
-        exclusive_scan(hist, hoff, 256u * nblocks, nullptr, st, tmp);
+        exclusive_scan(hist, hoff, 256u * nblocks, st, tmp);
         k_radix_scatter<<<nblocks, kB, 0, st>>>(ka, va, kb, vb, n, shift, hoff, nblocks);
         std::swap(ka, kb);
         std::swap(va, vb);
@@ -343,9 +408,8 @@ __device__ inline int kdelta(const uint32_t *codes, int n, int i, int j) {
     return __clz((int)(ci ^ cj));
 }
 
-__global__ void k_karras(const uint32_t *codes, int n, rt_bvh_node *nodes, uint32_t *parent, uint2 *range) {
+__global__ void k_karras(const uint32_t *codes, int n, rt_bvh_node *nodes, uint2 *range) {
     int id = blockIdx.x * blockDim.x + threadIdx.x;
-    if (id == 0) parent[0] = 0;
     if (id >= n - 1) return;
     int dl = kdelta(codes, n, id, id - 1), dr = kdelta(codes, n, id, id + 1);
     int dir = (dr >= dl) ? 1 : -1;
@@ -374,18 +438,11 @@ __global__ void k_karras(const uint32_t *codes, int n, rt_bvh_node *nodes, uint3
     nd.primitiveIndex = 0;
     nd.primitiveType = 0;
     nodes[id] = nd;
-    parent[left] = (uint32_t)id;
-    parent[right] = (uint32_t)id;
     range[id] = make_uint2((uint32_t)first, (uint32_t)last);
 }
 
-// leaf slot -> primitive (A11 selects the reference's unsorted placement)
-__global__ void k_slots(const uint32_t *sorted_vals, uint32_t n, uint32_t ntri, uint32_t ref_leaves,
-                        uint32_t *slot_prim) {
-    uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= n) return;
-    uint32_t p = ref_leaves ? i : sorted_vals[i];
-    slot_prim[i] = p < ntri ? p : (RT_SPHERE_BIT | (p - ntri));
+__device__ inline bool has_nan3(const rt_bvh_node &b) {
+    return has_nan(v3{b.minX, b.minY, b.minZ}) || has_nan(v3{b.maxX, b.maxY, b.maxZ});
 }
 
 // leaf boxes (ConstructHLBVH.comp:33-56, 134-169), leaf records and material table
@@ -433,10 +490,20 @@ __device__ inline void leaf_body(const rt_triangle *tris, const rt_sphere *sph, 
     if (leaf_nodes) leaf_nodes[i] = nd;
     records[i] = rec;
 }
-__global__ void k_leaves(const rt_triangle *tris, const rt_sphere *sph, const float2 *sph_uv, const uint32_t *slot_prim,
-                         uint32_t n, rt_bvh_node *leaf_nodes, LeafRecord *records, uint32_t *slot_mat) {
-    uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i < n) leaf_body(tris, sph, sph_uv, slot_prim, i, leaf_nodes, records, slot_mat);
+// Also the leaf slot -> primitive table (sorted_vals, or the reference's unsorted placement), and *has_nan = 1
+// when some box has a NaN plane (one store per wave; box_union needs to know).
+__global__ void k_leaves(const rt_triangle *tris, uint32_t ntri, const rt_sphere *sph, const float2 *sph_uv,
+                         const uint32_t *sorted_vals, uint32_t ref_leaves, uint32_t n, uint32_t *slot_prim,
+                         rt_bvh_node *leaf_nodes, LeafRecord *records, uint32_t *slot_mat, uint32_t *has_nan) {
+    const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
+    if (i >= n) return;
+    const uint32_t p = ref_leaves ? i : sorted_vals[i];
+    slot_prim[i] = p < ntri ? p : (RT_SPHERE_BIT | (p - ntri));
+    leaf_body(tris, sph, sph_uv, slot_prim, i, leaf_nodes, records, slot_mat);
+    const rt_bvh_node nd = leaf_nodes[i];
+    const bool nan = has_nan3(nd);
+    const unsigned long long m = __ballot(nan);
+    if (m != 0ull && __lane_id() == (uint32_t)__ffsll((long long)m) - 1u) *has_nan = 1u;
 }
 // leaf records only (caller-supplied node buffer: boxes come from that buffer)
 __global__ void k_records(const rt_triangle *tris, const rt_sphere *sph, const float2 *sph_uv, const uint32_t *slot_prim,
@@ -445,96 +512,129 @@ __global__ void k_records(const rt_triangle *tris, const rt_sphere *sph, const f
     if (i < n) leaf_body(tris, sph, sph_uv, slot_prim, i, nullptr, records, slot_mat);
 }
 
-// ConstructAABBsOfInternalNodes.comp:27-65 computes each internal box as the union of
-// its children's, bottom-up, with an atomic visit counter per node (the second visitor
-// writes the union).  Here the same unions are computed level by level instead, deepest
-// level first, one launch per level: on this device the eight XCDs keep separate L2
-// caches, so each of the counter scheme's release/acquire pairs writes back and
-// invalidates a whole L2, while launch boundaries make a level's boxes visible for free.
-// Depths come from pointer jumping over the parent links.  In a Karras tree every child's
-// range shares a strictly longer prefix of the 64-bit (code, index) key than its parent's
-// (kdelta below), so the depth is at most 64 and the per-level launches stay few.
+// ConstructAABBsOfInternalNodes.comp:27-65 computes each internal box as the union of its children's,
+// bottom-up, with an atomic visit counter per node.  On this device the eight XCDs keep separate L2 caches,
+// so each of that scheme's release/acquire pairs writes back and invalidates a whole L2; one launch per
+// level needs every node's depth first and ~60 launches and 6 host waits in all.  Here no node waits
+// for another: an internal node's box is the union of the leaf boxes of its slot range, taken from a
+// table of the unions of 2^k aligned slots (k = 1, 2, ...), 8 levels of it per launch, in at most 2 loads per level.
+// The reference's min and max keep their left operand on ties and both trees keep the slots' order, so the
+// bits are the same, -0 and +0 included.  With a NaN plane they are not associative: see k_refit_pass.
+// 1 M triangles: 0.05 ms in 4 launches (before: 0.25 ms of kernels in 39 launches).
+struct Box {
+    float v[6];  // minX maxX minY maxY minZ maxZ
+};
+__device__ inline Box box_union(const Box &a, const Box &b) {
+    Box r;
+    for (int k = 0; k < 6; k += 2) {
+        r.v[k] = gmin(a.v[k], b.v[k]);
+        r.v[k + 1] = gmax(a.v[k + 1], b.v[k + 1]);
+    }
+    return r;
+}
+__device__ inline Box node_box(const rt_bvh_node &n) { return Box{{n.minX, n.maxX, n.minY, n.maxY, n.minZ, n.maxZ}}; }
 
-// internal node i: jump = parent (the root points at itself), dist = 1 (root 0)
-__global__ void k_depth_init(const uint32_t *parent, uint32_t m, uint32_t *jump, uint32_t *dist) {
-    const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= m) return;
-    jump[i] = i == 0 ? 0u : parent[i];
-    dist[i] = i == 0 ? 0u : 1u;
+// Level k of the table holds n >> k boxes (whole ones only) at offset(k), k >= 1.
+struct BoxTable {
+    const rt_bvh_node *leaves;
+    Box *boxes;
+    uint32_t n;
+    __host__ __device__ static uint64_t boxes_before(uint32_t n, uint32_t k) {  // in levels 1..k-1
+        uint64_t s = 0;
+        for (uint32_t l = 1; l < k; ++l) s += n >> l;
+        return s;
+    }
+};
+
+// Levels level+1 .. level+8 from level `level` (0: the leaves).  A block takes 256 of its boxes.
+__global__ __launch_bounds__(kB) void k_box_table(BoxTable t, uint32_t level) {
+    __shared__ Box sh[kB];
+    const uint32_t have = t.n >> level, i = blockIdx.x * kB + threadIdx.x;
+    if (i < have) {
+        if (level == 0) sh[threadIdx.x] = node_box(t.leaves[i]);
+        else sh[threadIdx.x] = t.boxes[BoxTable::boxes_before(t.n, level) + i];
+    }
+    uint64_t at = BoxTable::boxes_before(t.n, level + 1u);
+    for (uint32_t k = 1; k <= 8u; ++k) {
+        const uint32_t count = t.n >> (level + k), j = blockIdx.x * (kB >> k) + threadIdx.x;
+        const bool mine = threadIdx.x < (kB >> k) && j < count;
+        Box b;
+        __syncthreads();
+        if (mine) b = box_union(sh[2u * threadIdx.x], sh[2u * threadIdx.x + 1u]);
+        __syncthreads();
+        if (mine) {
+            sh[threadIdx.x] = b;
+            t.boxes[at + j] = b;
+        }
+        at += count;
+    }
 }
 
-// one doubling step: dist(i) += dist(jump(i)), jump(i) = jump(jump(i)); *more = 1 (one
-// store per wave) while a jump has not reached the root
-__global__ void k_depth_jump(const uint32_t *jump, const uint32_t *dist, uint32_t *jump2, uint32_t *dist2, uint32_t m,
-                             uint32_t *more) {
-    const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= m) return;
-    const uint32_t j = jump[i];
-    dist2[i] = dist[i] + dist[j];
-    const uint32_t jj = jump[j];
-    jump2[i] = jj;
-    const unsigned long long pending = __ballot(jj != 0u);
-    if (pending != 0ull && __lane_id() == (uint32_t)__ffsll((long long)pending) - 1u) *more = 1u;
-}
-
-// largest depth: block maximum in LDS, one global atomic per block
-__global__ void k_depth_max(const uint32_t *depth, uint32_t m, uint32_t *out) {
-    __shared__ uint32_t best;
-    if (threadIdx.x == 0) best = 0u;
-    __syncthreads();
-    const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i < m) atomicMax(&best, depth[i]);
-    __syncthreads();
-    if (threadIdx.x == 0) atomicMax(out, best);
-}
-
-// the union for every node at depth d (its children are leaves or deeper nodes)
-__global__ void k_refit_level(rt_bvh_node *nodes, const uint32_t *depth, uint32_t m, uint32_t d) {
+__global__ void k_refit(rt_bvh_node *nodes, const uint2 *range, BoxTable t) {
     const uint32_t id = blockIdx.x * blockDim.x + threadIdx.x;
-    if (id >= m || depth[id] != d) return;
-    rt_bvh_node nd = nodes[id];
-    const rt_bvh_node a = nodes[nd.left], b = nodes[nd.right];
-    nd.minX = gmin(a.minX, b.minX); nd.maxX = gmax(a.maxX, b.maxX);
-    nd.minY = gmin(a.minY, b.minY); nd.maxY = gmax(a.maxY, b.maxY);
-    nd.minZ = gmin(a.minZ, b.minZ); nd.maxZ = gmax(a.maxZ, b.maxZ);
-    nodes[id] = nd;
+    if (id + 1u >= t.n) return;
+    uint32_t l = range[id].x, r = range[id].y + 1u, level = 0;
+    uint64_t at = 0;  // of level `level` in the table
+    Box left, right;
+    bool hl = false, hr = false;
+    while (l < r) {
+        if (l & 1u) {
+            const Box b = level ? t.boxes[at + l] : node_box(t.leaves[l]);
+            left = hl ? box_union(left, b) : b;
+            hl = true;
+            ++l;
+        }
+        if (r & 1u) {
+            --r;
+            const Box b = level ? t.boxes[at + r] : node_box(t.leaves[r]);
+            right = hr ? box_union(b, right) : b;
+            hr = true;
+        }
+        l >>= 1;
+        r >>= 1;
+        at += level ? t.n >> level : 0u;
+        ++level;
+    }
+    const Box b = hl && hr ? box_union(left, right) : hl ? left : right;
+    rt_bvh_node &nd = nodes[id];
+    nd.minX = b.v[0]; nd.maxX = b.v[1]; nd.minY = b.v[2]; nd.maxY = b.v[3]; nd.minZ = b.v[4]; nd.maxZ = b.v[5];
 }
+
+// Every node's union of its children's present boxes, from `in` to `out`.  As many passes as the tree is deep make
+// every box final whatever the union's rules for NaN; an LBVH is at most 64 deep (each child's range shares a
+// strictly longer prefix of the 64-bit (code, index) key than its parent's).  Scenes with NaN vertices only.
+__global__ void k_refit_pass(const rt_bvh_node *in, rt_bvh_node *out, uint32_t n) {
+    const uint32_t id = blockIdx.x * blockDim.x + threadIdx.x;
+    if (id >= 2u * n - 1u) return;
+    rt_bvh_node nd = in[id];
+    if (id < n - 1u) {
+        const Box b = box_union(node_box(in[nd.left]), node_box(in[nd.right]));
+        nd.minX = b.v[0]; nd.maxX = b.v[1]; nd.minY = b.v[2]; nd.maxY = b.v[3]; nd.minZ = b.v[4]; nd.maxZ = b.v[5];
+    }
+    out[id] = nd;
+}
+
+uint64_t refit_temp_bytes(uint64_t n) { return round256(sizeof(Box) * n); }
 
 // Internal boxes of the n-1 internal nodes (leaf boxes are already written).
-uint64_t refit_temp_bytes(uint64_t n) { return 4 * round256(4 * n) + round256(4); }
-
-void refit_levels(rt_bvh_node *nodes, const uint32_t *parent, uint32_t n, hipStream_t st, Temps &tmp) {
-    const uint32_t m = n - 1;
+void refit(rt_bvh_node *nodes, const uint2 *range, uint32_t n, hipStream_t st, Temps &tmp) {
     const uint64_t mk = tmp.mark();
-    uint32_t *jump = tmp.take<uint32_t>(m), *dist = tmp.take<uint32_t>(m), *jump2 = tmp.take<uint32_t>(m),
-             *dist2 = tmp.take<uint32_t>(m), *flag = tmp.take<uint32_t>(1);
-    k_depth_init<<<grid_for(m), kB, 0, st>>>(parent, m, jump, dist);
-    for (uint32_t round = 0; round < 32; ++round) {  // 2^32 exceeds any depth
-        k_fill_u32<<<1, kB, 0, st>>>(flag, 0u, 1u);
-        k_depth_jump<<<grid_for(m), kB, 0, st>>>(jump, dist, jump2, dist2, m, flag);
-        std::swap(jump, jump2);
-        std::swap(dist, dist2);
-        uint32_t more = 0;
-        RT_HIP(hipMemcpyAsync(&more, flag, sizeof more, hipMemcpyDeviceToHost, st));
-        RT_HIP(hipStreamSynchronize(st));
-        if (!more) break;
-    }
-    k_fill_u32<<<1, kB, 0, st>>>(flag, 0u, 1u);
-    k_depth_max<<<grid_for(m), kB, 0, st>>>(dist, m, flag);
-    uint32_t deepest = 0;
-    RT_HIP(hipMemcpyAsync(&deepest, flag, sizeof deepest, hipMemcpyDeviceToHost, st));
-    RT_HIP(hipStreamSynchronize(st));
-    RT_REQUIRE(deepest < m, "internal: LBVH parent links do not form a tree");
-    for (uint32_t d = deepest + 1; d-- > 0;) k_refit_level<<<grid_for(m), kB, 0, st>>>(nodes, dist, m, d);
+    BoxTable t{nodes + (n - 1), tmp.take<Box>(n), n};
+    for (uint32_t level = 0; (n >> level) > 1u; level += 8) k_box_table<<<grid_for(n >> level), kB, 0, st>>>(t, level);
+    k_refit<<<grid_for(n - 1), kB, 0, st>>>(nodes, range, t);
     tmp.release(mk);
 }
 
 // ---------------------------------------------------------------------------
-// Collapse binary -> wide, one BFS level per launch pair.  A wide node made
+// Collapse binary -> wide, breadth first.  A wide node made
 // from binary node b takes b's children and repeatedly opens the child with the
 // largest surface area until W children exist; a child whose subtree holds at
 // most leaf_size primitives becomes a leaf over its contiguous slot range.
-// ---------------------------------------------------------------------------
+//
+// Wide nodes are numbered in queue order: queue[i] is the binary node of wide node i, and a level's nodes are
+// consecutive.  Level sizes stay on the device (CollapseState), so levels are launched ahead without
+// the host reading each one; a launch past the last level finds an empty one.  A level takes two launches
+// (choose children and count; number and write), a small tree one launch in all.
 struct CollapseArgs {
     const rt_bvh_node *nodes;
     const uint2 *range;  // internal nodes: leaf-slot range of the subtree
@@ -587,55 +687,153 @@ __device__ inline bool becomes_node(const CollapseArgs &a, uint32_t c) {
     return is_internal(a, c) && subtree_count(a, c) > a.leaf_size;
 }
 
-__global__ void k_collapse_count(CollapseArgs a, const uint32_t *queue, uint32_t qn, uint32_t *newcount) {
-    uint32_t e = blockIdx.x * blockDim.x + threadIdx.x;
-    if (e >= qn) return;
-    uint32_t cand[8];
-    int nc = choose_children(a, queue[e], cand);
-    uint32_t k = 0;
-    for (int i = 0; i < nc; ++i) k += becomes_node(a, cand[i]) ? 1u : 0u;
-    newcount[e] = k;
+// [level & 1]: the level's first wide node and its size; the other entry receives the next level's
+struct CollapseState {
+    uint32_t base[2], count[2];
+    uint32_t depth, bad;  // levels with nodes so far; 1 when a level would not fit
+};
+
+constexpr uint32_t kCollapseBlocks = 2048;  // at most, per launch
+
+// the entries of the level that block `b` of `blocks` handles
+__device__ inline uint2 collapse_chunk(uint32_t count, uint32_t b, uint32_t blocks) {
+    const uint32_t chunk = ((count + blocks - 1u) / blocks + kB - 1u) / kB * kB;
+    return make_uint2(min(b * chunk, count), min(b * chunk + chunk, count));
 }
 
-__global__ void k_collapse_emit(CollapseArgs a, const uint32_t *queue, uint32_t qn, uint32_t level_base,
-                                uint32_t next_base, const uint32_t *child_base, uint32_t *next_queue,
-                                uint32_t *wide) {
-    uint32_t e = blockIdx.x * blockDim.x + threadIdx.x;
-    if (e >= qn) return;
+__device__ inline uint32_t child_nodes(const CollapseArgs &a, const uint32_t *cand, int nc) {
+    uint32_t k = 0;
+    for (int i = 0; i < nc; ++i) k += becomes_node(a, cand[i]) ? 1u : 0u;
+    return k;
+}
+
+// Writes wide node `node` of queue entry with children cand[0..nc); its node children are numbered from `j` on.
+__device__ inline void write_wide(const CollapseArgs &a, const uint32_t *cand, int nc, uint32_t node, uint32_t j,
+                                  uint32_t *queue, uint32_t *wide) {
     const uint32_t W = a.width;
-    uint32_t cand[8];
-    int nc = choose_children(a, queue[e], cand);
-    uint32_t *nd = wide + (size_t)(level_base + e) * 8u * W;
+    uint32_t *nd = wide + (size_t)node * 8u * W;
     float *f = reinterpret_cast<float *>(nd);
-    uint32_t j = child_base[e];
     const float inf = __uint_as_float(0x7F800000u);
     for (uint32_t k = 0; k < W; ++k) {
-        if ((int)k >= nc) {
-            f[0 * W + k] = inf; f[1 * W + k] = inf;
-            f[2 * W + k] = inf; f[3 * W + k] = inf;
-            f[4 * W + k] = inf; f[5 * W + k] = inf;
-            nd[6 * W + k] = kEmpty;
-            nd[7 * W + k] = 0u;
-            continue;
+        float box[6] = {inf, inf, inf, inf, inf, inf};
+        uint32_t ce = kEmpty;
+        if ((int)k < nc) {
+            const uint32_t c = cand[k];
+            const rt_bvh_node bn = a.nodes[c];
+            box[0] = bn.minX; box[1] = bn.maxX;
+            box[2] = bn.minY; box[3] = bn.maxY;
+            box[4] = bn.minZ; box[5] = bn.maxZ;
+            if (becomes_node(a, c)) {
+                ce = j;
+                queue[j] = c;
+                ++j;
+            } else if (is_internal(a, c)) {
+                const uint2 r = a.range[c];
+                ce = leaf_entry(r.x, r.y - r.x + 1u);
+            } else {
+                ce = leaf_entry(c - (a.n - 1u), 1u);
+            }
         }
-        uint32_t c = cand[k];
-        const rt_bvh_node bn = a.nodes[c];
-        f[0 * W + k] = bn.minX; f[1 * W + k] = bn.maxX;
-        f[2 * W + k] = bn.minY; f[3 * W + k] = bn.maxY;
-        f[4 * W + k] = bn.minZ; f[5 * W + k] = bn.maxZ;
-        uint32_t ce;
-        if (becomes_node(a, c)) {
-            ce = next_base + j;
-            next_queue[j] = c;
-            ++j;
-        } else if (is_internal(a, c)) {
-            uint2 r = a.range[c];
-            ce = leaf_entry(r.x, r.y - r.x + 1u);
-        } else {
-            ce = leaf_entry(c - (a.n - 1u), 1u);
-        }
+        for (int q = 0; q < 6; ++q) f[q * W + k] = box[q];
         nd[6 * W + k] = ce;
         nd[7 * W + k] = 0u;
+    }
+}
+
+// children of the level's entries -> chosen (8 words per entry), node children per block -> block_sums
+__global__ __launch_bounds__(kB) void k_collapse_choose(CollapseArgs a, uint32_t level, const CollapseState *st,
+                                                        const uint32_t *queue, uint32_t *chosen, uint32_t *block_sums) {
+    const uint32_t base = st->base[level & 1u];
+    const uint2 c = collapse_chunk(st->count[level & 1u], blockIdx.x, gridDim.x);
+    uint32_t sum = 0;
+    for (uint32_t e = c.x + threadIdx.x; e < c.y; e += kB) {
+        uint32_t cand[8];
+        const int nc = choose_children(a, level ? queue[base + e] : 0u, cand);  // level 0: the root
+        sum += child_nodes(a, cand, nc);
+        for (uint32_t k = 0; k < a.width; ++k) chosen[(size_t)e * a.width + k] = (int)k < nc ? cand[k] : kEmpty;
+    }
+    uint32_t total;
+    (void)block_exclusive_scan(sum, &total);
+    if (threadIdx.x == 0) block_sums[blockIdx.x] = total;
+}
+
+__global__ __launch_bounds__(kB) void k_collapse_emit(CollapseArgs a, uint32_t level, CollapseState *st, uint32_t *queue,
+                                                      const uint32_t *chosen, const uint32_t *block_sums, uint32_t *wide,
+                                                      uint32_t max_nodes) {
+    const uint32_t base = st->base[level & 1u], count = st->count[level & 1u];
+    if (count == 0u) {
+        if (blockIdx.x == 0 && threadIdx.x == 0) st->count[(level + 1u) & 1u] = 0u;
+        return;
+    }
+    const uint2 c = collapse_chunk(count, blockIdx.x, gridDim.x);
+    uint32_t before = 0, all = 0;  // node children of the earlier blocks, and of all
+    for (uint32_t b = threadIdx.x; b < gridDim.x; b += kB) {
+        const uint32_t v = block_sums[b];
+        all += v;
+        if (b < blockIdx.x) before += v;
+    }
+    uint32_t total_before, total;
+    (void)block_exclusive_scan(before, &total_before);
+    (void)block_exclusive_scan(all, &total);
+    if ((uint64_t)base + count + total > max_nodes) {  // cannot happen: a wide node is made from its own binary node
+        if (blockIdx.x == 0 && threadIdx.x == 0) { st->bad = 1u; st->count[(level + 1u) & 1u] = 0u; }
+        return;
+    }
+    uint32_t j0 = base + count + total_before;
+    for (uint32_t e0 = c.x; e0 < c.y; e0 += kB) {
+        const uint32_t e = e0 + threadIdx.x;
+        uint32_t cand[8], k = 0;
+        int nc = 0;
+        if (e < c.y) {
+            for (; nc < (int)a.width && chosen[(size_t)e * a.width + nc] != kEmpty; ++nc) cand[nc] = chosen[(size_t)e * a.width + nc];
+            k = child_nodes(a, cand, nc);
+        }
+        uint32_t tile;
+        const uint32_t pre = block_exclusive_scan(k, &tile);
+        if (e < c.y) write_wide(a, cand, nc, base + e, j0 + pre, queue, wide);
+        j0 += tile;
+    }
+    if (blockIdx.x == 0 && threadIdx.x == 0) {
+        st->base[(level + 1u) & 1u] = base + count;
+        st->count[(level + 1u) & 1u] = total;
+        st->depth = level + 1u;
+    }
+}
+
+// All levels of a small tree in one block.
+constexpr uint32_t kSmallCollapse = 16384;  // primitives
+__global__ __launch_bounds__(kB) void k_collapse_small(CollapseArgs a, CollapseState *st, uint32_t *queue, uint32_t *wide,
+                                                       uint32_t max_nodes) {
+    uint32_t base = 0, count = 1, level = 0;
+    if (threadIdx.x == 0) queue[0] = 0u;  // the root
+    for (; count > 0u; ++level) {
+        __syncthreads();  // the queue entries of this level are written
+        uint32_t j0 = base + count;
+        for (uint32_t e0 = 0; e0 < count; e0 += kB) {
+            const uint32_t e = e0 + threadIdx.x;
+            uint32_t cand[8], k = 0;
+            int nc = 0;
+            if (e < count) {
+                nc = choose_children(a, queue[base + e], cand);
+                k = child_nodes(a, cand, nc);
+            }
+            uint32_t tile;
+            const uint32_t pre = block_exclusive_scan(k, &tile);
+            if ((uint64_t)j0 + tile > max_nodes) {  // cannot happen, as above
+                if (threadIdx.x == 0) st->bad = 1u;
+                return;
+            }
+            if (e < count) write_wide(a, cand, nc, base + e, j0 + pre, queue, wide);
+            j0 += tile;
+        }
+        const uint32_t next = base + count;
+        count = j0 - next;
+        base = next;
+    }
+    if (threadIdx.x == 0) {
+        st->base[level & 1u] = base;
+        st->count[level & 1u] = 0u;
+        st->depth = level;
     }
 }
 
@@ -742,6 +940,12 @@ __global__ void k_compress(const uint32_t *wide, uint32_t nwide, uint32_t *qwide
         info[1] = __float_as_uint(far);
         info[2] = __float_as_uint(ext);
     }
+}
+
+// the first level is the root; info: see build_scene
+__global__ void k_build_init(CollapseState *st, uint32_t *info) {
+    if (threadIdx.x == 0) *st = CollapseState{{0u, 0u}, {1u, 0u}, 0u, 0u};
+    if (threadIdx.x < 4) info[threadIdx.x] = 0u;
 }
 
 template <class T> void upload(DevBuf &b, const T *src, size_t count) {
@@ -872,9 +1076,9 @@ void build_scene(rt_context *ctx, Scene &sc, const rt_triangle *tris, uint32_t n
     const uint32_t max_nodes = std::max<uint32_t>(n - 1, 1);
     const uint64_t temp_bytes =
         (keep_binary ? 0 : round256(sizeof(rt_bvh_node) * (2ull * n - 1))) + round256(sizeof(uint2) * max_nodes) +
-        round256(24) + round256(36) + 2 * round256(4ull * n) + round256(4ull * (2ull * n - 1)) +
-        std::max(radix_temp_bytes(n), refit_temp_bytes(n)) +                      // sort, then refit
-        round256(32ull * W * max_nodes) + 4 * round256(4ull * max_nodes) + round256(4) + scan_temp_bytes(max_nodes);
+        round256(24ull * kBoundsBlocks) + 2 * round256(4ull * n) + std::max(radix_temp_bytes(n), refit_temp_bytes(n)) +
+        round256(32ull * W * max_nodes) + round256(4ull * max_nodes) + round256(4ull * W * max_nodes) +
+        round256(4ull * kCollapseBlocks) + round256(sizeof(CollapseState)) + round256(16);
     Temps tmp(ctx, temp_bytes, st);
     DevBuf kept;  // the binary nodes, when they stay resident
     rt_bvh_node *binary = nullptr;
@@ -885,6 +1089,9 @@ void build_scene(rt_context *ctx, Scene &sc, const rt_triangle *tris, uint32_t n
         binary = tmp.take<rt_bvh_node>(2ull * n - 1);
     }
     uint2 *range = tmp.take<uint2>(max_nodes);
+    CollapseState *state = tmp.take<CollapseState>(1);
+    uint32_t *info = tmp.take<uint32_t>(4);  // k_compress's three words, then k_leaves' NaN flag
+    k_build_init<<<1, 64, 0, st>>>(state, info);
     if (nodes) {
         std::vector<uint32_t> hslots;
         std::vector<uint2> hrange;
@@ -897,49 +1104,64 @@ void build_scene(rt_context *ctx, Scene &sc, const rt_triangle *tris, uint32_t n
                                               sc.slot_mat.as<uint32_t>());
     } else {
         const uint64_t mk = tmp.mark();
-        uint32_t *bkeys = tmp.take<uint32_t>(6);
-        float *bounds = tmp.take<float>(9);
-        uint32_t *keys = tmp.take<uint32_t>(n), *vals = tmp.take<uint32_t>(n), *parent = tmp.take<uint32_t>(2ull * n - 1);
-        k_bounds_init<<<1, 64, 0, st>>>(bkeys);
-        uint32_t g = std::min<uint32_t>(grid_for(n), 4096);
-        k_centroid_bounds<<<g, kB, 0, st>>>(dtris.as<rt_triangle>(), ntri, dsph.as<rt_sphere>(), n, bkeys);
-        k_bounds_finalize<<<1, 64, 0, st>>>(bkeys, bounds);
-        k_morton<<<grid_for(n), kB, 0, st>>>(dtris.as<rt_triangle>(), ntri, dsph.as<rt_sphere>(), n, bounds,
+        uint32_t *partial = tmp.take<uint32_t>(6ull * kBoundsBlocks);
+        uint32_t *keys = tmp.take<uint32_t>(n), *vals = tmp.take<uint32_t>(n);
+        const uint32_t g = std::min<uint32_t>(grid_for(n), kBoundsBlocks);
+        k_centroid_bounds<<<g, kB, 0, st>>>(dtris.as<rt_triangle>(), ntri, dsph.as<rt_sphere>(), n, partial);
+        k_morton<<<grid_for(n), kB, 0, st>>>(dtris.as<rt_triangle>(), ntri, dsph.as<rt_sphere>(), n, partial, g,
                                              (opts.flags & RT_BUILD_REFERENCE_MORTON) ? 1u : 0u, keys, vals);
         radix_sort(keys, vals, n, st, tmp);
-        if (n > 1) k_karras<<<grid_for(n - 1), kB, 0, st>>>(keys, (int)n, binary, parent, range);
-        k_slots<<<grid_for(n), kB, 0, st>>>(vals, n, ntri, (opts.flags & RT_BUILD_REFERENCE_LEAVES) ? 1u : 0u,
-                                            sc.slot_prim.as<uint32_t>());
-        k_leaves<<<grid_for(n), kB, 0, st>>>(dtris.as<rt_triangle>(), dsph.as<rt_sphere>(), duv.as<float2>(),
-                                             sc.slot_prim.as<uint32_t>(), n, binary + (n - 1),
-                                             sc.records.as<LeafRecord>(), sc.slot_mat.as<uint32_t>());
-        if (n > 1) refit_levels(binary, parent, n, st, tmp);
+        if (n > 1) k_karras<<<grid_for(n - 1), kB, 0, st>>>(keys, (int)n, binary, range);
+        k_leaves<<<grid_for(n), kB, 0, st>>>(dtris.as<rt_triangle>(), ntri, dsph.as<rt_sphere>(), duv.as<float2>(), vals,
+                                             (opts.flags & RT_BUILD_REFERENCE_LEAVES) ? 1u : 0u, n,
+                                             sc.slot_prim.as<uint32_t>(), binary + (n - 1), sc.records.as<LeafRecord>(),
+                                             sc.slot_mat.as<uint32_t>(), info + 3);
+        if (n > 1) refit(binary, range, n, st, tmp);
         tmp.release(mk);
     }
     RT_HIP(hipGetLastError());
 
-    // collapse into the wide layout, BFS order
     CollapseArgs a{binary, range, n, W, L};
     uint32_t *wide_tmp = tmp.take<uint32_t>(8ull * W * max_nodes);
-    uint32_t *qa = tmp.take<uint32_t>(max_nodes), *qb = tmp.take<uint32_t>(max_nodes);
-    uint32_t *newcount = tmp.take<uint32_t>(max_nodes), *child_base = tmp.take<uint32_t>(max_nodes);
-    uint32_t *d_total = tmp.take<uint32_t>(3);
-    k_fill_u32<<<1, 64, 0, st>>>(qa, 0u, 1u);  // the root
-    uint32_t qn = 1, level_base = 0, depth = 0;
-    uint32_t *qcur = qa, *qnext = qb;
-    while (qn > 0) {
-        k_collapse_count<<<grid_for(qn), kB, 0, st>>>(a, qcur, qn, newcount);
-        exclusive_scan(newcount, child_base, qn, d_total, st, tmp);
-        uint32_t next_n = 0;
-        RT_HIP(hipMemcpy(&next_n, d_total, sizeof(uint32_t), hipMemcpyDeviceToHost));
-        RT_REQUIRE(level_base + qn + next_n <= max_nodes, "internal: wide node count exceeds bound");
-        k_collapse_emit<<<grid_for(qn), kB, 0, st>>>(a, qcur, qn, level_base, level_base + qn, child_base, qnext,
-                                                     wide_tmp);
-        level_base += qn;
-        qn = next_n;
-        std::swap(qcur, qnext);
-        ++depth;
+    uint32_t *queue = tmp.take<uint32_t>(max_nodes), *chosen = tmp.take<uint32_t>((uint64_t)W * max_nodes);
+    uint32_t *block_sums = tmp.take<uint32_t>(kCollapseBlocks);
+    struct { CollapseState state; uint32_t pad[58]; uint32_t info[4]; } out{};  // as the two lie in the temporaries
+    static_assert(sizeof(CollapseState) == 24 && offsetof(decltype(out), info) == 256, "state and info are read together");
+    const auto collapse = [&] {
+        if (n <= kSmallCollapse && !nodes) {
+            k_collapse_small<<<1, kB, 0, st>>>(a, state, queue, wide_tmp, max_nodes);
+            RT_HIP(hipMemcpy(&out, state, sizeof out, hipMemcpyDeviceToHost));
+            return;
+        }
+        // about log2(n) levels of a width-4 tree; the host looks after the first ones and then after every eight
+        uint32_t level = 0, ahead = 2;
+        for (uint64_t m = n; m > 1; m >>= 1) ++ahead;
+        uint64_t widest = 1;  // no level can hold more nodes
+        do {
+            for (uint32_t end = level + ahead; level < end; ++level) {
+                const uint32_t grid = std::min<uint32_t>(grid_for(widest), kCollapseBlocks);
+                k_collapse_choose<<<grid, kB, 0, st>>>(a, level, state, queue, chosen, block_sums);
+                k_collapse_emit<<<grid, kB, 0, st>>>(a, level, state, queue, chosen, block_sums, wide_tmp, max_nodes);
+                widest = std::min<uint64_t>(widest * W, max_nodes);
+            }
+            ahead = 8;
+            RT_HIP(hipMemcpy(&out, state, sizeof out, hipMemcpyDeviceToHost));
+        } while (out.state.count[level & 1u] != 0u);
+    };
+    collapse();
+    if (out.info[3] && n > 1) {  // NaN planes: unions in the tree's own order, then the collapse again
+        DevBuf other(sizeof(rt_bvh_node) * (2ull * n - 1));
+        for (int pass = 0; pass < 64; pass += 2) {
+            k_refit_pass<<<grid_for(2ull * n - 1), kB, 0, st>>>(binary, other.as<rt_bvh_node>(), n);
+            k_refit_pass<<<grid_for(2ull * n - 1), kB, 0, st>>>(other.as<rt_bvh_node>(), binary, n);
+        }
+        k_build_init<<<1, 64, 0, st>>>(state, info);
+        collapse();
+        RT_HIP(hipStreamSynchronize(st));  // `other` is freed
     }
+    RT_REQUIRE(!out.state.bad, "internal: wide node count exceeds bound");
+    const uint32_t depth = out.state.depth;
+    const uint32_t nwide = std::max(out.state.base[0], out.state.base[1]);
     RT_HIP(hipEventRecord(ev1, st));
     RT_HIP(hipEventSynchronize(ev1));
     RT_HIP(hipGetLastError());
@@ -948,25 +1170,24 @@ void build_scene(rt_context *ctx, Scene &sc, const rt_triangle *tris, uint32_t n
     (void)hipEventDestroy(ev0);
     (void)hipEventDestroy(ev1);
 
-    sc.nwide = level_base;
+    sc.nwide = nwide;
     sc.wide.alloc((size_t)sc.nwide * 32u * W);
     RT_HIP(hipMemcpy(sc.wide.p, wide_tmp, (size_t)sc.nwide * 32u * W, hipMemcpyDeviceToDevice));
     if (W == 4) {
         sc.qwide.alloc((size_t)sc.nwide * 64u);
         sc.slot_ref.alloc(sizeof(uint32_t) * n);
-        k_fill_u32<<<1, 64, 0, st>>>(d_total, 0u, 1u);
         if (nodes)
             k_check_boxes<<<grid_for(2ull * n - 1), kB, 0, st>>>(binary, n, dtris.as<rt_triangle>(), dsph.as<rt_sphere>(),
-                                                                 sc.slot_prim.as<uint32_t>(), d_total);
+                                                                 sc.slot_prim.as<uint32_t>(), info);
         k_compress<<<grid_for(sc.nwide), kB, 0, st>>>(sc.wide.as<uint32_t>(), sc.nwide, sc.qwide.as<uint32_t>(),
-                                                      sc.slot_ref.as<uint32_t>(), d_total);
+                                                      sc.slot_ref.as<uint32_t>(), info);
         RT_HIP(hipGetLastError());
-        struct { uint32_t bad; float far, extent; } info{};
-        RT_HIP(hipMemcpy(&info, d_total, sizeof info, hipMemcpyDeviceToHost));
+        struct { uint32_t bad; float far, extent; } whole{};
+        RT_HIP(hipMemcpy(&whole, info, sizeof whole, hipMemcpyDeviceToHost));
         // see Scene::far_limit: origins may lie this far outside the scene's coordinates
-        const float reach = std::min(1000.0f * info.extent, 512.0f * min_radius);
-        sc.far_limit = info.far + reach;
-        if (info.bad || !(reach >= 1.8f * info.extent)) {  // also where a sphere is too small to be seen across the scene
+        const float reach = std::min(1000.0f * whole.extent, 512.0f * min_radius);
+        sc.far_limit = whole.far + reach;
+        if (whole.bad || !(reach >= 1.8f * whole.extent)) {  // also where a sphere is too small to be seen across the scene
             sc.qwide.release();
             sc.slot_ref.release();
         }

@@ -1,0 +1,105 @@
+"""The device builder at the sizes where it changes its kernels, byte for byte against the oracle's: one primitive,
+whole and ragged powers of two (the table of aligned unions), both sides of the single-block sort, scan and collapse,
+every width and leaf size, signed zeros, NaN vertices, identical primitives."""
+import numpy as np
+import pytest
+
+import oracle as OR
+from raytracergpu_mastersproject_amd import layouts as L
+from raytracergpu_mastersproject_amd import workloads as W
+
+from helpers import gpu_trace, with_spheres
+
+pytestmark = pytest.mark.gpu
+
+MATS = W.make_materials([0.5, 0.5, 0.5], L.DIFFUSE)
+
+
+def _tris(n, seed=61):
+    tris, _ = W.cluster_scene(max(1, min(16, n // 8)), -(-n // max(1, min(16, n // 8))), seed=seed)
+    return np.ascontiguousarray(tris[:n])
+
+
+def _build(ctx, native, tris, sph=None, **kw):
+    sid = ctx.upload(tris, sph, MATS, flags=native.BUILD_KEEP_BINARY, **kw)
+    nodes, slots = ctx.nodes(sid), ctx.slots(sid)
+    onodes, _, oslots, _, _ = OR.build_lbvh(tris, sph)
+    assert np.array_equal(nodes.view(np.uint8), onodes.view(np.uint8))
+    assert np.array_equal(slots, oslots)
+    return sid, nodes, slots
+
+
+def _check_wide(ctx, sid, n, slots_leaf):
+    """Every leaf slot lies in exactly one wide leaf, every wide node but the root in one parent, breadth first."""
+    inf = ctx.info(sid)
+    w = ctx.wide(sid).reshape(inf.nwide, 8, inf.width)[:, 6, :]
+    child = w[w != 0xFFFFFFFF]
+    node = child[(child >> 31) == 0]
+    assert np.array_equal(node, np.arange(1, inf.nwide, dtype=np.uint32))
+    leaf = child[(child >> 31) == 1]
+    first, cnt = leaf & 0x07FFFFFF, ((leaf >> 27) & 15) + 1
+    assert cnt.max() <= slots_leaf
+    held = np.concatenate([np.arange(f, f + c) for f, c in zip(first, cnt)])
+    assert np.array_equal(np.sort(held), np.arange(n))
+
+
+@pytest.mark.parametrize("n", [1, 2, 3, 5, 255, 256, 257, 511, 512, 513, 4095, 4096, 4097, 16384, 16385, 65535, 65536, 70001,
+                               1048577, 1050000])
+def test_sizes(ctx, native, n):
+    tris = _tris(n)
+    sid, _, _ = _build(ctx, native, tris)
+    _check_wide(ctx, sid, n, 1)
+    ctx.release(sid)
+
+
+@pytest.mark.parametrize("n", [7, 3000, 20000])
+@pytest.mark.parametrize("width,leaf", [(2, 1), (2, 8), (4, 3), (8, 1), (8, 4)])
+def test_widths_and_leaves(ctx, native, n, width, leaf):
+    tris = _tris(n, 62)
+    sid, _, _ = _build(ctx, native, tris, with_spheres(tris, MATS, 3), width=width, leaf_size=leaf)
+    _check_wide(ctx, sid, n + 3, leaf)
+    ctx.release(sid)
+
+
+@pytest.mark.parametrize("n", [600, 5000])
+def test_signed_zeros_and_identical(ctx, native, n):
+    tris = _tris(n, 63)
+    for k in ("v0", "v1", "v2"):
+        tris[k][::2, 1] = np.where(np.arange(len(tris[k][::2])) % 3 == 0, 0.0, -0.0)
+    tris[n // 2:n // 2 + 300] = tris[n // 2]
+    sid, _, _ = _build(ctx, native, tris)
+    ctx.release(sid)
+
+
+def _tree_unions(nodes, n):
+    """Internal boxes as the reference's shader makes them: each the union of its two children's, left operand kept
+    on ties and against NaN (min(x, y) = y < x ? y : x)."""
+    box = np.stack([nodes[k] for k in ("minX", "maxX", "minY", "maxY", "minZ", "maxZ")], 1)
+    order, stack = [], [0]
+    while stack:
+        i = stack.pop()
+        if i < n - 1:
+            order.append(i)
+            stack += [int(nodes["left"][i]), int(nodes["right"][i])]
+    for i in reversed(order):
+        a, b = box[nodes["left"][i]], box[nodes["right"][i]]
+        box[i, 0::2] = np.where(b[0::2] < a[0::2], b[0::2], a[0::2])
+        box[i, 1::2] = np.where(a[1::2] < b[1::2], b[1::2], a[1::2])
+    return box
+
+
+@pytest.mark.parametrize("vertex", ["v0", "v1"])
+@pytest.mark.parametrize("n", [300, 9000])
+def test_nan_vertices(ctx, native, n, vertex):
+    """NaN planes: unions in the tree's own order (the rule is not associative then), and the launch still runs."""
+    tris = _tris(n, 64)
+    tris[vertex][5::n // 4, 0] = np.nan
+    sid = ctx.upload(tris, None, MATS, flags=native.BUILD_KEEP_BINARY)
+    nodes = ctx.nodes(sid)
+    box = np.stack([nodes[k] for k in ("minX", "maxX", "minY", "maxY", "minZ", "maxZ")], 1)
+    want = _tree_unions(nodes, n)
+    assert np.array_equal(np.isnan(box), np.isnan(want)) and np.array_equal(np.nan_to_num(box), np.nan_to_num(want))
+    assert np.any(np.isnan(box)) == (vertex == "v0")
+    rays = W.incoherent_rays(2000, [-1, -1, -1], [1, 1, 1], seed=65)
+    assert np.any(gpu_trace(ctx, sid, rays)["prim"] != L.NO_HIT)
+    ctx.release(sid)
