@@ -9,10 +9,13 @@
 // leaf slot (LeafRecord).  The reference's single-workgroup reduction and sort
 // are replaced by device-wide kernels.
 #include <algorithm>
+#include <atomic>
 #include <cmath>
 #include <cstddef>
 #include <cstring>
 #include <limits>
+#include <system_error>
+#include <thread>
 #include <vector>
 
 #include "rt_internal.hpp"
@@ -36,17 +39,19 @@ inline uint32_t grid_for(uint64_t n, int block = kB) {
 }
 
 // ModelSpaceToWorldSpace.comp:32-48: v' = M * vec4(v, 1) evaluated left to right
-__device__ inline void mat_vec1(const float *m, float *v) {
+__host__ __device__ inline void mat_vec1(const float *m, float *v) {
     float x = v[0], y = v[1], z = v[2];
     float r[4];
     for (int i = 0; i < 4; ++i) r[i] = m[0 + i] * x + m[4 + i] * y + m[8 + i] * z + m[12 + i] * 1.0f;
     v[0] = r[0]; v[1] = r[1]; v[2] = r[2]; v[3] = r[3];
 }
+// (a primitive with a model index out of range stays as it is; the build reports it)
 __global__ void k_model_to_world(rt_triangle *tris, uint32_t ntri, rt_sphere *sph, uint32_t nsph,
-                                 const float *models) {
+                                 const float *models, uint32_t nmodels) {
     uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
     if (i < ntri) {
         rt_triangle t = tris[i];
+        if (t.modelIndex >= nmodels) return;
         const float *m = models + 16u * t.modelIndex;
         mat_vec1(m, t.v0);
         mat_vec1(m, t.v1);
@@ -54,6 +59,7 @@ __global__ void k_model_to_world(rt_triangle *tris, uint32_t ntri, rt_sphere *sp
         tris[i] = t;
     } else if (i < ntri + nsph) {
         rt_sphere s = sph[i - ntri];
+        if (s.modelIndex >= nmodels) return;
         float c[4] = {s.center[0], s.center[1], s.center[2], s.center[3]};
         mat_vec1(models + 16u * s.modelIndex, c);  // radius stays unscaled
         s.center[0] = c[0]; s.center[1] = c[1]; s.center[2] = c[2]; s.center[3] = c[3];
@@ -943,14 +949,36 @@ __global__ void k_compress(const uint32_t *wide, uint32_t nwide, uint32_t *qwide
 }
 
 // the first level is the root; info: see build_scene
-__global__ void k_build_init(CollapseState *st, uint32_t *info) {
+__global__ void k_build_init(CollapseState *st, uint32_t *info, uint32_t all) {
     if (threadIdx.x == 0) *st = CollapseState{{0u, 0u}, {1u, 0u}, 0u, 0u};
-    if (threadIdx.x < 4) info[threadIdx.x] = 0u;
+    if (all && threadIdx.x < 6) info[threadIdx.x] = threadIdx.x < 4 ? 0u : 0xFFFFFFFFu;
 }
 
-template <class T> void upload(DevBuf &b, const T *src, size_t count) {
-    b.alloc(sizeof(T) * count);
-    if (count) RT_HIP(hipMemcpy(b.p, src, sizeof(T) * count, hipMemcpyHostToDevice));
+template <class T> void upload(rt_context *ctx, DevBuf &b, const T *src, size_t count) {
+    const size_t bytes = sizeof(T) * count;
+    b.alloc(bytes, &ctx->pool);
+    if (bytes >= HostStage::kMin) ctx->stage.copy(ctx->device, b.p, src, bytes);
+    else if (count) RT_HIP(hipMemcpy(b.p, src, bytes, hipMemcpyHostToDevice));
+}
+
+// The first primitive with an index out of range, as 2 * index + kind (0 material, 1 model): the smallest into
+// bad[0] for triangles and bad[1] for spheres.  One pass over the host's arrays took 1.2 ms for 1 M triangles.
+__global__ void k_check_indices(const rt_triangle *tris, uint32_t ntri, const rt_sphere *sph, uint32_t nsph, uint32_t nmat,
+                                uint32_t nmodels, uint32_t has_models, uint32_t *bad) {
+    const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
+    if (i >= ntri + nsph) return;
+    const bool tri = i < ntri;
+    const uint32_t k = tri ? i : i - ntri;
+    const uint32_t mat = tri ? tris[k].materialIndex : sph[k].materialIndex;
+    const uint32_t model = tri ? tris[k].modelIndex : sph[k].modelIndex;
+    if (mat >= nmat) atomicMin(&bad[tri ? 0 : 1], 2u * k);
+    else if (has_models && model >= nmodels) atomicMin(&bad[tri ? 0 : 1], 2u * k + 1u);
+}
+
+void throw_bad_index(const uint32_t *bad) {
+    for (int s = 0; s < 2; ++s)
+        RT_REQUIRE(bad[s] == 0xFFFFFFFFu, (s ? "sphere " : "triangle ") + std::to_string(bad[s] >> 1) +
+                                              ((bad[s] & 1u) ? ": modelIndex out of range" : ": materialIndex out of range"));
 }
 
 // Validate a caller-supplied binary node buffer and derive leaf slots and subtree ranges.
@@ -1009,10 +1037,41 @@ void validate_nodes(const rt_bvh_node *nodes, uint32_t n, uint32_t ntri, uint32_
 
 }  // namespace
 
+void HostStage::copy(int device, void *dst, const void *src, size_t bytes) {
+    const size_t chunks = (bytes + kChunk - 1) / kChunk;
+    std::atomic<size_t> next{0};
+    hipError_t status[kThreads] = {};
+    const auto work = [&](int id) {
+        hipError_t &e = status[id];
+        if ((e = hipSetDevice(device)) != hipSuccess) return;
+        for (int turn = 0;; turn ^= 1) {
+            const size_t c = next.fetch_add(1);
+            if (c >= chunks) return;
+            Buf &b = bufs_[id][turn];
+            if (!b.done && (e = hipEventCreateWithFlags(&b.done, hipEventDisableTiming)) != hipSuccess) return;
+            if (!b.host && (e = hipHostMalloc(&b.host, kChunk, hipHostMallocDefault)) != hipSuccess) return;
+            if (b.pending && (e = hipEventSynchronize(b.done)) != hipSuccess) return;
+            b.pending = false;
+            const size_t at = c * kChunk, len = std::min(kChunk, bytes - at);
+            std::memcpy(b.host, static_cast<const char *>(src) + at, len);
+            if ((e = hipMemcpyAsync(static_cast<char *>(dst) + at, b.host, len, hipMemcpyHostToDevice, nullptr)) != hipSuccess) return;
+            if ((e = hipEventRecord(b.done, nullptr)) != hipSuccess) return;
+            b.pending = true;
+        }
+    };
+    std::vector<std::thread> others;
+    try {
+        for (int id = 1; id < kThreads; ++id) others.emplace_back(work, id);
+    } catch (const std::system_error &) {  // fewer threads then: whoever runs takes the chunks
+    }
+    work(0);
+    for (std::thread &t : others) t.join();
+    for (hipError_t e : status) RT_HIP(e);
+}
+
 void build_scene(rt_context *ctx, Scene &sc, const rt_triangle *tris, uint32_t ntri, const rt_sphere *sph,
                  uint32_t nsph, const rt_material *mats, uint32_t nmat, const float *models, uint32_t nmodels,
                  const rt_bvh_node *nodes, uint32_t nnodes, const rt_build_options &opts) {
-    (void)ctx;
     const uint32_t W = opts.width ? opts.width : 4u;
     RT_REQUIRE(W == 2 || W == 4 || W == 8, "width must be 2, 4 or 8");
     uint32_t L = opts.leaf_size ? opts.leaf_size : 1u;
@@ -1024,21 +1083,13 @@ void build_scene(rt_context *ctx, Scene &sc, const rt_triangle *tris, uint32_t n
     RT_REQUIRE(nsph == 0 || sph, "spheres is NULL");
     RT_REQUIRE(nmat == 0 || mats, "materials is NULL");
     RT_REQUIRE(nmodels == 0 || models, "models is NULL");
-    for (uint32_t i = 0; i < ntri; ++i) {
-        RT_REQUIRE(tris[i].materialIndex < nmat, "triangle " + std::to_string(i) + ": materialIndex out of range");
-        RT_REQUIRE(!models || tris[i].modelIndex < nmodels,
-                   "triangle " + std::to_string(i) + ": modelIndex out of range");
-    }
-    for (uint32_t i = 0; i < nsph; ++i) {
-        RT_REQUIRE(sph[i].materialIndex < nmat, "sphere " + std::to_string(i) + ": materialIndex out of range");
-        RT_REQUIRE(!models || sph[i].modelIndex < nmodels, "sphere " + std::to_string(i) + ": modelIndex out of range");
-    }
-    if (nodes) RT_REQUIRE(n > 0 && nnodes == 2u * n - 1u, "node buffer must hold 2N-1 nodes");
+    const bool wrong_nodes = nodes && !(n > 0 && nnodes == 2u * n - 1u);  // reported after a bad index
 
     sc.ntri = ntri; sc.nsph = nsph; sc.nmat = nmat; sc.nprim = n;
     sc.width = W; sc.flags = opts.flags;
-    upload(sc.materials, mats, nmat);
+    upload(ctx, sc.materials, mats, nmat);
     if (n == 0) {
+        RT_REQUIRE(!wrong_nodes, "node buffer must hold 2N-1 nodes");
         sc.nwide = 0; sc.wide_depth = 0; sc.stack_bound = 0; sc.leaf_size = L;
         return;
     }
@@ -1047,30 +1098,32 @@ void build_scene(rt_context *ctx, Scene &sc, const rt_triangle *tris, uint32_t n
     RT_HIP(hipEventCreate(&ev0));
     RT_HIP(hipEventCreate(&ev1));
     DevBuf dtris, dsph, dmodels;
-    upload(dtris, tris, ntri);
-    upload(dsph, sph, nsph);
+    upload(ctx, dtris, tris, ntri);
+    upload(ctx, dsph, sph, nsph);
     RT_HIP(hipEventRecord(ev0, st));
     if (models) {
-        upload(dmodels, models, 16ull * nmodels);
+        upload(ctx, dmodels, models, 16ull * nmodels);
         k_model_to_world<<<grid_for(n), kB, 0, st>>>(dtris.as<rt_triangle>(), ntri, dsph.as<rt_sphere>(), nsph,
-                                                     dmodels.as<float>());
+                                                     dmodels.as<float>(), nmodels);
     }
     // centre-based u, v of every sphere (raytraceBVH.comp:172-173), from its world-space centre
     DevBuf duv;
     float min_radius = std::numeric_limits<float>::max();
     if (nsph) {
         std::vector<rt_sphere> world(sph, sph + nsph);
-        if (models) RT_HIP(hipMemcpy(world.data(), dsph.p, sizeof(rt_sphere) * nsph, hipMemcpyDeviceToHost));
+        if (models)  // as k_model_to_world, the same operations in the same order
+            for (rt_sphere &s : world)
+                if (s.modelIndex < nmodels) mat_vec1(models + 16u * s.modelIndex, s.center);
         std::vector<float2> uv(nsph);
         for (uint32_t i = 0; i < nsph; ++i) {
             sphere_uv(world[i].center, uv[i].x, uv[i].y);
             min_radius = std::fmin(min_radius, std::fabs(world[i].radius));
         }
-        upload(duv, uv.data(), nsph);
+        upload(ctx, duv, uv.data(), nsph);
     }
-    sc.slot_prim.alloc(sizeof(uint32_t) * n);
-    sc.slot_mat.alloc(sizeof(uint32_t) * n);
-    sc.records.alloc(sizeof(LeafRecord) * n);
+    sc.slot_prim.alloc(sizeof(uint32_t) * n, &ctx->pool);
+    sc.slot_mat.alloc(sizeof(uint32_t) * n, &ctx->pool);
+    sc.records.alloc(sizeof(LeafRecord) * n, &ctx->pool);
     // every temporary of the build from one block of the scratch cache
     const bool keep_binary = (opts.flags & RT_BUILD_KEEP_BINARY) != 0;
     const uint32_t max_nodes = std::max<uint32_t>(n - 1, 1);
@@ -1078,21 +1131,27 @@ void build_scene(rt_context *ctx, Scene &sc, const rt_triangle *tris, uint32_t n
         (keep_binary ? 0 : round256(sizeof(rt_bvh_node) * (2ull * n - 1))) + round256(sizeof(uint2) * max_nodes) +
         round256(24ull * kBoundsBlocks) + 2 * round256(4ull * n) + std::max(radix_temp_bytes(n), refit_temp_bytes(n)) +
         round256(32ull * W * max_nodes) + round256(4ull * max_nodes) + round256(4ull * W * max_nodes) +
-        round256(4ull * kCollapseBlocks) + round256(sizeof(CollapseState)) + round256(16);
+        round256(4ull * kCollapseBlocks) + round256(sizeof(CollapseState)) + round256(24);
     Temps tmp(ctx, temp_bytes, st);
     DevBuf kept;  // the binary nodes, when they stay resident
     rt_bvh_node *binary = nullptr;
     if (keep_binary) {
-        kept.alloc(sizeof(rt_bvh_node) * (2ull * n - 1));
+        kept.alloc(sizeof(rt_bvh_node) * (2ull * n - 1), &ctx->pool);
         binary = kept.as<rt_bvh_node>();
     } else {
         binary = tmp.take<rt_bvh_node>(2ull * n - 1);
     }
     uint2 *range = tmp.take<uint2>(max_nodes);
     CollapseState *state = tmp.take<CollapseState>(1);
-    uint32_t *info = tmp.take<uint32_t>(4);  // k_compress's three words, then k_leaves' NaN flag
-    k_build_init<<<1, 64, 0, st>>>(state, info);
+    uint32_t *info = tmp.take<uint32_t>(6);  // k_compress's three words, k_leaves' NaN flag, k_check_indices' two words
+    k_build_init<<<1, 64, 0, st>>>(state, info, 1u);
+    k_check_indices<<<grid_for(n), kB, 0, st>>>(dtris.as<rt_triangle>(), ntri, dsph.as<rt_sphere>(), nsph, nmat, nmodels,
+                                                models ? 1u : 0u, info + 4);
     if (nodes) {
+        uint32_t bad[2];
+        RT_HIP(hipMemcpy(bad, info + 4, sizeof bad, hipMemcpyDeviceToHost));
+        throw_bad_index(bad);
+        RT_REQUIRE(!wrong_nodes, "node buffer must hold 2N-1 nodes");
         std::vector<uint32_t> hslots;
         std::vector<uint2> hrange;
         validate_nodes(nodes, n, ntri, nsph, hslots, hrange, L);
@@ -1125,7 +1184,7 @@ void build_scene(rt_context *ctx, Scene &sc, const rt_triangle *tris, uint32_t n
     uint32_t *wide_tmp = tmp.take<uint32_t>(8ull * W * max_nodes);
     uint32_t *queue = tmp.take<uint32_t>(max_nodes), *chosen = tmp.take<uint32_t>((uint64_t)W * max_nodes);
     uint32_t *block_sums = tmp.take<uint32_t>(kCollapseBlocks);
-    struct { CollapseState state; uint32_t pad[58]; uint32_t info[4]; } out{};  // as the two lie in the temporaries
+    struct { CollapseState state; uint32_t pad[58]; uint32_t info[6]; } out{};  // as the two lie in the temporaries
     static_assert(sizeof(CollapseState) == 24 && offsetof(decltype(out), info) == 256, "state and info are read together");
     const auto collapse = [&] {
         if (n <= kSmallCollapse && !nodes) {
@@ -1149,13 +1208,14 @@ void build_scene(rt_context *ctx, Scene &sc, const rt_triangle *tris, uint32_t n
         } while (out.state.count[level & 1u] != 0u);
     };
     collapse();
+    throw_bad_index(out.info + 4);
     if (out.info[3] && n > 1) {  // NaN planes: unions in the tree's own order, then the collapse again
         DevBuf other(sizeof(rt_bvh_node) * (2ull * n - 1));
         for (int pass = 0; pass < 64; pass += 2) {
             k_refit_pass<<<grid_for(2ull * n - 1), kB, 0, st>>>(binary, other.as<rt_bvh_node>(), n);
             k_refit_pass<<<grid_for(2ull * n - 1), kB, 0, st>>>(other.as<rt_bvh_node>(), binary, n);
         }
-        k_build_init<<<1, 64, 0, st>>>(state, info);
+        k_build_init<<<1, 64, 0, st>>>(state, info, 0u);
         collapse();
         RT_HIP(hipStreamSynchronize(st));  // `other` is freed
     }
@@ -1171,11 +1231,11 @@ void build_scene(rt_context *ctx, Scene &sc, const rt_triangle *tris, uint32_t n
     (void)hipEventDestroy(ev1);
 
     sc.nwide = nwide;
-    sc.wide.alloc((size_t)sc.nwide * 32u * W);
+    sc.wide.alloc((size_t)sc.nwide * 32u * W, &ctx->pool);
     RT_HIP(hipMemcpy(sc.wide.p, wide_tmp, (size_t)sc.nwide * 32u * W, hipMemcpyDeviceToDevice));
     if (W == 4) {
-        sc.qwide.alloc((size_t)sc.nwide * 64u);
-        sc.slot_ref.alloc(sizeof(uint32_t) * n);
+        sc.qwide.alloc((size_t)sc.nwide * 64u, &ctx->pool);
+        sc.slot_ref.alloc(sizeof(uint32_t) * n, &ctx->pool);
         if (nodes)
             k_check_boxes<<<grid_for(2ull * n - 1), kB, 0, st>>>(binary, n, dtris.as<rt_triangle>(), dsph.as<rt_sphere>(),
                                                                  sc.slot_prim.as<uint32_t>(), info);

@@ -37,28 +37,101 @@ struct Error : std::runtime_error {
         if (!(cond)) throw ::rtgpu::Error(RT_ERR_INVALID, (msg));                                       \
     } while (0)
 
-// Owning device allocation.
+// Device memory of released scenes, kept for the next ones: hipMalloc and hipFree of a scene's buffers took 2 ms
+// of the 6.7 ms that a 1 M-triangle scene takes to come, answer a query and leave.  At most kKeep bytes stay,
+// the oldest given back first.  Used under the context's lock.  Whoever gives a block has waited for the
+// work that used it, except work of the null stream, on which every build that takes a block runs.
+class DevPool {
+  public:
+    static constexpr uint64_t kKeep = 1ull << 30;
+
+    DevPool() = default;
+    DevPool(const DevPool &) = delete;
+    DevPool &operator=(const DevPool &) = delete;
+    ~DevPool() { trim(0); }
+
+    // a block of at least `bytes`, its size in `cap`: sizes are rounded up to 4..7 times a power of two
+    void *take(size_t bytes, size_t &cap) {
+        cap = 4096;
+        while (cap * 2 < bytes) cap *= 2;
+        for (size_t step = cap / 4, c = cap; c <= 2 * cap; c += step)
+            if (c >= bytes) {
+                cap = c;
+                break;
+            }
+        for (size_t i = 0; i < free_.size(); ++i)
+            if (free_[i].second == cap) {
+                void *p = free_[i].first;
+                free_.erase(free_.begin() + (ptrdiff_t)i);
+                held_ -= cap;
+                return p;
+            }
+        void *p = nullptr;
+        hipError_t e = hipMalloc(&p, cap);
+        if (e == hipErrorOutOfMemory && !free_.empty()) {
+            trim(0);
+            e = hipMalloc(&p, cap);
+        }
+        RT_HIP(e);
+        return p;
+    }
+    void give(void *p, size_t cap) noexcept {
+        try {
+            free_.emplace_back(p, cap);
+        } catch (...) {
+            (void)hipFree(p);
+            return;
+        }
+        held_ += cap;
+        trim(kKeep);
+    }
+
+  private:
+    std::vector<std::pair<void *, size_t>> free_;  // oldest first
+    uint64_t held_ = 0;
+
+    void trim(uint64_t keep) noexcept {
+        size_t n = 0;
+        for (; n < free_.size() && held_ > keep; ++n) {
+            (void)hipFree(free_[n].first);
+            held_ -= free_[n].second;
+        }
+        free_.erase(free_.begin(), free_.begin() + (ptrdiff_t)n);
+    }
+};
+
+// Owning device allocation, from a pool or from hipMalloc.
 struct DevBuf {
     void *p = nullptr;
-    size_t bytes = 0;
+    size_t bytes = 0, cap = 0;
+    DevPool *pool = nullptr;
     DevBuf() = default;
-    explicit DevBuf(size_t n) { alloc(n); }
+    explicit DevBuf(size_t n, DevPool *from = nullptr) { alloc(n, from); }
     DevBuf(const DevBuf &) = delete;
     DevBuf &operator=(const DevBuf &) = delete;
-    DevBuf(DevBuf &&o) noexcept : p(o.p), bytes(o.bytes) { o.p = nullptr; o.bytes = 0; }
+    DevBuf(DevBuf &&o) noexcept { *this = std::move(o); }
     DevBuf &operator=(DevBuf &&o) noexcept {
-        if (this != &o) { release(); p = o.p; bytes = o.bytes; o.p = nullptr; o.bytes = 0; }
+        if (this != &o) {
+            release();
+            p = o.p; bytes = o.bytes; cap = o.cap; pool = o.pool;
+            o.p = nullptr; o.bytes = 0;
+        }
         return *this;
     }
     ~DevBuf() { release(); }
-    void alloc(size_t n) {
+    void alloc(size_t n, DevPool *from = nullptr) {
         release();
         if (n == 0) return;
-        RT_HIP(hipMalloc(&p, n));
+        pool = from;
+        if (pool) p = pool->take(n, cap);
+        else RT_HIP(hipMalloc(&p, n));
         bytes = n;
     }
     void release() {
-        if (p) (void)hipFree(p);
+        if (p) {
+            if (pool) pool->give(p, cap);
+            else (void)hipFree(p);
+        }
         p = nullptr;
         bytes = 0;
     }
@@ -73,6 +146,36 @@ struct LaunchCfg {
     uint32_t refill = 16;
     uint32_t leaf_weight = 2;  // leaf phase when leaf lanes * weight >= node lanes
     uint32_t shade_min = 24;   // render: shade when this many lanes hold a resolved segment
+};
+
+// Copies large host arrays to the device through pinned buffers that a few threads fill while the copies of
+// earlier chunks run: 64 MB of pageable memory in 1.5 ms, where hipMemcpy alone takes 3.0 (one thread fills its
+// staging memory).  The copies go to the null stream; the pinned memory stays with the context.
+class HostStage {
+    static constexpr int kThreads = 4;
+    static constexpr size_t kChunk = 1ull << 21;
+    struct Buf {
+        void *host = nullptr;
+        hipEvent_t done = nullptr;
+        bool pending = false;
+    };
+    Buf bufs_[kThreads][2];
+
+  public:
+    static constexpr size_t kMin = 8ull << 20;  // smaller arrays: hipMemcpy (8 MB 0.4 ms either way)
+
+    HostStage() = default;
+    HostStage(const HostStage &) = delete;
+    HostStage &operator=(const HostStage &) = delete;
+    ~HostStage() {
+        for (auto &t : bufs_)
+            for (Buf &b : t) {
+                if (b.pending) (void)hipEventSynchronize(b.done);
+                if (b.done) (void)hipEventDestroy(b.done);
+                if (b.host) (void)hipHostFree(b.host);
+            }
+    }
+    void copy(int device, void *dst, const void *src, size_t bytes);
 };
 
 // A scene resident in HBM.
@@ -321,6 +424,8 @@ struct rt_context {
     int device = 0;
     std::string last_error;
     uint32_t next_scene = 1;
+    rtgpu::DevPool pool;      // scenes' memory; outlives them
+    rtgpu::HostStage stage;  // pinned memory for large uploads
     std::map<uint32_t, std::unique_ptr<rtgpu::Scene>> scenes;
     int num_cus = 256;
     // small device area for per-launch work counters (one slot per launch, round robin)
@@ -390,8 +495,8 @@ struct rt_context {
 namespace rtgpu {
 
 inline void Scene::note_use(hipStream_t stream, int recorded) {
-    if (recorded == rt_context::kUseCaptured) return;
-    if (recorded == rt_context::kUseUnrecorded) {
+    // a graph may still run when the scene is released, and its memory then goes to the next scene
+    if (recorded == rt_context::kUseCaptured || recorded == rt_context::kUseUnrecorded) {
         unmarked_use = true;
         return;
     }

@@ -171,7 +171,9 @@ int rt_autotune_build(rt_context *ctx, const rt_tune_scene *scenes, uint32_t nsc
         for (uint32_t width : {2u, 4u, 8u})
             for (uint32_t leaf : {1u, 2u, 4u}) {
                 const rt_build_options opts{0u, width, leaf, 0u};
-                std::vector<std::unique_ptr<Scene>> built;
+                struct Built : std::vector<std::unique_ptr<Scene>> {
+                    ~Built() { (void)hipDeviceSynchronize(); }  // their memory goes back to the pool next
+                } built;
                 std::vector<TraceItem> items;
                 float build_ms = 0.0f;
                 uint64_t bytes = 0;
@@ -190,7 +192,6 @@ int rt_autotune_build(rt_context *ctx, const rt_tune_scene *scenes, uint32_t nsc
                 const Best b = search(timer, launch_space(bound, false, false), [&](const LaunchCfg &c, hipStream_t st) {
                     launch_trace_items(ctx, items, flags, c, st);
                 });
-                RT_HIP(hipStreamSynchronize(timer.stream()));  // the trees are freed next
                 cands.push_back(rt_build_candidate{width, leaf, build_ms, b.ms, to_abi(b.cfg), bytes});
             }
         std::stable_sort(cands.begin(), cands.end(),

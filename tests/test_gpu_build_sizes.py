@@ -103,3 +103,51 @@ def test_nan_vertices(ctx, native, n, vertex):
     rays = W.incoherent_rays(2000, [-1, -1, -1], [1, 1, 1], seed=65)
     assert np.any(gpu_trace(ctx, sid, rays)["prim"] != L.NO_HIT)
     ctx.release(sid)
+
+
+@pytest.mark.parametrize("n", [50, 140_000])  # one copy, and staged in chunks by several threads
+@pytest.mark.parametrize("what", ["material", "model", "sphere material", "sphere model", "first of several"])
+def test_bad_indices_are_refused(ctx, native, n, what):
+    tris, sph = _tris(n, 66), with_spheres(_tris(50), MATS, 5)
+    models = np.tile(np.eye(4, dtype=np.float32).reshape(1, 16), (2, 1))
+    if what == "material":
+        tris["materialIndex"][n - 7] = 1
+        said = f"triangle {n - 7}: materialIndex out of range"
+    elif what == "model":
+        tris["modelIndex"][n // 2] = 2
+        said = f"triangle {n // 2}: modelIndex out of range"
+    elif what == "sphere material":
+        sph["materialIndex"][3] = 0xFFFFFFFF
+        said = "sphere 3: materialIndex out of range"
+    elif what == "sphere model":
+        sph["modelIndex"][2] = 7
+        said = "sphere 2: modelIndex out of range"
+    else:
+        sph["modelIndex"][0] = 7
+        tris["modelIndex"][n // 3], tris["materialIndex"][n // 3], tris["materialIndex"][n // 3 + 1:] = 9, 9, 9
+        said = f"triangle {n // 3}: materialIndex out of range"
+    with pytest.raises(native.RTError, match=said) as e:
+        ctx.upload(tris, sph, MATS, models=models)
+    assert e.value.status == 1
+    tris, sph = _tris(n, 66), with_spheres(_tris(50), MATS, 5)
+    ctx.release(ctx.upload(tris, sph, MATS, models=models))
+
+
+def test_memory_of_released_scenes_is_reused_safely(ctx, native):
+    """Scenes of changing sizes come and go while queries on another stream still read the last one."""
+    stream = native.Stream()
+    want = {}
+    rays = W.incoherent_rays(300_000, [-1.2] * 3, [1.2] * 3, seed=67)
+    dr = native.DeviceArray.from_numpy(rays)
+    outs = []
+    for k in range(12):
+        n = (3000, 90_000, 3001, 200_000)[k % 4]
+        sid = ctx.upload(_tris(n, 68 + k % 4), None, MATS)
+        dh = native.DeviceArray(16 * len(rays))
+        ctx.trace(sid, dr, len(rays), dh, stream=stream)
+        ctx.release(sid)
+        outs.append((k % 4, dh))
+    stream.synchronize()
+    for k, dh in outs:
+        got = dh.to_numpy(np.uint32)
+        assert np.array_equal(want.setdefault(k, got), got)
