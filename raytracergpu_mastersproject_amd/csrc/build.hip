@@ -164,24 +164,19 @@ __global__ __launch_bounds__(kB) void k_morton(const rt_triangle *tris, uint32_t
     vals[i] = i;
 }
 
-// ---------------------------------------------------------------------------
-// Exclusive scan of u32 (one block, or device-wide and recursive over 2048-element blocks)
-// ---------------------------------------------------------------------------
-constexpr int kScanItems = 8;
-constexpr int kScanTile = kB * kScanItems;
-
-__device__ inline uint32_t block_exclusive_scan(uint32_t v, uint32_t *total) {
-    __shared__ uint32_t wsum[kB / 64];
-    int lane = threadIdx.x % 64, wave = threadIdx.x / 64;
+// exclusive sum of v over the block's threads, and the block's total
+template <int THREADS> __device__ inline uint32_t block_exclusive_scan(uint32_t v, uint32_t *total) {
+    __shared__ uint32_t wsum[THREADS / 64];
+    const int lane = threadIdx.x % 64, wave = threadIdx.x / 64;
     uint32_t x = v;
     for (int off = 1; off < 64; off <<= 1) {
-        uint32_t y = (uint32_t)__shfl_up((int)x, off);
+        const uint32_t y = (uint32_t)__shfl_up((int)x, off);
         if (lane >= off) x += y;
     }
     if (lane == 63) wsum[wave] = x;
     __syncthreads();
     uint32_t base = 0, all = 0;
-    for (int w = 0; w < kB / 64; ++w) {
+    for (int w = 0; w < THREADS / 64; ++w) {
         if (w < wave) base += wsum[w];
         all += wsum[w];
     }
@@ -190,58 +185,6 @@ __device__ inline uint32_t block_exclusive_scan(uint32_t v, uint32_t *total) {
     return base + x - v;
 }
 
-__global__ void k_scan_block(const uint32_t *in, uint32_t *out, uint32_t n, uint32_t *block_sums) {
-    uint64_t base = (uint64_t)blockIdx.x * kScanTile + (uint64_t)threadIdx.x * kScanItems;
-    uint32_t v[kScanItems], s = 0;
-    for (int k = 0; k < kScanItems; ++k) {
-        v[k] = (base + k < n) ? in[base + k] : 0u;
-        s += v[k];
-    }
-    uint32_t tot;
-    uint32_t pre = block_exclusive_scan(s, &tot);
-    for (int k = 0; k < kScanItems; ++k) {
-        if (base + k < n) out[base + k] = pre;
-        pre += v[k];
-    }
-    if (threadIdx.x == 0) block_sums[blockIdx.x] = tot;
-}
-// one block over up to kScanOne elements, in tiles of 8,192
-constexpr uint32_t kScanOne = 1u << 17;
-__global__ __launch_bounds__(1024) void k_scan_one(const uint32_t *in, uint32_t *out, uint32_t n) {
-    __shared__ uint32_t wsum[2][16];
-    const uint32_t lane = threadIdx.x % 64u, wave = threadIdx.x / 64u;
-    uint32_t run = 0;
-    for (uint32_t t0 = 0, phase = 0; t0 < n; t0 += 8192u, phase ^= 1u) {
-        const uint32_t base = t0 + threadIdx.x * 8u;
-        uint32_t v[8], s = 0;
-        for (int k = 0; k < 8; ++k) {
-            v[k] = base + k < n ? in[base + k] : 0u;
-            s += v[k];
-        }
-        uint32_t x = s;
-        for (int off = 1; off < 64; off <<= 1) {
-            const uint32_t y = (uint32_t)__shfl_up((int)x, off);
-            if (lane >= (uint32_t)off) x += y;
-        }
-        if (lane == 63u) wsum[phase][wave] = x;
-        __syncthreads();  // the other phase's sums are read before the next tile's barrier, so two sets suffice
-        uint32_t pre = run + x - s;
-        for (uint32_t w = 0; w < 16u; ++w) {
-            if (w < wave) pre += wsum[phase][w];
-            run += wsum[phase][w];
-        }
-        for (int k = 0; k < 8; ++k) {
-            if (base + k < n) out[base + k] = pre;
-            pre += v[k];
-        }
-    }
-}
-__global__ void k_scan_add(uint32_t *out, uint32_t n, const uint32_t *block_offsets) {
-    uint64_t i = (uint64_t)blockIdx.x * kScanTile + threadIdx.x;
-    uint32_t add = block_offsets[blockIdx.x];
-    for (int k = 0; k < kScanItems; ++k, i += kB)
-        if (i < n) out[i] += add;
-}
 // Temporaries of one build, carved from one block of the context's scratch cache.  Every
 // launch of a build is on one stream, so a range can be handed out again as soon as the
 // launches using it have been enqueued (mark / release); the block itself returns to the
@@ -266,30 +209,10 @@ class Temps {
 
 uint64_t round256(uint64_t b) { return (b + 255u) & ~uint64_t(255); }
 
-// bytes exclusive_scan takes from Temps for n elements
-uint64_t scan_temp_bytes(uint64_t n) {
-    const uint64_t nb = (n + kScanTile - 1) / kScanTile;
-    return n <= kScanOne ? 0 : 2 * round256(4 * nb) + scan_temp_bytes(nb);
-}
-
-void exclusive_scan(const uint32_t *in, uint32_t *out, uint32_t n, hipStream_t st, Temps &tmp) {
-    if (n <= kScanOne) {
-        k_scan_one<<<1, 1024, 0, st>>>(in, out, n);
-        return;
-    }
-    const uint32_t nb = (n + kScanTile - 1) / kScanTile;
-    const uint64_t m = tmp.mark();
-    uint32_t *sums = tmp.take<uint32_t>(nb), *sums_scan = tmp.take<uint32_t>(nb);
-    k_scan_block<<<nb, kB, 0, st>>>(in, out, n, sums);
-    exclusive_scan(sums, sums_scan, nb, st, tmp);
-    k_scan_add<<<nb, kB, 0, st>>>(out, n, sums_scan);
-    tmp.release(m);
-}
-
 // ---------------------------------------------------------------------------
 // Stable LSD radix sort, 4 passes x 8 bits (RadixSortSimple.comp's intent, A14):
-// per-tile digit histograms -> digit-major exclusive scan -> stable scatter in
-// which each round ranks 256 keys with wave ballots (keys keep tile order).
+// per-tile digit histograms -> exclusive scan of each digit's row of tiles -> stable
+// scatter in which each round ranks 256 keys with wave ballots (keys keep tile order).
 // ---------------------------------------------------------------------------
 constexpr int kSortItems = 8;
 constexpr int kSortTile = kB * kSortItems;
@@ -307,13 +230,39 @@ __global__ void k_radix_hist(const uint32_t *keys, uint32_t n, uint32_t shift, u
     ghist[(uint64_t)threadIdx.x * nblocks + blockIdx.x] = h[threadIdx.x];
 }
 
-__global__ void k_radix_scatter(const uint32_t *keys_in, const uint32_t *vals_in, uint32_t *keys_out,
-                                uint32_t *vals_out, uint32_t n, uint32_t shift, const uint32_t *goff,
-                                uint32_t nblocks) {
+// One block per digit: its tiles' counts -> the sums of the tiles before, and the digit's total.  The scatter adds
+// the smaller digits' totals itself.  A block's row is read in tiles of 2,048, so 1 M keys (489 tiles of keys) take
+// 5 us; one block over all 125,000 counts took 117 us, most of a 1 M-key sort.
+__global__ __launch_bounds__(kB) void k_radix_scan(const uint32_t *hist, uint32_t nblocks, uint32_t *before, uint32_t *totals) {
+    const uint32_t *in = hist + (uint64_t)blockIdx.x * nblocks;
+    uint32_t *out = before + (uint64_t)blockIdx.x * nblocks;
+    uint32_t run = 0;
+    for (uint32_t t0 = 0; t0 < nblocks; t0 += kB * 8u) {
+        const uint32_t base = t0 + threadIdx.x * 8u;
+        uint32_t v[8], s = 0, total;
+        for (int k = 0; k < 8; ++k) {
+            v[k] = base + k < nblocks ? in[base + k] : 0u;
+            s += v[k];
+        }
+        uint32_t pre = run + block_exclusive_scan<kB>(s, &total);
+        for (int k = 0; k < 8; ++k) {
+            if (base + k < nblocks) out[base + k] = pre;
+            pre += v[k];
+        }
+        run += total;
+    }
+    if (threadIdx.x == 0) totals[blockIdx.x] = run;
+}
+
+__global__ __launch_bounds__(kB) void k_radix_scatter(const uint32_t *keys_in, const uint32_t *vals_in, uint32_t *keys_out,
+                                                      uint32_t *vals_out, uint32_t n, uint32_t shift,
+                                                      const uint32_t *before, const uint32_t *totals, uint32_t nblocks) {
+    static_assert(kB == 256, "a thread per digit");
     __shared__ uint32_t off[256];
     __shared__ uint32_t cnt[kB / 64][256];
     const int tid = threadIdx.x, lane = tid % 64, wave = tid / 64;
-    off[tid] = goff[(uint64_t)tid * nblocks + blockIdx.x];
+    uint32_t all;
+    off[tid] = block_exclusive_scan<kB>(totals[tid], &all) + before[(uint64_t)tid * nblocks + blockIdx.x];
     const unsigned long long lt = (lane == 0) ? 0ull : ((~0ull) >> (64 - lane));
     uint64_t base = (uint64_t)blockIdx.x * kSortTile;
     for (int r = 0; r < kSortItems; ++r) {
@@ -346,62 +295,63 @@ __global__ void k_radix_scatter(const uint32_t *keys_in, const uint32_t *vals_in
     }
 }
 
-uint64_t radix_temp_bytes(uint64_t n) {
+uint64_t sort_temp_bytes(uint64_t n) {
     const uint64_t nblocks = (n + kSortTile - 1) / kSortTile;
-    return 2 * round256(4 * n) + 2 * round256(4 * 256 * nblocks) + scan_temp_bytes(256 * nblocks);
+    return 2 * round256(4 * n) + 2 * round256(4 * 256 * nblocks) + round256(4 * 256);
 }
 
-// The whole sort of few keys in one block: a bitonic network over (key, value) pairs in LDS.  The values are
-// the keys' original places, so equal keys keep their order and the result is the stable sort's.  4,096
-// keys in one launch, against twelve or more of the multi-block passes.
-constexpr uint32_t kSmallSort = 4096;
+// Few keys: each finds its place in the sorted order by counting the keys before it, the smaller ones and
+// the equal ones of smaller index.  A block ranks 64 keys, one per lane; each of its 16 waves counts over a sixteenth of
+// the keys, which it reads as scalars.  n^2 comparisons at two instructions each, but one launch and no
+// dependent passes.  A build of 4,096 triangles takes 90 us with it and 140 with the passes, of 16,384 131 and 164, of
+// 32,768 183 and 169: the line lies between.
+constexpr uint32_t kRankSort = 16384;
 
-__global__ __launch_bounds__(1024) void k_sort_small(uint32_t *keys, uint32_t *vals, uint32_t n, uint32_t padded) {
-    __shared__ uint64_t k[kSmallSort];
-    for (uint32_t i = threadIdx.x; i < padded; i += blockDim.x)
-        k[i] = i < n ? ((uint64_t)keys[i] << 32) | vals[i] : ~0ull;
-    for (uint32_t size = 2; size <= padded; size <<= 1)
-        for (uint32_t stride = size >> 1; stride > 0; stride >>= 1) {
-            __syncthreads();
-            for (uint32_t t = threadIdx.x; t < padded / 2; t += blockDim.x) {
-                const uint32_t i = 2u * t - (t & (stride - 1u)), j = i + stride;
-                const uint64_t a = k[i], b = k[j];
-                if ((a > b) == ((i & size) == 0u)) {
-                    k[i] = b;
-                    k[j] = a;
-                }
-            }
-        }
+__global__ __launch_bounds__(1024) void k_rank_sort(const uint32_t *__restrict__ keys, const uint32_t *__restrict__ vals,
+                                                    uint32_t n, uint32_t *__restrict__ keys_out,
+                                                    uint32_t *__restrict__ vals_out) {
+    __shared__ uint32_t part[16][64];
+    const uint32_t lane = threadIdx.x % 64u, wave = __builtin_amdgcn_readfirstlane(threadIdx.x / 64u);
+    const uint32_t first = blockIdx.x * 64u, i = first + lane;
+    const uint32_t key = i < n ? keys[i] : 0u;  // Morton codes have 30 bits: key + 1 does not wrap
+    const uint32_t chunk = (n + 15u) / 16u, lo = min(wave * chunk, n), hi = min(lo + chunk, n);
+    // keys before this block's: also the equal ones are before; keys after it: only the smaller ones
+    const uint32_t a = min(max(first, lo), hi), b = min(max(first + 64u, lo), hi);
+    uint32_t rank = 0;
+#pragma unroll 8
+    for (uint32_t j = lo; j < a; ++j) rank += keys[j] <= key ? 1u : 0u;
+    for (uint32_t j = a; j < b; ++j) rank += keys[j] < key + (j < i ? 1u : 0u) ? 1u : 0u;
+#pragma unroll 8
+    for (uint32_t j = b; j < hi; ++j) rank += keys[j] < key ? 1u : 0u;
+    part[wave][lane] = rank;
     __syncthreads();
-    for (uint32_t i = threadIdx.x; i < n; i += blockDim.x) {
-        keys[i] = (uint32_t)(k[i] >> 32);
-        vals[i] = (uint32_t)k[i];
+    if (wave == 0u && i < n) {
+        for (uint32_t w = 1; w < 16u; ++w) rank += part[w][lane];
+        keys_out[rank] = key;
+        vals_out[rank] = vals[i];
     }
 }
 
-// vals: 0..n-1 in order
-void radix_sort(uint32_t *keys, uint32_t *vals, uint32_t n, hipStream_t st, Temps &tmp) {
+// Sorts keys, and vals with them; the two pointers are then the result's, in the given arrays or in `tmp`.
+void sort_pairs(uint32_t *&keys, uint32_t *&vals, uint32_t n, hipStream_t st, Temps &tmp) {
     if (n <= 1) return;
-    if (n <= kSmallSort) {
-        uint32_t padded = 2;
-        while (padded < n) padded <<= 1;
-        k_sort_small<<<1, std::min(1024u, std::max(64u, padded / 2)), 0, st>>>(keys, vals, n, padded);
+    uint32_t *k2 = tmp.take<uint32_t>(n), *v2 = tmp.take<uint32_t>(n);
+    if (n <= kRankSort) {
+        k_rank_sort<<<(n + 63u) / 64u, 1024, 0, st>>>(keys, vals, n, k2, v2);
+        keys = k2;
+        vals = v2;
         return;
     }
-    uint32_t nblocks = (n + kSortTile - 1) / kSortTile;
-    const uint64_t m = tmp.mark();
-    uint32_t *k2 = tmp.take<uint32_t>(n), *v2 = tmp.take<uint32_t>(n);
-    uint32_t *hist = tmp.take<uint32_t>(256ull * nblocks), *hoff = tmp.take<uint32_t>(256ull * nblocks);
-    uint32_t *ka = keys, *va = vals, *kb = k2, *vb = v2;
-    for (int pass = 0; pass < 4; ++pass) {  // an even number of passes: the result is back in keys/vals
-        uint32_t shift = 8u * pass;
-        k_radix_hist<<<nblocks, kB, 0, st>>>(ka, n, shift, hist, nblocks);
-        exclusive_scan(hist, hoff, 256u * nblocks, st, tmp);
-        k_radix_scatter<<<nblocks, kB, 0, st>>>(ka, va, kb, vb, n, shift, hoff, nblocks);
-        std::swap(ka, kb);
-        std::swap(va, vb);
+    const uint32_t nblocks = (n + kSortTile - 1) / kSortTile;
+    uint32_t *hist = tmp.take<uint32_t>(256ull * nblocks), *before = tmp.take<uint32_t>(256ull * nblocks);
+    uint32_t *totals = tmp.take<uint32_t>(256);
+    for (uint32_t shift = 0; shift < 32u; shift += 8u) {
+        k_radix_hist<<<nblocks, kB, 0, st>>>(keys, n, shift, hist, nblocks);
+        k_radix_scan<<<256, kB, 0, st>>>(hist, nblocks, before, totals);
+        k_radix_scatter<<<nblocks, kB, 0, st>>>(keys, vals, k2, v2, n, shift, before, totals, nblocks);
+        std::swap(keys, k2);
+        std::swap(vals, v2);
     }
-    tmp.release(m);
 }
 
 // ---------------------------------------------------------------------------
@@ -637,10 +587,10 @@ void refit(rt_bvh_node *nodes, const uint2 *range, uint32_t n, hipStream_t st, T
 // largest surface area until W children exist; a child whose subtree holds at
 // most leaf_size primitives becomes a leaf over its contiguous slot range.
 //
-// Wide nodes are numbered in queue order: queue[i] is the binary node of wide node i, and a level's nodes are
-// consecutive.  Level sizes stay on the device (CollapseState), so levels are launched ahead without
-// the host reading each one; a launch past the last level finds an empty one.  A level takes two launches
-// (choose children and count; number and write), a small tree one launch in all.
+// Three steps: every binary node's choice of children (k_collapse_choose, all at once), the numbering of the wide
+// nodes level by level (k_collapse_levels), which then only follows the choices, and the wide nodes themselves
+// with their compressed copies (k_collapse_emit, all at once).  Wide nodes are numbered in queue order: queue[i] is the
+// binary node of wide node i, a level's nodes are consecutive, and first[i] is the number of node i's first node child.
 struct CollapseArgs {
     const rt_bvh_node *nodes;
     const uint2 *range;  // internal nodes: leaf-slot range of the subtree
@@ -661,216 +611,194 @@ __device__ inline float box_area(const rt_bvh_node &nd) {
     return dx * dy + dy * dz + dz * dx;
 }
 
-__device__ int choose_children(const CollapseArgs &a, uint32_t b, uint32_t *cand) {
-    int nc;
-    if (!is_internal(a, b)) {
-        cand[0] = b;
-        return 1;
-    }
-    cand[0] = a.nodes[b].left;
-    cand[1] = a.nodes[b].right;
-    nc = 2;
-    while (nc < (int)a.width) {
-        int best = -1;
-        float best_area = -1.0f;
-        for (int k = 0; k < nc; ++k) {
-            uint32_t c = cand[k];
-            if (!is_internal(a, c) || subtree_count(a, c) <= a.leaf_size) continue;
-            float ar = box_area(a.nodes[c]);
-            if (ar > best_area) { best_area = ar; best = k; }
-        }
-        if (best < 0) break;
-        uint32_t c = cand[best];
-        for (int k = nc; k > best + 1; --k) cand[k] = cand[k - 1];
-        cand[best] = a.nodes[c].left;
-        cand[best + 1] = a.nodes[c].right;
-        ++nc;
-    }
-    return nc;
-}
-
 __device__ inline bool becomes_node(const CollapseArgs &a, uint32_t c) {
     return is_internal(a, c) && subtree_count(a, c) > a.leaf_size;
 }
 
-// [level & 1]: the level's first wide node and its size; the other entry receives the next level's
+// chosen[W * b + k]: binary node b's children in a wide node (kEmpty behind the last); mask[b]: bit k is set when child k
+// becomes a node itself.  Nodes that never become one (subtrees of at most leaf_size) are left out.
+template <int W>
+__global__ __launch_bounds__(kB) void k_collapse_choose(CollapseArgs a, uint32_t *chosen, uint8_t *mask) {
+    const uint32_t b = blockIdx.x * kB + threadIdx.x;
+    if (b >= max(a.n - 1u, 1u) || (b != 0u && !becomes_node(a, b))) return;
+    uint32_t cand[W], l[W], r[W];  // child, its own children
+    float area[W];                 // -1 when it cannot be opened
+    int nc = 1;
+    const auto load = [&](uint32_t c, uint32_t &id, uint32_t &left, uint32_t &right, float &ar) {
+        const rt_bvh_node nd = a.nodes[c];
+        id = c;
+        left = nd.left;
+        right = nd.right;
+        ar = becomes_node(a, c) ? box_area(nd) : -1.0f;
+    };
+#pragma unroll
+    for (int k = 0; k < W; ++k) cand[k] = kEmpty, l[k] = r[k] = 0u, area[k] = -1.0f;
+    if (!is_internal(a, b)) {
+        cand[0] = b;
+    } else {
+        const uint32_t bl = a.nodes[b].left, br = a.nodes[b].right;
+        load(bl, cand[0], l[0], r[0], area[0]);
+        load(br, cand[1], l[1], r[1], area[1]);
+        for (nc = 2; nc < W; ++nc) {
+            int best = -1;
+            float best_area = -1.0f;
+            uint32_t ol = 0, orr = 0;
+#pragma unroll
+            for (int k = 0; k < W; ++k)
+                if (area[k] > best_area) best_area = area[k], best = k, ol = l[k], orr = r[k];
+            if (best < 0) break;
+            // the two children take the opened one's place
+#pragma unroll
+            for (int k = W - 1; k > 0; --k)
+                if (k > best + 1) cand[k] = cand[k - 1], l[k] = l[k - 1], r[k] = r[k - 1], area[k] = area[k - 1];
+            uint32_t c0, l0, r0, c1, l1, r1;
+            float a0, a1;
+            load(ol, c0, l0, r0, a0);
+            load(orr, c1, l1, r1, a1);
+#pragma unroll
+            for (int k = 0; k < W; ++k) {
+                if (k == best) cand[k] = c0, l[k] = l0, r[k] = r0, area[k] = a0;
+                if (k == best + 1) cand[k] = c1, l[k] = l1, r[k] = r1, area[k] = a1;
+            }
+        }
+    }
+    uint32_t m = 0;
+#pragma unroll
+    for (int k = 0; k < W; ++k) {
+        if (cand[k] != kEmpty && becomes_node(a, cand[k])) m |= 1u << k;
+        chosen[(size_t)b * W + k] = cand[k];
+    }
+    mask[b] = (uint8_t)m;
+}
+
+// [launch & 1]: the first wide node and the size of the level that the launch begins with; the other entry receives the
+// next launch's.
 struct CollapseState {
     uint32_t base[2], count[2];
     uint32_t depth, bad;  // levels with nodes so far; 1 when a level would not fit
 };
 
-constexpr uint32_t kCollapseBlocks = 2048;  // at most, per launch
+constexpr uint32_t kLevelThreads = 1024;
+constexpr uint32_t kLevelBlocks = 1024;  // at most, per launch
 
-// the entries of the level that block `b` of `blocks` handles
-__device__ inline uint2 collapse_chunk(uint32_t count, uint32_t b, uint32_t blocks) {
-    const uint32_t chunk = ((count + blocks - 1u) / blocks + kB - 1u) / kB * kB;
-    return make_uint2(min(b * chunk, count), min(b * chunk + chunk, count));
+// A level is split into equal chunks, one per block; chunk sums are kept in three sets of kLevelBlocks words, by
+// launch % 3: of the node children of this level's chunks (complete), of the next level's (added up here), and the
+// one that the next launch adds to (cleared here).
+__device__ inline uint32_t collapse_chunk(uint32_t count) {
+    return ((count + kLevelBlocks - 1u) / kLevelBlocks + kLevelThreads - 1u) / kLevelThreads * kLevelThreads;
 }
 
-__device__ inline uint32_t child_nodes(const CollapseArgs &a, const uint32_t *cand, int nc) {
-    uint32_t k = 0;
-    for (int i = 0; i < nc; ++i) k += becomes_node(a, cand[i]) ? 1u : 0u;
-    return k;
-}
-
-// Writes wide node `node` of queue entry with children cand[0..nc); its node children are numbered from `j` on.
-__device__ inline void write_wide(const CollapseArgs &a, const uint32_t *cand, int nc, uint32_t node, uint32_t j,
-                                  uint32_t *queue, uint32_t *wide) {
-    const uint32_t W = a.width;
-    uint32_t *nd = wide + (size_t)node * 8u * W;
-    float *f = reinterpret_cast<float *>(nd);
-    const float inf = __uint_as_float(0x7F800000u);
-    for (uint32_t k = 0; k < W; ++k) {
-        float box[6] = {inf, inf, inf, inf, inf, inf};
-        uint32_t ce = kEmpty;
-        if ((int)k < nc) {
-            const uint32_t c = cand[k];
-            const rt_bvh_node bn = a.nodes[c];
-            box[0] = bn.minX; box[1] = bn.maxX;
-            box[2] = bn.minY; box[3] = bn.maxY;
-            box[4] = bn.minZ; box[5] = bn.maxZ;
-            if (becomes_node(a, c)) {
-                ce = j;
-                queue[j] = c;
-                ++j;
-            } else if (is_internal(a, c)) {
-                const uint2 r = a.range[c];
-                ce = leaf_entry(r.x, r.y - r.x + 1u);
-            } else {
-                ce = leaf_entry(c - (a.n - 1u), 1u);
-            }
-        }
-        for (int q = 0; q < 6; ++q) f[q * W + k] = box[q];
-        nd[6 * W + k] = ce;
-        nd[7 * W + k] = 0u;
-    }
-}
-
-// children of the level's entries -> chosen (8 words per entry), node children per block -> block_sums
-__global__ __launch_bounds__(kB) void k_collapse_choose(CollapseArgs a, uint32_t level, const CollapseState *st,
-                                                        const uint32_t *queue, uint32_t *chosen, uint32_t *block_sums) {
-    const uint32_t base = st->base[level & 1u];
-    const uint2 c = collapse_chunk(st->count[level & 1u], blockIdx.x, gridDim.x);
-    uint32_t sum = 0;
-    for (uint32_t e = c.x + threadIdx.x; e < c.y; e += kB) {
-        uint32_t cand[8];
-        const int nc = choose_children(a, level ? queue[base + e] : 0u, cand);  // level 0: the root
-        sum += child_nodes(a, cand, nc);
-        for (uint32_t k = 0; k < a.width; ++k) chosen[(size_t)e * a.width + k] = (int)k < nc ? cand[k] : kEmpty;
-    }
-    uint32_t total;
-    (void)block_exclusive_scan(sum, &total);
-    if (threadIdx.x == 0) block_sums[blockIdx.x] = total;
-}
-
-__global__ __launch_bounds__(kB) void k_collapse_emit(CollapseArgs a, uint32_t level, CollapseState *st, uint32_t *queue,
-                                                      const uint32_t *chosen, const uint32_t *block_sums, uint32_t *wide,
-                                                      uint32_t max_nodes) {
-    const uint32_t base = st->base[level & 1u], count = st->count[level & 1u];
-    if (count == 0u) {
-        if (blockIdx.x == 0 && threadIdx.x == 0) st->count[(level + 1u) & 1u] = 0u;
-        return;
-    }
-    const uint2 c = collapse_chunk(count, blockIdx.x, gridDim.x);
-    uint32_t before = 0, all = 0;  // node children of the earlier blocks, and of all
-    for (uint32_t b = threadIdx.x; b < gridDim.x; b += kB) {
-        const uint32_t v = block_sums[b];
-        all += v;
-        if (b < blockIdx.x) before += v;
-    }
-    uint32_t total_before, total;
-    (void)block_exclusive_scan(before, &total_before);
-    (void)block_exclusive_scan(all, &total);
-    if ((uint64_t)base + count + total > max_nodes) {  // cannot happen: a wide node is made from its own binary node
-        if (blockIdx.x == 0 && threadIdx.x == 0) { st->bad = 1u; st->count[(level + 1u) & 1u] = 0u; }
-        return;
-    }
-    uint32_t j0 = base + count + total_before;
-    for (uint32_t e0 = c.x; e0 < c.y; e0 += kB) {
-        const uint32_t e = e0 + threadIdx.x;
-        uint32_t cand[8], k = 0;
-        int nc = 0;
-        if (e < c.y) {
-            for (; nc < (int)a.width && chosen[(size_t)e * a.width + nc] != kEmpty; ++nc) cand[nc] = chosen[(size_t)e * a.width + nc];
-            k = child_nodes(a, cand, nc);
-        }
-        uint32_t tile;
-        const uint32_t pre = block_exclusive_scan(k, &tile);
-        if (e < c.y) write_wide(a, cand, nc, base + e, j0 + pre, queue, wide);
-        j0 += tile;
-    }
-    if (blockIdx.x == 0 && threadIdx.x == 0) {
-        st->base[(level + 1u) & 1u] = base + count;
-        st->count[(level + 1u) & 1u] = total;
-        st->depth = level + 1u;
-    }
-}
-
-// All levels of a small tree in one block.
-constexpr uint32_t kSmallCollapse = 16384;  // primitives
-__global__ __launch_bounds__(kB) void k_collapse_small(CollapseArgs a, CollapseState *st, uint32_t *queue, uint32_t *wide,
-                                                       uint32_t max_nodes) {
-    uint32_t base = 0, count = 1, level = 0;
-    if (threadIdx.x == 0) queue[0] = 0u;  // the root
-    for (; count > 0u; ++level) {
-        __syncthreads();  // the queue entries of this level are written
-        uint32_t j0 = base + count;
-        for (uint32_t e0 = 0; e0 < count; e0 += kB) {
+// The numbering of one level, or of as many as fit one block each (block 0 then goes through them in one
+// launch, a microsecond or two for each).  Levels are launched ahead without the host reading their sizes; a
+// launch past the last finds an empty one.  What bounds a level is its chain of dependent loads: queue entry ->
+// choice -> the children's masks.  1 M triangles: 0.10 ms in 11 launches, and 0.05 ms for the choices (before, with
+// the choices and the nodes inside the level launches: 0.47 ms in 42).
+template <int W>
+__global__ __launch_bounds__(kLevelThreads) void k_collapse_levels(uint32_t launch, CollapseState *st, uint32_t *queue,
+                                                                   uint32_t *first, const uint32_t *chosen,
+                                                                   const uint8_t *mask, uint32_t *sums,
+                                                                   uint32_t max_nodes) {
+    uint32_t base = st->base[launch & 1u], count = st->count[launch & 1u];
+    const uint32_t *now = sums + (launch % 3u) * kLevelBlocks;
+    uint32_t *next = sums + ((launch + 1u) % 3u) * kLevelBlocks, *later = sums + ((launch + 2u) % 3u) * kLevelBlocks;
+    if (blockIdx.x == 0) later[threadIdx.x] = 0u;
+    static_assert(kLevelBlocks == kLevelThreads, "a thread per chunk");
+    const auto number = [&](uint32_t lo, uint32_t hi, uint32_t j, uint32_t next_base, uint32_t next_chunk) {
+        for (uint32_t e0 = lo; e0 < hi; e0 += kLevelThreads) {
             const uint32_t e = e0 + threadIdx.x;
-            uint32_t cand[8], k = 0;
-            int nc = 0;
-            if (e < count) {
-                nc = choose_children(a, queue[base + e], cand);
-                k = child_nodes(a, cand, nc);
+            uint32_t m = 0, c[W];
+            if (e < hi) {
+                const uint32_t b = queue[base + e];
+                m = mask[b];
+                for (int k = 0; k < W; ++k) c[k] = chosen[(size_t)b * W + k];
             }
-            uint32_t tile;
-            const uint32_t pre = block_exclusive_scan(k, &tile);
-            if ((uint64_t)j0 + tile > max_nodes) {  // cannot happen, as above
-                if (threadIdx.x == 0) st->bad = 1u;
-                return;
+            uint32_t tile, at = j + block_exclusive_scan<kLevelThreads>((uint32_t)__popc(m), &tile);
+            j += tile;
+            if (j > max_nodes) return j;  // cannot happen: a wide node is made from its own binary node
+            // a wave's children lie in at most two chunks: their sums take two atomics instead of one a child, which
+            // would go to few addresses (175 us on a level of 70,000 nodes, against 11)
+            const uint32_t chunk0 = next_chunk ? (__builtin_amdgcn_readfirstlane(at) - next_base) / next_chunk : 0u;
+            const uint32_t split = next_base + (chunk0 + 1u) * next_chunk;
+            uint32_t below0 = 0, below1 = 0;
+            if (e < hi) {
+                first[base + e] = at;
+                for (int k = 0; k < W; ++k)
+                    if (m >> k & 1u) {
+                        queue[at] = c[k];
+                        if (next_chunk) (at < split ? below0 : below1) += (uint32_t)__popc((uint32_t)mask[c[k]]);
+                        ++at;
+                    }
             }
-            if (e < count) write_wide(a, cand, nc, base + e, j0 + pre, queue, wide);
-            j0 += tile;
+            if (next_chunk) {
+                for (int o = 1; o < 64; o <<= 1) {
+                    below0 += (uint32_t)__shfl_xor((int)below0, o);
+                    below1 += (uint32_t)__shfl_xor((int)below1, o);
+                }
+                if (threadIdx.x % 64u == 0u) {
+                    if (below0) atomicAdd(&next[chunk0], below0);
+                    if (below1) atomicAdd(&next[chunk0 + 1u], below1);
+                }
+            }
         }
-        const uint32_t next = base + count;
-        count = j0 - next;
-        base = next;
+        return j;
+    };
+    if (count <= kLevelThreads) {
+        if (blockIdx.x != 0) return;
+        uint32_t depth = st->depth;
+        for (; count > 0u && count <= kLevelThreads; ++depth) {
+            const uint32_t end = base + count, j = number(0, count, end, 0u, 0u);
+            if (j > max_nodes) {
+                if (threadIdx.x == 0) st->bad = 1u;
+                count = 0u;
+                base = end;
+                break;
+            }
+            __syncthreads();  // the next level's queue entries are written
+            base = end;
+            count = j - end;
+        }
+        const uint32_t chunk = collapse_chunk(count);
+        for (uint32_t e0 = 0; e0 < count; e0 += kLevelThreads) {  // chunk is a multiple of kLevelThreads
+            uint32_t sum;
+            const uint32_t e = e0 + threadIdx.x;
+            (void)block_exclusive_scan<kLevelThreads>(e < count ? (uint32_t)__popc((uint32_t)mask[queue[base + e]]) : 0u, &sum);
+            if (threadIdx.x == 0) atomicAdd(&next[e0 / chunk], sum);
+        }
+        if (threadIdx.x == 0) {
+            st->base[(launch + 1u) & 1u] = base;
+            st->count[(launch + 1u) & 1u] = count;
+            st->depth = depth;
+        }
+        return;
     }
-    if (threadIdx.x == 0) {
-        st->base[level & 1u] = base;
-        st->count[level & 1u] = 0u;
-        st->depth = level;
+    const uint32_t chunk = collapse_chunk(count), lo = min(blockIdx.x * chunk, count), hi = min(lo + chunk, count);
+    const uint32_t v = threadIdx.x * (uint64_t)chunk < count ? now[threadIdx.x] : 0u;
+    uint32_t total, before;
+    (void)block_exclusive_scan<kLevelThreads>(v, &total);
+    (void)block_exclusive_scan<kLevelThreads>(threadIdx.x < blockIdx.x ? v : 0u, &before);
+    const uint32_t end = base + count;
+    const bool bad = (uint64_t)end + total > max_nodes;  // cannot happen, as above
+    if (!bad && lo < hi) (void)number(lo, hi, end + before, end, collapse_chunk(total));
+    if (blockIdx.x == 0 && threadIdx.x == 0) {
+        if (bad) st->bad = 1u;
+        st->base[(launch + 1u) & 1u] = end;
+        st->count[(launch + 1u) & 1u] = bad ? 0u : total;
+        st->depth += 1u;
     }
 }
 
-// One axis of a compressed node (rt_device.hpp): lo, hi are the planes of its nc children.  False when a
-// plane is not finite or too large, or a box is inverted: its exact tests do not order the two planes.
-__device__ inline bool compress_axis(const float *lo, const float *hi, const uint32_t *child, float &org, float &scale,
-                                     uint32_t &qlo, uint32_t &qhi) {
-    float mn = 0x1p24f, mx = -0x1p24f;
-    bool ok = true;
-    for (int k = 0; k < 4; ++k)
-        if (child[k] != kEmpty) {
-            ok = ok && fabsf(lo[k]) < 0x1p24f && fabsf(hi[k]) < 0x1p24f && lo[k] <= hi[k];
-            mn = fminf(mn, lo[k]);
-            mx = fmaxf(mx, hi[k]);
-        }
-    qlo = qhi = 0u;
-    // 248 steps over the extent; a step is no finer than the origin's rounding, at most a quarter of it
-    scale = fmaxf(fmaxf((mx - mn) * (1.0f / 248.0f), 0x1p-22f * fmaxf(fabsf(mn), fabsf(mx))), 0x1p-100f);
-    org = (float)((double)mn - 1026.0 * (double)scale);
-    const double s = 1.0 / (double)scale;
-    for (int k = 0; k < 4; ++k) {
-        double l = 255.0, h = 0.0;
-        if (child[k] != kEmpty) {
-            l = floor(((double)lo[k] - (double)org) * s - (1024.0 + kPlaneMargin));
-            h = ceil(((double)hi[k] - (double)org) * s - (1024.0 - kPlaneMargin));
-            ok = ok && l >= 0.0 && h <= 255.0;
-        }
-        qlo |= ((uint32_t)l & 255u) << (8 * k);
-        qhi |= ((uint32_t)h & 255u) << (8 * k);
-    }
-    return ok;
+// min, max and bitwise or over the four lanes of a quad
+__device__ inline float quad_min(float x) {
+    x = fminf(x, __shfl_xor(x, 1, 4));
+    return fminf(x, __shfl_xor(x, 2, 4));
+}
+__device__ inline float quad_max(float x) {
+    x = fmaxf(x, __shfl_xor(x, 1, 4));
+    return fmaxf(x, __shfl_xor(x, 2, 4));
+}
+__device__ inline uint32_t quad_or(uint32_t x) {
+    x |= (uint32_t)__shfl_xor((int)x, 1, 4);
+    return x | (uint32_t)__shfl_xor((int)x, 2, 4);
 }
 
 // A caller's node buffer may hold any boxes; compressed nodes need every box to hold what is below it.
@@ -906,51 +834,93 @@ __global__ void k_check_boxes(const rt_bvh_node *nodes, uint32_t n, const rt_tri
     if (fail != 0ull && __lane_id() == (uint32_t)__ffsll((long long)fail) - 1u) *bad = 1u;
 }
 
-// Compressed copies of the width-4 nodes, and the node and child that hold each leaf slot.  info[0] = 1 when
-// some node cannot be compressed (one store per wave); info[1], info[2]: the scene's largest coordinate in
-// magnitude and its largest extent (the root's planes).
-__global__ void k_compress(const uint32_t *wide, uint32_t nwide, uint32_t *qwide, uint32_t *slot_ref, uint32_t *info) {
-    const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= nwide) return;
-    const uint32_t *nd = wide + (size_t)i * 32u;
-    const float *f = reinterpret_cast<const float *>(nd);
-    const uint4 ch = reinterpret_cast<const uint4 *>(nd)[6];
-    const uint32_t child[4] = {ch.x, ch.y, ch.z, ch.w};
-    float org[3], scale[3];
-    uint32_t lo[3], hi[3];
+// Writes the wide nodes, a lane per child, and of width-4 ones (qwide non-null) the compressed copies (rt_device.hpp) and the
+// node and child that hold each leaf slot.  info[0] = 1 when some node cannot be compressed, because a plane
+// is not finite or too large or a box is inverted: its exact tests do not order the two planes (one store per
+// wave); info[1], info[2]: the scene's largest coordinate in magnitude and its largest extent (the root's planes).
+// 330,000 nodes in 43 us (42 MB and 21 MB written); writing them by level, copying them and compressing the copies took
+// 16 us for the copy and 69 us for the compression alone.
+template <int W>
+__global__ __launch_bounds__(kB) void k_collapse_emit(CollapseArgs a, uint32_t nwide, const uint32_t *queue,
+                                                      const uint32_t *first, const uint32_t *chosen, const uint8_t *mask,
+                                                      uint32_t *wide, uint32_t *qwide, uint32_t *slot_ref,
+                                                      uint32_t *info) {
+    const uint64_t t = (uint64_t)blockIdx.x * kB + threadIdx.x;
+    const uint32_t node = (uint32_t)(t / W), k = (uint32_t)(t % W);
+    if (t / W >= nwide) return;
+    const uint32_t b = queue[node], c = chosen[(size_t)b * W + k], m = mask[b];
+    const float inf = __uint_as_float(0x7F800000u);
+    float lo[3] = {inf, inf, inf}, hi[3] = {inf, inf, inf};
+    uint32_t ce = kEmpty;
+    if (c != kEmpty) {
+        const rt_bvh_node nd = a.nodes[c];
+        lo[0] = nd.minX; hi[0] = nd.maxX;
+        lo[1] = nd.minY; hi[1] = nd.maxY;
+        lo[2] = nd.minZ; hi[2] = nd.maxZ;
+        if (m >> k & 1u) {
+            ce = first[node] + (uint32_t)__popc(m & ((1u << k) - 1u));
+        } else if (is_internal(a, c)) {
+            const uint2 r = a.range[c];
+            ce = leaf_entry(r.x, r.y - r.x + 1u);
+        } else {
+            ce = leaf_entry(c - (a.n - 1u), 1u);
+        }
+    }
+    uint32_t *nd = wide + (size_t)node * 8u * W + k;
+    for (int q = 0; q < 3; ++q) {
+        nd[2 * q * W] = __float_as_uint(lo[q]);
+        nd[(2 * q + 1) * W] = __float_as_uint(hi[q]);
+    }
+    nd[6 * W] = ce;
+    nd[7 * W] = 0u;
+    if (W != 4 || !qwide) return;
     bool ok = true;
-    for (int a = 0; a < 3; ++a)
-        ok = compress_axis(f + 8 * a, f + 8 * a + 4, child, org[a], scale[a], lo[a], hi[a]) && ok;
-    uint4 *q = reinterpret_cast<uint4 *>(qwide) + (size_t)i * 4u;
-    q[0] = make_uint4(__float_as_uint(org[0]), __float_as_uint(org[1]), __float_as_uint(org[2]), __float_as_uint(scale[0]));
-    q[1] = make_uint4(child[0], lo[0], child[1], hi[0]);
-    q[2] = make_uint4(child[2], lo[1], child[3], hi[1]);
-    q[3] = make_uint4(lo[2], hi[2], __float_as_uint(scale[1]), __float_as_uint(scale[2]));
-    for (uint32_t k = 0; k < 4; ++k)
-        if (child[k] != kEmpty && (child[k] & kLeafBit))
-            for (uint32_t s = leaf_first(child[k]), e = s + leaf_count(child[k]); s < e; ++s) slot_ref[s] = 4u * i + k;
+    float org[3], scale[3], far = 0.0f, ext = 0.0f;
+    uint32_t qlo[3], qhi[3];
+    for (int q = 0; q < 3; ++q) {
+        const bool have = c != kEmpty;
+        ok = ok && (!have || (fabsf(lo[q]) < 0x1p24f && fabsf(hi[q]) < 0x1p24f && lo[q] <= hi[q]));
+        const float mn = quad_min(have ? lo[q] : inf), mx = quad_max(have ? hi[q] : -inf);
+        far = fmaxf(far, fmaxf(fabsf(mn), fabsf(mx)));
+        ext = fmaxf(ext, mx - mn);
+        // 248 steps over the extent; a step is no finer than the origin's rounding, at most a quarter of it
+        scale[q] = fmaxf(fmaxf((mx - mn) * (1.0f / 248.0f), 0x1p-22f * fmaxf(fabsf(mn), fabsf(mx))), 0x1p-100f);
+        org[q] = (float)((double)mn - 1026.0 * (double)scale[q]);
+        double l = 255.0, h = 0.0;
+        if (have) {
+            const double s = 1.0 / (double)scale[q];
+            l = floor(((double)lo[q] - (double)org[q]) * s - (1024.0 + kPlaneMargin));
+            h = ceil(((double)hi[q] - (double)org[q]) * s - (1024.0 - kPlaneMargin));
+            ok = ok && l >= 0.0 && h <= 255.0;
+        }
+        qlo[q] = quad_or(((uint32_t)l & 255u) << (8 * k));
+        qhi[q] = quad_or(((uint32_t)h & 255u) << (8 * k));
+    }
+    const uint32_t first_of_pair = (uint32_t)__shfl((int)ce, k == 2u ? 2 : 0, 4);
+    const uint32_t second_of_pair = (uint32_t)__shfl((int)ce, k == 2u ? 3 : 1, 4);
+    uint4 w;
+    if (k == 0u)
+        w = make_uint4(__float_as_uint(org[0]), __float_as_uint(org[1]), __float_as_uint(org[2]), __float_as_uint(scale[0]));
+    else if (k == 3u)
+        w = make_uint4(qlo[2], qhi[2], __float_as_uint(scale[1]), __float_as_uint(scale[2]));
+    else
+        w = make_uint4(first_of_pair, qlo[k - 1u], second_of_pair, qhi[k - 1u]);
+    reinterpret_cast<uint4 *>(qwide)[t] = w;
+    if (ce != kEmpty && (ce & kLeafBit))
+        for (uint32_t s = leaf_first(ce), e = s + leaf_count(ce); s < e; ++s) slot_ref[s] = (uint32_t)t;
     const unsigned long long fail = __ballot(!ok);
     if (fail != 0ull && __lane_id() == (uint32_t)__ffsll((long long)fail) - 1u) info[0] = 1u;
-    if (i == 0) {
-        float far = 0.0f, ext = 0.0f;
-        for (int a = 0; a < 3; ++a) {
-            float mn = f[8 * a], mx = f[8 * a + 4];
-            for (int k = 1; k < 4; ++k)
-                if (child[k] != kEmpty) {
-                    mn = fminf(mn, f[8 * a + k]);
-                    mx = fmaxf(mx, f[8 * a + 4 + k]);
-                }
-            far = fmaxf(far, fmaxf(fabsf(mn), fabsf(mx)));
-            ext = fmaxf(ext, mx - mn);
-        }
+    if (t == 0) {
         info[1] = __float_as_uint(far);
         info[2] = __float_as_uint(ext);
     }
 }
 
 // the first level is the root; info: see build_scene
-__global__ void k_build_init(CollapseState *st, uint32_t *info, uint32_t all) {
+__global__ void k_build_init(CollapseState *st, uint32_t *queue, uint32_t *sums, uint32_t *info, uint32_t all) {
     if (threadIdx.x == 0) *st = CollapseState{{0u, 0u}, {1u, 0u}, 0u, 0u};
+    if (threadIdx.x == 0) queue[0] = 0u;
+    for (uint32_t i = threadIdx.x; i < 3u * kLevelBlocks; i += blockDim.x) sums[i] = 0u;
     if (all && threadIdx.x < 6) info[threadIdx.x] = threadIdx.x < 4 ? 0u : 0xFFFFFFFFu;
 }
 
@@ -1127,11 +1097,13 @@ void build_scene(rt_context *ctx, Scene &sc, const rt_triangle *tris, uint32_t n
     // every temporary of the build from one block of the scratch cache
     const bool keep_binary = (opts.flags & RT_BUILD_KEEP_BINARY) != 0;
     const uint32_t max_nodes = std::max<uint32_t>(n - 1, 1);
-    const uint64_t temp_bytes =
-        (keep_binary ? 0 : round256(sizeof(rt_bvh_node) * (2ull * n - 1))) + round256(sizeof(uint2) * max_nodes) +
-        round256(24ull * kBoundsBlocks) + 2 * round256(4ull * n) + std::max(radix_temp_bytes(n), refit_temp_bytes(n)) +
-        round256(32ull * W * max_nodes) + round256(4ull * max_nodes) + round256(4ull * W * max_nodes) +
-        round256(4ull * kCollapseBlocks) + round256(sizeof(CollapseState)) + round256(24);
+    const uint64_t sort_bytes = round256(24ull * kBoundsBlocks) + 2 * round256(4ull * n) +
+                                std::max(sort_temp_bytes(n), refit_temp_bytes(n));
+    const uint64_t collapse_bytes = round256(4ull * W * max_nodes) + round256(4ull * max_nodes) + round256(max_nodes);
+    const uint64_t temp_bytes = (keep_binary ? 0 : round256(sizeof(rt_bvh_node) * (2ull * n - 1))) +
+                                round256(sizeof(uint2) * max_nodes) + round256(sizeof(CollapseState)) + round256(24) +
+                                round256(4ull * max_nodes) + round256(12ull * kLevelBlocks) +
+                                std::max(sort_bytes, collapse_bytes);
     Temps tmp(ctx, temp_bytes, st);
     DevBuf kept;  // the binary nodes, when they stay resident
     rt_bvh_node *binary = nullptr;
@@ -1144,9 +1116,11 @@ void build_scene(rt_context *ctx, Scene &sc, const rt_triangle *tris, uint32_t n
     uint2 *range = tmp.take<uint2>(max_nodes);
     CollapseState *state = tmp.take<CollapseState>(1);
     uint32_t *info = tmp.take<uint32_t>(6);  // k_compress's three words, k_leaves' NaN flag, k_check_indices' two words
-    k_build_init<<<1, 64, 0, st>>>(state, info, 1u);
+    uint32_t *queue = tmp.take<uint32_t>(max_nodes), *sums = tmp.take<uint32_t>(3ull * kLevelBlocks);
+    k_build_init<<<1, 1024, 0, st>>>(state, queue, sums, info, 1u);
     k_check_indices<<<grid_for(n), kB, 0, st>>>(dtris.as<rt_triangle>(), ntri, dsph.as<rt_sphere>(), nsph, nmat, nmodels,
                                                 models ? 1u : 0u, info + 4);
+    const uint64_t mk = tmp.mark();
     if (nodes) {
         uint32_t bad[2];
         RT_HIP(hipMemcpy(bad, info + 4, sizeof bad, hipMemcpyDeviceToHost));
@@ -1162,50 +1136,54 @@ void build_scene(rt_context *ctx, Scene &sc, const rt_triangle *tris, uint32_t n
                                               sc.slot_prim.as<uint32_t>(), n, sc.records.as<LeafRecord>(),
                                               sc.slot_mat.as<uint32_t>());
     } else {
-        const uint64_t mk = tmp.mark();
         uint32_t *partial = tmp.take<uint32_t>(6ull * kBoundsBlocks);
         uint32_t *keys = tmp.take<uint32_t>(n), *vals = tmp.take<uint32_t>(n);
         const uint32_t g = std::min<uint32_t>(grid_for(n), kBoundsBlocks);
         k_centroid_bounds<<<g, kB, 0, st>>>(dtris.as<rt_triangle>(), ntri, dsph.as<rt_sphere>(), n, partial);
         k_morton<<<grid_for(n), kB, 0, st>>>(dtris.as<rt_triangle>(), ntri, dsph.as<rt_sphere>(), n, partial, g,
                                              (opts.flags & RT_BUILD_REFERENCE_MORTON) ? 1u : 0u, keys, vals);
-        radix_sort(keys, vals, n, st, tmp);
+        const uint64_t sort_mk = tmp.mark();
+        sort_pairs(keys, vals, n, st, tmp);
         if (n > 1) k_karras<<<grid_for(n - 1), kB, 0, st>>>(keys, (int)n, binary, range);
         k_leaves<<<grid_for(n), kB, 0, st>>>(dtris.as<rt_triangle>(), ntri, dsph.as<rt_sphere>(), duv.as<float2>(), vals,
                                              (opts.flags & RT_BUILD_REFERENCE_LEAVES) ? 1u : 0u, n,
                                              sc.slot_prim.as<uint32_t>(), binary + (n - 1), sc.records.as<LeafRecord>(),
                                              sc.slot_mat.as<uint32_t>(), info + 3);
+        tmp.release(sort_mk);
         if (n > 1) refit(binary, range, n, st, tmp);
         tmp.release(mk);
     }
     RT_HIP(hipGetLastError());
 
     CollapseArgs a{binary, range, n, W, L};
-    uint32_t *wide_tmp = tmp.take<uint32_t>(8ull * W * max_nodes);
-    uint32_t *queue = tmp.take<uint32_t>(max_nodes), *chosen = tmp.take<uint32_t>((uint64_t)W * max_nodes);
-    uint32_t *block_sums = tmp.take<uint32_t>(kCollapseBlocks);
+    uint32_t *chosen = tmp.take<uint32_t>((uint64_t)W * max_nodes), *first = tmp.take<uint32_t>(max_nodes);
+    uint8_t *mask = tmp.take<uint8_t>(max_nodes);
     struct { CollapseState state; uint32_t pad[58]; uint32_t info[6]; } out{};  // as the two lie in the temporaries
     static_assert(sizeof(CollapseState) == 24 && offsetof(decltype(out), info) == 256, "state and info are read together");
+    const auto with_width = [&](auto f) {
+        if (W == 2) f(std::integral_constant<int, 2>{});
+        else if (W == 4) f(std::integral_constant<int, 4>{});
+        else f(std::integral_constant<int, 8>{});
+    };
     const auto collapse = [&] {
-        if (n <= kSmallCollapse && !nodes) {
-            k_collapse_small<<<1, kB, 0, st>>>(a, state, queue, wide_tmp, max_nodes);
-            RT_HIP(hipMemcpy(&out, state, sizeof out, hipMemcpyDeviceToHost));
-            return;
-        }
-        // about log2(n) levels of a width-4 tree; the host looks after the first ones and then after every eight
-        uint32_t level = 0, ahead = 2;
-        for (uint64_t m = n; m > 1; m >>= 1) ++ahead;
+        // The levels of up to kLevelThreads nodes at both ends take one launch each, and about log2(n) / 2 levels lie
+        // between them; the host looks after these and then after every four more.
+        uint32_t launch = 0, ahead = 1;
+        for (uint64_t m = n; m > 1024; m >>= 1) ++ahead;
         uint64_t widest = 1;  // no level can hold more nodes
+        with_width([&](auto w) { k_collapse_choose<w.value><<<grid_for(max_nodes), kB, 0, st>>>(a, chosen, mask); });
         do {
-            for (uint32_t end = level + ahead; level < end; ++level) {
-                const uint32_t grid = std::min<uint32_t>(grid_for(widest), kCollapseBlocks);
-                k_collapse_choose<<<grid, kB, 0, st>>>(a, level, state, queue, chosen, block_sums);
-                k_collapse_emit<<<grid, kB, 0, st>>>(a, level, state, queue, chosen, block_sums, wide_tmp, max_nodes);
-                widest = std::min<uint64_t>(widest * W, max_nodes);
+            for (uint32_t end = launch + ahead; launch < end; ++launch) {
+                widest = launch == 0 ? std::min<uint64_t>(kLevelThreads * W, max_nodes) : std::min<uint64_t>(widest * W, max_nodes);
+                const uint32_t grid = launch == 0 ? 1u : std::min<uint32_t>((widest + kLevelThreads - 1u) / kLevelThreads, kLevelBlocks);
+                with_width([&](auto w) {
+                    k_collapse_levels<w.value><<<grid, kLevelThreads, 0, st>>>(launch, state, queue, first, chosen, mask, sums,
+                                                                              max_nodes);
+                });
             }
-            ahead = 8;
+            ahead = 4;
             RT_HIP(hipMemcpy(&out, state, sizeof out, hipMemcpyDeviceToHost));
-        } while (out.state.count[level & 1u] != 0u);
+        } while (out.state.count[launch & 1u] != 0u);
     };
     collapse();
     throw_bad_index(out.info + 4);
@@ -1215,33 +1193,35 @@ void build_scene(rt_context *ctx, Scene &sc, const rt_triangle *tris, uint32_t n
             k_refit_pass<<<grid_for(2ull * n - 1), kB, 0, st>>>(binary, other.as<rt_bvh_node>(), n);
             k_refit_pass<<<grid_for(2ull * n - 1), kB, 0, st>>>(other.as<rt_bvh_node>(), binary, n);
         }
-        k_build_init<<<1, 64, 0, st>>>(state, info, 0u);
+        k_build_init<<<1, 1024, 0, st>>>(state, queue, sums, info, 0u);
         collapse();
         RT_HIP(hipStreamSynchronize(st));  // `other` is freed
     }
     RT_REQUIRE(!out.state.bad, "internal: wide node count exceeds bound");
     const uint32_t depth = out.state.depth;
-    const uint32_t nwide = std::max(out.state.base[0], out.state.base[1]);
-    RT_HIP(hipEventRecord(ev1, st));
-    RT_HIP(hipEventSynchronize(ev1));
-    RT_HIP(hipGetLastError());
-    float ms = 0.0f;
-    RT_HIP(hipEventElapsedTime(&ms, ev0, ev1));
-    (void)hipEventDestroy(ev0);
-    (void)hipEventDestroy(ev1);
-
-    sc.nwide = nwide;
+    sc.nwide = std::max(out.state.base[0], out.state.base[1]);
     sc.wide.alloc((size_t)sc.nwide * 32u * W, &ctx->pool);
-    RT_HIP(hipMemcpy(sc.wide.p, wide_tmp, (size_t)sc.nwide * 32u * W, hipMemcpyDeviceToDevice));
     if (W == 4) {
         sc.qwide.alloc((size_t)sc.nwide * 64u, &ctx->pool);
         sc.slot_ref.alloc(sizeof(uint32_t) * n, &ctx->pool);
         if (nodes)
             k_check_boxes<<<grid_for(2ull * n - 1), kB, 0, st>>>(binary, n, dtris.as<rt_triangle>(), dsph.as<rt_sphere>(),
                                                                  sc.slot_prim.as<uint32_t>(), info);
-        k_compress<<<grid_for(sc.nwide), kB, 0, st>>>(sc.wide.as<uint32_t>(), sc.nwide, sc.qwide.as<uint32_t>(),
-                                                      sc.slot_ref.as<uint32_t>(), info);
-        RT_HIP(hipGetLastError());
+    }
+    with_width([&](auto w) {
+        k_collapse_emit<w.value><<<grid_for((uint64_t)sc.nwide * W), kB, 0, st>>>(
+            a, sc.nwide, queue, first, chosen, mask, sc.wide.as<uint32_t>(), sc.qwide.as<uint32_t>(),
+            sc.slot_ref.as<uint32_t>(), info);
+    });
+    RT_HIP(hipGetLastError());
+    RT_HIP(hipEventRecord(ev1, st));
+    RT_HIP(hipEventSynchronize(ev1));
+    float ms = 0.0f;
+    RT_HIP(hipEventElapsedTime(&ms, ev0, ev1));
+    (void)hipEventDestroy(ev0);
+    (void)hipEventDestroy(ev1);
+
+    if (W == 4) {
         struct { uint32_t bad; float far, extent; } whole{};
         RT_HIP(hipMemcpy(&whole, info, sizeof whole, hipMemcpyDeviceToHost));
         // see Scene::far_limit: origins may lie this far outside the scene's coordinates

@@ -1,5 +1,5 @@
 """The device builder at the sizes where it changes its kernels, byte for byte against the oracle's: one primitive,
-whole and ragged powers of two (the table of aligned unions), both sides of the single-block sort, scan and collapse,
+whole and ragged powers of two (the table of aligned unions), both sides of the ranking sort, wide and narrow levels,
 every width and leaf size, signed zeros, NaN vertices, identical primitives."""
 import numpy as np
 import pytest
@@ -151,3 +151,24 @@ def test_memory_of_released_scenes_is_reused_safely(ctx, native):
     for k, dh in outs:
         got = dh.to_numpy(np.uint32)
         assert np.array_equal(want.setdefault(k, got), got)
+
+
+def test_level_wider_than_the_blocks(ctx, native):
+    """A binary tree whose widest level has more than 2^20 nodes, so that each block of it takes several tiles."""
+    n = 6_000_000
+    rng = np.random.default_rng(66)
+    tris = np.zeros(n, L.TRIANGLE)
+    at = rng.random((n, 3), dtype=np.float32) * 100
+    for k in ("v0", "v1", "v2"):
+        tris[k][:, :3] = at + rng.random((n, 3), dtype=np.float32)
+    sid = ctx.upload(tris, None, MATS, width=2, leaf_size=1)
+    inf = ctx.info(sid)
+    _check_wide(ctx, sid, n, 1)
+    child = ctx.wide(sid).reshape(inf.nwide, 8, 2)[:, 6, :]
+    nodes = np.concatenate([[0], np.cumsum(((child >> 31) == 0).sum(1))])  # node children of the nodes before
+    base, size, widest, depth = 0, 1, 0, 0
+    while size:
+        widest, depth = max(widest, size), depth + 1
+        base, size = base + size, int(nodes[base + size] - nodes[base])
+    assert base == inf.nwide and depth == inf.wide_depth and widest > 1 << 20
+    ctx.release(sid)
