@@ -53,7 +53,7 @@ int rt_create(rt_context **out, int device) {
     ctx->device = device;
     int st = guarded(ctx, [&] {
         RT_HIP(hipDeviceGetAttribute(&ctx->num_cus, hipDeviceAttributeMultiprocessorCount, device));
-        ctx->counters.alloc(16ull * rt_context::kCounterSlots);
+        ctx->counters.alloc(4ull * kCounterLines * kCounterStride * rt_context::kCounterSlots);
         RT_HIP(hipMemset(ctx->counters.p, 0, ctx->counters.bytes));
         ctx->noalloc_scratch = static_cast<char *>(noalloc_scratch_address());  // this device's copy
     });

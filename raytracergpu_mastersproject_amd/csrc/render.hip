@@ -360,21 +360,24 @@ __global__ __launch_bounds__(256) void k_render(RenderArgs a) {
     uint32_t segs = 0;
     bool exhausted = false;
     uint32_t q_next = 0, q_end = 0, q_job = 0;  // the wave's current chunk of work items (wave-uniform)
+    const uint32_t wpb = blockDim.x / 64u;
+    WorkLines lines(blockIdx.x * wpb + __builtin_amdgcn_readfirstlane(threadIdx.x / 64u), gridDim.x * wpb);
     for (;;) {
         const unsigned long long idle = __ballot(ps.phase == kIdle);
         const uint32_t nidle = (uint32_t)__popcll(idle);
         if (!exhausted && nidle >= a.refill) {
-            if (q_next == q_end) {
+            while (q_next == q_end && !exhausted) {
                 const int leader = __ffsll((unsigned long long)idle) - 1;
-                uint32_t base = 0;
-                if ((int)lane == leader) base = atomicAdd(a.work, kRenderChunk);
-                base = (uint32_t)__builtin_amdgcn_readfirstlane(__shfl((int)base, leader));
+                uint32_t v = 0;
+                if ((int)lane == leader) v = atomicAdd(lines.counter(a.work), 1u);
+                v = (uint32_t)__builtin_amdgcn_readfirstlane(__shfl((int)v, leader));
+                const uint64_t base = lines.item(v) * kRenderChunk;
                 if (base >= a.nitems) {
-                    exhausted = true;
+                    exhausted = !lines.next();
                 } else {
-                    q_next = base;
-                    q_end = (uint32_t)min((uint64_t)base + kRenderChunk, (uint64_t)a.nitems);
-                    if constexpr (MULTI) q_job = find_job(a.jobs, a.njobs, base);
+                    q_next = (uint32_t)base;
+                    q_end = (uint32_t)min(base + kRenderChunk, (uint64_t)a.nitems);
+                    if constexpr (MULTI) q_job = find_job(a.jobs, a.njobs, q_next);
                 }
             }
             const uint32_t take = exhausted ? 0u : min(nidle, q_end - q_next);
@@ -692,6 +695,7 @@ constexpr uint32_t kYieldPoll = 32;
 struct FinishArgs {
     WaveArgs w;
     unsigned int *work;  // work[0]: the counter; work[1]: its value when the launch yielded
+    uint32_t lines;      // counters at most; 1 for a launch that can yield
     uint32_t refill, leaf_weight, shade_min;
     uint32_t *yield;  // host-written yield requests (fine-grained host memory), or nullptr
     uint32_t yield_at;
@@ -717,15 +721,17 @@ template <int W, int S> __global__ __launch_bounds__(256) void k_wave_finish(Fin
     uint32_t segs = 0;  // continuation segments (the queue's own were counted when queued)
     bool exhausted = false;
     uint32_t q_next = 0, q_end = 0;
+    const uint32_t wpb = blockDim.x / 64u;
+    WorkLines lines(blockIdx.x * wpb + __builtin_amdgcn_readfirstlane(threadIdx.x / 64u), gridDim.x * wpb, f.lines);
     for (;;) {
         const unsigned long long idle = __ballot(phase == kIdle);
         const uint32_t nidle = (uint32_t)__popcll(idle);
         if (!exhausted && nidle >= f.refill) {
-            if (q_next == q_end) {
+            while (q_next == q_end && !exhausted) {
                 const int leader = __ffsll((unsigned long long)idle) - 1;
                 uint32_t base = 0;
                 if ((int)lane == leader) {
-                    base = atomicAdd(f.work, chunk);
+                    base = atomicAdd(lines.counter(f.work), chunk);
                     if (f.yield && !(base & kYieldBit) && (base / chunk) % kYieldPoll == 0u &&
                         __hip_atomic_load(f.yield, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM) >= f.yield_at) {
                         const uint32_t before = atomicOr(f.work, kYieldBit);
@@ -733,8 +739,9 @@ template <int W, int S> __global__ __launch_bounds__(256) void k_wave_finish(Fin
                     }
                 }
                 base = (uint32_t)__shfl((int)base, leader);
-                if (base >= n) exhausted = true;  // taken after a yield (kYieldBit), or past the end
-                else { q_next = base; q_end = min(base + chunk, n); }
+                const uint64_t first = lines.item(base / chunk) * chunk;
+                if (first >= n) exhausted = !lines.next();  // taken after a yield (kYieldBit), or past the end
+                else { q_next = (uint32_t)first; q_end = (uint32_t)min(first + chunk, (uint64_t)n); }
             }
             if (!exhausted) {
                 const uint32_t take = min(nidle, q_end - q_next);
@@ -804,6 +811,7 @@ template <int W, int S> __global__ __launch_bounds__(256) void k_wave_finish(Fin
 struct TeamPathArgs {
     WaveArgs w;
     unsigned int *work;
+    uint32_t lines;  // counters at most
     uint32_t limit;  // team_trace's
 };
 
@@ -815,6 +823,7 @@ template <int T> __global__ __launch_bounds__(64) void k_path_team(TeamPathArgs 
     const uint32_t n = *a.n_in + n2;
     const uint32_t lane = threadIdx.x, first_lane = lane & ~(uint32_t)(T - 1);
     bool live = false, more = true;
+    WorkLines lines(blockIdx.x, gridDim.x, f.lines);
     uint32_t p = 0, bounce = 0, st = 0, segs = 0;
     float next = 0.0f;
     v3 color{0.0f, 0.0f, 0.0f}, atten{1.0f, 1.0f, 1.0f}, o{0.0f, 0.0f, 0.0f}, d{0.0f, 0.0f, 0.0f};
@@ -823,13 +832,13 @@ template <int T> __global__ __launch_bounds__(64) void k_path_team(TeamPathArgs 
         if (more && idle != 0ull) {
             const uint32_t want = (uint32_t)__popcll(idle) / T;
             uint32_t base = 0;
-            if (lane == 0) base = atomicAdd(f.work, want);
+            if (lane == 0) base = atomicAdd(lines.counter(f.work), want);
             base = (uint32_t)__builtin_amdgcn_readfirstlane((int)base);
-            const uint32_t i = base + (uint32_t)__popcll(idle & ((1ull << first_lane) - 1ull)) / T;
-            more = base + want < n;
+            const uint64_t i = lines.item(base + (uint32_t)__popcll(idle & ((1ull << first_lane) - 1ull)) / T);
+            const bool ran_out = lines.item((uint64_t)base + want) >= n;
             if (!live && i < n) {
                 const bool second = i < n2;
-                const uint32_t qi = second ? i : i - n2;
+                const uint32_t qi = (uint32_t)(second ? i : i - n2);
                 p = (second ? a.ids_in2 : a.ids_in)[qi];
                 const float4 *q = reinterpret_cast<const float4 *>((second ? a.rays_in2 : a.rays_in) + qi);
                 const float4 r0 = q[0], r1 = q[1];
@@ -842,6 +851,10 @@ template <int T> __global__ __launch_bounds__(64) void k_path_team(TeamPathArgs 
                 st = __float_as_uint(at.w);
                 bounce = a.bounce;
                 live = true;
+            }
+            if (ran_out) {
+                more = lines.next();
+                if (more && __ballot(!live) != 0ull) continue;
             }
         }
         if (__ballot(live) == 0ull) break;
@@ -906,6 +919,10 @@ __global__ void k_zero(unsigned int *c) {
     if (threadIdx.x == 0) c[0] = 0u;
 }
 
+__global__ void k_zero_lines(unsigned int *work) {
+    if (threadIdx.x < kCounterLines) work[threadIdx.x * kCounterStride] = 0u;
+}
+
 // Before a yielded finish launch is resumed: its work counter back to where the yield left it.
 __global__ void k_resume_counter(unsigned int *work) {
     if (threadIdx.x == 0 && (work[0] & kYieldBit)) work[0] = work[1];
@@ -930,7 +947,7 @@ void launch_render_kernel(rt_context *ctx, RenderArgs &a, uint32_t layout, bool 
     a.leaf_weight = c.leaf_weight;
     a.shade_min = c.shade_min;
     a.work = ctx->counter_slot();
-    k_zero<<<1, 64, 0, stream>>>(a.work);
+    k_zero_lines<<<1, 64, 0, stream>>>(a.work);
     const size_t lds = stack_lds_bytes(c.lds_stack, c.block);
     void *k = pick_render(layout, c.lds_stack, multi);
     int per_cu = 0;
@@ -1064,16 +1081,19 @@ uint32_t wave_finish_bounce() {
 
 namespace {
 // Lanes per path of a pass of `paths` paths, at most a quarter of which usually queue after the first
-// bounce; 0: the finish kernel's one lane per path.  Whole frames (us; 256 CUs; 200 k triangles unless stated),
-// one lane -> 32 / 16 / 8 lanes per path:
-//   4,096 paths    900 -> 164 / 171 / 184  (1,024 triangles 238 -> 79 / 80 / 83)
-//   65,536 paths   1,054 -> 350 / 353 / 371 (1,024 triangles 260 -> 243 / 230 / 225, 1 M 1,244 -> 391 / 389 / 401)
-//   262,144 paths  1,181 -> -- / 764 / 641  (1,024 triangles 297 -> -- / 511 / 349, 1 M 1,256 -> -- / 905 / 749)
-//   1,048,576      1,343 -> -- / 2,055 / 1,327 (1,024 triangles 411 -> -- / 1,575 / 900)
+// bounce; 0: the finish kernel's one lane per path.  Whole frames (us; 256 CUs), one lane -> 32 / 16 / 8 lanes per
+// path, on 1,024 triangles, 200 k and 600 k:
+//   4,096 paths    156 -> 71 / 74 / 82     662 -> 121 / 152 / 198     705 -> 129 / 154 / 226
+//   65,536         188 -> 108 / 106 / 110  892 -> 206 / 236 / 310     959 -> 225 / 258 / 336
+//   262,144        214 -> 161 / 143 / 145  981 -> 310 / 308 / 376     1,056 -> 372 / 357 / 429
+//   1,048,576      335 -> 421 / 333 / 310  1,131 -> 765 / 665 / 672   1,342 -> 1,012 / 866 / 847
+//   2,001,996      377 -> -- / 430 / 384   1,185 -> -- / 842 / 820    1,383 -> -- / 1,085 / 1,045
+//   4,194,304      554 -> -- / 902 / 771   1,586 -> -- / 1,952 / 1,792
+// (64 lanes: 117 at 4,096 paths on 200 k triangles, but 118 at 65,536 on 1,024.)
 uint32_t path_team_size(const rt_context *ctx, uint32_t layout, uint32_t stack_bound, uint64_t paths) {
     const uint64_t cus = (uint64_t)ctx->num_cus;
-    if (layout != kQ4 || paths > 1024u * cus) return 0;
-    const uint32_t t = paths <= 32u * cus ? 32u : paths <= 128u * cus ? 16u : 8u;
+    if (layout != kQ4 || paths > 8192u * cus) return 0;
+    const uint32_t t = paths <= 512u * cus ? 32u : paths <= 2048u * cus ? 16u : 8u;
     return team_limit(t, stack_bound) ? t : 0u;
 }
 }  // namespace
@@ -1199,9 +1219,16 @@ void launch_render_wave(rt_context *ctx, const Scene &sc, const RenderJob &j, un
                 a.rays_in = rays[cur];
                 a.ids_in = ids[cur];
                 a.n_in = count + cur;
+                // the hits are no longer needed: their storage holds the work counters.  A launch that can yield
+                // has one, among the pass's counters, and so has a pass of few paths.
+                const bool many = !yield && 16ull * maxp >= 4ull * kCounterLines * kCounterStride + 128u;
+                unsigned int *work = count + 2;
+                if (many) work = reinterpret_cast<unsigned int *>((reinterpret_cast<uintptr_t>(hits) + 127u) & ~uintptr_t(127));
+                const uint32_t lines = many ? kCounterLines : 1u;
+                if (many) k_zero_lines<<<1, 64, 0, stream>>>(work);
+                else k_zero<<<1, 64, 0, stream>>>(work);
                 if (const uint32_t team = yield ? 0u : path_team_size(ctx, j.layout, sc.stack_bound, paths)) {
-                    TeamPathArgs ta{a, count + 2, team_limit(team, sc.stack_bound)};
-                    k_zero<<<1, 64, 0, stream>>>(ta.work);
+                    TeamPathArgs ta{a, work, lines, team_limit(team, sc.stack_bound)};
                     void *k = pick_path_team(team);
                     int per_cu = 0;
                     RT_HIP(hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, k, 64, 0));
@@ -1214,9 +1241,8 @@ void launch_render_wave(rt_context *ctx, const Scene &sc, const RenderJob &j, un
                     break;
                 }
                 WaveResume w{};
-                w.fa = FinishArgs{a, count + 2, tc.refill, tc.leaf_weight, tc.shade_min,
+                w.fa = FinishArgs{a, work, lines, tc.refill, tc.leaf_weight, tc.shade_min,
                                   yield ? yield->flag : nullptr, yield ? yield->yield_at : 0u};
-                k_zero<<<1, 64, 0, stream>>>(w.fa.work);
                 w.lds = stack_lds_bytes(tc.lds_stack, tc.block);
                 w.kernel = pick_finish(j.layout, tc.lds_stack);
                 int per_cu = 0;
@@ -1264,10 +1290,9 @@ bool wave_schedule(uint32_t width, uint32_t height, uint32_t spp, uint32_t flags
     return (flags & RT_RENDER_WAVEFRONT) || (!layout && (uint64_t)width * height * spp >= kWaveMinSamples);
 }
 
-// rt_render's own choice.  One image is faster bounce by bounce at every size on compressed nodes: from
-// 1,024 paths per CU with one lane per path (2 M samples on 200 k triangles 1,905 us in one persistent
-// launch, 1,475 bounce by bounce; 1 M samples on 1,024 triangles 638 and 411), below with a team
-// per path (path_team_size).  Other layouts keep wave_schedule's line.
+// rt_render's own choice.  One image is faster bounce by bounce at every size on compressed nodes: with a team per
+// path (path_team_size), and with one lane per path above 1,024 paths per CU (2 M samples on 200 k triangles
+// 1,905 us in one persistent launch, 1,185 bounce by bounce; 1 M samples on 1,024 triangles 638 and 335).  Other layouts keep wave_schedule's line.
 static bool bounce_by_bounce(rt_context *ctx, const Scene &sc, const RenderJob &j, uint32_t flags) {
     const bool layout_flags = (flags & (RT_RENDER_SPLIT_SAMPLES | RT_RENDER_NO_SPLIT | RT_RENDER_PERSISTENT_PATHS)) != 0;
     if (wave_schedule(j.width, j.height, j.spp, flags)) return true;

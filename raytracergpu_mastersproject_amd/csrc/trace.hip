@@ -2,7 +2,7 @@
 //
 // Two schedules:
 //   persistent: a grid sized to fill every CU once; each wave takes chunks of rays
-//     from a global counter, one atomic per chunk (ChunkSchedule: smaller chunks for
+//     from global counters (WorkLines), one atomic per chunk (ChunkSchedule: smaller chunks for
 //     the last rays).  When at least `refill` lanes of a wave are idle they take the
 //     next rays of the wave's chunk (ballot + popcount + lane prefix), so finished
 //     lanes are refilled while long rays keep traversing.
@@ -178,7 +178,9 @@ __global__ __launch_bounds__(256) void k_trace_persistent(TraceArgs a) {
     bool exhausted = false;
     uint32_t q_next = 0, q_end = 0;  // the wave's current chunk of ray indices (wave-uniform)
     const uint32_t n = a.n_dev ? min(*a.n_dev, a.n) : a.n;
-    const ChunkSchedule<uint32_t> sched(n, gridDim.x * (blockDim.x / 64u), true);
+    const uint32_t wpb = blockDim.x / 64u;
+    const ChunkSchedule<uint32_t> sched(n, gridDim.x * wpb, true);
+    WorkLines lines(blockIdx.x * wpb + __builtin_amdgcn_readfirstlane(threadIdx.x / 64u), gridDim.x * wpb);
     Trav t;
     t.have = false;
     t.top = 0;
@@ -194,14 +196,14 @@ __global__ __launch_bounds__(256) void k_trace_persistent(TraceArgs a) {
                 store((uint32_t)done);
                 done = -1;
             }
-            if (q_next == q_end) {  // one atomic per chunk keeps the shared counter off the critical path
+            while (q_next == q_end && !exhausted) {  // one atomic per chunk
                 const int leader = __ffsll((unsigned long long)idle) - 1;
                 uint32_t base = 0;
-                if ((int)lane == leader) base = atomicAdd(a.work, 1u);
+                if ((int)lane == leader) base = atomicAdd(lines.counter(a.work), 1u);
                 base = (uint32_t)__shfl((int)base, leader);
                 uint64_t lo, hi;
-                if (!sched.range(base, lo, hi)) exhausted = true;
-                else { q_next = (uint32_t)lo; q_end = (uint32_t)hi; }
+                if (sched.range((uint32_t)lines.item(base), lo, hi)) { q_next = (uint32_t)lo; q_end = (uint32_t)hi; }
+                else exhausted = !lines.next();
             }
             if (!exhausted) {
                 const uint32_t take = min(nidle, q_end - q_next);
@@ -316,7 +318,9 @@ __global__ __launch_bounds__(256) void k_trace_batch(BatchArgs a) {
     // latency to every step
     const uint32_t *nodes = nullptr;
     const LeafRecord *rec = nullptr;
-    const ChunkSchedule<uint64_t> sched(a.total, gridDim.x * (blockDim.x / 64u), false);
+    const uint32_t wpb = blockDim.x / 64u;
+    const ChunkSchedule<uint64_t> sched(a.total, gridDim.x * wpb, false);
+    WorkLines lines(blockIdx.x * wpb + __builtin_amdgcn_readfirstlane(threadIdx.x / 64u), gridDim.x * wpb);
     Trav t;
     t.have = false;
     t.top = 0;
@@ -333,14 +337,17 @@ __global__ __launch_bounds__(256) void k_trace_batch(BatchArgs a) {
                 store();
                 pending = false;
             }
-            if (q_next == q_end) {
+            while (q_next == q_end && !exhausted) {
                 const int leader = __ffsll((unsigned long long)idle) - 1;
                 unsigned long long base = 0;
-                if ((int)lane == leader) base = atomicAdd(a.work, 1ull);
+                if ((int)lane == leader) base = atomicAdd(lines.counter(a.work), 1ull);
                 base = __shfl(base, leader);
-                if (!sched.range(base, q_next, q_end)) {
-                    exhausted = true;
+                uint64_t lo, hi;
+                if (!sched.range(lines.item(base), lo, hi)) {
+                    exhausted = !lines.next();
                 } else {  // chunks are short: usually one item, found once per chunk
+                    q_next = lo;
+                    q_end = hi;
                     c_lo = find_item(a.items, 0u, a.nitems, q_next);
                     c_hi = find_item(a.items, c_lo, a.nitems, q_end - 1u) + 1u;
                 }
@@ -379,7 +386,7 @@ __global__ __launch_bounds__(256) void k_trace_batch(BatchArgs a) {
 }
 
 __global__ void k_zero_counter(unsigned int *c) {
-    if (threadIdx.x == 0) { c[0] = 0u; c[1] = 0u; }
+    if (threadIdx.x < kCounterLines) c[threadIdx.x * kCounterStride] = c[threadIdx.x * kCounterStride + 1u] = 0u;
 }
 
 SceneView view_of(const Scene &sc) {
@@ -460,16 +467,16 @@ LaunchCfg resolve_cfg(const rt_context *ctx, const Scene &sc, const rt_launch_co
 // cross (us; 256 CUs; closest hit, 1 M triangles unless stated):
 //   24 rays per CU     a wave per ray, every wave resident: 4,096 rays 21.4 with 64 lanes, 22.6 with 32
 //   128 rays per CU    16,384 rays 33.0 with 32 lanes, 42.5 with 16; 65,536 rays 80.1 and 75.0
-//   1,024 rays per CU  131,072 rays 114.8 with 16 lanes, 126.7 with 8; 524,288 rays 359 and 347
-//   3,072 rays per CU  524,288 rays 347 with 8 lanes, 472 with one; 1,000,000 rays 632 and 604
-//                      (4 M triangles 426 and 579, 768 and 715; 1,024 triangles 113 and 230, 202 and 323)
+//   1,024 rays per CU  131,072 rays 118 with 16 lanes, 128 with 8; 400,000 rays 287 and 281
+//   1,536 rays per CU  400,000 rays 281 with 8 lanes, 296 with one; 524,288 rays 348 and 304
+//                      (4 M triangles 333 and 376, 427 and 392; 1,024 triangles 82 and 89, 102 and 93)
 // Four lanes per ray were slower than eight at every size.  A launch that counts tests per ray keeps
 // one lane per ray (its counts are those of the ordered traversal), as do the widths 2 and 8, a
 // caller's one-lane-per-ray configuration, and a tree too deep for the team's stack.
 static uint32_t team_size(const rt_context *ctx, const Scene &sc, uint32_t n, const LaunchCfg &c, bool count) {
     if (sc.layout() != kQ4 || count || !c.persistent) return 0;
     const uint64_t cus = (uint64_t)ctx->num_cus;
-    if (n > 3072u * cus) return 0;
+    if (n > 1536u * cus) return 0;
     const uint32_t t = n <= 24u * cus ? 64u : n <= 128u * cus ? 32u : n <= 1024u * cus ? 16u : 8u;
     return team_limit(t, sc.stack_bound) ? t : 0u;
 }

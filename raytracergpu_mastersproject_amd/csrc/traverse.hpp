@@ -68,6 +68,31 @@ template <typename T> struct ChunkSchedule {
     }
 };
 
+// A wave's place among a launch's work counters.  Wave w of `waves` takes from counter w % lines; value v of counter k
+// stands for item v * lines + k, so the items are taken nearly in order.  When its counter has run out, a wave
+// helps one other before it stops.  A counter per 32 waves or more: a few waves share one.
+struct WorkLines {
+    uint32_t lines, home;
+    bool helping;
+    __device__ __forceinline__ WorkLines(uint32_t wave, uint32_t waves, uint32_t max_lines = kCounterLines) {
+        lines = 1u;
+        while (lines < max_lines && lines * 64u <= waves) lines *= 2u;
+        home = wave & (lines - 1u);
+        helping = lines == 1u;
+    }
+    template <typename T> __device__ __forceinline__ T *counter(T *work) const {
+        return work + home * (kCounterStride * 4u / (uint32_t)sizeof(T));
+    }
+    __device__ __forceinline__ uint64_t item(uint64_t value) const { return value * lines + home; }
+    // the counter has run out: false when there is no other to try
+    __device__ __forceinline__ bool next() {
+        if (helping) return false;
+        helping = true;
+        home ^= lines / 2u;
+        return true;
+    }
+};
+
 template <int W> struct WideNode {
     float lo[3][W], hi[3][W];
     uint32_t child[W];

@@ -28,7 +28,8 @@ def _scene(ctx, ntri=6000, leaf_size=1):
 
 @pytest.mark.parametrize("w,h,calls", [(1, 1, (1,)), (64, 128, (1,)), (8193, 1, (1,)), (128, 64, (2, 2)),
                                        (181, 181, (1,)), (256, 128, (1,)), (32769, 1, (1,)), (200, 111, (3, 8)),
-                                       (512, 512, (1,)), (262145, 1, (1,)), (600, 600, (1, 2))])
+                                       (512, 512, (1,)), (262145, 1, (1,)), (600, 600, (1, 2)), (131073, 1, (1,)),
+                                       (512, 512, (2,)), (524289, 1, (1,)), (2048, 256, (4,)), (2097153, 1, (1,))])
 def test_sizes_agree_with_one_lane_per_path(ctx, native, w, h, calls):
     sid, params = _scene(ctx)
     a, segs = _image(ctx, native, sid, params, w, h, calls)

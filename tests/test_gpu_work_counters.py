@@ -1,0 +1,61 @@
+"""Persistent launches at the numbers of waves at which they use one, two, ... 32 work counters: every ray, pixel and
+path is taken exactly once, so results equal those of one lane per ray and of the other schedule, bit for bit."""
+import numpy as np
+import pytest
+
+from raytracergpu_mastersproject_amd import layouts as L
+from raytracergpu_mastersproject_amd import workloads as W
+
+from helpers import gpu_trace, small_cluster_scene
+
+pytestmark = pytest.mark.gpu
+
+SIZES = [1, 63, 64, 65, 64 * 63, 64 * 64 + 1, 64 * 128 - 1, 64 * 1024 + 7, 64 * 2048, 300_001]
+
+
+@pytest.mark.parametrize("n", SIZES)
+@pytest.mark.parametrize("width", [2, 8])
+def test_trace(ctx, native, n, width):
+    tris, mats = small_cluster_scene(4, 500, seed=91)
+    sid = ctx.upload(tris, None, mats, width=width)
+    rays = W.incoherent_rays(n, *W.scene_bounds(tris), seed=92)
+    one = native.launch_config(block=64, lds_stack=8, persistent=0)
+    for block, refill in ((64, 1), (256, 16), (256, 64)):
+        cfg = native.launch_config(block=block, lds_stack=8, refill=refill, persistent=1)
+        for any_hit in (False, True):
+            a = gpu_trace(ctx, sid, rays, any_hit=any_hit, cfg=cfg)
+            b = gpu_trace(ctx, sid, rays, any_hit=any_hit, cfg=one)
+            assert np.array_equal(a.view(np.uint32), b.view(np.uint32))
+    ctx.release(sid)
+
+
+@pytest.mark.parametrize("sizes", [[1], [64] * 7, [4096, 1, 0, 33_000], [70_001] * 9])
+def test_batch(ctx, native, sizes):
+    tris, mats = small_cluster_scene(4, 500, seed=93)
+    sids = [ctx.upload(tris[k:], None, mats) for k in range(2)]
+    items, want = [], []
+    for k, n in enumerate(sizes):
+        rays = W.incoherent_rays(max(n, 1), *W.scene_bounds(tris), seed=94 + k)
+        items.append((sids[k % 2], n, native.DeviceArray.from_numpy(rays), native.DeviceArray(16 * max(n, 1))))
+        want.append(gpu_trace(ctx, sids[k % 2], rays[:n]))
+    ctx.trace_batch(items)
+    for (_, n, _, hits), w in zip(items, want):
+        assert np.array_equal(hits.to_numpy(L.HIT, n).view(np.uint32), w.view(np.uint32))
+    for s in sids:
+        ctx.release(s)
+
+
+@pytest.mark.parametrize("w,h,spp", [(1, 1, 1), (8, 8, 4), (24, 11, 1), (33, 8, 1), (64, 63, 1), (91, 90, 1), (300, 200, 2)])
+@pytest.mark.parametrize("width", [2, 4])
+def test_render(ctx, native, w, h, spp, width):
+    s = W.served_scene(3000, 95)
+    sid = ctx.upload(s["tris"], None, s["materials"], width=width)
+    images = []
+    for flags in (native.RENDER_WAVEFRONT, native.RENDER_PERSISTENT_PATHS, native.RENDER_NO_SPLIT):
+        acc, seg = native.DeviceArray(16 * w * h), native.DeviceArray(8)
+        seg.zero()
+        ctx.accum_clear(acc, w * h)
+        ctx.render(sid, s["params"], w, h, spp, acc, flags=flags, segments=seg)
+        images.append(acc.to_numpy(np.uint32))
+    assert all(np.array_equal(images[0], i) for i in images[1:])
+    ctx.release(sid)
