@@ -47,8 +47,6 @@ __device__ __forceinline__ void wave_fence() {
     __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
 }
 
-// A wave's team stacks take 6 KB of LDS, so 26 waves fit a CU.
-constexpr uint32_t kTeamStackWave = 768;  // entries of 8 bytes per wave
 constexpr uint32_t team_stack(uint32_t t) { return kTeamStackWave / 64u * t; }
 
 // The stack holds at most 3 entries more per entry taken than before it.  While it holds more than
@@ -165,6 +163,18 @@ __device__ __forceinline__ TeamHit team_trace(bool live, v3 o, v3 d, float tmin,
     // the smallest (t, slot); a slot is tested by one lane only
     const uint32_t slot = team_min<T>(lt == bt ? ls : kEmpty);
     return TeamHit{bt, slot, lu, lv, slot != kEmpty && ls == slot && lt == bt};
+}
+
+// The end of a launch whose waves trace a ray (path) per lane: once a wave finds no more work and at most kLastRays of its
+// lanes are live, each of these rays goes on with a team of kLastTeam lanes.  A lane alone would take as long as
+// its ray's chain of loads, while the device empties: 1 M any-hit rays on 1 M triangles
+// 432 -> 375 us.  Rays start over; fewer rays (6: 386 us) or more in two rounds (12: 404) are slower.
+constexpr uint32_t kLastTeam = 8, kLastRays = 64 / kLastTeam;
+
+// The lane whose ray this lane's team takes over; `live`: at most kLastRays lanes, and not none.
+__device__ __forceinline__ uint32_t last_ray_lane(unsigned long long live) {
+    for (uint32_t k = (threadIdx.x & 63u) / kLastTeam; k > 0u && (live & (live - 1ull)) != 0ull; --k) live &= live - 1ull;
+    return (uint32_t)__ffsll(live) - 1u;
 }
 
 }  // namespace rtgpu

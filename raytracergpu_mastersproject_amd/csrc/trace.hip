@@ -1,13 +1,14 @@
 // trace.hip -- ray-query kernels (closest-hit / any-hit) over the resident wide BVH.
 //
-// Two schedules:
+// Two schedules of one lane per ray:
 //   persistent: a grid sized to fill every CU once; each wave takes chunks of rays
 //     from global counters (WorkLines), one atomic per chunk (ChunkSchedule: smaller chunks for
 //     the last rays).  When at least `refill` lanes of a wave are idle they take the
 //     next rays of the wave's chunk (ballot + popcount + lane prefix), so finished
 //     lanes are refilled while long rays keep traversing.
 //   direct: one lane per ray (a launch-tuner candidate; the camera rays of renders).
-// The batched variant runs many scenes' ray batches in one persistent launch.
+// A launch of few rays, and the last rays of each persistent wave, are traced by a team of lanes per ray (team.hpp).
+// The batched variants run many scenes' ray batches in one launch.
 #include <algorithm>
 #include <cstdlib>
 #include <vector>
@@ -40,6 +41,7 @@ struct TraceArgs {
     unsigned int *work;
     uint32_t leaf_weight;
     const uint32_t *n_dev;  // when set, the ray count is min(*n_dev, n)
+    uint32_t limit;         // of a team of kLastTeam lanes; 0: the last rays stay with their lanes
 };
 
 // Rays are read once and hits written once per launch: non-temporal accesses keep them from
@@ -114,72 +116,85 @@ __device__ __forceinline__ void store_refined(const SceneView &sc, const Trav &t
     if (counts) reinterpret_cast<uint2 *>(counts)[i] = make_uint2(t.nbox, t.ntri);
 }
 
-// One team of T lanes per ray, one wave per block, every ray at once: no work counter, no refill.
-template <int T, bool ANY, bool REFINE> __global__ __launch_bounds__(64) void k_trace_team(TraceArgs a, uint32_t limit) {
-    __shared__ uint2 stacks[64 / T * team_stack(T)];
-    const uint32_t i = blockIdx.x * (64u / T) + threadIdx.x / T;
-    bool live = i < a.n;
+// A team's result, by the lane that holds it.
+template <int T, bool REFINE>
+__device__ __forceinline__ void store_team(const SceneView &sc, const TeamHit &h, v3 o, v3 d, rt_hit *hits, uint32_t i) {
+    if (!h.owner && !(h.slot == kEmpty && threadIdx.x % T == 0)) return;
+    Trav t;
+    t.o = o;
+    t.d = d;
+    t.bt = h.t;
+    t.bslot = h.slot;
+    t.bu = h.u;
+    t.bv = h.v;
+    if constexpr (REFINE) store_refined(sc, t, hits, nullptr, i);
+    else store_hit(sc, t, hits, nullptr, i);
+}
+
+// The last rays of a wave, one per lane in `live`, from their start: ray i of that lane.
+template <int S, bool ANY, bool REFINE>
+__device__ __forceinline__ void trace_last(unsigned long long live, const SceneView &sc, const rt_ray *rays,
+                                           rt_hit *hits, uint32_t i, void *lds, uint32_t limit) {
+    const bool on = (threadIdx.x & 63u) / kLastTeam < (uint32_t)__popcll(live);
+    v3 o, d;
+    float tmin, tmax;
+    load_ray(rays, i, o, tmin, d, tmax);
+    const TeamHit h = team_trace<kLastTeam, ANY>(on, o, d, tmin, tmax, sc.wide, sc.nwide, sc.rec,
+                                                 reinterpret_cast<uint2 *>(wave_lds<S>(lds)), limit);
+    if (on) store_team<kLastTeam, REFINE>(sc, h, o, d, hits, i);
+}
+
+// Ray i by a team of T lanes; every lane of the wave calls it.
+template <int T, bool ANY, bool REFINE>
+__device__ __forceinline__ void trace_by_team(bool live, const SceneView &sc, const rt_ray *rays, rt_hit *hits, uint32_t i,
+                                              uint2 *stacks, uint32_t limit, uint32_t leaf_weight) {
     v3 o{0.0f, 0.0f, 0.0f}, d{0.0f, 0.0f, 0.0f};
     float tmin = 0.0f, tmax = 0.0f;
-    if (live) load_ray(a.rays, i, o, tmin, d, tmax);
-    const bool ordered = live && needs_exact_nodes(o, d, a.sc.far_limit);
+    if (live) load_ray(rays, i, o, tmin, d, tmax);
+    const bool ordered = live && needs_exact_nodes(o, d, sc.far_limit);
     if (__ballot(ordered) != 0ull) {  // rare: a team's first lane runs such a ray alone, in the stacks' memory
         uint2 spill[kSpillCap];
         if (ordered && threadIdx.x % T == 0) {
             Trav t;
-            trav_init<4>(t, o, d, tmin, tmax, a.sc.nwide);
-            trav_run<4, 16, ANY, false>(t, stack_mem<16>(stacks, spill), a.sc.wide, a.sc.rec, a.sc, a.leaf_weight);
-            if constexpr (REFINE) store_refined(a.sc, t, a.hits, nullptr, i);
-            else store_hit(a.sc, t, a.hits, nullptr, i);
+            trav_init<4>(t, o, d, tmin, tmax, sc.nwide);
+            trav_run<4, 16, ANY, false>(t, stack_mem<16>(stacks, spill), sc.wide, sc.rec, sc, leaf_weight);
+            if constexpr (REFINE) store_refined(sc, t, hits, nullptr, i);
+            else store_hit(sc, t, hits, nullptr, i);
         }
         live = live && !ordered;
     }
-    const TeamHit h = team_trace<T, ANY>(live, o, d, tmin, tmax, a.sc.wide, a.sc.nwide, a.sc.rec, stacks, limit);
-    if (!live) return;
-    if (h.owner || (h.slot == kEmpty && threadIdx.x % T == 0)) {
-        Trav t;
-        t.o = o;
-        t.d = d;
-        t.bt = h.t;
-        t.bslot = h.slot;
-        t.bu = h.u;
-        t.bv = h.v;
-        if constexpr (REFINE) store_refined(a.sc, t, a.hits, nullptr, i);
-        else store_hit(a.sc, t, a.hits, nullptr, i);
-    }
+    const TeamHit h = team_trace<T, ANY>(live, o, d, tmin, tmax, sc.wide, sc.nwide, sc.rec, stacks, limit);
+    if (live) store_team<T, REFINE>(sc, h, o, d, hits, i);
 }
 
-template <int T> void *team_kernel_t(bool any, bool refine) {
-    if (any) return refine ? (void *)k_trace_team<T, true, true> : (void *)k_trace_team<T, true, false>;
-    return refine ? (void *)k_trace_team<T, false, true> : (void *)k_trace_team<T, false, false>;
+// One team of T lanes per ray, one wave per block, every ray at once: no work counter, no refill.
+template <int T, bool ANY, bool REFINE> __global__ __launch_bounds__(64) void k_trace_team(TraceArgs a, uint32_t limit) {
+    __shared__ uint2 stacks[64 / T * team_stack(T)];
+    const uint32_t i = blockIdx.x * (64u / T) + threadIdx.x / T;
+    trace_by_team<T, ANY, REFINE>(i < a.n, a.sc, a.rays, a.hits, i, stacks, limit, a.leaf_weight);
 }
-void *team_kernel(uint32_t t, bool any, bool refine) {
-    switch (t) {
-        case 8: return team_kernel_t<8>(any, refine);
-        case 16: return team_kernel_t<16>(any, refine);
-        case 32: return team_kernel_t<32>(any, refine);
-        default: return team_kernel_t<64>(any, refine);
-    }
-}
+
+constexpr uint32_t kNoRay = ~0u;
 
 // REFINE: store each hit with t, u, v refined in double (store_refined) instead of the fp32 values.
-template <int W, int S, bool ANY, bool COUNT, bool REFINE>
-__global__ __launch_bounds__(256) void k_trace_persistent(TraceArgs a) {
+// LAST: the wave's last rays go on with teams of lanes (trace_last).
+template <int W, int S, bool ANY, bool COUNT, bool REFINE, bool LAST>
+__global__ __launch_bounds__(256, W == kQ4 ? 5 : 1) void k_trace_persistent(TraceArgs a) {
     extern __shared__ uint32_t lds[];
     uint2 spill[kSpillCap];
     const StackMem m = stack_mem<S>(lds, spill);
     const uint32_t lane = threadIdx.x & 63u;
     const unsigned long long lt = lane ? (~0ull >> (64u - lane)) : 0ull;
-    int64_t rid = -1;
+    uint32_t rid = kNoRay;  // a launch has fewer rays than this
     // REFINE: a finished ray's result is stored at the wave's next refill (or at the end), where the
     // lanes that finished since the last refill refine together; refining as each lane finishes would
     // run the double-precision code on almost every iteration.  Without refinement a lane stores at once.
-    int64_t done = -1;
+    uint32_t done = kNoRay;
     bool exhausted = false;
     uint32_t q_next = 0, q_end = 0;  // the wave's current chunk of ray indices (wave-uniform)
     const uint32_t n = a.n_dev ? min(*a.n_dev, a.n) : a.n;
     const uint32_t wpb = blockDim.x / 64u;
-    const ChunkSchedule<uint32_t> sched(n, gridDim.x * wpb, true);
+    const ChunkSchedule<uint32_t> sched(n, gridDim.x * wpb);
     WorkLines lines(blockIdx.x * wpb + __builtin_amdgcn_readfirstlane(threadIdx.x / 64u), gridDim.x * wpb);
     Trav t;
     t.have = false;
@@ -189,12 +204,12 @@ __global__ __launch_bounds__(256) void k_trace_persistent(TraceArgs a) {
         else store_hit(a.sc, t, a.hits, a.counts, i);
     };
     for (;;) {
-        const unsigned long long idle = __ballot(rid < 0);
+        const unsigned long long idle = __ballot(rid == kNoRay);
         const uint32_t nidle = (uint32_t)__popcll(idle);
         if (!exhausted && nidle >= a.refill) {
-            if (done >= 0) {
-                store((uint32_t)done);
-                done = -1;
+            if (done != kNoRay) {
+                store(done);
+                done = kNoRay;
             }
             while (q_next == q_end && !exhausted) {  // one atomic per chunk
                 const int leader = __ffsll((unsigned long long)idle) - 1;
@@ -208,31 +223,39 @@ __global__ __launch_bounds__(256) void k_trace_persistent(TraceArgs a) {
             if (!exhausted) {
                 const uint32_t take = min(nidle, q_end - q_next);
                 const uint32_t r = (uint32_t)__popcll(idle & lt);
-                if (rid < 0 && r < take) {
-                    rid = (int64_t)(q_next + r);
+                if (rid == kNoRay && r < take) {
+                    rid = q_next + r;
                     v3 o, d;
                     float tmin, tmax;
-                    load_ray(a.rays, (uint32_t)rid, o, tmin, d, tmax);
+                    load_ray(a.rays, rid, o, tmin, d, tmax);
                     walk_init<W, S, ANY>(t, m, o, d, tmin, tmax, a.sc.nwide, a.sc.far_limit, a.sc.rec, a.sc, a.leaf_weight);
                 }
                 q_next += take;
             }
         }
-        if (__ballot(rid >= 0) == 0ull) break;  // every lane idle and the queue is drained
-        const bool on_node = rid >= 0 && at_node(t), on_leaf = rid >= 0 && at_leaf(t);
+        const unsigned long long live = __ballot(rid != kNoRay);
+        if (live == 0ull) break;  // every lane idle and the queue is drained
+        if (LAST && exhausted && a.limit && (uint32_t)__popcll(live) <= kLastRays) break;
+        const bool on_node = rid != kNoRay && at_node(t), on_leaf = rid != kNoRay && at_leaf(t);
         if (choose_leaf_phase(on_node, on_leaf, a.leaf_weight)) {
             if (on_leaf) leaf_step<W, S, ANY, COUNT>(t, m, a.sc.rec, a.sc);
         } else {
             if (on_node) walk_node<W, S, ANY, COUNT>(t, m, a.sc.nodes);
         }
         walk_pop<W, S, ANY>(t, m);
-        if (rid >= 0 && trav_done(t)) {
+        if (rid != kNoRay && trav_done(t)) {
             if constexpr (REFINE) done = rid;
-            else store((uint32_t)rid);
-            rid = -1;
+            else store(rid);
+            rid = kNoRay;
         }
     }
-    if (done >= 0) store((uint32_t)done);
+    if (done != kNoRay) store(done);
+    if constexpr (LAST) {
+        const unsigned long long live = __ballot(rid != kNoRay);
+        if (live == 0ull) return;
+        const uint32_t i = (uint32_t)__shfl((int)rid, (int)last_ray_lane(live));
+        trace_last<S, ANY, REFINE>(live, a.sc, a.rays, a.hits, i, lds, a.limit);
+    }
 }
 
 // ---------------------------------------------------------------------------
@@ -289,6 +312,7 @@ struct BatchArgs {
     uint64_t total;
     unsigned long long *work;
     uint32_t leaf_weight;
+    uint32_t limit;  // as in TraceArgs
 };
 
 // the last item in [lo, hi) whose first ray is at or before g
@@ -302,8 +326,8 @@ __device__ __forceinline__ uint32_t find_item(const BatchItemDev *items, uint32_
 }
 
 // REFINE: store each hit with t, u, v refined in double (store_refined).
-template <int W, int S, bool ANY, bool REFINE>
-__global__ __launch_bounds__(256) void k_trace_batch(BatchArgs a) {
+template <int W, int S, bool ANY, bool REFINE, bool LAST>
+__global__ __launch_bounds__(256, W == kQ4 ? 5 : 1) void k_trace_batch(BatchArgs a) {
     extern __shared__ uint32_t lds[];
     uint2 spill[kSpillCap];
     const StackMem m = stack_mem<S>(lds, spill);
@@ -319,7 +343,7 @@ __global__ __launch_bounds__(256) void k_trace_batch(BatchArgs a) {
     const uint32_t *nodes = nullptr;
     const LeafRecord *rec = nullptr;
     const uint32_t wpb = blockDim.x / 64u;
-    const ChunkSchedule<uint64_t> sched(a.total, gridDim.x * wpb, false);
+    const ChunkSchedule<uint64_t> sched(a.total, gridDim.x * wpb);
     WorkLines lines(blockIdx.x * wpb + __builtin_amdgcn_readfirstlane(threadIdx.x / 64u), gridDim.x * wpb);
     Trav t;
     t.have = false;
@@ -368,7 +392,9 @@ __global__ __launch_bounds__(256) void k_trace_batch(BatchArgs a) {
                 active = true;
             }
         }
-        if (__ballot(active) == 0ull) break;
+        const unsigned long long live = __ballot(active);
+        if (live == 0ull) break;
+        if (LAST && exhausted && a.limit && (uint32_t)__popcll(live) <= kLastRays) break;
         const bool on_node = active && at_node(t), on_leaf = active && at_leaf(t);
         if (choose_leaf_phase(on_node, on_leaf, a.leaf_weight)) {
             if (on_leaf) leaf_step<W, S, ANY, false>(t, m, rec, a.items[item].sc);
@@ -383,6 +409,39 @@ __global__ __launch_bounds__(256) void k_trace_batch(BatchArgs a) {
         }
     }
     if (pending) store();
+    if constexpr (LAST) {
+        const unsigned long long live = __ballot(active);
+        if (live == 0ull) return;
+        const int from = (int)last_ray_lane(live);
+        const BatchItemDev &it = a.items[(uint32_t)__shfl((int)item, from)];
+        trace_last<S, ANY, REFINE>(live, it.sc, it.rays, it.hits, (uint32_t)__shfl((int)local, from), lds, a.limit);
+    }
+}
+
+// The same for few rays in all: a team of T lanes per ray, every ray at once.
+template <int T, bool ANY, bool REFINE>
+__global__ __launch_bounds__(64) void k_trace_team_batch(BatchArgs a, uint32_t limit) {
+    __shared__ uint2 stacks[64 / T * team_stack(T)];
+    const uint32_t g = blockIdx.x * (64u / T) + threadIdx.x / T;
+    const BatchItemDev &it = a.items[find_item(a.items, 0u, a.nitems, min((uint64_t)g, a.total - 1u))];
+    trace_by_team<T, ANY, REFINE>(g < a.total, it.sc, it.rays, it.hits, (uint32_t)(g - it.first), stacks, limit,
+                                  a.leaf_weight);
+}
+
+template <int T, bool ANY, bool REFINE> void *team_kernel_t(bool batch) {
+    return batch ? (void *)k_trace_team_batch<T, ANY, REFINE> : (void *)k_trace_team<T, ANY, REFINE>;
+}
+template <int T> void *team_kernel_t(bool any, bool refine, bool batch) {
+    if (any) return refine ? team_kernel_t<T, true, true>(batch) : team_kernel_t<T, true, false>(batch);
+    return refine ? team_kernel_t<T, false, true>(batch) : team_kernel_t<T, false, false>(batch);
+}
+void *team_kernel(uint32_t t, bool any, bool refine, bool batch) {
+    switch (t) {
+        case 8: return team_kernel_t<8>(any, refine, batch);
+        case 16: return team_kernel_t<16>(any, refine, batch);
+        case 32: return team_kernel_t<32>(any, refine, batch);
+        default: return team_kernel_t<64>(any, refine, batch);
+    }
 }
 
 __global__ void k_zero_counter(unsigned int *c) {
@@ -399,38 +458,51 @@ template <int W, int S> struct Kernels {
         if constexpr (W == kQ4) return (void *)k_trace_direct<W, S, ANY, false>;
         else return count ? (void *)k_trace_direct<W, S, ANY, true> : (void *)k_trace_direct<W, S, ANY, false>;
     }
-    template <bool ANY, bool REFINE> static void *persistent(bool count) {
-        if constexpr (W == kQ4) return (void *)k_trace_persistent<W, S, ANY, false, REFINE>;
-        else return count ? (void *)k_trace_persistent<W, S, ANY, true, REFINE>
-                     : (void *)k_trace_persistent<W, S, ANY, false, REFINE>;
+    template <bool ANY, bool REFINE> static void *persistent(bool count, bool last) {
+        if constexpr (W == kQ4)
+            return last ? (void *)k_trace_persistent<W, S, ANY, false, REFINE, true>
+                        : (void *)k_trace_persistent<W, S, ANY, false, REFINE, false>;
+        else return count ? (void *)k_trace_persistent<W, S, ANY, true, REFINE, false>
+                     : (void *)k_trace_persistent<W, S, ANY, false, REFINE, false>;
     }
-    static void *get(int which, bool any, bool count) {
+    template <bool ANY, bool REFINE> static void *batch(bool last) {
+        if constexpr (W == kQ4)
+            if (last) return (void *)k_trace_batch<W, S, ANY, REFINE, true>;
+        return (void *)k_trace_batch<W, S, ANY, REFINE, false>;
+    }
+    static void *get(int which, bool any, bool count, bool last) {
         if (which == 0) return any ? direct<true>(count) : direct<false>(count);
-        if (which == 1) return any ? persistent<true, false>(count) : persistent<false, false>(count);
-        if (which == 3) return persistent<false, true>(count);  // closest hit only
-        if (which == 2) return any ? (void *)k_trace_batch<W, S, true, false> : (void *)k_trace_batch<W, S, false, false>;
-        return any ? (void *)k_trace_batch<W, S, true, true> : (void *)k_trace_batch<W, S, false, true>;
+        if (which == 1) return any ? persistent<true, false>(count, last) : persistent<false, false>(count, last);
+        if (which == 3) return persistent<false, true>(count, last);  // closest hit only
+        if (which == 2) return any ? batch<true, false>(last) : batch<false, false>(last);
+        return any ? batch<true, true>(last) : batch<false, true>(last);
     }
 };
 
-template <int W> void *pick(uint32_t s, int which, bool any, bool count) {
+template <int W> void *pick(uint32_t s, int which, bool any, bool count, bool last) {
     switch (s) {
-        case 4: return Kernels<W, 4>::get(which, any, count);
-        case 16: return Kernels<W, 16>::get(which, any, count);
-        default: return Kernels<W, 8>::get(which, any, count);
+        case 4: return Kernels<W, 4>::get(which, any, count, last);
+        case 16: return Kernels<W, 16>::get(which, any, count, last);
+        default: return Kernels<W, 8>::get(which, any, count, last);
     }
 }
 
-// layout: Scene::layout (compressed nodes never count); which: 0 one lane per ray, 1 persistent, 2 persistent over many scenes (never counts), 3 persistent
-// storing refined hits, 4 persistent over many scenes storing refined hits
-void *pick_kernel(uint32_t layout, uint32_t s, int which, bool any, bool count) {
+// layout: Scene::layout (compressed nodes never count); which: 0 one lane per ray, 1 persistent, 2 persistent over many
+// scenes (never counts), 3 persistent storing refined hits, 4 persistent over many scenes storing refined hits; last:
+// the waves' last rays by teams (compressed nodes only)
+void *pick_kernel(uint32_t layout, uint32_t s, int which, bool any, bool count, bool last) {
     switch (layout) {
-        case kQ4: return pick<kQ4>(s, which, any, count);
-        case 2: return pick<2>(s, which, any, count);
-        case 8: return pick<8>(s, which, any, count);
-        default: return pick<4>(s, which, any, count);
+        case kQ4: return pick<kQ4>(s, which, any, count, last);
+        case 2: return pick<2>(s, which, any, count, last);
+        case 8: return pick<8>(s, which, any, count, last);
+        default: return pick<4>(s, which, any, count, last);
     }
 }
+
+// Whether a persistent launch of n rays ends with teams.  Up to 16,384 rays per CU: 2 M rays on 1 M triangles 530 us and
+// 549 without, 4 M 865 and 874.  Beyond, the share of the end is small and the larger kernel's main loop costs about
+// 1 %: 8 M rays 1,482 and 1,467, 16 M on 4 M triangles 3,444 and 3,387.
+bool ends_with_teams(const rt_context *ctx, uint64_t n) { return n <= 16384ull * (uint64_t)ctx->num_cus; }
 
 uint32_t persistent_grid(rt_context *ctx, const void *kernel, uint32_t block, size_t lds) {
     int per_cu = 0;
@@ -473,12 +545,12 @@ LaunchCfg resolve_cfg(const rt_context *ctx, const Scene &sc, const rt_launch_co
 // Four lanes per ray were slower than eight at every size.  A launch that counts tests per ray keeps
 // one lane per ray (its counts are those of the ordered traversal), as do the widths 2 and 8, a
 // caller's one-lane-per-ray configuration, and a tree too deep for the team's stack.
-static uint32_t team_size(const rt_context *ctx, const Scene &sc, uint32_t n, const LaunchCfg &c, bool count) {
-    if (sc.layout() != kQ4 || count || !c.persistent) return 0;
+static uint32_t team_size(const rt_context *ctx, uint32_t layout, uint32_t stack_bound, uint64_t n, const LaunchCfg &c) {
+    if (layout != kQ4 || !c.persistent) return 0;
     const uint64_t cus = (uint64_t)ctx->num_cus;
     if (n > 1536u * cus) return 0;
     const uint32_t t = n <= 24u * cus ? 64u : n <= 128u * cus ? 32u : n <= 1024u * cus ? 16u : 8u;
-    return team_limit(t, sc.stack_bound) ? t : 0u;
+    return team_limit(t, stack_bound) ? t : 0u;
 }
 
 void launch_trace(rt_context *ctx, const Scene &sc, const rt_ray *rays, uint32_t n, rt_hit *hits, uint32_t *counts,
@@ -492,29 +564,29 @@ void launch_trace(rt_context *ctx, const Scene &sc, const rt_ray *rays, uint32_t
     // and feel the refining kernel's registers (90 VGPRs, 5 waves per SIMD instead of 6) more: 3,270
     // against 3,410 Mrays/s, so they keep the separate pass.
     const bool refine_in_kernel = refine && !any && c.persistent;
-    TraceArgs a{view_of(sc), rays, hits, counts, n, c.refill, nullptr, c.leaf_weight, nullptr};
+    TraceArgs a{view_of(sc), rays, hits, counts, n, c.refill, nullptr, c.leaf_weight, nullptr, team_limit(kLastTeam, sc.stack_bound)};
     uint32_t layout = sc.layout();
     if (counts) {  // the counts are those of the exact boxes
         layout = sc.width;
         a.sc.nodes = a.sc.wide;
     }
     const size_t lds = stack_lds_bytes(c.lds_stack, c.block);
-    if (const uint32_t team = team_size(ctx, sc, n, c, counts != nullptr)) {
+    if (const uint32_t team = counts ? 0u : team_size(ctx, layout, sc.stack_bound, n, c)) {
         uint32_t limit = team_limit(team, sc.stack_bound);
         void *args[] = {&a, &limit};
-        RT_HIP(hipLaunchKernel(team_kernel(team, any, refine), dim3((n + 64u / team - 1) / (64u / team)), dim3(64), args, 0, stream));
+        RT_HIP(hipLaunchKernel(team_kernel(team, any, refine, false), dim3((n + 64u / team - 1) / (64u / team)), dim3(64), args, 0, stream));
         RT_HIP(hipGetLastError());
         return;
     }
     if (!c.persistent) {
-        void *k = pick_kernel(layout, c.lds_stack, 0, any, counts != nullptr);
+        void *k = pick_kernel(layout, c.lds_stack, 0, any, counts != nullptr, false);
         const uint32_t grid = (uint32_t)(((uint64_t)n + c.block - 1) / c.block);
         void *args[] = {&a};
         RT_HIP(hipLaunchKernel(k, dim3(grid), dim3(c.block), args, lds, stream));
     } else {
         a.work = ctx->counter_slot();
         k_zero_counter<<<1, 64, 0, stream>>>(a.work);
-        void *k = pick_kernel(layout, c.lds_stack, refine_in_kernel ? 3 : 1, any, counts != nullptr);
+        void *k = pick_kernel(layout, c.lds_stack, refine_in_kernel ? 3 : 1, any, counts != nullptr, ends_with_teams(ctx, n));
         // no more lanes than rays: a small batch would otherwise launch the whole device's worth of
         // waves, nearly all of which find no chunk and exit
         const uint32_t grid = (uint32_t)std::min<uint64_t>(persistent_grid(ctx, k, c.block, lds),
@@ -533,13 +605,14 @@ void launch_trace_queue(rt_context *ctx, const Scene &sc, const rt_ray *rays, ui
     check_stack(sc, c);
     SceneView v = view_of(sc);
     v.slot_prim = nullptr;  // hits carry leaf slots
-    TraceArgs a{v, rays, hits, nullptr, n_max, c.refill, ctx->counter_slot(), c.leaf_weight, n_dev};
+    TraceArgs a{v, rays, hits, nullptr, n_max, c.refill, ctx->counter_slot(), c.leaf_weight, n_dev,
+                team_limit(kLastTeam, sc.stack_bound)};
     const size_t lds = stack_lds_bytes(c.lds_stack, c.block);
     // camera rays of a small image: a team per ray (65,536 pixels on 200 k triangles: the frame 353 against 483 us)
-    if (const uint32_t team = n_dev || n_max > 1024u * (uint64_t)ctx->num_cus ? 0u : team_size(ctx, sc, n_max, c, false)) {
+    if (const uint32_t team = n_dev || n_max > 1024u * (uint64_t)ctx->num_cus ? 0u : team_size(ctx, sc.layout(), sc.stack_bound, n_max, c)) {
         uint32_t limit = team_limit(team, sc.stack_bound);
         void *args[] = {&a, &limit};
-        RT_HIP(hipLaunchKernel(team_kernel(team, false, false), dim3((n_max + 64u / team - 1) / (64u / team)), dim3(64),
+        RT_HIP(hipLaunchKernel(team_kernel(team, false, false, false), dim3((n_max + 64u / team - 1) / (64u / team)), dim3(64),
                                args, 0, stream));
         RT_HIP(hipGetLastError());
         return;
@@ -549,14 +622,14 @@ void launch_trace_queue(rt_context *ctx, const Scene &sc, const rt_ray *rays, ui
         // pixels, and about two thirds of them leave the scene at once.  One thread per ray lets
         // such waves retire and new ones start (0.45 vs 0.69 ms for the 1080p frame's primaries);
         // refilling lanes in a persistent wave mixes rays at different depths instead.
-        void *k = pick_kernel(sc.layout(), c.lds_stack, 0, false, false);
+        void *k = pick_kernel(sc.layout(), c.lds_stack, 0, false, false, false);
         void *args[] = {&a};
         RT_HIP(hipLaunchKernel(k, dim3((uint32_t)(((uint64_t)n_max + c.block - 1) / c.block)), dim3(c.block), args, lds, stream));
         RT_HIP(hipGetLastError());
         return;
     }
     k_zero_counter<<<1, 64, 0, stream>>>(a.work);
-    void *k = pick_kernel(sc.layout(), c.lds_stack, 1, false, false);
+    void *k = pick_kernel(sc.layout(), c.lds_stack, 1, false, false, ends_with_teams(ctx, n_max));
     const uint32_t grid = persistent_grid(ctx, k, c.block, lds);
     void *args[] = {&a};
     RT_HIP(hipLaunchKernel(k, dim3(grid), dim3(c.block), args, lds, stream));
@@ -569,28 +642,36 @@ void launch_trace_items(rt_context *ctx, const std::vector<TraceItem> &items, ui
     for (uint32_t layout : {2u, 4u, 8u, (uint32_t)kQ4}) {
         std::vector<BatchItemDev> hv;
         uint64_t total = 0;
+        uint32_t bound = 0;
         for (const TraceItem &it : items) {
             if (it.sc->layout() != layout) continue;
             RT_REQUIRE(it.n == 0 || (it.rays && it.hits), "batch item with NULL rays/hits");
             check_stack(*it.sc, c);
             hv.push_back(BatchItemDev{view_of(*it.sc), it.rays, it.hits, total});
             total += it.n;
+            bound = std::max(bound, it.sc->stack_bound);
         }
         if (total == 0) continue;
         int slot = 0;
         void *table = ctx->tables.stage(hv.data(), sizeof(BatchItemDev) * hv.size(), stream, slot);
-        unsigned long long *work = reinterpret_cast<unsigned long long *>(ctx->counter_slot());
-        k_zero_counter<<<1, 64, 0, stream>>>(reinterpret_cast<unsigned int *>(work));
-        BatchArgs a{static_cast<const BatchItemDev *>(table), (uint32_t)hv.size(), c.refill, total, work,
-                    c.leaf_weight};
-        const bool any = (flags & RT_TRACE_ANY) != 0;
-        const size_t lds = stack_lds_bytes(c.lds_stack, c.block);
-        void *k = pick_kernel(layout, c.lds_stack, (flags & RT_TRACE_FP32) ? 2 : 4, any, false);
-        const uint64_t chunks = (total + kChunk - 1) / kChunk, wpb = c.block / 64u;
-        const uint32_t grid = (uint32_t)std::max<uint64_t>(
-            1, std::min<uint64_t>(persistent_grid(ctx, k, c.block, lds), (chunks + wpb - 1) / wpb));
-        void *args[] = {&a};
-        RT_HIP(hipLaunchKernel(k, dim3(grid), dim3(c.block), args, lds, stream));
+        BatchArgs a{static_cast<const BatchItemDev *>(table), (uint32_t)hv.size(), c.refill, total, nullptr,
+                    c.leaf_weight, team_limit(kLastTeam, bound)};
+        const bool any = (flags & RT_TRACE_ANY) != 0, refine = (flags & RT_TRACE_FP32) == 0;
+        if (const uint32_t team = team_size(ctx, layout, bound, total, c)) {  // as for one scene
+            uint32_t limit = team_limit(team, bound);
+            void *args[] = {&a, &limit};
+            RT_HIP(hipLaunchKernel(team_kernel(team, any, refine, true), dim3(((uint32_t)total + 64u / team - 1) / (64u / team)),
+                                   dim3(64), args, 0, stream));
+        } else {
+            a.work = reinterpret_cast<unsigned long long *>(ctx->counter_slot());
+            k_zero_counter<<<1, 64, 0, stream>>>(reinterpret_cast<unsigned int *>(a.work));
+            const size_t lds = stack_lds_bytes(c.lds_stack, c.block);
+            void *k = pick_kernel(layout, c.lds_stack, refine ? 4 : 2, any, false, ends_with_teams(ctx, total));
+            const uint32_t grid = (uint32_t)std::min<uint64_t>(persistent_grid(ctx, k, c.block, lds),
+                                                               (total + c.block - 1) / c.block);
+            void *args[] = {&a};
+            RT_HIP(hipLaunchKernel(k, dim3(grid), dim3(c.block), args, lds, stream));
+        }
         RT_HIP(hipGetLastError());
         ctx->tables.commit(slot, stream);
     }

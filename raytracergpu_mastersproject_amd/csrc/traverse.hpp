@@ -40,11 +40,11 @@ template <typename T> struct ChunkSchedule {
     T n, nA, nB, KA, KB;
     uint32_t chunk;
 
-    // shrink: fewer rays per chunk when there are too few for every wave to take two chunks
+    // Fewer rays per chunk when there are too few for every wave to take two chunks
     // (a small launch then ends with its longest ray, not with a wave's run of rays)
-    __device__ __forceinline__ ChunkSchedule(T n_, uint32_t waves, bool shrink) {
+    __device__ __forceinline__ ChunkSchedule(T n_, uint32_t waves) {
         n = n_;
-        chunk = shrink ? (uint32_t)max((T)64u, min((T)kChunk, (T)(n / (2u * waves)) & ~(T)63u)) : kChunk;
+        chunk = (uint32_t)max((T)64u, min((T)kChunk, (T)(n / (2u * waves)) & ~(T)63u));
         const T lanes = (T)waves * 64u;
         const T nC = chunk > 64u ? min(n, (T)(2u * lanes)) : (T)0u;
         nB = chunk > 128u ? min((T)(n - nC), (T)(8u * lanes)) : (T)0u;
@@ -169,30 +169,37 @@ struct Trav {
 constexpr uint32_t kStackSlotBytes = 6;
 
 struct StackMem {
-    uint32_t *ent;    // this lane's LDS entry column: slot k at ent[k * stride]
+    uint32_t *ent;    // this lane's LDS entry column: slot k at ent[k * 64]
     uint16_t *key;    // this lane's LDS key column, same indexing
-    uint32_t stride;  // block size
     uint2 *spill;     // private spill array (kSpillCap entries of (entry, key << 16))
 };
 
-// LDS layout of a block: S x block entries, then S x block keys
+// A wave's LDS: S x 64 entries, then S x 64 keys; at least what the team stacks of its last rays need, which take
+// the same place (team.hpp).  6 KB a wave: 26 waves fit a CU, more than the registers let in.
+constexpr uint32_t kTeamStackWave = 768;  // team stack entries of 8 bytes per wave
+__host__ __device__ constexpr uint32_t wave_lds_bytes(uint32_t lds_stack) {
+    return lds_stack * 64u * kStackSlotBytes > kTeamStackWave * 8u ? lds_stack * 64u * kStackSlotBytes : kTeamStackWave * 8u;
+}
+template <int S> __device__ __forceinline__ uint32_t *wave_lds(void *lds) {
+    return static_cast<uint32_t *>(lds) + (threadIdx.x / 64u) * (wave_lds_bytes(S) / 4u);
+}
 template <int S> __device__ __forceinline__ StackMem stack_mem(void *lds, uint2 *spill) {
-    uint32_t *ent = static_cast<uint32_t *>(lds);
-    uint16_t *key = reinterpret_cast<uint16_t *>(ent + (size_t)S * blockDim.x);
-    return StackMem{ent + threadIdx.x, key + threadIdx.x, blockDim.x, spill};
+    uint32_t *ent = wave_lds<S>(lds);
+    uint16_t *key = reinterpret_cast<uint16_t *>(ent + (size_t)S * 64u);
+    return StackMem{ent + threadIdx.x % 64u, key + threadIdx.x % 64u, spill};
 }
 
 inline size_t stack_lds_bytes(uint32_t lds_stack, uint32_t block) {
-    return (size_t)kStackSlotBytes * lds_stack * block;
+    return (size_t)wave_lds_bytes(lds_stack) * (block / 64u);
 }
 
 template <int S> __device__ __forceinline__ void push(Trav &t, const StackMem &m, uint32_t e, uint32_t tnkey) {
     if (t.top - t.nspill == (uint32_t)S) {  // LDS part full: move its oldest entry out
-        const uint32_t o = (t.nspill & (S - 1)) * m.stride;
+        const uint32_t o = (t.nspill & (S - 1)) * 64u;
         if (t.nspill < kSpillCap) m.spill[t.nspill] = make_uint2(m.ent[o], (uint32_t)m.key[o] << 16);
         t.nspill++;
     }
-    const uint32_t o = (t.top & (S - 1)) * m.stride;
+    const uint32_t o = (t.top & (S - 1)) * 64u;
     m.ent[o] = e;
     m.key[o] = (uint16_t)(tnkey >> 16);
     t.top++;
@@ -202,7 +209,7 @@ template <int S> __device__ __forceinline__ void pop(Trav &t, const StackMem &m)
     uint2 v;
     if (t.top > t.nspill) {
         t.top--;
-        const uint32_t o = (t.top & (S - 1)) * m.stride;
+        const uint32_t o = (t.top & (S - 1)) * 64u;
         v = make_uint2(m.ent[o], (uint32_t)m.key[o] << 16);
     } else {
         t.nspill--;
@@ -484,7 +491,7 @@ __device__ __forceinline__ void node_step_q(Trav &t, const StackMem &m, const ui
     t.have = __double2hiint(key[0]) < (int)kMissKey;
     if (t.have) {
         while (t.top + 3u - t.nspill > (uint32_t)S) {  // room for three in the LDS part: move its oldest entries out
-            const uint32_t o = (t.nspill & (S - 1)) * m.stride;
+            const uint32_t o = (t.nspill & (S - 1)) * 64u;
             if (t.nspill < kSpillCap) m.spill[t.nspill] = make_uint2(m.ent[o], (uint32_t)m.key[o] << 16);
             t.nspill++;
         }
@@ -492,7 +499,7 @@ __device__ __forceinline__ void node_step_q(Trav &t, const StackMem &m, const ui
         for (int k = 3; k >= 1; --k) {
             const uint32_t hi = (uint32_t)__double2hiint(key[k]);
             if ((int)hi < (int)kMissKey) {
-                const uint32_t o = (t.top & (S - 1)) * m.stride;
+                const uint32_t o = (t.top & (S - 1)) * 64u;
                 m.ent[o] = (uint32_t)__double2loint(key[k]);
                 m.key[o] = (uint16_t)(hi >> 16);
                 t.top++;
@@ -512,7 +519,7 @@ template <int S, bool ANY> __device__ __forceinline__ void pop_q(Trav &t, const 
     uint32_t e;
     float tn;
     if (t.top >= t.nspill) {
-        const uint32_t o = (t.top & (S - 1)) * m.stride;
+        const uint32_t o = (t.top & (S - 1)) * 64u;
         e = m.ent[o];
         asm("" : "+v"(e));  // else this load and the other become one through a generic pointer
         tn = __uint_as_float((uint32_t)m.key[o] << 16);

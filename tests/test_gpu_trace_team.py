@@ -17,7 +17,8 @@ def _same(a, b):
 
 
 @pytest.mark.parametrize("any_hit", [False, True])
-@pytest.mark.parametrize("n", [1, 63, 6144, 6145, 32768, 32769, 262144, 262145, 393216, 393217, 786432, 786433])
+@pytest.mark.parametrize("n", [1, 63, 6144, 6145, 32768, 32769, 262144, 262145, 393216, 393217, 786432, 786433, 4194304,
+                               4194305])
 def test_sizes_agree_with_one_lane_per_ray(ctx, native, n, any_hit):
     tris, mats = small_cluster_scene(16, 4096, seed=31)
     sid = ctx.upload(tris, with_spheres(tris, mats, 7), mats)

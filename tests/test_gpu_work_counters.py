@@ -1,5 +1,5 @@
 """Persistent launches at the numbers of waves at which they use one, two, ... 32 work counters: every ray, pixel and
-path is taken exactly once, so results equal those of one lane per ray and of the other schedule, bit for bit."""
+path is taken exactly once (batches of few rays: several lanes per ray), so results equal those of one lane per ray and of the other schedule, bit for bit."""
 import numpy as np
 import pytest
 
@@ -29,18 +29,20 @@ def test_trace(ctx, native, n, width):
     ctx.release(sid)
 
 
-@pytest.mark.parametrize("sizes", [[1], [64] * 7, [4096, 1, 0, 33_000], [70_001] * 9])
-def test_batch(ctx, native, sizes):
+@pytest.mark.parametrize("any_hit,fp32", [(False, False), (False, True), (True, False), (True, True)])
+@pytest.mark.parametrize("sizes", [[1], [0, 5, 0], [64] * 7, [4096, 1, 0, 33_000], [3] * 200 + [200_000], [70_001] * 9])
+def test_batch(ctx, native, sizes, any_hit, fp32):
     tris, mats = small_cluster_scene(4, 500, seed=93)
     sids = [ctx.upload(tris[k:], None, mats) for k in range(2)]
     items, want = [], []
     for k, n in enumerate(sizes):
         rays = W.incoherent_rays(max(n, 1), *W.scene_bounds(tris), seed=94 + k)
         items.append((sids[k % 2], n, native.DeviceArray.from_numpy(rays), native.DeviceArray(16 * max(n, 1))))
-        want.append(gpu_trace(ctx, sids[k % 2], rays[:n]))
-    ctx.trace_batch(items)
+        want.append(gpu_trace(ctx, sids[k % 2], rays[:n], any_hit=any_hit, fp32=fp32,
+                              cfg=native.launch_config(block=64, lds_stack=8, persistent=0)) if n else None)
+    ctx.trace_batch(items, any_hit=any_hit, fp32=fp32)
     for (_, n, _, hits), w in zip(items, want):
-        assert np.array_equal(hits.to_numpy(L.HIT, n).view(np.uint32), w.view(np.uint32))
+        assert n == 0 or np.array_equal(hits.to_numpy(L.HIT, n).view(np.uint32), w.view(np.uint32))
     for s in sids:
         ctx.release(s)
 
