@@ -241,6 +241,7 @@ struct RenderJob {
     uint32_t nwide, width, height, spp;
     uint32_t depth, random_state, flags, tiles_x;
     uint32_t first_item, nitems, group;
+    uint32_t stack_bound;  // the scene's
     uint32_t layout;  // of `nodes` (Scene::layout, or the width from a camera beyond Scene::far_limit); group: samples per split item (0 = whole pixels)
     float cam[12];  // pixel00, deltaU, deltaV, origin
 };

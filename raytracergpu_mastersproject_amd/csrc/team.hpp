@@ -171,10 +171,15 @@ __device__ __forceinline__ TeamHit team_trace(bool live, v3 o, v3 d, float tmin,
 // 432 -> 375 us.  Rays start over; fewer rays (6: 386 us) or more in two rounds (12: 404) are slower.
 constexpr uint32_t kLastTeam = 8, kLastRays = 64 / kLastTeam;
 
-// The lane whose ray this lane's team takes over; `live`: at most kLastRays lanes, and not none.
-__device__ __forceinline__ uint32_t last_ray_lane(unsigned long long live) {
-    for (uint32_t k = (threadIdx.x & 63u) / kLastTeam; k > 0u && (live & (live - 1ull)) != 0ull; --k) live &= live - 1ull;
+// The lane whose ray this lane's team of T takes over; `live`: at most 64 / T lanes, and not none.
+template <int T> __device__ __forceinline__ uint32_t last_ray_lane(unsigned long long live) {
+    for (uint32_t k = (threadIdx.x & 63u) / T; k > 0u && (live & (live - 1ull)) != 0ull; --k) live &= live - 1ull;
     return (uint32_t)__ffsll(live) - 1u;
+}
+
+// team_limit of T lanes, from that of kLastTeam
+template <int T> __device__ __forceinline__ uint32_t last_limit(uint32_t limit) {
+    return limit + (team_stack(T) - 3u * (T / 4u)) - (team_stack(kLastTeam) - 3u * (kLastTeam / 4u));
 }
 
 }  // namespace rtgpu

@@ -253,7 +253,7 @@ __global__ __launch_bounds__(256, W == kQ4 ? 5 : 1) void k_trace_persistent(Trac
     if constexpr (LAST) {
         const unsigned long long live = __ballot(rid != kNoRay);
         if (live == 0ull) return;
-        const uint32_t i = (uint32_t)__shfl((int)rid, (int)last_ray_lane(live));
+        const uint32_t i = (uint32_t)__shfl((int)rid, (int)last_ray_lane<kLastTeam>(live));
         trace_last<S, ANY, REFINE>(live, a.sc, a.rays, a.hits, i, lds, a.limit);
     }
 }
@@ -412,7 +412,7 @@ __global__ __launch_bounds__(256, W == kQ4 ? 5 : 1) void k_trace_batch(BatchArgs
     if constexpr (LAST) {
         const unsigned long long live = __ballot(active);
         if (live == 0ull) return;
-        const int from = (int)last_ray_lane(live);
+        const int from = (int)last_ray_lane<kLastTeam>(live);
         const BatchItemDev &it = a.items[(uint32_t)__shfl((int)item, from)];
         trace_last<S, ANY, REFINE>(live, it.sc, it.rays, it.hits, (uint32_t)__shfl((int)local, from), lds, a.limit);
     }

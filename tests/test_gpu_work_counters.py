@@ -61,3 +61,27 @@ def test_render(ctx, native, w, h, spp, width):
         images.append(acc.to_numpy(np.uint32))
     assert all(np.array_equal(images[0], i) for i in images[1:])
     ctx.release(sid)
+
+
+@pytest.mark.parametrize("flags", [0, 4, 8, 10])  # split as the launch chooses, samples, whole pixels, no cached primaries
+@pytest.mark.parametrize("sizes", [[(1, 1, 3)], [(8, 8, 1), (64, 48, 4)], [(256, 256, 2), (100, 70, 5), (33, 9, 12)]])
+def test_last_items_of_fused_images(ctx, native, sizes, flags):
+    """The last items of each wave go on with several lanes each: images and segment counts as from single calls."""
+    setups = [W.served_scene(2000 + 9000 * k, 96 + k) for k in range(len(sizes))]
+    sids = [ctx.upload(s["tris"], None, s["materials"], leaf_size=1 + k) for k, s in enumerate(setups)]
+    seg, one = native.DeviceArray(8), native.DeviceArray(8)
+    seg.zero(), one.zero()
+    accs = [native.DeviceArray(16 * w * h) for w, h, _ in sizes]
+    for a, (w, h, _) in zip(accs, sizes):
+        ctx.accum_clear(a, w * h)
+    ctx.render_batch([(sid, s["params"], w, h, spp, a, flags)
+                      for sid, s, a, (w, h, spp) in zip(sids, setups, accs, sizes)], segments=seg)
+    wave = native.RENDER_WAVEFRONT | (flags & native.RENDER_NO_PRIMARY_CACHE)
+    for sid, s, a, (w, h, spp) in zip(sids, setups, accs, sizes):
+        ref = native.DeviceArray(16 * w * h)
+        ctx.accum_clear(ref, w * h)
+        ctx.render(sid, s["params"], w, h, spp, ref, flags=wave, segments=one)
+        assert np.array_equal(a.to_numpy(np.uint32), ref.to_numpy(np.uint32))
+        ctx.release(sid)
+    if flags & native.RENDER_NO_SPLIT:  # an item holds all samples of its pixel
+        assert int(seg.to_numpy(np.uint64, 1)[0]) == int(one.to_numpy(np.uint64, 1)[0])
