@@ -176,6 +176,11 @@ template <int T, bool ANY, bool REFINE> __global__ __launch_bounds__(64) void k_
 
 constexpr uint32_t kNoRay = ~0u;
 
+// Whether fp32 results wait for the refill too.  16.8 M rays on compressed nodes: closest hit 3,777 -> 3,300 us, any hit
+// 3,452 -> 3,090; exact width-4 nodes with counts, 4 M rays 947 -> 906.  Width 2 is slower with it (1,116 -> 1,180 us)
+// and width 8's any hit too (1,052 -> 1,078).
+template <int W> constexpr bool kDefer = W == kQ4 || W == 4;
+
 // REFINE: store each hit with t, u, v refined in double (store_refined) instead of the fp32 values.
 // LAST: the wave's last rays go on with teams of lanes (trace_last).
 template <int W, int S, bool ANY, bool COUNT, bool REFINE, bool LAST>
@@ -186,9 +191,9 @@ __global__ __launch_bounds__(256, W == kQ4 ? 5 : 1) void k_trace_persistent(Trac
     const uint32_t lane = threadIdx.x & 63u;
     const unsigned long long lt = lane ? (~0ull >> (64u - lane)) : 0ull;
     uint32_t rid = kNoRay;  // a launch has fewer rays than this
-    // REFINE: a finished ray's result is stored at the wave's next refill (or at the end), where the
-    // lanes that finished since the last refill refine together; refining as each lane finishes would
-    // run the double-precision code on almost every iteration.  Without refinement a lane stores at once.
+    // A finished ray's result is stored at the wave's next refill (or at the end), with those of the lanes that finished
+    // since the last one: storing, and refining in double, as each lane finishes would run that code on almost every
+    // iteration.  See kDefer for fp32 results.
     uint32_t done = kNoRay;
     bool exhausted = false;
     uint32_t q_next = 0, q_end = 0;  // the wave's current chunk of ray indices (wave-uniform)
@@ -244,7 +249,7 @@ __global__ __launch_bounds__(256, W == kQ4 ? 5 : 1) void k_trace_persistent(Trac
         }
         walk_pop<W, S, ANY>(t, m);
         if (rid != kNoRay && trav_done(t)) {
-            if constexpr (REFINE) done = rid;
+            if constexpr (REFINE || kDefer<W>) done = rid;
             else store(rid);
             rid = kNoRay;
         }
@@ -334,7 +339,7 @@ __global__ __launch_bounds__(256, W == kQ4 ? 5 : 1) void k_trace_batch(BatchArgs
     const uint32_t lane = threadIdx.x & 63u;
     const unsigned long long lt = lane ? (~0ull >> (64u - lane)) : 0ull;
     bool active = false, exhausted = false;
-    bool pending = false;  // REFINE: a finished ray (item, local) whose result waits for the wave's next refill
+    bool pending = false;  // a finished ray (item, local) whose result waits for the wave's next refill
     uint32_t item = 0, local = 0;
     uint64_t q_next = 0, q_end = 0;  // the wave's current chunk of global ray indices
     uint32_t c_lo = 0, c_hi = 1;     // the items the chunk's rays belong to: [c_lo, c_hi)
@@ -403,7 +408,7 @@ __global__ __launch_bounds__(256, W == kQ4 ? 5 : 1) void k_trace_batch(BatchArgs
         }
         walk_pop<W, S, ANY>(t, m);
         if (active && trav_done(t)) {
-            if constexpr (REFINE) pending = true;
+            if constexpr (REFINE || kDefer<W>) pending = true;
             else store();
             active = false;
         }
@@ -473,7 +478,7 @@ template <int W, int S> struct Kernels {
     static void *get(int which, bool any, bool count, bool last) {
         if (which == 0) return any ? direct<true>(count) : direct<false>(count);
         if (which == 1) return any ? persistent<true, false>(count, last) : persistent<false, false>(count, last);
-        if (which == 3) return persistent<false, true>(count, last);  // closest hit only
+        if (which == 3) return any ? persistent<true, true>(count, last) : persistent<false, true>(count, last);
         if (which == 2) return any ? batch<true, false>(last) : batch<false, false>(last);
         return any ? batch<true, true>(last) : batch<false, true>(last);
     }
@@ -559,11 +564,10 @@ void launch_trace(rt_context *ctx, const Scene &sc, const rt_ray *rays, uint32_t
     RT_REQUIRE(rays && hits, "rays/hits must be device pointers");
     check_stack(sc, c);
     const bool any = (flags & RT_TRACE_ANY) != 0, refine = (flags & RT_TRACE_FP32) == 0;
-    // Closest-hit persistent launches refine in the kernel, at each wave's refills: measured on one box,
-    // 5.11-5.14 ms per 16M-ray query against 5.19 ms with the separate pass.  Any-hit rays end sooner
-    // and feel the refining kernel's registers (90 VGPRs, 5 waves per SIMD instead of 6) more: 3,270
-    // against 3,410 Mrays/s, so they keep the separate pass.
-    const bool refine_in_kernel = refine && !any && c.persistent;
+    // Persistent launches refine in the kernel, at each wave's refills: a separate pass reads every ray and hit again
+    // (16.8 M any-hit rays 3,390 us with it, 3,295 without; 1 M on 1,024 triangles 106 and 100).  Width 8's any hit, with
+    // its larger kernel, keeps the pass (4 M rays 1,093 us, 1,118 in the kernel).
+    const bool refine_in_kernel = refine && c.persistent && !(any && sc.width == 8);
     TraceArgs a{view_of(sc), rays, hits, counts, n, c.refill, nullptr, c.leaf_weight, nullptr, team_limit(kLastTeam, sc.stack_bound)};
     uint32_t layout = sc.layout();
     if (counts) {  // the counts are those of the exact boxes
