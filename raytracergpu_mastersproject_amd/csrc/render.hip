@@ -1036,8 +1036,8 @@ __global__ void k_resolve(const float4 *accum, uint32_t npix, uint32_t spp, floa
     }
 }
 
-__global__ void k_zero(unsigned int *c) {
-    if (threadIdx.x == 0) c[0] = 0u;
+__global__ void k_zero(unsigned int *c, uint32_t words) {
+    if (threadIdx.x < words) c[threadIdx.x] = 0u;
 }
 
 __global__ void k_zero_lines(unsigned int *work) {
@@ -1315,14 +1315,13 @@ void launch_render_wave(rt_context *ctx, const Scene &sc, const RenderJob &j, un
         }
         int cur = 0;
         const uint32_t finish_at = wave_finish_bounce();
-        k_zero<<<1, 64, 0, stream>>>(count + cur);
+        k_zero<<<1, 64, 0, stream>>>(count, 2u);  // both queues, in one launch
         a.bounce = 0;
         a.hits_in = first_hits;
         a.rays_out = rays[cur];
         a.ids_out = ids[cur];
         a.n_out = count + cur;
         if (finish_at == 1) {  // dielectric scatters into the second queue, which the finish kernel takes first
-            k_zero<<<1, 64, 0, stream>>>(count + 1);
             a.rays_out2 = rays[1];
             a.ids_out2 = ids[1];
             a.n_out2 = count + 1;
@@ -1348,7 +1347,7 @@ void launch_render_wave(rt_context *ctx, const Scene &sc, const RenderJob &j, un
                 if (many) work = reinterpret_cast<unsigned int *>((reinterpret_cast<uintptr_t>(hits) + 127u) & ~uintptr_t(127));
                 const uint32_t lines = many ? kCounterLines : 1u;
                 if (many) k_zero_lines<<<1, 64, 0, stream>>>(work);
-                else k_zero<<<1, 64, 0, stream>>>(work);
+                else k_zero<<<1, 64, 0, stream>>>(work, 1u);
                 if (const uint32_t team = yield ? 0u : path_team_size(ctx, j.layout, sc.stack_bound, paths)) {
                     TeamPathArgs ta{a, work, lines, team_limit(team, sc.stack_bound)};
                     void *k = pick_path_team(team);
@@ -1381,7 +1380,7 @@ void launch_render_wave(rt_context *ctx, const Scene &sc, const RenderJob &j, un
                 break;
             }
             launch_trace_queue(ctx, sc, rays[cur], (uint32_t)paths, count + cur, hits, tc, stream);
-            k_zero<<<1, 64, 0, stream>>>(count + (cur ^ 1));
+            k_zero<<<1, 64, 0, stream>>>(count + (cur ^ 1), 1u);
             a.bounce = b;
             a.rays_in = rays[cur];
             a.ids_in = ids[cur];
