@@ -362,7 +362,7 @@ __global__ __launch_bounds__(256, W == kQ4 ? 5 : 1) void k_trace_batch(BatchArgs
         const unsigned long long idle = __ballot(!active);
         const uint32_t nidle = (uint32_t)__popcll(idle);
         if (!exhausted && nidle >= a.refill) {
-            if (pending) {  // as in k_trace_persistent: the lanes that finished refine together
+            if (pending) {  // as in k_trace_persistent: the lanes that finished store together
                 store();
                 pending = false;
             }
@@ -612,7 +612,7 @@ void launch_trace_queue(rt_context *ctx, const Scene &sc, const rt_ray *rays, ui
     TraceArgs a{v, rays, hits, nullptr, n_max, c.refill, ctx->counter_slot(), c.leaf_weight, n_dev,
                 team_limit(kLastTeam, sc.stack_bound)};
     const size_t lds = stack_lds_bytes(c.lds_stack, c.block);
-    // camera rays of a small image: a team per ray (65,536 pixels on 200 k triangles: the frame 353 against 483 us)
+    // camera rays of a small image: a team per ray (65,536 pixels on 200 k triangles: 130 us less per frame)
     if (const uint32_t team = n_dev || n_max > 1024u * (uint64_t)ctx->num_cus ? 0u : team_size(ctx, sc.layout(), sc.stack_bound, n_max, c)) {
         uint32_t limit = team_limit(team, sc.stack_bound);
         void *args[] = {&a, &limit};
