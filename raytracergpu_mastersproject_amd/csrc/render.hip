@@ -127,7 +127,7 @@ __device__ __forceinline__ void begin_segment(const RenderArgs &a, PixelState &p
         ps.phase = kResolved;
         return;
     }
-    trav_init<W>(t, ps.o, ps.d, 0.001f, 10000000.0f, job_of<MULTI>(a, ps).nwide);
+    trav_init<W, false>(t, ps.o, ps.d, 0.001f, 10000000.0f, job_of<MULTI>(a, ps).nwide, job_of<MULTI>(a, ps).reach);
     ps.phase = kTracing;
     segs++;
 }
@@ -345,6 +345,14 @@ struct JobBoxes {
     __device__ LeafBoxes operator()() const { return LeafBoxes{j.wide, j.slot_ref}; }
 };
 
+// A finished segment: again in the exact nodes' order if its hit depends on the order (rare).
+template <int W, int S>
+__device__ __forceinline__ void end_segment(Trav &t, const StackMem &m, const RenderJob &J, uint32_t leaf_weight) {
+    if constexpr (W == kQ4)
+        if (__builtin_expect(t.bslot == kRedo, 0))
+            walk_exact<S, false>(t, m, t.o, t.d, 0.001f, 10000000.0f, J.nwide, J.wide, J.rec, JobBoxes{J}, leaf_weight);
+}
+
 __device__ __forceinline__ uint32_t from_lane(uint32_t v, int lane) { return (uint32_t)__shfl((int)v, lane); }
 __device__ __forceinline__ float from_lane(float v, int lane) { return __shfl(v, lane); }
 __device__ __forceinline__ v3 from_lane(v3 v, int lane) {
@@ -360,7 +368,7 @@ constexpr int kFewTeam = 32;
 
 template <int S, bool MULTI, int T>
 __device__ __forceinline__ void render_last(const RenderArgs &a, unsigned long long live, const PixelState &ps,
-                                            uint32_t &segs, uint32_t *lds) {
+                                            uint32_t &segs, uint32_t *lds, const StackMem &m) {
     const int src = (int)last_ray_lane<T>(live);
     PixelState q;  // every lane reads, whether its team takes an item or not: the source lanes are any
     q.phase = from_lane(ps.phase, src);
@@ -395,8 +403,8 @@ __device__ __forceinline__ void render_last(const RenderArgs &a, unsigned long l
         live = __ballot(q.phase != kIdle && threadIdx.x % T == 0u);
         if (live == 0ull || (T < kFewTeam && (uint32_t)__popcll(live) <= 64u / kFewTeam)) break;
         const bool tracing = q.phase == kTracing;
-        const TeamHit h = team_trace<T, false>(tracing, q.o, q.d, 0.001f, 10000000.0f, J.wide, J.nwide, J.rec, stacks,
-                                               last_limit<T>(a.limit));
+        const TeamHit h = team_closest<T, S>(tracing, q.o, q.d, 0.001f, 10000000.0f, J.wide, J.nwide, J.rec, stacks,
+                                             last_limit<T>(a.limit), J.reach, m, JobBoxes{J});
         if (tracing) {
             q.hslot = h.slot;
             q.ht = h.t;
@@ -405,7 +413,7 @@ __device__ __forceinline__ void render_last(const RenderArgs &a, unsigned long l
     }
     if (threadIdx.x % T == 0u) segs += traced;
     if constexpr (T < kFewTeam)
-        if (live != 0ull) render_last<S, MULTI, kFewTeam>(a, live, q, segs, lds);
+        if (live != 0ull) render_last<S, MULTI, kFewTeam>(a, live, q, segs, lds, m);
 }
 
 template <int W, int S, bool MULTI>
@@ -490,6 +498,7 @@ __global__ __launch_bounds__(256, W == kQ4 ? 3 : 1) void k_render(RenderArgs a) 
             }
             if (tracing) walk_pop<W, S, false>(t, m);
             if (tracing && trav_done(t)) {
+                end_segment<W, S>(t, m, job_of<MULTI>(a, ps), a.leaf_weight);
                 ps.hslot = t.bslot;
                 ps.ht = t.bt;
                 ps.phase = kResolved;
@@ -498,7 +507,7 @@ __global__ __launch_bounds__(256, W == kQ4 ? 3 : 1) void k_render(RenderArgs a) 
     }
     if constexpr (W == kQ4) {
         const unsigned long long live = __ballot(ps.phase != kIdle);
-        if (live != 0ull) render_last<S, MULTI, kLastTeam>(a, live, ps, segs, lds);
+        if (live != 0ull) render_last<S, MULTI, kLastTeam>(a, live, ps, segs, lds, m);
     }
     if (a.segments) {
         unsigned long long s = segs;
@@ -572,8 +581,31 @@ struct WaveArgs {
     const uint32_t *n_in2;
     float4 *col;  // [path] {colour, carry out}
     float4 *att;  // [path] {attenuation, RNG state bits}
+    // Paths that k_wave_finish or k_path_team leaves to k_path_redo: their number, and the queue buffer other than rays_in
+    // (left_cap entries), see left_entry.
+    uint32_t *left;
+    rt_ray *left_rays;
+    uint32_t left_cap;
     unsigned long long *segments;
 };
+
+// The place of the k-th path left, behind the two queues' entries: the queues hold at most left_cap paths together, so
+// there is room for all of them.
+__device__ __forceinline__ float4 *left_entry(const WaveArgs &a, uint32_t k) {
+    const uint32_t n2 = a.n_in2 ? *a.n_in2 : 0u, first = a.left_cap - n2;
+    rt_ray *r = k < first ? a.left_rays + n2 + k : const_cast<rt_ray *>(a.rays_in) + *a.n_in + (k - first);
+    return reinterpret_cast<float4 *>(r);
+}
+
+// A path whose segment must be traced in the exact nodes' order (kRedo): its state as the segment begins.
+__device__ __forceinline__ void leave_path(const WaveArgs &a, uint32_t p, uint32_t bounce, uint32_t st, float next, v3 color,
+                                           v3 atten, v3 o, v3 d) {
+    a.col[p] = make_float4(color.x, color.y, color.z, next);
+    a.att[p] = make_float4(atten.x, atten.y, atten.z, __uint_as_float(st));
+    float4 *q = left_entry(a, atomicAdd(a.left, 1u));
+    q[0] = make_float4(o.x, o.y, o.z, __uint_as_float(bounce));
+    q[1] = make_float4(d.x, d.y, d.z, __uint_as_float(p));
+}
 
 __device__ __forceinline__ void store_ray(rt_ray *rays, uint32_t i, v3 o, v3 d) {
     float4 *q = reinterpret_cast<float4 *>(rays + i);
@@ -791,6 +823,10 @@ __device__ __forceinline__ void finish_last(const FinishArgs &f, unsigned long l
     if ((threadIdx.x & 63u) / T >= (uint32_t)__popcll(live)) q.phase = kIdle;
     uint2 *stacks = reinterpret_cast<uint2 *>(wave_lds<S>(lds));
     for (;;) {
+        if (q.phase == kResolved && q.hslot == kRedo) {
+            if (threadIdx.x % T == 0u) leave_path(f.w, q.p, q.bounce, q.st, q.next, q.color, q.atten, q.o, q.d);
+            q.phase = kIdle;
+        }
         if (q.phase == kResolved) {
             if (shade_segment(J, J.rec, q.hslot, q.ht, q.o, q.d, q.st, q.color, q.atten) && q.bounce + 1 < J.depth) {
                 q.bounce++;
@@ -805,9 +841,9 @@ __device__ __forceinline__ void finish_last(const FinishArgs &f, unsigned long l
         if (live == 0ull || (T < kFewTeam && (uint32_t)__popcll(live) <= 64u / kFewTeam)) break;
         const bool tracing = q.phase == kTracing;
         const TeamHit h = team_trace<T, false>(tracing, q.o, q.d, 0.001f, 10000000.0f, J.wide, J.nwide, J.rec, stacks,
-                                               last_limit<T>(f.limit));
+                                               last_limit<T>(f.limit), J.reach);
         if (tracing) {
-            q.hslot = h.slot;
+            q.hslot = h.redo ? kRedo : h.slot;
             q.ht = h.t;
             q.phase = kResolved;
         }
@@ -874,7 +910,7 @@ template <int W, int S> __global__ __launch_bounds__(256, W == kQ4 ? 5 : 1) void
                     atten = v3{at.x, at.y, at.z};
                     st = __float_as_uint(at.w);
                     bounce = a.bounce;
-                    trav_init<W>(t, v3{r0.x, r0.y, r0.z}, v3{r1.x, r1.y, r1.z}, r0.w, r1.w, J.nwide);
+                    trav_init<W, false>(t, v3{r0.x, r0.y, r0.z}, v3{r1.x, r1.y, r1.z}, r0.w, r1.w, J.nwide, J.reach);
                     phase = kTracing;
                 }
                 q_next += take;
@@ -885,11 +921,15 @@ template <int W, int S> __global__ __launch_bounds__(256, W == kQ4 ? 5 : 1) void
         if (W == kQ4 && exhausted && f.limit && (uint32_t)__popcll(live) <= kLastRays) break;
         const unsigned long long mres = __ballot(phase == kResolved), mtr = __ballot(phase == kTracing);
         if (shade_now(mres, mtr, f.shade_min)) {
+            if (W == kQ4 && phase == kResolved && hslot == kRedo) {
+                leave_path(a, p, bounce, st, next, color, atten, t.o, t.d);
+                phase = kIdle;
+            }
             if (phase == kResolved) {
                 v3 o = t.o, d = t.d;
                 if (shade_segment(J, J.rec, hslot, ht, o, d, st, color, atten) && bounce + 1 < J.depth) {
                     bounce++;
-                    trav_init<W>(t, o, d, 0.001f, 10000000.0f, J.nwide);
+                    trav_init<W, false>(t, o, d, 0.001f, 10000000.0f, J.nwide, J.reach);
                     phase = kTracing;
                     segs++;
                 } else {
@@ -936,7 +976,7 @@ struct TeamPathArgs {
     uint32_t limit;  // team_trace's
 };
 
-template <int T> __global__ __launch_bounds__(64) void k_path_team(TeamPathArgs f) {
+template <int T> __global__ __launch_bounds__(64, 6) void k_path_team(TeamPathArgs f) {
     __shared__ uint2 stacks[64 / T * team_stack(T)];
     const WaveArgs &a = f.w;
     const RenderJob &J = a.J;
@@ -979,8 +1019,11 @@ template <int T> __global__ __launch_bounds__(64) void k_path_team(TeamPathArgs 
             }
         }
         if (__ballot(live) == 0ull) break;
-        const TeamHit h = team_trace<T, false>(live, o, d, 0.001f, 10000000.0f, J.wide, J.nwide, J.rec, stacks, f.limit);
-        if (live) {
+        const TeamHit h = team_trace<T, false>(live, o, d, 0.001f, 10000000.0f, J.wide, J.nwide, J.rec, stacks, f.limit, J.reach);
+        if (live && h.redo) {
+            if (lane == first_lane) leave_path(a, p, bounce, st, next, color, atten, o, d);
+            live = false;
+        } else if (live) {
             if (shade_segment(J, J.rec, h.slot, h.t, o, d, st, color, atten) && bounce + 1 < J.depth) {
                 bounce++;
                 segs++;
@@ -995,6 +1038,43 @@ template <int T> __global__ __launch_bounds__(64) void k_path_team(TeamPathArgs 
         for (int off = 32; off > 0; off >>= 1) sg += __shfl_xor(sg, off);
         if (lane == 0 && sg) atomicAdd(a.segments, sg);
     }
+}
+
+// The paths left over, a lane each, in the exact nodes' order to their ends.  Usually there are none (an empty launch takes
+// 3 us; with this walk in the kernels before, frames of 1 M paths took 7 % longer and of 33 M 2 %).
+__global__ __launch_bounds__(128) void k_path_redo(WaveArgs a, uint32_t leaf_weight) {
+    extern __shared__ uint32_t lds[];
+    const uint32_t n = *a.left;
+    if (n == 0u) return;
+    uint2 spill[kSpillCap];
+    const StackMem m = stack_mem<16>(lds, spill);
+    const RenderJob &J = a.J;
+    uint32_t segs = 0;
+    for (uint32_t i = blockIdx.x * blockDim.x + threadIdx.x; i < n; i += gridDim.x * blockDim.x) {
+        const float4 *q = left_entry(a, i);
+        const float4 r0 = q[0], r1 = q[1];
+        const uint32_t p = __float_as_uint(r1.w);
+        uint32_t bounce = __float_as_uint(r0.w);
+        v3 o{r0.x, r0.y, r0.z}, d{r1.x, r1.y, r1.z};
+        const float4 c = a.col[p], at = a.att[p];
+        v3 color{c.x, c.y, c.z}, atten{at.x, at.y, at.z};
+        uint32_t st = __float_as_uint(at.w);
+        for (;;) {
+            Trav t;
+            walk_exact<16, false>(t, m, o, d, 0.001f, 10000000.0f, J.nwide, J.wide, J.rec, JobBoxes{J}, leaf_weight);
+            if (!shade_segment(J, J.rec, t.bslot, t.bt, o, d, st, color, atten) || bounce + 1 >= J.depth) break;
+            bounce++;
+            segs++;
+        }
+        a.col[p] = make_float4(color.x, color.y, color.z, c.w);
+    }
+    if (a.segments && segs) atomicAdd(a.segments, (unsigned long long)segs);
+}
+
+void launch_path_redo(rt_context *ctx, const WaveArgs &a, uint32_t leaf_weight, hipStream_t stream) {
+    if (a.J.layout != (uint32_t)kQ4) return;
+    k_path_redo<<<(uint32_t)ctx->num_cus * 8u, 128, stack_lds_bytes(16, 128), stream>>>(a, leaf_weight);
+    RT_HIP(hipGetLastError());
 }
 
 void *pick_path_team(uint32_t t) {
@@ -1044,9 +1124,10 @@ __global__ void k_zero_lines(unsigned int *work) {
     if (threadIdx.x < kCounterLines) work[threadIdx.x * kCounterStride] = 0u;
 }
 
-// Before a yielded finish launch is resumed: its work counter back to where the yield left it.
-__global__ void k_resume_counter(unsigned int *work) {
+// Before a yielded finish launch is resumed: its work counter back to where the yield left it, and no paths left over.
+__global__ void k_resume_counter(unsigned int *work, uint32_t *left) {
     if (threadIdx.x == 0 && (work[0] & kYieldBit)) work[0] = work[1];
+    if (threadIdx.x == 0) *left = 0u;
 }
 
 template <int W, bool MULTI> void *pick_render_s(uint32_t s) {
@@ -1149,7 +1230,7 @@ RenderJob make_render_job(const Scene &sc, const rt_params &p, uint32_t width, u
     RT_REQUIRE((uint64_t)width * height < (1ull << 31), "image too large");
     RenderJob j{};
     const float far = std::max(std::max(std::fabs(p.camPos[0]), std::fabs(p.camPos[1])), std::fabs(p.camPos[2]));
-    const bool exact = sc.qwide.p && !(far <= sc.far_limit);
+    const bool exact = sc.qwide.p && !(far <= sc.reach.far_limit);
     j.layout = exact ? sc.width : sc.layout();
     j.nodes = exact ? sc.wide.as<uint32_t>() : sc.nodes();
     j.wide = sc.wide.as<uint32_t>();
@@ -1159,6 +1240,7 @@ RenderJob make_render_job(const Scene &sc, const rt_params &p, uint32_t width, u
     j.mats = sc.materials.as<rt_material>();
     j.accum = accum;
     j.nwide = sc.nwide;
+    j.reach = sc.reach;
     j.stack_bound = sc.stack_bound;
     j.width = width;
     j.height = height;
@@ -1222,6 +1304,7 @@ uint32_t path_team_size(const rt_context *ctx, uint32_t layout, uint32_t stack_b
 
 // A yieldable pass: its finish launch and gated sum, launched again until the pass is complete.
 struct WaveResume {
+    rt_context *ctx;
     FinishArgs fa;
     void *kernel;
     uint32_t grid, block;
@@ -1237,6 +1320,7 @@ void launch_finish(const WaveResume &r, hipStream_t stream) {
     void *args[] = {&fa};
     RT_HIP(hipLaunchKernel(r.kernel, dim3(r.grid), dim3(r.block), args, r.lds, stream));
     RT_HIP(hipGetLastError());
+    launch_path_redo(r.ctx, fa.w, fa.leaf_weight, stream);
 }
 }  // namespace
 
@@ -1244,7 +1328,7 @@ void resume_render_wave(const WaveResume &r, const WaveYield &yield, hipStream_t
     WaveResume again = r;
     again.fa.yield = yield.flag;
     again.fa.yield_at = yield.yield_at;
-    k_resume_counter<<<1, 64, 0, stream>>>(again.fa.work);
+    k_resume_counter<<<1, 64, 0, stream>>>(again.fa.work, again.fa.w.left);
     RT_HIP(hipGetLastError());
     launch_finish(again, stream);
     RenderArgs sa = r.sum;
@@ -1286,7 +1370,7 @@ void launch_render_wave(rt_context *ctx, const Scene &sc, const RenderJob &j, un
     rt_hit *hits = reinterpret_cast<rt_hit *>(rays[1] + maxp);
     uint32_t *ids[2] = {reinterpret_cast<uint32_t *>(hits + maxp), nullptr};
     ids[1] = ids[0] + maxp;
-    uint32_t *count = ids[1] + maxp;  // two queue counters, a work counter and its value at a yield
+    uint32_t *count = ids[1] + maxp;  // two queue counters, a work counter and its value at a yield, the number of paths left over
     const bool cache = !(j.flags & RT_RENDER_NO_PRIMARY_CACHE);
     if (!cache) primary = nullptr;
     const uint32_t block = kShadeBlock;
@@ -1315,7 +1399,7 @@ void launch_render_wave(rt_context *ctx, const Scene &sc, const RenderJob &j, un
         }
         int cur = 0;
         const uint32_t finish_at = wave_finish_bounce();
-        k_zero<<<1, 64, 0, stream>>>(count, 2u);  // both queues, in one launch
+        k_zero<<<1, 64, 0, stream>>>(count, 5u);  // in one launch
         a.bounce = 0;
         a.hits_in = first_hits;
         a.rays_out = rays[cur];
@@ -1340,6 +1424,9 @@ void launch_render_wave(rt_context *ctx, const Scene &sc, const RenderJob &j, un
                 a.rays_in = rays[cur];
                 a.ids_in = ids[cur];
                 a.n_in = count + cur;
+                a.left = count + 4;
+                a.left_rays = rays[cur ^ 1];
+                a.left_cap = (uint32_t)maxp;
                 // the hits are no longer needed: their storage holds the work counters.  A launch that can yield
                 // has one, among the pass's counters, and so has a pass of few paths.
                 const bool many = !yield && 16ull * maxp >= 4ull * kCounterLines * kCounterStride + 128u;
@@ -1359,9 +1446,11 @@ void launch_render_wave(rt_context *ctx, const Scene &sc, const RenderJob &j, un
                     void *args[] = {&ta};
                     RT_HIP(hipLaunchKernel(k, dim3(g), dim3(64), args, 0, stream));
                     RT_HIP(hipGetLastError());
+                    launch_path_redo(ctx, a, tc.leaf_weight, stream);
                     break;
                 }
                 WaveResume w{};
+                w.ctx = ctx;
                 w.fa = FinishArgs{a, work, lines, tc.refill, tc.leaf_weight, tc.shade_min,
                                   yield ? yield->flag : nullptr, yield ? yield->yield_at : 0u,
                                   team_limit(kLastTeam, sc.stack_bound)};

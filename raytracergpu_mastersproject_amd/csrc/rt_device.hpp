@@ -305,6 +305,13 @@ constexpr uint32_t kSlotMask = 0x07FFFFFFu;
 // slab-test robustness: exit distance scaled by 1 + 2*gamma(3) (Ize 2013), rounded up
 constexpr float kRobust = 0x1.000006p+0f;
 
+// What bounds a scene's roundings (Scene::reach, and ray_pad in traverse.hpp)
+struct Reach {
+    float far_limit;
+    float coord;       // the largest coordinate in magnitude
+    float inv_radius;  // of the smallest sphere; 0 without spheres
+};
+
 __host__ __device__ inline uint32_t leaf_entry(uint32_t first, uint32_t count) {
     return kLeafBit | ((count - 1u) << 27) | first;
 }

@@ -208,11 +208,10 @@ struct Scene {
     Scene(const Scene &) = delete;
     Scene &operator=(const Scene &) = delete;
 
-    // Rays whose origin has a coordinate beyond this are traced in the exact nodes' order (with qwide).
-    // fp32 intersection at great distances gives a hit a t outside its own box by more than the slab test
-    // allows for; which of two such hits a traversal keeps depends on its order.  Rays from up to 1,000 scene extents
-    // away, spheres from up to 512 radii: no hit differed between orders below 19,000 extents (12 M rays).
-    float far_limit = 0.0f;
+    // reach.far_limit: rays whose origin has a coordinate beyond this are traced in the exact nodes' order (with qwide).  From
+    // great distances fp32 hits lie far outside their boxes: ray_pad's larger boxes would hold too much, and many rays would
+    // have to be traced again.  1,000 scene extents, 512 radii of the smallest sphere.
+    Reach reach{};
     // the node layout that the traversal kernels read: the width, or 44 (kQ4) for compressed width-4 nodes
     uint32_t layout() const { return qwide.p ? 44u : width; }
     const uint32_t *nodes() const { return qwide.p ? qwide.as<uint32_t>() : wide.as<uint32_t>(); }
@@ -239,10 +238,11 @@ struct RenderJob {
     float *accum;
     float4 *samples;   // split jobs: per (pixel, sample) {colour, next carry}, [sample][pixel]
     uint32_t nwide, width, height, spp;
+    Reach reach;
     uint32_t depth, random_state, flags, tiles_x;
     uint32_t first_item, nitems, group;
     uint32_t stack_bound;  // the scene's
-    uint32_t layout;  // of `nodes` (Scene::layout, or the width from a camera beyond Scene::far_limit); group: samples per split item (0 = whole pixels)
+    uint32_t layout;  // of `nodes` (Scene::layout, or the width from a camera beyond Scene::reach.far_limit); group: samples per split item (0 = whole pixels)
     float cam[12];  // pixel00, deltaU, deltaV, origin
 };
 // Split jobs give every (pixel, group of `group` consecutive samples) its own work item; the

@@ -6,9 +6,9 @@
 // from the team's stack, one per quad of lanes; a quad's lane c tests child c, and a leaf child is
 // tested by the lane that found it, at once.  Node children go back on the stack.
 //   Closest hit: the nearest quad's children on top, each quad's nearest first.  More nodes are
-//   visited than one after the other would (a hit culls only what has not been started), but every
-//   box that the ordered traversal enters is entered, and the closest hit is the smallest
-//   (t, leaf slot) of all hits whatever the order (Scene::far_limit says for which rays that holds).
+//   visited than one after the other would (a hit culls only what has not been started).  The result is
+//   that of the ordered traversal, or the team says that it must be traced in that order
+//   (traverse.hpp: closest hits out of another order).
 //   Any hit: the stack keeps depth-first child order, first entry on top, and lanes follow it.  A
 //   hit discards everything later in that order and the search goes on with what is earlier, so the
 //   result is the hit that the depth-first traversal finds first.
@@ -62,14 +62,14 @@ struct TeamHit {
     uint32_t slot;  // in every lane; kEmpty: a miss
     float u, v;     // in the owner
     bool owner;     // the lane that found the hit
+    bool redo;      // closest hit, in every lane: the ray must be traced in the exact nodes' order (team_ordered)
 };
 
 // Every lane of the wave calls it; `live` teams trace, all lanes of a team with the same ray.
-
 template <int T, bool ANY>
 __device__ __forceinline__ TeamHit team_trace(bool live, v3 o, v3 d, float tmin, float tmax, const uint32_t *wide,
                                               uint32_t nwide, const LeafRecord *__restrict__ rec, uint2 *stacks,
-                                              uint32_t limit) {
+                                              uint32_t limit, const Reach &reach) {
     constexpr uint32_t Q = T / 4;
     const uint32_t lane = threadIdx.x & 63u, c = lane & 3u;
     const uint32_t quad = (lane % T) >> 2, team0 = lane & ~(uint32_t)(T - 1);
@@ -78,9 +78,11 @@ __device__ __forceinline__ TeamHit team_trace(bool live, v3 o, v3 d, float tmin,
     slab_axis(d.x, o.x, idir.x, nlo.x, nhi.x);
     slab_axis(d.y, o.y, idir.y, nlo.y, nhi.y);
     slab_axis(d.z, o.z, idir.z, nlo.z, nhi.z);
-    float bt = tmax;                        // closest hit: the team's best t
-    float lt = tmax, lu = 0.0f, lv = 0.0f;  // this lane's best (any hit: last) hit
+    const float pad = ANY ? 0.0f : ray_pad(o, reach);
+    float bt = tmax, cull = tmax;           // closest hit: the team's best t, and the end of its window (hit_window)
+    float lt = tmax, lw = tmax, lu = 0.0f, lv = 0.0f;  // this lane's best (any hit: last) hit
     uint32_t ls = kEmpty;
+    bool redo = false;                      // closest hit: this lane saw two hits in one window
     bool owner = false;                     // any hit: this lane holds the team's hit
     uint32_t top = live && nwide > 0 && !has_nan(d) ? 1u : 0u;
     if (top) st[0] = make_uint2(0u, __float_as_uint(tmin));  // the root (the same from every lane)
@@ -90,7 +92,7 @@ __device__ __forceinline__ TeamHit team_trace(bool live, v3 o, v3 d, float tmin,
         bool alive = quad < take;
         uint2 e = make_uint2(0u, 0u);
         if (alive) e = st[top - 1u - quad];
-        if constexpr (!ANY) alive = alive && __uint_as_float(e.y) <= bt * kRobust;
+        if constexpr (!ANY) alive = alive && __uint_as_float(e.y) <= cull * kRobust;
         wave_fence();
         bool push = false, found = false;
         float tn = 0.0f;
@@ -103,24 +105,46 @@ __device__ __forceinline__ TeamHit team_trace(bool live, v3 o, v3 d, float tmin,
             const float x0 = fmaf(lox, idir.x, nlo.x), x1 = fmaf(hix, idir.x, nhi.x);
             const float y0 = fmaf(loy, idir.y, nlo.y), y1 = fmaf(hiy, idir.y, nhi.y);
             const float z0 = fmaf(loz, idir.z, nlo.z), z1 = fmaf(hiz, idir.z, nhi.z);
-            tn = fmaxf(fmaxf(fminf(x0, x1), fminf(y0, y1)), fmaxf(fminf(z0, z1), tmin));
-            const float tf = fminf(fminf(fmaxf(x0, x1), fmaxf(y0, y1)), fminf(fmaxf(z0, z1), bt));
+            const float nx = fminf(x0, x1), ny = fminf(y0, y1), nz = fminf(z0, z1);
+            const float fx = fmaxf(x0, x1), fy = fmaxf(y0, y1), fz = fmaxf(z0, z1);
+            float tf, entry = 0.0f;
+            if constexpr (ANY) {
+                tn = fmaxf(fmaxf(nx, ny), fmaxf(nz, tmin));
+                tf = fminf(fminf(fx, fy), fminf(fz, bt));
+            } else {  // the box larger by the ray's pad
+                tn = fmaxf(fmaxf(fmaf(-pad, fabsf(idir.x), nx), fmaf(-pad, fabsf(idir.y), ny)),
+                           fmaxf(fmaf(-pad, fabsf(idir.z), nz), tmin));
+                tf = fminf(fminf(fmaf(pad, fabsf(idir.x), fx), fmaf(pad, fabsf(idir.y), fy)),
+                           fminf(fmaf(pad, fabsf(idir.z), fz), cull));
+            }
             const bool hit = child != kEmpty && tn <= tf * kRobust;
             push = hit && !(child & kLeafBit);
-            if (hit && (child & kLeafBit)) {
+            bool leaf = hit && (child & kLeafBit);
+            if constexpr (!ANY) {  // leaves by their exact boxes
+                entry = fmaxf(fmaxf(nx, ny), fmaxf(nz, tmin));
+                leaf = leaf && entry <= fminf(fminf(fx, fy), fz) * kRobust;
+            }
+            if (leaf) {
                 const uint32_t first = leaf_first(child), end = first + leaf_count(child);
                 for (uint32_t s = first; s < end; ++s) {
                     const LeafRecord r = rec[s];
                     float th = 0.0f, u = 0.0f, v = 0.0f;
                     bool h;
                     if (is_sphere_record(r)) {
-                        h = sphere_test(r, o, d, tmin, bt, th);
+                        h = sphere_test(r, o, d, tmin, cull, th);
                         u = r.r1.y;
                         v = r.r1.z;
                     } else {
-                        h = triangle_test(r, o, d, tmin, bt, th, u, v);
+                        h = triangle_test(r, o, d, tmin, cull, th, u, v);
                     }
-                    if (h && (ANY ? th <= bt : th < lt || (th == lt && s < ls))) {
+                    if constexpr (!ANY) {
+                        const float window = hit_window(th, entry);
+                        const bool best = th < lt || (th == lt && s < ls);
+                        if (h && (best ? window > th && lt <= window : lw > lt && th <= lw)) redo = true;
+                        h = h && best;
+                        if (h) lw = window;
+                    }
+                    if (h && (!ANY || th <= bt)) {
                         lt = th;
                         ls = s;
                         lu = u;
@@ -146,7 +170,11 @@ __device__ __forceinline__ TeamHit team_trace(bool live, v3 o, v3 d, float tmin,
             }
             if (push) st[base + (uint32_t)__popcll((pushing >> (lane - team0)) >> 1)] = make_uint2(child, 0u);
         } else {
-            if (__ballot(found) != 0ull) bt = ord_dec(team_min<T>(ord_key(lt)));
+            if (__ballot(found) != 0ull) {
+                cull = bt = ord_dec(team_min<T>(ord_key(lt)));
+                if (__ballot(lw > lt) != 0ull)  // rare
+                    cull = ord_dec(~team_min<T>(~ord_key(lt == bt ? fmaxf(lw, bt) : bt)));
+            }
             const uint32_t k = push ? ((__float_as_uint(tn) & ~3u) | c) : 0u;
             const uint32_t farther = (dpp<quad_perm(1, 2, 3, 0)>(k) > k ? 1u : 0u) +
                                      (dpp<quad_perm(2, 3, 0, 1)>(k) > k ? 1u : 0u) +
@@ -158,11 +186,42 @@ __device__ __forceinline__ TeamHit team_trace(bool live, v3 o, v3 d, float tmin,
     }
     if constexpr (ANY) {
         const uint32_t slot = team_min<T>(owner ? ls : kEmpty);
-        return TeamHit{owner ? lt : tmax, slot, lu, lv, owner};
+        return TeamHit{owner ? lt : tmax, slot, lu, lv, owner, false};
     }
     // the smallest (t, slot); a slot is tested by one lane only
     const uint32_t slot = team_min<T>(lt == bt ? ls : kEmpty);
-    return TeamHit{bt, slot, lu, lv, slot != kEmpty && ls == slot && lt == bt};
+    redo = redo || (cull > bt && ls != kEmpty && ls != slot && lt <= cull);  // another lane's hit in the window
+    const unsigned long long rm = (__ballot(redo) >> team0) & (~0ull >> (64 - T));
+    return TeamHit{bt, slot, lu, lv, slot != kEmpty && ls == slot && lt == bt, rm != 0ull};
+}
+
+// The rays of the `on` teams in the exact nodes' order, by their first lanes (rare).  Every lane of the wave calls it; `m` takes
+// the team stacks' place.
+template <int T, int S, bool ANY, class B>
+__device__ __forceinline__ TeamHit team_ordered(bool on, v3 o, v3 d, float tmin, float tmax, const uint32_t *wide, uint32_t nwide,
+                                                const LeafRecord *rec, const StackMem &m, const B &boxes) {
+    Trav t;
+    t.bt = tmax;
+    t.bslot = kEmpty;
+    t.bu = t.bv = 0.0f;
+    const bool first = threadIdx.x % T == 0;
+    if (on && first) walk_exact<S, ANY>(t, m, o, d, tmin, tmax, nwide, wide, rec, boxes, 2u);
+    wave_fence();
+    const int from = (int)(threadIdx.x & 63u & ~(uint32_t)(T - 1));
+    return TeamHit{__shfl(t.bt, from), (uint32_t)__shfl((int)t.bslot, from), t.bu, t.bv, first && t.bslot != kEmpty, false};
+}
+
+// The closest hit of each live team's ray, in the ordered traversal's terms.
+template <int T, int S, class B>
+__device__ __forceinline__ TeamHit team_closest(bool live, v3 o, v3 d, float tmin, float tmax, const uint32_t *wide, uint32_t nwide,
+                                                const LeafRecord *rec, uint2 *stacks, uint32_t limit, const Reach &reach,
+                                                const StackMem &m, const B &boxes) {
+    TeamHit h = team_trace<T, false>(live, o, d, tmin, tmax, wide, nwide, rec, stacks, limit, reach);
+    if (__ballot(live && h.redo) != 0ull) {
+        const TeamHit again = team_ordered<T, S, false>(live && h.redo, o, d, tmin, tmax, wide, nwide, rec, m, boxes);
+        if (h.redo) h = again;
+    }
+    return h;
 }
 
 // The end of a launch whose waves trace a ray (path) per lane: once a wave finds no more work and at most kLastRays of its

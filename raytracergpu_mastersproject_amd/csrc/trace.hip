@@ -27,7 +27,7 @@ struct SceneView {
     const rt_triangle *tris;  // world-space primitives, for the refined results
     const rt_sphere *sph;
     uint32_t nwide;
-    float far_limit;
+    Reach reach;
     __device__ LeafBoxes operator()() const { return LeafBoxes{wide, slot_ref}; }
 };
 
@@ -44,6 +44,15 @@ struct TraceArgs {
     uint32_t limit;         // of a team of kLastTeam lanes; 0: the last rays stay with their lanes
 };
 
+// A counter slot's words: per line, 0 and 1 the launch's work counter, 2 and 3 that of the launch over the marked rays
+// (which must be traced in the exact nodes' order, kRedo); word kMarks of the first line counts the marked
+// rays, and the words from kMarkList of every line hold the indices of the first kMarkCap of them.
+constexpr uint32_t kMarks = 4, kMarkList = 16, kMarkPerLine = kCounterStride - kMarkList, kMarkCap = kMarkPerLine * kCounterLines;
+
+template <typename T> __device__ __forceinline__ uint32_t *mark_count(T *work) { return reinterpret_cast<uint32_t *>(work) + kMarks; }
+template <typename T> __device__ __forceinline__ uint32_t *mark_entry(T *work, uint32_t k) {
+    return reinterpret_cast<uint32_t *>(work) + (k / kMarkPerLine) * kCounterStride + kMarkList + k % kMarkPerLine;
+}
 // Rays are read once and hits written once per launch: non-temporal accesses keep them from
 // displacing the BVH nodes and leaf records in L2 and the MALL (refined closest-hit query on
 // 4M triangles: 5.10 against 5.13 ms).
@@ -53,6 +62,18 @@ typedef unsigned int nt_u4 __attribute__((ext_vector_type(4)));
 __device__ __forceinline__ void store_hit_nt(rt_hit *hits, uint32_t i, uint4 h) {
     const nt_u4 v = {h.x, h.y, h.z, h.w};
     __builtin_nontemporal_store(v, reinterpret_cast<nt_u4 *>(hits) + i);
+}
+
+// The ray's hit record says that it is to be traced again; g: its index in the launch.  `full`: the lane has seen the list full,
+// and the count no longer matters (one counter for all would hold up a launch that marks every ray).
+template <typename T> __device__ __forceinline__ void mark_ray(T *work, rt_hit *hits, uint32_t i, uint64_t g, bool &full) {
+    store_hit_nt(hits, i, make_uint4(kRedo, 0u, 0u, 0u));
+    if (full) return;
+    uint32_t *n = mark_count(work);
+    full = __hip_atomic_load(n, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) > kMarkCap;
+    if (full) return;
+    const uint32_t k = atomicAdd(n, g > 0xFFFFFFFFull ? kMarkCap + 1u : 1u);
+    if (k < kMarkCap) *mark_entry(work, k) = (uint32_t)g;
 }
 
 __device__ __forceinline__ void load_ray(const rt_ray *rays, uint32_t i, v3 &o, float &tmin, v3 &d, float &tmax) {
@@ -85,8 +106,17 @@ __global__ __launch_bounds__(256) void k_trace_direct(TraceArgs a) {
     float tmin, tmax;
     load_ray(a.rays, i, o, tmin, d, tmax);
     Trav t;
-    walk_init<W, S, ANY>(t, m, o, d, tmin, tmax, a.sc.nwide, a.sc.far_limit, a.sc.rec, a.sc, a.leaf_weight);
+    trav_init<W, ANY>(t, o, d, tmin, tmax, a.sc.nwide, a.sc.reach);
+    bool exact = false;
+    if constexpr (W == kQ4) {
+        exact = needs_exact_nodes(o, d, a.sc.reach.far_limit);
+        if (exact) t.have = false;
+    }
     trav_run<W, S, ANY, COUNT>(t, m, a.sc.nodes, a.sc.rec, a.sc, a.leaf_weight);
+    if constexpr (W == kQ4) {
+        if (exact || t.bslot == kRedo)
+            walk_exact<S, ANY>(t, m, o, d, tmin, tmax, a.sc.nwide, a.sc.wide, a.sc.rec, a.sc, a.leaf_weight);
+    }
     store_hit(a.sc, t, a.hits, a.counts, i);
 }
 
@@ -131,47 +161,79 @@ __device__ __forceinline__ void store_team(const SceneView &sc, const TeamHit &h
     else store_hit(sc, t, hits, nullptr, i);
 }
 
-// The last rays of a wave, one per lane in `live`, from their start: ray i of that lane.
-template <int S, bool ANY, bool REFINE>
+// The last rays of a wave, one per lane in `live`, from their start: ray i of that lane, g in the launch.
+template <int S, bool ANY, bool REFINE, typename W>
 __device__ __forceinline__ void trace_last(unsigned long long live, const SceneView &sc, const rt_ray *rays,
-                                           rt_hit *hits, uint32_t i, void *lds, uint32_t limit) {
+                                           rt_hit *hits, uint32_t i, uint64_t g, W *work, void *lds, uint32_t limit) {
     const bool on = (threadIdx.x & 63u) / kLastTeam < (uint32_t)__popcll(live);
     v3 o, d;
     float tmin, tmax;
     load_ray(rays, i, o, tmin, d, tmax);
     const TeamHit h = team_trace<kLastTeam, ANY>(on, o, d, tmin, tmax, sc.wide, sc.nwide, sc.rec,
-                                                 reinterpret_cast<uint2 *>(wave_lds<S>(lds)), limit);
-    if (on) store_team<kLastTeam, REFINE>(sc, h, o, d, hits, i);
+                                                 reinterpret_cast<uint2 *>(wave_lds<S>(lds)), limit, sc.reach);
+    if (on && h.redo) {
+        bool full = false;
+        if (threadIdx.x % kLastTeam == 0) mark_ray(work, hits, i, g, full);
+    } else if (on) {
+        store_team<kLastTeam, REFINE>(sc, h, o, d, hits, i);
+    }
 }
 
-// Ray i by a team of T lanes; every lane of the wave calls it.
+// Ray i by a team of T lanes; every lane of the wave calls it.  A closest-hit ray that must be traced in the exact nodes' order:
+// by the team's first lane with 32 lanes or more, whose launches are short; else it is marked for k_trace_marked.
+constexpr bool team_marks(uint32_t t) { return t <= 16u; }
+
 template <int T, bool ANY, bool REFINE>
 __device__ __forceinline__ void trace_by_team(bool live, const SceneView &sc, const rt_ray *rays, rt_hit *hits, uint32_t i,
-                                              uint2 *stacks, uint32_t limit, uint32_t leaf_weight) {
+                                              uint2 *stacks, uint32_t limit) {
     v3 o{0.0f, 0.0f, 0.0f}, d{0.0f, 0.0f, 0.0f};
     float tmin = 0.0f, tmax = 0.0f;
     if (live) load_ray(rays, i, o, tmin, d, tmax);
-    const bool ordered = live && needs_exact_nodes(o, d, sc.far_limit);
-    if (__ballot(ordered) != 0ull) {  // rare: a team's first lane runs such a ray alone, in the stacks' memory
-        uint2 spill[kSpillCap];
-        if (ordered && threadIdx.x % T == 0) {
-            Trav t;
-            trav_init<4>(t, o, d, tmin, tmax, sc.nwide);
-            trav_run<4, 16, ANY, false>(t, stack_mem<16>(stacks, spill), sc.wide, sc.rec, sc, leaf_weight);
-            if constexpr (REFINE) store_refined(sc, t, hits, nullptr, i);
-            else store_hit(sc, t, hits, nullptr, i);
+    // any hit: the teams read the exact nodes, and no order changes its result
+    const bool exact = !ANY && live && needs_exact_nodes(o, d, sc.reach.far_limit);
+    TeamHit h = team_trace<T, ANY>(live && !exact, o, d, tmin, tmax, sc.wide, sc.nwide, sc.rec, stacks, limit, sc.reach);
+    bool stored = !live;
+    if constexpr (!ANY) {
+        const bool ordered = live && (exact || h.redo);
+        if constexpr (team_marks(T)) {
+            if (ordered && threadIdx.x % T == 0) hits[i].prim = kRedo;
+            stored = stored || ordered;
+        } else if (__ballot(ordered) != 0ull) {
+            uint2 spill[kSpillCap];
+            const TeamHit again = team_ordered<T, 16, ANY>(ordered, o, d, tmin, tmax, sc.wide, sc.nwide, sc.rec,
+                                                           stack_mem<16>(stacks, spill), sc);
+            if (ordered) h = again;
         }
-        live = live && !ordered;
     }
-    const TeamHit h = team_trace<T, ANY>(live, o, d, tmin, tmax, sc.wide, sc.nwide, sc.rec, stacks, limit);
-    if (live) store_team<T, REFINE>(sc, h, o, d, hits, i);
+    if (!stored) store_team<T, REFINE>(sc, h, o, d, hits, i);
 }
 
 // One team of T lanes per ray, one wave per block, every ray at once: no work counter, no refill.
 template <int T, bool ANY, bool REFINE> __global__ __launch_bounds__(64) void k_trace_team(TraceArgs a, uint32_t limit) {
     __shared__ uint2 stacks[64 / T * team_stack(T)];
     const uint32_t i = blockIdx.x * (64u / T) + threadIdx.x / T;
-    trace_by_team<T, ANY, REFINE>(i < a.n, a.sc, a.rays, a.hits, i, stacks, limit, a.leaf_weight);
+    trace_by_team<T, ANY, REFINE>(i < a.n, a.sc, a.rays, a.hits, i, stacks, limit);
+}
+
+// The rays that a launch of teams has marked, a lane per ray.
+template <bool REFINE>
+__device__ __forceinline__ void trace_marked(const SceneView &sc, const rt_ray *rays, rt_hit *hits, uint32_t i, const StackMem &m,
+                                             uint32_t leaf_weight) {
+    if (hits[i].prim != kRedo) return;
+    v3 o, d;
+    float tmin, tmax;
+    load_ray(rays, i, o, tmin, d, tmax);
+    Trav t;
+    walk_exact<16, false>(t, m, o, d, tmin, tmax, sc.nwide, sc.wide, sc.rec, sc, leaf_weight);
+    if constexpr (REFINE) store_refined(sc, t, hits, nullptr, i);
+    else store_hit(sc, t, hits, nullptr, i);
+}
+
+template <bool REFINE> __global__ __launch_bounds__(128) void k_trace_marked(TraceArgs a) {
+    extern __shared__ uint32_t lds[];
+    uint2 spill[kSpillCap];
+    const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
+    if (i < a.n) trace_marked<REFINE>(a.sc, a.rays, a.hits, i, stack_mem<16>(lds, spill), a.leaf_weight);
 }
 
 constexpr uint32_t kNoRay = ~0u;
@@ -183,7 +245,8 @@ template <int W> constexpr bool kDefer = W == kQ4 || W == 4;
 
 // REFINE: store each hit with t, u, v refined in double (store_refined) instead of the fp32 values.
 // LAST: the wave's last rays go on with teams of lanes (trace_last).
-template <int W, int S, bool ANY, bool COUNT, bool REFINE, bool LAST>
+// MARKED: only the rays that the launch before has marked (mark_ray).
+template <int W, int S, bool ANY, bool COUNT, bool REFINE, bool LAST, bool MARKED>
 __global__ __launch_bounds__(256, W == kQ4 ? 5 : 1) void k_trace_persistent(TraceArgs a) {
     extern __shared__ uint32_t lds[];
     uint2 spill[kSpillCap];
@@ -197,15 +260,26 @@ __global__ __launch_bounds__(256, W == kQ4 ? 5 : 1) void k_trace_persistent(Trac
     uint32_t done = kNoRay;
     bool exhausted = false;
     uint32_t q_next = 0, q_end = 0;  // the wave's current chunk of ray indices (wave-uniform)
-    const uint32_t n = a.n_dev ? min(*a.n_dev, a.n) : a.n;
+    uint32_t n = a.n_dev ? min(*a.n_dev, a.n) : a.n;
+    bool listed = false;  // the marked rays' indices are in the list
+    unsigned int *work = a.work;
+    if constexpr (MARKED) {
+        const uint32_t marks = *mark_count(a.work);
+        if (marks == 0u) return;
+        listed = marks <= kMarkCap;
+        if (listed) n = marks;
+        work += 2;
+    }
     const uint32_t wpb = blockDim.x / 64u;
     const ChunkSchedule<uint32_t> sched(n, gridDim.x * wpb);
     WorkLines lines(blockIdx.x * wpb + __builtin_amdgcn_readfirstlane(threadIdx.x / 64u), gridDim.x * wpb);
     Trav t;
     t.have = false;
     t.top = 0;
+    bool full = false;  // mark_ray's
     const auto store = [&](uint32_t i) {
-        if constexpr (REFINE) store_refined(a.sc, t, a.hits, a.counts, i);
+        if (W == kQ4 && !ANY && t.bslot == kRedo) mark_ray(a.work, a.hits, i, i, full);
+        else if constexpr (REFINE) store_refined(a.sc, t, a.hits, a.counts, i);
         else store_hit(a.sc, t, a.hits, a.counts, i);
     };
     for (;;) {
@@ -219,7 +293,7 @@ __global__ __launch_bounds__(256, W == kQ4 ? 5 : 1) void k_trace_persistent(Trac
             while (q_next == q_end && !exhausted) {  // one atomic per chunk
                 const int leader = __ffsll((unsigned long long)idle) - 1;
                 uint32_t base = 0;
-                if ((int)lane == leader) base = atomicAdd(lines.counter(a.work), 1u);
+                if ((int)lane == leader) base = atomicAdd(lines.counter(work), 1u);
                 base = (uint32_t)__shfl((int)base, leader);
                 uint64_t lo, hi;
                 if (sched.range((uint32_t)lines.item(base), lo, hi)) { q_next = (uint32_t)lo; q_end = (uint32_t)hi; }
@@ -230,16 +304,25 @@ __global__ __launch_bounds__(256, W == kQ4 ? 5 : 1) void k_trace_persistent(Trac
                 const uint32_t r = (uint32_t)__popcll(idle & lt);
                 if (rid == kNoRay && r < take) {
                     rid = q_next + r;
-                    v3 o, d;
-                    float tmin, tmax;
-                    load_ray(a.rays, rid, o, tmin, d, tmax);
-                    walk_init<W, S, ANY>(t, m, o, d, tmin, tmax, a.sc.nwide, a.sc.far_limit, a.sc.rec, a.sc, a.leaf_weight);
+                    if constexpr (MARKED) {
+                        if (listed) rid = *mark_entry(a.work, rid);
+                        else if (a.hits[rid].prim != kRedo) rid = kNoRay;
+                    }
+                    if (!MARKED || rid != kNoRay) {
+                        v3 o, d;
+                        float tmin, tmax;
+                        load_ray(a.rays, rid, o, tmin, d, tmax);
+                        walk_init<W, S, ANY>(t, m, o, d, tmin, tmax, a.sc.nwide, a.sc.reach, a.sc.rec, a.sc, a.leaf_weight);
+                    }
                 }
                 q_next += take;
             }
         }
         const unsigned long long live = __ballot(rid != kNoRay);
-        if (live == 0ull) break;  // every lane idle and the queue is drained
+        if (live == 0ull) {  // every lane idle
+            if (exhausted) break;  // and the queue is drained
+            continue;  // no ray of those taken was started
+        }
         if (LAST && exhausted && a.limit && (uint32_t)__popcll(live) <= kLastRays) break;
         const bool on_node = rid != kNoRay && at_node(t), on_leaf = rid != kNoRay && at_leaf(t);
         if (choose_leaf_phase(on_node, on_leaf, a.leaf_weight)) {
@@ -259,7 +342,7 @@ __global__ __launch_bounds__(256, W == kQ4 ? 5 : 1) void k_trace_persistent(Trac
         const unsigned long long live = __ballot(rid != kNoRay);
         if (live == 0ull) return;
         const uint32_t i = (uint32_t)__shfl((int)rid, (int)last_ray_lane<kLastTeam>(live));
-        trace_last<S, ANY, REFINE>(live, a.sc, a.rays, a.hits, i, lds, a.limit);
+        trace_last<S, ANY, REFINE>(live, a.sc, a.rays, a.hits, i, i, a.work, lds, a.limit);
     }
 }
 
@@ -330,8 +413,8 @@ __device__ __forceinline__ uint32_t find_item(const BatchItemDev *items, uint32_
     return lo;
 }
 
-// REFINE: store each hit with t, u, v refined in double (store_refined).
-template <int W, int S, bool ANY, bool REFINE, bool LAST>
+// REFINE: store each hit with t, u, v refined in double (store_refined); LAST, MARKED: as in k_trace_persistent.
+template <int W, int S, bool ANY, bool REFINE, bool LAST, bool MARKED>
 __global__ __launch_bounds__(256, W == kQ4 ? 5 : 1) void k_trace_batch(BatchArgs a) {
     extern __shared__ uint32_t lds[];
     uint2 spill[kSpillCap];
@@ -347,15 +430,27 @@ __global__ __launch_bounds__(256, W == kQ4 ? 5 : 1) void k_trace_batch(BatchArgs
     // latency to every step
     const uint32_t *nodes = nullptr;
     const LeafRecord *rec = nullptr;
+    uint64_t total = a.total;
+    bool listed = false;
+    unsigned long long *work = a.work;
+    if constexpr (MARKED) {
+        const uint32_t marks = *mark_count(a.work);
+        if (marks == 0u) return;
+        listed = marks <= kMarkCap;
+        if (listed) total = marks;
+        work += 1;
+    }
     const uint32_t wpb = blockDim.x / 64u;
-    const ChunkSchedule<uint64_t> sched(a.total, gridDim.x * wpb);
+    const ChunkSchedule<uint64_t> sched(total, gridDim.x * wpb);
     WorkLines lines(blockIdx.x * wpb + __builtin_amdgcn_readfirstlane(threadIdx.x / 64u), gridDim.x * wpb);
     Trav t;
     t.have = false;
     t.top = 0;
+    bool full = false;
     const auto store = [&]() {
         const BatchItemDev &it = a.items[item];
-        if constexpr (REFINE) store_refined(it.sc, t, it.hits, nullptr, local);
+        if (W == kQ4 && !ANY && t.bslot == kRedo) mark_ray(a.work, it.hits, local, it.first + local, full);
+        else if constexpr (REFINE) store_refined(it.sc, t, it.hits, nullptr, local);
         else store_hit(it.sc, t, it.hits, nullptr, local);
     };
     for (;;) {
@@ -369,7 +464,7 @@ __global__ __launch_bounds__(256, W == kQ4 ? 5 : 1) void k_trace_batch(BatchArgs
             while (q_next == q_end && !exhausted) {
                 const int leader = __ffsll((unsigned long long)idle) - 1;
                 unsigned long long base = 0;
-                if ((int)lane == leader) base = atomicAdd(lines.counter(a.work), 1ull);
+                if ((int)lane == leader) base = atomicAdd(lines.counter(work), 1ull);
                 base = __shfl(base, leader);
                 uint64_t lo, hi;
                 if (!sched.range(lines.item(base), lo, hi)) {
@@ -377,28 +472,35 @@ __global__ __launch_bounds__(256, W == kQ4 ? 5 : 1) void k_trace_batch(BatchArgs
                 } else {  // chunks are short: usually one item, found once per chunk
                     q_next = lo;
                     q_end = hi;
-                    c_lo = find_item(a.items, 0u, a.nitems, q_next);
-                    c_hi = find_item(a.items, c_lo, a.nitems, q_end - 1u) + 1u;
+                    c_lo = listed ? 0u : find_item(a.items, 0u, a.nitems, q_next);
+                    c_hi = listed ? a.nitems : find_item(a.items, c_lo, a.nitems, q_end - 1u) + 1u;
                 }
             }
             const uint32_t take = exhausted ? 0u : (uint32_t)min((uint64_t)nidle, q_end - q_next);
             const uint32_t r = (uint32_t)__popcll(idle & lt);
-            const uint64_t g = q_next + r;
+            uint64_t g = q_next + r;
             q_next += take;
             if (!active && r < take) {
+                if (MARKED && listed) g = *mark_entry(a.work, (uint32_t)g);
                 item = find_item(a.items, c_lo, c_hi, g);
                 local = (uint32_t)(g - a.items[item].first);
-                nodes = a.items[item].sc.nodes;
-                rec = a.items[item].sc.rec;
-                v3 o, d;
-                float tmin, tmax;
-                load_ray(a.items[item].rays, local, o, tmin, d, tmax);
-                walk_init<W, S, ANY>(t, m, o, d, tmin, tmax, a.items[item].sc.nwide, a.items[item].sc.far_limit, rec, a.items[item].sc, a.leaf_weight);
-                active = true;
+                if (!MARKED || listed || a.items[item].hits[local].prim == kRedo) {
+                    nodes = MARKED ? a.items[item].sc.wide : a.items[item].sc.nodes;
+                    rec = a.items[item].sc.rec;
+                    v3 o, d;
+                    float tmin, tmax;
+                    load_ray(a.items[item].rays, local, o, tmin, d, tmax);
+                    walk_init<W, S, ANY>(t, m, o, d, tmin, tmax, a.items[item].sc.nwide, a.items[item].sc.reach, rec,
+                                         a.items[item].sc, a.leaf_weight);
+                    active = true;
+                }
             }
         }
         const unsigned long long live = __ballot(active);
-        if (live == 0ull) break;
+        if (live == 0ull) {
+            if (exhausted) break;
+            continue;
+        }
         if (LAST && exhausted && a.limit && (uint32_t)__popcll(live) <= kLastRays) break;
         const bool on_node = active && at_node(t), on_leaf = active && at_leaf(t);
         if (choose_leaf_phase(on_node, on_leaf, a.leaf_weight)) {
@@ -419,7 +521,8 @@ __global__ __launch_bounds__(256, W == kQ4 ? 5 : 1) void k_trace_batch(BatchArgs
         if (live == 0ull) return;
         const int from = (int)last_ray_lane<kLastTeam>(live);
         const BatchItemDev &it = a.items[(uint32_t)__shfl((int)item, from)];
-        trace_last<S, ANY, REFINE>(live, it.sc, it.rays, it.hits, (uint32_t)__shfl((int)local, from), lds, a.limit);
+        const uint32_t i = (uint32_t)__shfl((int)local, from);
+        trace_last<S, ANY, REFINE>(live, it.sc, it.rays, it.hits, i, it.first + i, a.work, lds, a.limit);
     }
 }
 
@@ -429,8 +532,16 @@ __global__ __launch_bounds__(64) void k_trace_team_batch(BatchArgs a, uint32_t l
     __shared__ uint2 stacks[64 / T * team_stack(T)];
     const uint32_t g = blockIdx.x * (64u / T) + threadIdx.x / T;
     const BatchItemDev &it = a.items[find_item(a.items, 0u, a.nitems, min((uint64_t)g, a.total - 1u))];
-    trace_by_team<T, ANY, REFINE>(g < a.total, it.sc, it.rays, it.hits, (uint32_t)(g - it.first), stacks, limit,
-                                  a.leaf_weight);
+    trace_by_team<T, ANY, REFINE>(g < a.total, it.sc, it.rays, it.hits, (uint32_t)(g - it.first), stacks, limit);
+}
+
+template <bool REFINE> __global__ __launch_bounds__(128) void k_trace_marked_batch(BatchArgs a) {
+    extern __shared__ uint32_t lds[];
+    uint2 spill[kSpillCap];
+    const uint64_t g = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
+    if (g >= a.total) return;
+    const BatchItemDev &it = a.items[find_item(a.items, 0u, a.nitems, g)];
+    trace_marked<REFINE>(it.sc, it.rays, it.hits, (uint32_t)(g - it.first), stack_mem<16>(lds, spill), a.leaf_weight);
 }
 
 template <int T, bool ANY, bool REFINE> void *team_kernel_t(bool batch) {
@@ -450,12 +561,13 @@ void *team_kernel(uint32_t t, bool any, bool refine, bool batch) {
 }
 
 __global__ void k_zero_counter(unsigned int *c) {
-    if (threadIdx.x < kCounterLines) c[threadIdx.x * kCounterStride] = c[threadIdx.x * kCounterStride + 1u] = 0u;
+    if (threadIdx.x < kCounterLines) reinterpret_cast<uint4 *>(c + threadIdx.x * kCounterStride)[0] = make_uint4(0u, 0u, 0u, 0u);
+    if (threadIdx.x == 0) c[kMarks] = 0u;
 }
 
 SceneView view_of(const Scene &sc) {
     return SceneView{sc.nodes(), sc.wide.as<uint32_t>(), sc.slot_ref.as<uint32_t>(), sc.records.as<LeafRecord>(), sc.slot_prim.as<uint32_t>(),
-                     sc.tris.as<rt_triangle>(), sc.spheres.as<rt_sphere>(), sc.nwide, sc.far_limit};
+                     sc.tris.as<rt_triangle>(), sc.spheres.as<rt_sphere>(), sc.nwide, sc.reach};
 }
 
 template <int W, int S> struct Kernels {
@@ -465,15 +577,15 @@ template <int W, int S> struct Kernels {
     }
     template <bool ANY, bool REFINE> static void *persistent(bool count, bool last) {
         if constexpr (W == kQ4)
-            return last ? (void *)k_trace_persistent<W, S, ANY, false, REFINE, true>
-                        : (void *)k_trace_persistent<W, S, ANY, false, REFINE, false>;
-        else return count ? (void *)k_trace_persistent<W, S, ANY, true, REFINE, false>
-                     : (void *)k_trace_persistent<W, S, ANY, false, REFINE, false>;
+            return last ? (void *)k_trace_persistent<W, S, ANY, false, REFINE, true, false>
+                        : (void *)k_trace_persistent<W, S, ANY, false, REFINE, false, false>;
+        else return count ? (void *)k_trace_persistent<W, S, ANY, true, REFINE, false, false>
+                     : (void *)k_trace_persistent<W, S, ANY, false, REFINE, false, false>;
     }
     template <bool ANY, bool REFINE> static void *batch(bool last) {
         if constexpr (W == kQ4)
-            if (last) return (void *)k_trace_batch<W, S, ANY, REFINE, true>;
-        return (void *)k_trace_batch<W, S, ANY, REFINE, false>;
+            if (last) return (void *)k_trace_batch<W, S, ANY, REFINE, true, false>;
+        return (void *)k_trace_batch<W, S, ANY, REFINE, false, false>;
     }
     static void *get(int which, bool any, bool count, bool last) {
         if (which == 0) return any ? direct<true>(count) : direct<false>(count);
@@ -513,6 +625,38 @@ uint32_t persistent_grid(rt_context *ctx, const void *kernel, uint32_t block, si
     int per_cu = 0;
     RT_HIP(hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, kernel, (int)block, lds));
     return (uint32_t)std::max(1, per_cu) * (uint32_t)ctx->num_cus;
+}
+
+// After a launch for closest hits: the rays that it has marked, if any, over the exact nodes.  An empty launch takes 3 us.
+template <class A> void launch_marked(rt_context *ctx, A &a, void *k, uint64_t n, hipStream_t stream) {
+    constexpr uint32_t block = 128, lds_stack = 16;  // holds any stack that the launch before could
+    const size_t lds = stack_lds_bytes(lds_stack, block);
+    const uint32_t grid = (uint32_t)std::min<uint64_t>(persistent_grid(ctx, k, block, lds), (n + block - 1) / block);
+    void *args[] = {&a};
+    RT_HIP(hipLaunchKernel(k, dim3(grid), dim3(block), args, lds, stream));
+}
+void launch_marked(rt_context *ctx, TraceArgs a, bool refine, hipStream_t stream) {
+    a.sc.nodes = a.sc.wide;
+    launch_marked(ctx, a, refine ? (void *)k_trace_persistent<4, 16, false, false, true, false, true>
+                                 : (void *)k_trace_persistent<4, 16, false, false, false, false, true>, a.n, stream);
+}
+void launch_marked(rt_context *ctx, BatchArgs a, bool refine, hipStream_t stream) {
+    launch_marked(ctx, a, refine ? (void *)k_trace_batch<4, 16, false, true, false, true>
+                                 : (void *)k_trace_batch<4, 16, false, false, false, true>, a.total, stream);
+}
+
+
+// A launch of a team per ray, and one over the rays that it has marked.
+template <class A>
+void launch_team(uint32_t team, bool any, bool refine, bool batch, A &a, uint64_t n, uint32_t stack_bound, hipStream_t stream) {
+    uint32_t limit = team_limit(team, stack_bound);
+    void *args[] = {&a, &limit};
+    RT_HIP(hipLaunchKernel(team_kernel(team, any, refine, batch), dim3(((uint32_t)n + 64u / team - 1) / (64u / team)), dim3(64), args, 0,
+                           stream));
+    if (any || !team_marks(team)) return;
+    void *k = batch ? (refine ? (void *)k_trace_marked_batch<true> : (void *)k_trace_marked_batch<false>)
+                    : (refine ? (void *)k_trace_marked<true> : (void *)k_trace_marked<false>);
+    RT_HIP(hipLaunchKernel(k, dim3(((uint32_t)n + 127u) / 128u), dim3(128), args, stack_lds_bytes(16, 128), stream));
 }
 
 }  // namespace
@@ -576,9 +720,7 @@ void launch_trace(rt_context *ctx, const Scene &sc, const rt_ray *rays, uint32_t
     }
     const size_t lds = stack_lds_bytes(c.lds_stack, c.block);
     if (const uint32_t team = counts ? 0u : team_size(ctx, layout, sc.stack_bound, n, c)) {
-        uint32_t limit = team_limit(team, sc.stack_bound);
-        void *args[] = {&a, &limit};
-        RT_HIP(hipLaunchKernel(team_kernel(team, any, refine, false), dim3((n + 64u / team - 1) / (64u / team)), dim3(64), args, 0, stream));
+        launch_team(team, any, refine, false, a, n, sc.stack_bound, stream);
         RT_HIP(hipGetLastError());
         return;
     }
@@ -597,6 +739,7 @@ void launch_trace(rt_context *ctx, const Scene &sc, const rt_ray *rays, uint32_t
                                                            ((uint64_t)n + c.block - 1) / c.block);
         void *args[] = {&a};
         RT_HIP(hipLaunchKernel(k, dim3(grid), dim3(c.block), args, lds, stream));
+        if (layout == kQ4 && !any) launch_marked(ctx, a, refine, stream);
     }
     if (refine && !refine_in_kernel)
         k_refine_hits<<<(uint32_t)(((uint64_t)n + 255u) / 256u), 256, 0, stream>>>(rays, hits, n, a.sc.tris, a.sc.sph);
@@ -614,10 +757,7 @@ void launch_trace_queue(rt_context *ctx, const Scene &sc, const rt_ray *rays, ui
     const size_t lds = stack_lds_bytes(c.lds_stack, c.block);
     // camera rays of a small image: a team per ray (65,536 pixels on 200 k triangles: 130 us less per frame)
     if (const uint32_t team = n_dev || n_max > 1024u * (uint64_t)ctx->num_cus ? 0u : team_size(ctx, sc.layout(), sc.stack_bound, n_max, c)) {
-        uint32_t limit = team_limit(team, sc.stack_bound);
-        void *args[] = {&a, &limit};
-        RT_HIP(hipLaunchKernel(team_kernel(team, false, false, false), dim3((n_max + 64u / team - 1) / (64u / team)), dim3(64),
-                               args, 0, stream));
+        launch_team(team, false, false, false, a, n_max, sc.stack_bound, stream);
         RT_HIP(hipGetLastError());
         return;
     }
@@ -637,6 +777,7 @@ void launch_trace_queue(rt_context *ctx, const Scene &sc, const rt_ray *rays, ui
     const uint32_t grid = persistent_grid(ctx, k, c.block, lds);
     void *args[] = {&a};
     RT_HIP(hipLaunchKernel(k, dim3(grid), dim3(c.block), args, lds, stream));
+    if (sc.layout() == kQ4) launch_marked(ctx, a, false, stream);
     RT_HIP(hipGetLastError());
 }
 
@@ -662,10 +803,7 @@ void launch_trace_items(rt_context *ctx, const std::vector<TraceItem> &items, ui
                     c.leaf_weight, team_limit(kLastTeam, bound)};
         const bool any = (flags & RT_TRACE_ANY) != 0, refine = (flags & RT_TRACE_FP32) == 0;
         if (const uint32_t team = team_size(ctx, layout, bound, total, c)) {  // as for one scene
-            uint32_t limit = team_limit(team, bound);
-            void *args[] = {&a, &limit};
-            RT_HIP(hipLaunchKernel(team_kernel(team, any, refine, true), dim3(((uint32_t)total + 64u / team - 1) / (64u / team)),
-                                   dim3(64), args, 0, stream));
+            launch_team(team, any, refine, true, a, total, bound, stream);
         } else {
             a.work = reinterpret_cast<unsigned long long *>(ctx->counter_slot());
             k_zero_counter<<<1, 64, 0, stream>>>(reinterpret_cast<unsigned int *>(a.work));
@@ -675,6 +813,7 @@ void launch_trace_items(rt_context *ctx, const std::vector<TraceItem> &items, ui
                                                                (total + c.block - 1) / c.block);
             void *args[] = {&a};
             RT_HIP(hipLaunchKernel(k, dim3(grid), dim3(c.block), args, lds, stream));
+            if (layout == kQ4 && !any) launch_marked(ctx, a, refine, stream);
         }
         RT_HIP(hipGetLastError());
         ctx->tables.commit(slot, stream);

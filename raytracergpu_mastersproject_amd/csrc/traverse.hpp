@@ -151,7 +151,8 @@ struct Trav {
     v3 nlo, nhi;        // per-axis slab offsets of the low and high planes (see slab_axis); of the planes a
                         // ray enters and leaves through on compressed nodes
     float tmin, bt;     // ray start; best t so far (initially tmax)
-    uint32_t bslot;     // leaf slot of the best hit (kEmpty = none)
+    float cull;         // compressed nodes, closest hit: what lies beyond is skipped; bt, or more (test_leaf)
+    uint32_t bslot;     // leaf slot of the best hit (kEmpty = none, kRedo = the ray must be traced in the exact nodes' order)
     float bu, bv;       // barycentrics of the best hit
     uint32_t cur;       // current entry (node index or leaf entry)
     bool have;          // cur is valid
@@ -247,36 +248,72 @@ __device__ __forceinline__ void slab_axis(float d, float o, float &idir, float &
 
 constexpr int kQ4 = 44;  // layout code of width 4 with compressed nodes (see node_step_q); 2, 4, 8: exact nodes
 
-// slab_axis for compressed nodes: offsets of the planes the ray enters and leaves through
-__device__ __forceinline__ void slab_axis_q(float d, float o, float &idir, float &near, float &far) {
+// ---------------------------------------------------------------------------
+// Closest hits out of another order than the exact nodes'.
+//
+// A hit's t is rounded, so it can lie a little before the box of its own leaf.  The ordered traversal of the exact nodes
+// (node_step<4>) then finds it or not, depending on what it has found before: it skips boxes behind the best hit.  Traversals in
+// other orders (compressed nodes, teams of lanes) give the same result all the same:
+//   - Let H be the hits whose leaf's exact box the ray enters, M the smallest (t, slot) of them, and E the
+//     distance at which the ray enters M's leaf.  The ordered traversal finds M unless another hit's t lies before
+//     E: every box around M is entered no later than E, and nothing but such a hit skips it.
+//   - These traversals see every hit of H up to their best one's E: they skip what lies beyond it, and their boxes are larger by
+//     the most that rounding takes a hit out of its box (ray_pad).  Hits outside H are dropped (leaf_span).
+//   - When there is no other hit before E, their result is M.  When there is, the ray is traced
+//     again over the exact nodes in their order (kRedo).  That takes two hits a few roundings apart, at a corner
+//     that both triangles share: about one ray in 10^7 into a mesh, one in 10^6 aimed at its vertices.
+// ---------------------------------------------------------------------------
+constexpr uint32_t kRedo = 0xFFFFFFFEu;  // Trav::bslot
+
+// How far outside its box a hit of this ray can lie, by the roundings of triangle_test and sphere_test.  u = 2^-24, S the sum of
+// the scene's and the origin's largest coordinates.  Triangle: 14 u S off its plane (the numerator's two products
+// 7, the denominator's 5, the division 2), 2 u S in the point, and 25 u L^3 / |e1 x e2| in the
+// plane (L its longest side): in all below 32 u S, but for needles with L^3 / |e1 x e2| > S / 2.  Sphere of radius r: the discriminant is off by
+// 21 u times the squared distance to its centre (at most 3 S^2), so the point by at most 32 u S^2 / r, and
+// along the ray by 14 u S.
+__device__ __forceinline__ float ray_pad(v3 o, const Reach &reach) {
+    const float s = reach.coord + fmaxf(fmaxf(fabsf(o.x), fabsf(o.y)), fabsf(o.z));
+    return 0x1p-19f * s * (1.0f + s * reach.inv_radius);
+}
+
+// The end of the window before the leaf of a hit at `t`, entered at `entry`: another hit there makes the result
+// depend on the order.  None (t itself) when the box is entered before the hit.
+__device__ __forceinline__ float hit_window(float t, float entry) {
+    return entry <= t * kRobust ? t : fmaxf(t, fmaf(fabsf(entry), 0x1p-21f, entry));
+}
+
+// slab_axis for compressed nodes: offsets of the planes the ray enters and leaves through, boxes larger by `pad`
+__device__ __forceinline__ void slab_axis_q(float d, float o, float pad, float &idir, float &near, float &far) {
     float lo, hi;
     slab_axis(d, o, idir, lo, hi);
-    near = idir < 0.0f ? hi : lo;
-    far = idir < 0.0f ? lo : hi;
+    const float g = pad * fabsf(idir);
+    near = (idir < 0.0f ? hi : lo) - g;
+    far = (idir < 0.0f ? lo : hi) + g;
 }
 
 // A ray that compressed nodes are not made for: a direction component so small, and not zero, that plane
-// distances overflow, or an origin beyond the scene's limit (Scene::far_limit).  It is traced over the exact
-// nodes at once when its lane takes it up.
+// distances overflow, or an origin beyond the scene's limit (Scene::reach).
 __device__ __forceinline__ bool needs_exact_nodes(v3 o, v3 d, float far_limit) {
-    return fmaxf(fmaxf(fabsf(o.x), fabsf(o.y)), fabsf(o.z)) > far_limit || (d.x != 0.0f && fabsf(d.x) < 0x1p-90f) || (d.y != 0.0f && fabsf(d.y) < 0x1p-90f) ||
-           (d.z != 0.0f && fabsf(d.z) < 0x1p-90f);
+    return fmaxf(fmaxf(fabsf(o.x), fabsf(o.y)), fabsf(o.z)) > far_limit || (d.x != 0.0f && fabsf(d.x) < 0x1p-90f) ||
+           (d.y != 0.0f && fabsf(d.y) < 0x1p-90f) || (d.z != 0.0f && fabsf(d.z) < 0x1p-90f);
 }
 
-template <int W> __device__ __forceinline__ void trav_init(Trav &t, v3 o, v3 d, float tmin, float tmax, uint32_t nwide) {
+template <int W, bool ANY>
+__device__ __forceinline__ void trav_init(Trav &t, v3 o, v3 d, float tmin, float tmax, uint32_t nwide, const Reach &reach) {
     t.o = o;
     t.d = d;
-    if constexpr (W == kQ4) {
-        slab_axis_q(d.x, o.x, t.idir.x, t.nlo.x, t.nhi.x);
-        slab_axis_q(d.y, o.y, t.idir.y, t.nlo.y, t.nhi.y);
-        slab_axis_q(d.z, o.z, t.idir.z, t.nlo.z, t.nhi.z);
+    if constexpr (W == kQ4) {  // any hit: the first one in the order of the children, whatever boxes were entered before
+        const float pad = ANY ? 0.0f : ray_pad(o, reach);
+        slab_axis_q(d.x, o.x, pad, t.idir.x, t.nlo.x, t.nhi.x);
+        slab_axis_q(d.y, o.y, pad, t.idir.y, t.nlo.y, t.nhi.y);
+        slab_axis_q(d.z, o.z, pad, t.idir.z, t.nlo.z, t.nhi.z);
     } else {
         slab_axis(d.x, o.x, t.idir.x, t.nlo.x, t.nhi.x);
         slab_axis(d.y, o.y, t.idir.y, t.nlo.y, t.nhi.y);
         slab_axis(d.z, o.z, t.idir.z, t.nlo.z, t.nhi.z);
     }
     t.tmin = tmin;
-    t.bt = tmax;
+    t.bt = t.cull = tmax;
     t.bslot = kEmpty;
     t.bu = 0.0f;
     t.bv = 0.0f;
@@ -390,39 +427,45 @@ struct LeafBoxes {
 };
 
 // Entry and exit distances of one axis of a box lo <= hi, as slab_axis and node_step compute them.
-__device__ __forceinline__ void axis_span(float lo, float hi, float idir, float near, float far, float &tn, float &tf) {
-    tn = fmaf(idir < 0.0f ? hi : lo, idir, near);
-    tf = fmaf(idir < 0.0f ? lo : hi, idir, far);
+__device__ __forceinline__ void axis_span(float lo, float hi, float d, float o, float idir, float &tn, float &tf) {
+    const float n = -(o * idir), e = d != 0.0f ? 0x1p-22f * fabsf(n) : 0.0f;
+    tn = fmaf(idir < 0.0f ? hi : lo, idir, n - e);
+    tf = fmaf(idir < 0.0f ? lo : hi, idir, n + e);
 }
 
-// the exact slab test of the leaf that holds `slot`, as node_step makes it
-__device__ __forceinline__ bool leaf_entered(const LeafBoxes &b, const Trav &t, uint32_t slot) {
-    const uint32_t ref = b.slot_ref[slot];
-    const float *p = reinterpret_cast<const float *>(b.wide) + (size_t)(ref >> 2) * 32u + (ref & 3u);
+// the entry and exit distances of child box `p` of an exact width-4 node, as node_step has them without a best hit
+__device__ __forceinline__ void box_span(const float *p, v3 o, v3 d, v3 idir, float tmin, float &entry, float &exit) {
     float nx, fx, ny, fy, nz, fz;
-    axis_span(p[0], p[4], t.idir.x, t.nlo.x, t.nhi.x, nx, fx);
-    axis_span(p[8], p[12], t.idir.y, t.nlo.y, t.nhi.y, ny, fy);
-    axis_span(p[16], p[20], t.idir.z, t.nlo.z, t.nhi.z, nz, fz);
-    return fmaxf(fmaxf(nx, ny), fmaxf(nz, t.tmin)) <= fminf(fminf(fx, fy), fminf(fz, t.bt)) * kRobust;
+    axis_span(p[0], p[4], d.x, o.x, idir.x, nx, fx);
+    axis_span(p[8], p[12], d.y, o.y, idir.y, ny, fy);
+    axis_span(p[16], p[20], d.z, o.z, idir.z, nz, fz);
+    entry = fmaxf(fmaxf(nx, ny), fmaxf(nz, tmin));
+    exit = fminf(fminf(fx, fy), fz);
+}
+
+// those of the leaf that holds `slot`
+__device__ __forceinline__ void leaf_span(const LeafBoxes &b, const Trav &t, uint32_t slot, float &entry, float &exit) {
+    const uint32_t ref = b.slot_ref[slot];
+    box_span(reinterpret_cast<const float *>(b.wide) + (size_t)(ref >> 2) * 32u + (ref & 3u), t.o, t.d, t.idir, t.tmin, entry, exit);
 }
 
 // True when the ray enters the primitive's own box, from its record and drawn in by the record's
-// rounding, so that it lies inside the leaf's box: then the leaf is entered too.  Nearly every hit
+// rounding, so that it lies inside the leaf's box, and does so by `bound`: then the leaf is entered by then too.  Nearly every hit
 // passes; the others (a hit near the box's corner, a triangle in an axis plane) look the leaf's box up.
-__device__ __forceinline__ bool primitive_entered(const LeafRecord &r, const Trav &t) {
+__device__ __forceinline__ bool primitive_entered(const LeafRecord &r, const Trav &t, float bound) {
     const bool sphere = is_sphere_record(r);
-    const auto axis = [&](float v0, float a, float b, float idir, float near, float far, float &tn,
+    const auto axis = [&](float v0, float a, float b, float d, float o, float idir, float &tn,
                           float &tf) __attribute__((always_inline)) {
         const float v1 = sphere ? v0 - r.r0.w : v0 + a, v2 = sphere ? v0 + r.r0.w : v0 + b;
         const float lo = fminf(fminf(v0, v1), v2), hi = fmaxf(fmaxf(v0, v1), v2);
         const float in = 0x1p-21f * fmaxf(fabsf(lo), fabsf(hi));
-        axis_span(lo + in, hi - in, idir, near, far, tn, tf);
+        axis_span(lo + in, hi - in, d, o, idir, tn, tf);
     };
     float nx, fx, ny, fy, nz, fz;
-    axis(r.r0.x, r.r1.x, r.r2.x, t.idir.x, t.nlo.x, t.nhi.x, nx, fx);
-    axis(r.r0.y, r.r1.y, r.r2.y, t.idir.y, t.nlo.y, t.nhi.y, ny, fy);
-    axis(r.r0.z, r.r1.z, r.r2.z, t.idir.z, t.nlo.z, t.nhi.z, nz, fz);
-    return fmaxf(fmaxf(nx, ny), fmaxf(nz, t.tmin)) <= fminf(fminf(fx, fy), fminf(fz, t.bt)) * kRobust;
+    axis(r.r0.x, r.r1.x, r.r2.x, t.d.x, t.o.x, t.idir.x, nx, fx);
+    axis(r.r0.y, r.r1.y, r.r2.y, t.d.y, t.o.y, t.idir.y, ny, fy);
+    axis(r.r0.z, r.r1.z, r.r2.z, t.d.z, t.o.z, t.idir.z, nz, fz);
+    return fmaxf(fmaxf(nx, ny), fmaxf(nz, t.tmin)) <= fminf(fminf(fx, fy), fminf(fz, bound)) * kRobust;
 }
 
 __device__ __forceinline__ double sort_min(double a, double b) {  // no canonicalisation: the bits are a key
@@ -469,7 +512,7 @@ __device__ __forceinline__ void node_step_q(Trav &t, const StackMem &m, const ui
         const float tn = fmaxf(fmaxf(fmaxf(fmaf((float)hnx, sx, nx), fmaf((float)hny, sy, ny)),
                                      fmaf((float)hnz, sz, nz)), t.tmin);
         const float tf = fminf(fminf(fminf(fmaf((float)hfx, sx, fx), fmaf((float)hfy, sy, fy)),
-                                     fmaf((float)hfz, sz, fz)), t.bt);
+                                     fmaf((float)hfz, sz, fz)), ANY ? t.bt : t.cull);
         const bool hit = tn <= fmaf(fabsf(tf), kSlackQ, tf);
         key[c] = __hiloint2double((int)(hit ? (ANY ? (uint32_t)c : __float_as_uint(tn)) : kMissKey), (int)e);
     };
@@ -530,29 +573,57 @@ template <int S, bool ANY> __device__ __forceinline__ void pop_q(Trav &t, const 
         tn = __uint_as_float(v.y);
     }
     t.cur = e;
-    t.have = ANY || !(tn > fmaxf(t.bt * kRobust, 0.0f));
+    t.have = ANY || !(tn > fmaxf(t.cull * kRobust, 0.0f));
 }
 
-// Test the primitives of one leaf entry; true when an any-hit query has found its hit.
+// Test the primitives of one leaf entry; true when the ray's traversal is over: an any-hit query has its hit, or the closest
+// hit depends on the order (kRedo).
 // boxes(): the LeafBoxes of compressed layouts (W == kQ4), not called for the others.
 template <int W, bool ANY, bool COUNT, class B>
 __device__ __forceinline__ bool test_leaf(Trav &t, uint32_t entry, const LeafRecord *__restrict__ rec, const B &boxes) {
     const uint32_t first = leaf_first(entry), cnt = leaf_count(entry);
+    constexpr bool WINDOW = W == kQ4 && !ANY;
     for (uint32_t s = first; s < first + cnt; ++s) {
         if constexpr (COUNT) t.ntri++;
         const LeafRecord r = rec[s];
+        const float last = WINDOW ? t.cull : t.bt;
         float th = 0.0f, a = 0.0f, b = 0.0f;
         bool hit;
         if (is_sphere_record(r)) {
-            hit = sphere_test(r, t.o, t.d, t.tmin, t.bt, th);
+            hit = sphere_test(r, t.o, t.d, t.tmin, last, th);
             a = r.r1.y;  // the sphere's centre-based u, v
             b = r.r1.z;
         } else {
-            hit = triangle_test(r, t.o, t.d, t.tmin, t.bt, th, a, b);
+            hit = triangle_test(r, t.o, t.d, t.tmin, last, th, a, b);
         }
-        if (hit && (th < t.bt || (th == t.bt && s < t.bslot))) {
+        if constexpr (WINDOW) {
+            if (!hit) continue;
+            float window = th;
+            if (!primitive_entered(r, t, th)) {
+                float in, out;
+                leaf_span(boxes(), t, s, in, out);
+                if (!(in <= out * kRobust)) continue;
+                window = hit_window(th, in);
+            }
+            const bool best = th < t.bt || (th == t.bt && s < t.bslot);
+            // another hit (or the ray's end) in the window of the nearer one
+            if (best ? window > th && t.bt <= window : t.cull > t.bt && th <= t.cull) {
+                t.bslot = kRedo;
+                return true;
+            }
+            if (!best) continue;
+            t.bt = th;
+            t.cull = window;
+            t.bslot = s;
+            t.bu = a;
+            t.bv = b;
+        } else if (hit && (th < t.bt || (th == t.bt && s < t.bslot))) {
             if constexpr (W == kQ4) {
-                if (!primitive_entered(r, t) && !leaf_entered(boxes(), t, s)) continue;
+                if (!primitive_entered(r, t, t.bt)) {
+                    float in, out;
+                    leaf_span(boxes(), t, s, in, out);
+                    if (!(in <= fminf(out, t.bt) * kRobust)) continue;
+                }
             }
             t.bt = th;
             t.bslot = s;
@@ -618,19 +689,24 @@ __device__ __forceinline__ void trav_run(Trav &t, const StackMem &m, const uint3
     }
 }
 
+// A ray over the exact nodes in their own order, to its end.
+template <int S, bool ANY, class B>
+__device__ __forceinline__ void walk_exact(Trav &t, const StackMem &m, v3 o, v3 d, float tmin, float tmax, uint32_t nwide,
+                                           const uint32_t *wide, const LeafRecord *rec, const B &boxes, uint32_t leaf_weight) {
+    trav_init<4, ANY>(t, o, d, tmin, tmax, nwide, Reach{});
+    trav_run<4, S, ANY, false>(t, m, wide, rec, boxes, leaf_weight);
+}
+
 // Starts a ray; on compressed nodes a ray that needs the exact ones is run to its end here (rare: the other
 // lanes of its wave wait).
 template <int W, int S, bool ANY, class B>
 __device__ __forceinline__ void walk_init(Trav &t, const StackMem &m, v3 o, v3 d, float tmin, float tmax,
-                                          uint32_t nwide, float far_limit, const LeafRecord *rec, const B &boxes,
+                                          uint32_t nwide, const Reach &reach, const LeafRecord *rec, const B &boxes,
                                           uint32_t leaf_weight) {
-    trav_init<W>(t, o, d, tmin, tmax, nwide);
-    if constexpr (W == kQ4) {
-        if (needs_exact_nodes(o, d, far_limit)) {
-            trav_init<4>(t, o, d, tmin, tmax, nwide);
-            trav_run<4, S, ANY, false>(t, m, boxes().wide, rec, boxes, leaf_weight);
-        }
-    }
+    if (W == kQ4 && needs_exact_nodes(o, d, reach.far_limit))
+        walk_exact<S, ANY>(t, m, o, d, tmin, tmax, nwide, boxes().wide, rec, boxes, leaf_weight);
+    else
+        trav_init<W, ANY>(t, o, d, tmin, tmax, nwide, reach);
 }
 
 }  // namespace rtgpu
