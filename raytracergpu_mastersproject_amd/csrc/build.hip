@@ -1239,7 +1239,7 @@ void build_scene(rt_context *ctx, Scene &sc, const rt_triangle *tris, uint32_t n
         struct { uint32_t bad; float far, extent; uint32_t pad[3]; uint32_t small; } whole{};
         RT_HIP(hipMemcpy(&whole, info, sizeof whole, hipMemcpyDeviceToHost));
         // see Scene::reach: origins may lie this far outside the scene's coordinates
-        const float reach = std::min(1000.0f * whole.extent, 512.0f * min_radius);
+        const float reach = std::min(400.0f * whole.extent, 512.0f * min_radius);
         sc.reach = Reach{whole.far + reach, whole.far, inv_radius};
         // Where a third of the leaves or more are hardly larger than a hit's rounding, the larger boxes hold too much
         // (32,000 triangles of 0.03, shifted by 1,000 from the origin: 4.6 M paths 1.5 ms and 1.5 over the exact nodes; by 3,000 2.2

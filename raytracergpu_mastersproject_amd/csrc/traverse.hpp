@@ -292,9 +292,9 @@ __device__ __forceinline__ void slab_axis_q(float d, float o, float pad, float &
 }
 
 // A ray that compressed nodes are not made for: a direction component so small, and not zero, that plane
-// distances overflow, or an origin beyond the scene's limit (Scene::reach).
-__device__ __forceinline__ bool needs_exact_nodes(v3 o, v3 d, float far_limit) {
-    return fmaxf(fmaxf(fabsf(o.x), fabsf(o.y)), fabsf(o.z)) > far_limit || (d.x != 0.0f && fabsf(d.x) < 0x1p-90f) ||
+// distances overflow; and for a closest hit an origin beyond the scene's limit (Scene::reach).
+template <bool ANY> __device__ __forceinline__ bool needs_exact_nodes(v3 o, v3 d, float far_limit) {
+    return (!ANY && fmaxf(fmaxf(fabsf(o.x), fabsf(o.y)), fabsf(o.z)) > far_limit) || (d.x != 0.0f && fabsf(d.x) < 0x1p-90f) ||
            (d.y != 0.0f && fabsf(d.y) < 0x1p-90f) || (d.z != 0.0f && fabsf(d.z) < 0x1p-90f);
 }
 
@@ -697,16 +697,19 @@ __device__ __forceinline__ void walk_exact(Trav &t, const StackMem &m, v3 o, v3 
     trav_run<4, S, ANY, false>(t, m, wide, rec, boxes, leaf_weight);
 }
 
-// Starts a ray; on compressed nodes a ray that needs the exact ones is run to its end here (rare: the other
-// lanes of its wave wait).
+// Starts a ray.  On compressed nodes one that needs the exact ones: for a closest hit false (it is left to the launch over the
+// marked rays), an any hit is run to its end here (rare: the other lanes of its wave wait).
 template <int W, int S, bool ANY, class B>
-__device__ __forceinline__ void walk_init(Trav &t, const StackMem &m, v3 o, v3 d, float tmin, float tmax,
+__device__ __forceinline__ bool walk_init(Trav &t, const StackMem &m, v3 o, v3 d, float tmin, float tmax,
                                           uint32_t nwide, const Reach &reach, const LeafRecord *rec, const B &boxes,
                                           uint32_t leaf_weight) {
-    if (W == kQ4 && needs_exact_nodes(o, d, reach.far_limit))
+    if (W == kQ4 && needs_exact_nodes<ANY>(o, d, reach.far_limit)) {
+        if constexpr (!ANY) return false;
         walk_exact<S, ANY>(t, m, o, d, tmin, tmax, nwide, boxes().wide, rec, boxes, leaf_weight);
-    else
+    } else {
         trav_init<W, ANY>(t, o, d, tmin, tmax, nwide, reach);
+    }
+    return true;
 }
 
 }  // namespace rtgpu

@@ -104,3 +104,24 @@ def test_every_schedule_renders_the_ordered_image(ctx, native, shift):
         assert np.array_equal(acc.to_numpy(np.uint32, 4 * w * h), want)
     ctx.release(a)
     ctx.release(b)
+
+
+@pytest.mark.parametrize("far", [3, 512, 513, 5000, 0])  # rays from far outside; 0: all
+@pytest.mark.parametrize("n", [5_000, 30_000, 200_001, 700_001])
+def test_rays_from_far_outside(ctx, native, n, far):
+    """They are left to a launch of their own: by a list of 512, or by the marks in the hit records."""
+    tris = _mesh(48, 0.0)
+    sid = ctx.upload(tris, None, MATS)
+    rays = W.incoherent_rays(n, *W.scene_bounds(tris), seed=7, tmax=1e7)
+    which = np.random.default_rng(n + far).permutation(n)[:far or n]
+    rays["o"][which] -= rays["d"][which] * np.float32(4000.0)
+    rays["d"][which[::50], 1] = np.float32(1e-30)  # no compressed nodes for these either
+    dr, dh = native.DeviceArray.from_numpy(rays), native.DeviceArray(16 * n)
+    for any_hit in (False, True):
+        want, _ = gpu_trace(ctx, sid, rays, counts=True, any_hit=any_hit)
+        assert np.array_equal(gpu_trace(ctx, sid, rays, any_hit=any_hit).view(np.uint32), want.view(np.uint32))
+        third = n // 3
+        ctx.trace_batch([(sid, third, dr.ptr, dh.ptr), (sid, 0, dr.ptr, dh.ptr),
+                         (sid, n - third, dr.ptr + 32 * third, dh.ptr + 16 * third)], any_hit=any_hit)
+        assert np.array_equal(dh.to_numpy(np.uint32), want.view(np.uint32))
+    ctx.release(sid)
