@@ -84,8 +84,9 @@ __device__ __forceinline__ TeamHit team_trace(bool live, v3 o, v3 d, float tmin,
     uint32_t ls = kEmpty;
     bool redo = false;                      // closest hit: this lane saw two hits in one window
     bool owner = false;                     // any hit: this lane holds the team's hit
-    uint32_t top = live && nwide > 0 && !has_nan(d) ? 1u : 0u;
-    if (top) st[0] = make_uint2(0u, __float_as_uint(tmin));  // the root (the same from every lane)
+    // the root (the same from every lane), entered as node_step enters it: a NaN tmin bounds nothing
+    uint32_t top = live && nwide > 0 && !has_nan(d) && (ANY || !(tmin > tmax * kRobust)) ? 1u : 0u;
+    if (top) st[0] = make_uint2(0u, 0xFF800000u);
     wave_fence();
     while (__ballot(top > 0) != 0ull) {
         const uint32_t take = top > limit ? 1u : min(Q, top);

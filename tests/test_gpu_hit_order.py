@@ -125,3 +125,22 @@ def test_rays_from_far_outside(ctx, native, n, far):
                          (sid, n - third, dr.ptr + 32 * third, dh.ptr + 16 * third)], any_hit=any_hit)
         assert np.array_equal(dh.to_numpy(np.uint32), want.view(np.uint32))
     ctx.release(sid)
+
+
+@pytest.mark.parametrize("n", [5_000, 30_000, 200_001, 700_001])
+def test_bounds_that_are_not_numbers(ctx, native, n):
+    """A NaN tmin bounds nothing, a NaN tmax lets no hit through, whichever route traces the ray."""
+    tris = _mesh(24, 0.0)
+    sid = ctx.upload(tris, None, MATS)
+    rays = W.incoherent_rays(n, *W.scene_bounds(tris), seed=9, tmax=1e7)
+    rays["tmin"][::3] = np.nan
+    rays["tmax"][1::7] = np.nan
+    rays["tmin"][2::5] = -np.inf
+    rays["tmax"][3::11] = np.inf
+    rays["tmin"][4::13], rays["tmax"][4::13] = 3.0, 1.0
+    for any_hit in (False, True):
+        want, _ = gpu_trace(ctx, sid, rays, counts=True, any_hit=any_hit, fp32=True)
+        assert np.mean(want["prim"][::3] != L.NO_HIT) > 0.2
+        got = gpu_trace(ctx, sid, rays, any_hit=any_hit, fp32=True)
+        assert np.array_equal(got.view(np.uint32), want.view(np.uint32))
+    ctx.release(sid)
