@@ -152,8 +152,10 @@ int rt_trace(rt_context *ctx, uint32_t scene_id, const rt_ray *rays, uint32_t n,
         RT_REQUIRE((flags & ~kTraceFlags) == 0, "unknown trace flags");
         Scene &s = ctx->scene(scene_id);
         LaunchCfg c = resolve_cfg(ctx, s, cfg, (flags & RT_TRACE_ANY) != 0);
+        SceneUse use(ctx, static_cast<hipStream_t>(stream));
+        use.add(s);
         launch_trace(ctx, s, rays, n, hits, counts, flags, c, static_cast<hipStream_t>(stream));
-        s.note_use(static_cast<hipStream_t>(stream), ctx->record_use(static_cast<hipStream_t>(stream)));
+        use.done();
     });
 }
 
@@ -170,9 +172,11 @@ int rt_render(rt_context *ctx, uint32_t scene_id, const rt_params *params, uint3
         RT_REQUIRE((flags & ~kRenderFlags) == 0, "unknown render flags");
         Scene &s = ctx->scene(scene_id);
         LaunchCfg c = resolve_cfg(ctx, s, cfg, false);
+        SceneUse use(ctx, static_cast<hipStream_t>(stream));
+        use.add(s);
         launch_render(ctx, s, *params, width, height, spp, flags, accum, segments, c,
                       static_cast<hipStream_t>(stream));
-        s.note_use(static_cast<hipStream_t>(stream), ctx->record_use(static_cast<hipStream_t>(stream)));
+        use.done();
     });
 }
 
@@ -185,9 +189,11 @@ int rt_render_noalloc(rt_context *ctx, uint32_t scene_id, const rt_params *param
         RT_REQUIRE(ctx->noalloc_scratch != nullptr, "the static scratch array has no device address");
         Scene &s = ctx->scene(scene_id);
         LaunchCfg c = resolve_cfg(ctx, s, cfg, false);
+        SceneUse use(ctx, static_cast<hipStream_t>(stream), false);
+        use.add(s);
         launch_render(ctx, s, *params, width, height, spp, flags, accum, segments, c, static_cast<hipStream_t>(stream),
                       ctx->noalloc_scratch, noalloc_scratch_bytes());
-        s.note_use(static_cast<hipStream_t>(stream), ctx->record_use(static_cast<hipStream_t>(stream), false));
+        use.done();
     });
 }
 
@@ -236,10 +242,11 @@ int rt_render_batch(rt_context *ctx, const rt_render_job *jobs, uint32_t njobs, 
             make_split(*rj, reinterpret_cast<float4 *>(scratch + off), g);
             off += 16ull * rj->width * rj->height * rj->spp;
         }
+        SceneUse use(ctx, st);
+        for (uint32_t i = 0; i < njobs; ++i) use.add(ctx->scene(jobs[i].scene_id));
         for (auto &kv : by_layout) launch_render_jobs(ctx, kv.second, kv.first, segments, c, st);
         for (auto &[s, rj] : waves) launch_render_wave(ctx, *s, rj, segments, c, st, nullptr, 0);
-        const int used = ctx->record_use(st);
-        for (uint32_t i = 0; i < njobs; ++i) ctx->scene(jobs[i].scene_id).note_use(st, used);
+        use.done();
     });
 }
 
@@ -252,9 +259,10 @@ int rt_trace_batch(rt_context *ctx, const rt_batch_item *items, uint32_t nitems,
         const bool any = (flags & RT_TRACE_ANY) != 0;
         if (nitems) c = resolve_cfg(ctx, ctx->scene(items[0].scene_id), cfg, any);
         if (!cfg && ctx->has_batch_tuned) c = any ? ctx->batch_any : ctx->batch_closest;
+        SceneUse use(ctx, static_cast<hipStream_t>(stream));
+        for (uint32_t i = 0; items && i < nitems; ++i) use.add(ctx->scene(items[i].scene_id));
         launch_trace_batch(ctx, items, nitems, flags, c, static_cast<hipStream_t>(stream));
-        const int used = ctx->record_use(static_cast<hipStream_t>(stream));
-        for (uint32_t i = 0; i < nitems; ++i) ctx->scene(items[i].scene_id).note_use(static_cast<hipStream_t>(stream), used);
+        use.done();
     });
 }
 

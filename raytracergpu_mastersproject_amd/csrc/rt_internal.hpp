@@ -502,6 +502,31 @@ struct rt_context {
 
 namespace rtgpu {
 
+// The scenes that an entry point's launches read on `stream`.  Made before the first launch: when the entry point throws after some
+// of them, the scenes' releases wait for the device, since no use event covers what was enqueued.
+class SceneUse {
+  public:
+    SceneUse(rt_context *ctx, hipStream_t stream, bool may_create_event = true)
+        : ctx_(ctx), stream_(stream), may_create_(may_create_event) {}
+    SceneUse(const SceneUse &) = delete;
+    SceneUse &operator=(const SceneUse &) = delete;
+    ~SceneUse() {
+        for (Scene *s : scenes_) s->unmarked_use = true;
+    }
+    void add(Scene &s) { scenes_.push_back(&s); }
+    void done() {  // every launch is enqueued
+        const int used = ctx_->record_use(stream_, may_create_);
+        for (Scene *s : scenes_) s->note_use(stream_, used);
+        scenes_.clear();
+    }
+
+  private:
+    rt_context *ctx_;
+    hipStream_t stream_;
+    bool may_create_;
+    std::vector<Scene *> scenes_;
+};
+
 inline void Scene::note_use(hipStream_t stream, int recorded) {
     // a graph may still run when the scene is released, and its memory then goes to the next scene
     if (recorded == rt_context::kUseCaptured || recorded == rt_context::kUseUnrecorded) {

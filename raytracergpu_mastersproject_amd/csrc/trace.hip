@@ -791,6 +791,10 @@ void launch_trace_queue(rt_context *ctx, const Scene &sc, const rt_ray *rays, ui
 
 void launch_trace_items(rt_context *ctx, const std::vector<TraceItem> &items, uint32_t flags, const LaunchCfg &c,
                         hipStream_t stream) {
+    for (const TraceItem &it : items) {  // before the first launch: a bad item leaves every hit buffer as it was
+        RT_REQUIRE(it.n == 0 || (it.rays && it.hits), "batch item with NULL rays/hits");
+        check_stack(*it.sc, c);
+    }
     // one launch per node layout present, each over that layout's items in order
     for (uint32_t layout : {2u, 4u, 8u, (uint32_t)kQ4}) {
         std::vector<BatchItemDev> hv;
@@ -798,8 +802,6 @@ void launch_trace_items(rt_context *ctx, const std::vector<TraceItem> &items, ui
         uint32_t bound = 0;
         for (const TraceItem &it : items) {
             if (it.sc->layout() != layout) continue;
-            RT_REQUIRE(it.n == 0 || (it.rays && it.hits), "batch item with NULL rays/hits");
-            check_stack(*it.sc, c);
             hv.push_back(BatchItemDev{view_of(*it.sc), it.rays, it.hits, total});
             total += it.n;
             bound = std::max(bound, it.sc->stack_bound);

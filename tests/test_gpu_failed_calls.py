@@ -1,0 +1,85 @@
+"""Calls that fail after they have, or could have, enqueued work: what they read stays until that work has ended, and what
+they refuse they leave untouched."""
+import numpy as np
+import pytest
+import torch
+
+from raytracergpu_mastersproject_amd import layouts as L
+from raytracergpu_mastersproject_amd import workloads as W
+
+from helpers import gpu_trace, small_cluster_scene
+
+pytestmark = pytest.mark.gpu
+
+
+class _NonBlocking:
+    """A stream that the null stream does not wait for, as the binding takes streams."""
+
+    def __init__(self):
+        self.stream = torch.cuda.Stream()
+        self.handle = self.stream.cuda_stream
+
+    def idle(self):
+        return self.stream.query()
+
+
+@pytest.mark.parametrize("wrong", ["hits", "rays"])
+def test_batch_with_a_bad_item_traces_nothing(ctx, native, wrong):
+    tris, mats = small_cluster_scene(4, 500, seed=71)
+    sids = [ctx.upload(tris, None, mats, width=w) for w in (2, 4, 8)]
+    rays = W.incoherent_rays(5000, *W.scene_bounds(tris), seed=72)
+    dr = native.DeviceArray.from_numpy(rays)
+    hits = [native.DeviceArray.from_numpy(np.full(4 * 5000, 7, np.uint32)) for _ in sids]
+    items = [(s, 5000, dr.ptr, h.ptr) for s, h in zip(sids, hits)]
+    items[1] = (sids[1], 5000, None, hits[1].ptr) if wrong == "rays" else (sids[1], 5000, dr.ptr, None)
+    with pytest.raises(native.RTError, match="NULL rays/hits"):
+        ctx.trace_batch(items)
+    native.synchronize()
+    for h in hits:
+        assert np.all(h.to_numpy(np.uint32) == 7)
+    for s in sids:
+        ctx.release(s)
+
+
+def test_release_waits_for_a_batch_that_failed(ctx, native):
+    """The first image is enqueued, on a stream of its own, before the others turn out to be too many for one launch."""
+    s = W.served_scene(200_000, 3)
+    sid = ctx.upload(s["tris"], None, s["materials"], width=2)  # launched first
+    other = ctx.upload(s["tris"][:64], None, s["materials"])
+    w, h, spp = 256, 256, 2000  # 0.1 s
+    acc = native.DeviceArray(16 * w * h)
+    stream = _NonBlocking()
+    ctx.accum_clear(acc, w * h)
+    native.synchronize()
+    too_many = [(other, s["params"], 65536, 32767, 1, acc.ptr + k, native.RENDER_NO_SPLIT) for k in (1 << 40, 1 << 41, 1 << 42)]
+    with pytest.raises(native.RTError, match="too many work items"):
+        ctx.render_batch([(sid, s["params"], w, h, spp, acc, native.RENDER_NO_SPLIT)] + too_many, stream=stream)
+    assert not stream.idle()
+    ctx.release(sid)
+    assert stream.idle()
+    ctx.release(other)
+
+
+def test_scenes_come_and_go_beside_a_stream_of_its_own(ctx, native):
+    """Queries on a stream that uploads do not wait for: a release waits for them before the memory is used again."""
+    stream = _NonBlocking()
+    tris = {n: W.cluster_scene(16, n // 16, seed=n)[0] for n in (4096, 65_536, 8192, 200_000)}
+    mats = W.make_materials([0.5, 0.5, 0.5], L.DIFFUSE)
+    for t in tris.values():
+        t["materialIndex"] = 0
+    rays = W.incoherent_rays(1_000_000, [-1.2] * 3, [1.2] * 3, seed=73)
+    dr = native.DeviceArray.from_numpy(rays)
+    want, outs = {}, []
+    for n, t in tris.items():
+        sid = ctx.upload(t, None, mats)
+        want[n] = gpu_trace(ctx, sid, rays)
+        ctx.release(sid)
+    for n in list(tris) * 3:
+        sid = ctx.upload(tris[n], None, mats)
+        dh = native.DeviceArray(16 * len(rays))
+        ctx.trace(sid, dr, len(rays), dh, stream=stream)
+        ctx.release(sid)
+        assert stream.idle()
+        outs.append((n, dh))
+    for n, dh in outs:
+        assert np.array_equal(dh.to_numpy(np.uint32), want[n].view(np.uint32))
