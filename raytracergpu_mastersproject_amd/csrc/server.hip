@@ -668,6 +668,9 @@ void fail_all(rt_server *s, int status, const std::string &msg) {
     };
     for (auto &r : s->queue) fail(r);
     for (auto &r : s->active) fail(r);
+    // The steps in flight still read the scenes, which no use event covers, and the callers' device buffers.
+    for (hipStream_t st : {s->stream, s->small_stream})
+        if (st) (void)hipStreamSynchronize(st);
     {
         std::lock_guard<std::recursive_mutex> lk(s->ctx->mu);
         for (auto &r : s->queue) r->scene->users--;

@@ -83,3 +83,32 @@ def test_scenes_come_and_go_beside_a_stream_of_its_own(ctx, native):
         outs.append((n, dh))
     for n, dh in outs:
         assert np.array_equal(dh.to_numpy(np.uint32), want[n].view(np.uint32))
+
+
+def test_failed_server_lets_its_steps_end(ctx, native):
+    """An unbatched server fails on a request whose flags exclude each other, with a long ray query in flight: that query's
+    scene and buffers stay until it has ended."""
+    tris, mats = W.cluster_scene(64, 8192, seed=74)
+    tris["materialIndex"] = 0
+    sid = ctx.upload(tris, None, mats)
+    n = 24_000_000  # some 5 ms
+    rays = native.DeviceArray.from_numpy(np.tile(W.incoherent_rays(n // 8, *W.scene_bounds(tris), seed=75), 8))
+    before = native.DeviceArray(16 * n)
+    ctx.trace(sid, rays, n, before)
+    want = before.to_numpy(np.uint32)
+    hits = native.DeviceArray.from_numpy(np.full(4 * n, 7, np.uint32))
+    small = W.soup_scene(64)
+    other = ctx.upload(small["tris"], None, small["materials"])
+    srv = native.Server(ctx, serial=True)
+    zeroth = srv.submit(native.trace_request_device(sid, rays, n, before))  # the others wait behind it and are enqueued together
+    first = srv.submit(native.trace_request_device(sid, rays, n, hits))
+    second = srv.submit(native.render_request(other, small["params"], 32, 32, 1, flags=native.RENDER_WAVEFRONT | native.RENDER_SPLIT_SAMPLES))
+    srv.wait(zeroth)
+    for rid in (second, first):
+        with pytest.raises(native.RTError):
+            srv.wait(rid)
+    ctx.release(sid)
+    assert np.array_equal(hits.to_numpy(np.uint32), want)
+    with pytest.raises(native.RTError):
+        srv.close()
+    ctx.release(other)
