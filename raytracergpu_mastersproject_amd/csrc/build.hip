@@ -1200,7 +1200,8 @@ void build_scene(rt_context *ctx, Scene &sc, const rt_triangle *tris, uint32_t n
     collapse();
     throw_bad_index(out.info + 4);
     if (out.info[3] && n > 1) {  // NaN planes: unions in the tree's own order, then the collapse again
-        DevBuf other(sizeof(rt_bvh_node) * (2ull * n - 1));
+        DevBuf other;
+        other.alloc_own(sizeof(rt_bvh_node) * (2ull * n - 1), ctx->pool);
         for (int pass = 0; pass < 64; pass += 2) {
             k_refit_pass<<<grid_for(2ull * n - 1), kB, 0, st>>>(binary, other.as<rt_bvh_node>(), n);
             k_refit_pass<<<grid_for(2ull * n - 1), kB, 0, st>>>(other.as<rt_bvh_node>(), binary, n);

@@ -66,11 +66,16 @@ class DevPool {
                 held_ -= cap;
                 return p;
             }
+        return fresh(cap);
+    }
+    // a new allocation of `bytes`, for which the kept blocks make room if need be
+    void *fresh(size_t bytes) {
         void *p = nullptr;
-        hipError_t e = hipMalloc(&p, cap);
+        hipError_t e = hipMalloc(&p, bytes);
         if (e == hipErrorOutOfMemory && !free_.empty()) {
+            (void)hipGetLastError();
             trim(0);
-            e = hipMalloc(&p, cap);
+            e = hipMalloc(&p, bytes);
         }
         RT_HIP(e);
         return p;
@@ -100,7 +105,7 @@ class DevPool {
     }
 };
 
-// Owning device allocation, from a pool or from hipMalloc.
+// Owning device allocation, from a pool (alloc) or its own (alloc_own), for which a pool gives up what it keeps if need be.
 struct DevBuf {
     void *p = nullptr;
     size_t bytes = 0, cap = 0;
@@ -125,6 +130,13 @@ struct DevBuf {
         pool = from;
         if (pool) p = pool->take(n, cap);
         else RT_HIP(hipMalloc(&p, n));
+        bytes = n;
+    }
+    void alloc_own(size_t n, DevPool &spare) {
+        release();
+        if (n == 0) return;
+        pool = nullptr;
+        p = spare.fresh(n);
         bytes = n;
     }
     void release() {
@@ -271,6 +283,7 @@ constexpr uint32_t kRenderChunk = 64;  // work items (one 8x8 tile) per atomic o
 // waits on events recorded on the ring stream, which lives as long as the ring, never on
 // events of a caller's stream that may have been destroyed since.
 class TableRing {
+    DevPool &spare_;
     static constexpr int kSlots = 128;
     struct Slot {
         void *host = nullptr;
@@ -285,7 +298,7 @@ class TableRing {
     hipStream_t ring_ = nullptr;
 
 public:
-    TableRing() = default;
+    explicit TableRing(DevPool &spare) : spare_(spare) {}
     TableRing(const TableRing &) = delete;
     TableRing &operator=(const TableRing &) = delete;
     ~TableRing() {
@@ -316,7 +329,7 @@ public:
             s.host = nullptr;
             s.cap = 0;
             RT_HIP(hipHostMalloc(&s.host, cap, hipHostMallocDefault));
-            s.dev.alloc(cap);
+            s.dev.alloc_own(cap, spare_);
             s.cap = cap;
         }
         std::memcpy(s.host, src, bytes);
@@ -356,6 +369,7 @@ class ScratchCache {
         bool used = false, taken = false;
     };
 
+    explicit ScratchCache(DevPool &spare) : spare_(spare) {}
     ~ScratchCache() {
         for (auto &b : blocks_)
             if (b->done) (void)hipEventDestroy(b->done);
@@ -370,7 +384,7 @@ class ScratchCache {
         if (!best) {
             trim(bytes);
             auto b = std::make_unique<Block>();
-            b->buf.alloc((bytes + kGrain - 1) / kGrain * kGrain);
+            b->buf.alloc_own((bytes + kGrain - 1) / kGrain * kGrain, spare_);
             RT_HIP(hipEventCreateWithFlags(&b->done, hipEventDisableTiming));
             best = b.get();
             blocks_.push_back(std::move(b));
@@ -389,6 +403,7 @@ class ScratchCache {
     }
 
   private:
+    DevPool &spare_;
     std::vector<std::unique_ptr<Block>> blocks_;
 
     static bool usable(const Block &b, hipStream_t st) {
@@ -440,14 +455,14 @@ struct rt_context {
     rtgpu::DevBuf counters;
     uint32_t next_counter = 0;
     static constexpr uint32_t kCounterSlots = 4096;
-    rtgpu::TableRing tables;
+    rtgpu::TableRing tables{pool};
     // launch configuration chosen by rt_autotune_batch for fused multi-scene launches
     bool has_batch_tuned = false;
     rtgpu::LaunchCfg batch_closest, batch_any;
     // Held by every entry point for its duration and by a server's worker thread while
     // it enqueues a step, so a context may be shared by the caller and its servers.
     std::recursive_mutex mu;
-    rtgpu::ScratchCache scratch;  // launch scratch (split samples, path storage)
+    rtgpu::ScratchCache scratch{pool};  // launch scratch (split samples, path storage)
     // the device address of this GPU's static scratch array (rt_render_noalloc), taken at rt_create
     char *noalloc_scratch = nullptr;
 

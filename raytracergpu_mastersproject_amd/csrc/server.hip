@@ -791,7 +791,7 @@ int rt_server_create(rt_context *ctx, const rt_server_config *cfg, rt_server **o
         RT_REQUIRE((s->cfg.flags & ~(RT_SERVER_SERIAL | RT_SERVER_NO_YIELD)) == 0, "unknown server flags");
         std::lock_guard<std::recursive_mutex> lk(ctx->mu);
         RT_HIP(hipSetDevice(ctx->device));
-        s->arena_mem.alloc(s->cfg.arena_bytes);
+        s->arena_mem.alloc_own(s->cfg.arena_bytes, ctx->pool);
         s->scratch_base = s->cfg.arena_bytes / 2 / Arena::kAlign * Arena::kAlign;
         s->arena.reset(s->scratch_base);
         s->scratch.reset(s->cfg.arena_bytes - s->scratch_base);

@@ -1,0 +1,82 @@
+"""The host-side owners of device memory against a small device of their own: the HIP calls they make are replaced by ones
+that hand out host memory up to a limit (compiled for the host only; no GPU and no HIP runtime)."""
+import subprocess
+
+import pytest
+
+from raytracergpu_mastersproject_amd import build as B
+
+FAKE = r"""
+#include <cstdio>
+#include <cstdlib>
+#include <map>
+#include "rt_internal.hpp"
+using namespace rtgpu;
+
+static size_t limit = 1u << 30, used = 0;
+static int mallocs = 0, live_events = 0;
+static std::map<void *, size_t> blocks;
+extern "C" {
+hipError_t hipMalloc(void **p, size_t n) {
+    ++mallocs;
+    if (used + n > limit) return hipErrorOutOfMemory;
+    *p = std::malloc(1);
+    blocks[*p] = n;
+    used += n;
+    return hipSuccess;
+}
+hipError_t hipFree(void *p) {
+    auto it = blocks.find(p);
+    if (it == blocks.end()) std::abort();
+    used -= it->second;
+    blocks.erase(it);
+    std::free(p);
+    return hipSuccess;
+}
+hipError_t hipGetLastError() { return hipSuccess; }
+const char *hipGetErrorString(hipError_t) { return "error"; }
+hipError_t hipEventCreateWithFlags(hipEvent_t *e, unsigned) { ++live_events; *e = reinterpret_cast<hipEvent_t>(1); return hipSuccess; }
+hipError_t hipEventCreate(hipEvent_t *e) { ++live_events; *e = reinterpret_cast<hipEvent_t>(1); return hipSuccess; }
+hipError_t hipEventDestroy(hipEvent_t) { --live_events; return hipSuccess; }
+hipError_t hipEventQuery(hipEvent_t) { return hipSuccess; }
+hipError_t hipEventRecord(hipEvent_t, hipStream_t) { return hipSuccess; }
+}
+#define CHECK(c) do { if (!(c)) { std::printf("line %d: %s\n", __LINE__, #c); return 1; } } while (0)
+int main() {
+    constexpr size_t MB = 1u << 20;
+@BODY@
+    return 0;
+}
+"""
+
+
+def _run(tmp_path, body):
+    src = tmp_path / "fake.hip"
+    src.write_text(FAKE.replace("@BODY@", body))
+    flags = [f for f in B.COMMON if not f.startswith("--offload-arch")]
+    subprocess.run([B.HIPCC, "--offload-host-only", *flags, "-c", str(src), "-o", str(tmp_path / "fake.o")], check=True)
+    subprocess.run(["g++", str(tmp_path / "fake.o"), "-o", str(tmp_path / "fake"), "-pthread"], check=True)
+    r = subprocess.run([str(tmp_path / "fake")], capture_output=True, text=True)
+    assert r.returncode == 0, r.stdout
+
+
+MAKES_ROOM = {
+    "another scene": "DevBuf b(600 * MB, &pool); CHECK(b.p);",
+    "an arena": "DevBuf b; b.alloc_own(600 * MB, pool); CHECK(b.p && b.bytes == 600 * MB);",
+    "path storage": "ScratchCache c(pool); { ScratchLease l(c, 600 * MB, nullptr); CHECK(l.ptr()); }",
+}
+
+
+@pytest.mark.parametrize("what", MAKES_ROOM)
+def test_kept_memory_makes_room(tmp_path, what):
+    """700 MB kept of a released scene, 324 MB left: 600 MB for something else of the same context."""
+    _run(tmp_path, """
+    {
+        DevPool pool;
+        { DevBuf a(350 * MB, &pool), b(340 * MB, &pool); }
+        CHECK(used > 690 * MB);  // kept
+        %s
+        try { DevBuf b; b.alloc_own(2000 * MB, pool); CHECK(false); } catch (const Error &e) { CHECK(e.status == RT_ERR_NO_MEMORY); }
+    }
+    CHECK(used == 0 && live_events == 0);
+""" % MAKES_ROOM[what])
