@@ -147,6 +147,7 @@ struct DevBuf {
         p = nullptr;
         bytes = 0;
     }
+    size_t held() const { return p && pool ? cap : bytes; }  // what it takes of the device
     template <class T> T *as() const { return static_cast<T *>(p); }
 };
 
@@ -235,8 +236,8 @@ struct Scene {
     // rt_context::record_use for that stream.
     void note_use(hipStream_t stream, int recorded);
     uint64_t device_bytes() const {
-        return wide.bytes + qwide.bytes + slot_ref.bytes + records.bytes + slot_prim.bytes + slot_mat.bytes + materials.bytes + binary.bytes +
-               tris.bytes + spheres.bytes;
+        return wide.held() + qwide.held() + slot_ref.held() + records.held() + slot_prim.held() + slot_mat.held() + materials.held() +
+               binary.held() + tris.held() + spheres.held();
     }
 };
 

@@ -80,3 +80,20 @@ def test_kept_memory_makes_room(tmp_path, what):
     }
     CHECK(used == 0 && live_events == 0);
 """ % MAKES_ROOM[what])
+
+
+def test_scene_size_is_what_it_takes_of_the_device(tmp_path):
+    """Pooled blocks are rounded up to 4..7 times a power of two."""
+    _run(tmp_path, """
+    DevPool pool;
+    Scene s;
+    s.wide.alloc(33 * MB, &pool);
+    s.records.alloc(4097, &pool);
+    s.tris.alloc(100 * MB, &pool);
+    CHECK(s.device_bytes() == used);
+    s.spheres = DevBuf(5 * MB, &pool);  // moved, as the build does
+    s.qwide.alloc(9 * MB, &pool);
+    CHECK(s.device_bytes() == used);
+    s.qwide.release();
+    CHECK(s.device_bytes() < used);  // kept, but not the scene's
+""")
