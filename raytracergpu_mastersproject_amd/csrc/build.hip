@@ -1076,13 +1076,11 @@ void build_scene(rt_context *ctx, Scene &sc, const rt_triangle *tris, uint32_t n
         return;
     }
     hipStream_t st = nullptr;
-    hipEvent_t ev0, ev1;
-    RT_HIP(hipEventCreate(&ev0));
-    RT_HIP(hipEventCreate(&ev1));
+    Event ev0, ev1;
     DevBuf dtris, dsph, dmodels;
     upload(ctx, dtris, tris, ntri);
     upload(ctx, dsph, sph, nsph);
-    RT_HIP(hipEventRecord(ev0, st));
+    RT_HIP(hipEventRecord(ev0.e, st));
     if (models) {
         upload(ctx, dmodels, models, 16ull * nmodels);
         k_model_to_world<<<grid_for(n), kB, 0, st>>>(dtris.as<rt_triangle>(), ntri, dsph.as<rt_sphere>(), nsph,
@@ -1229,12 +1227,10 @@ void build_scene(rt_context *ctx, Scene &sc, const rt_triangle *tris, uint32_t n
                                                              sample);
     });
     RT_HIP(hipGetLastError());
-    RT_HIP(hipEventRecord(ev1, st));
-    RT_HIP(hipEventSynchronize(ev1));
+    RT_HIP(hipEventRecord(ev1.e, st));
+    RT_HIP(hipEventSynchronize(ev1.e));
     float ms = 0.0f;
-    RT_HIP(hipEventElapsedTime(&ms, ev0, ev1));
-    (void)hipEventDestroy(ev0);
-    (void)hipEventDestroy(ev1);
+    RT_HIP(hipEventElapsedTime(&ms, ev0.e, ev1.e));
 
     if (W == 4) {
         struct { uint32_t bad; float far, extent; uint32_t pad[3]; uint32_t small; } whole{};

@@ -151,6 +151,15 @@ struct DevBuf {
     template <class T> T *as() const { return static_cast<T *>(p); }
 };
 
+// Owning timing event.
+struct Event {
+    hipEvent_t e = nullptr;
+    Event() { RT_HIP(hipEventCreate(&e)); }
+    Event(const Event &) = delete;
+    Event &operator=(const Event &) = delete;
+    ~Event() { (void)hipEventDestroy(e); }
+};
+
 // Launch configuration actually used by a kernel (after defaults are applied).
 struct LaunchCfg {
     uint32_t block = 128;

@@ -97,3 +97,15 @@ def test_scene_size_is_what_it_takes_of_the_device(tmp_path):
     s.qwide.release();
     CHECK(s.device_bytes() < used);  // kept, but not the scene's
 """)
+
+
+def test_events_of_a_refused_build_are_destroyed(tmp_path):
+    _run(tmp_path, """
+    try {
+        Event a, b;
+        CHECK(live_events == 2);
+        throw Error(RT_ERR_INVALID, "triangle 3: materialIndex out of range");
+    } catch (const Error &) {
+    }
+    CHECK(live_events == 0);
+""")
