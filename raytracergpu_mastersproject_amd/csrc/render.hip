@@ -1360,6 +1360,7 @@ void launch_render_wave(rt_context *ctx, const Scene &sc, const RenderJob &j, un
     RT_REQUIRE(maxp < (1ull << 32), "too many paths in one pass");
     LaunchCfg tc = c;
     tc.persistent = 1;
+    tc.teams = true;
     std::unique_ptr<ScratchLease> lease;
     if (!scratch) lease = std::make_unique<ScratchLease>(ctx->scratch, wave_scratch_bytes(maxp), stream);
     char *mem = scratch ? scratch : lease->ptr();

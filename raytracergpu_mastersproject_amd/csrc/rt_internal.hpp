@@ -168,6 +168,7 @@ struct LaunchCfg {
     uint32_t refill = 16;
     uint32_t leaf_weight = 2;  // leaf phase when leaf lanes * weight >= node lanes
     uint32_t shade_min = 24;   // render: shade when this many lanes hold a resolved segment
+    bool teams = true;         // launches of few rays by several lanes per ray; not with a caller's one lane per ray
 };
 
 // Copies large host arrays to the device through pinned buffers that a few threads fill while the copies of

@@ -438,7 +438,7 @@ bool enqueue_step(rt_server *s, bool big_lane) {
         const uint32_t kflags = r->req.render_flags & ~RT_REQ_OUT_ACCUM;
         if (!rc_set) {
             rc = resolve_cfg(s->ctx, *r->scene, &s->cfg.render_cfg, false);
-            if (!s->cfg.render_cfg.persistent) rc.persistent = 1;
+            if (!s->cfg.render_cfg.persistent) rc.persistent = 1, rc.teams = true;
             rc_set = true;
         }
         check_stack(*r->scene, rc);
@@ -492,7 +492,7 @@ bool enqueue_step(rt_server *s, bool big_lane) {
             auto &items = groups[flags];
             if (items.empty()) continue;
             LaunchCfg tc = resolve_cfg(s->ctx, *items[0].sc, &s->cfg.trace_cfg, (flags & RT_TRACE_ANY) != 0);
-            if (!s->cfg.trace_cfg.persistent) tc.persistent = 1;
+            if (!s->cfg.trace_cfg.persistent) tc.persistent = 1, tc.teams = true;
             // a lone query goes through the single-scene kernel: the fused launch's item table and
             // per-chunk item lookup only pay off over several
             if (serial || items.size() == 1)

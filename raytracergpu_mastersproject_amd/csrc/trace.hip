@@ -682,6 +682,7 @@ LaunchCfg resolve_cfg(const rt_context *ctx, const Scene &sc, const rt_launch_co
         if (cfg->block) c.block = cfg->block;
         if (cfg->lds_stack) c.lds_stack = cfg->lds_stack;
         c.persistent = cfg->persistent;
+        c.teams = cfg->persistent != 0u;
         if (cfg->refill) c.refill = cfg->refill;
     }
     RT_REQUIRE(c.block == 64 || c.block == 128 || c.block == 256, "block must be 64, 128 or 256");
@@ -701,9 +702,10 @@ LaunchCfg resolve_cfg(const rt_context *ctx, const Scene &sc, const rt_launch_co
 //                      (4 M triangles 333 and 376, 427 and 392; 1,024 triangles 82 and 89, 102 and 93)
 // Four lanes per ray were slower than eight at every size.  A launch that counts tests per ray keeps
 // one lane per ray (its counts are those of the ordered traversal), as do the widths 2 and 8, a
-// caller's one-lane-per-ray configuration, and a tree too deep for the team's stack.
+// caller's one-lane-per-ray configuration, and a tree too deep for the team's stack.  A tuned configuration says
+// how the larger launches run: that one lane per ray was the best shape at the tuner's size says nothing about small ones.
 static uint32_t team_size(const rt_context *ctx, uint32_t layout, uint32_t stack_bound, uint64_t n, const LaunchCfg &c) {
-    if (layout != kQ4 || !c.persistent) return 0;
+    if (layout != kQ4 || !c.teams) return 0;
     const uint64_t cus = (uint64_t)ctx->num_cus;
     if (n > 1536u * cus) return 0;
     const uint32_t t = n <= 24u * cus ? 64u : n <= 128u * cus ? 32u : n <= 1024u * cus ? 16u : 8u;

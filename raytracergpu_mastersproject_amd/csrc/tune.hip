@@ -71,11 +71,14 @@ struct Best {
     uint32_t tried = 0;
 };
 
+// The shapes are timed without teams, which run a launch of few rays whatever its shape: else such a sample would choose
+// by chance, and larger launches run with that choice.  The time returned is that of a launch as it will run.
 Best search(Timer &timer, const std::vector<LaunchCfg> &space,
             const std::function<void(const LaunchCfg &, hipStream_t)> &launch) {
     Best b;
     b.cfg = space[0];
-    for (const LaunchCfg &c : space) {
+    for (LaunchCfg c : space) {
+        c.teams = false;
         const float ms = timer.median_ms([&](hipStream_t s) { launch(c, s); });
         b.tried++;
         if (ms < b.ms) {
@@ -83,6 +86,8 @@ Best search(Timer &timer, const std::vector<LaunchCfg> &space,
             b.cfg = c;
         }
     }
+    b.cfg.teams = true;
+    b.ms = timer.median_ms([&](hipStream_t s) { launch(b.cfg, s); });
     return b;
 }
 

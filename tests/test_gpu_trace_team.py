@@ -84,3 +84,33 @@ def test_deep_trees(ctx, native, ntri, n):
                                   cfg=native.launch_config(block=64, lds_stack=16, persistent=0)))
         assert np.mean(g["prim"] != L.NO_HIT) > 0.001
     ctx.release(sid)
+
+
+def test_a_tuned_shape_leaves_small_launches_to_teams(ctx, native):
+    """Tuned with more rays than teams are best at, where one lane per ray wins; a small query then takes as long as before."""
+    s = W.soup_scene(1024)
+    sid = ctx.upload(s["tris"], None, s["materials"])
+    lo, hi = W.scene_bounds(s["tris"])
+    n = 300_000
+    many = native.DeviceArray.from_numpy(W.incoherent_rays(n, lo, hi, seed=38))
+    few = native.DeviceArray.from_numpy(W.incoherent_rays(4096, lo, hi, seed=39))
+    hits = native.DeviceArray(16 * n)
+
+    def small_us():
+        t = []
+        for _ in range(40):
+            a, b = native.Event(), native.Event()
+            a.record()
+            ctx.trace(sid, few, 4096, hits)
+            b.record()
+            t.append(a.elapsed_ms(b) * 1e3)
+        return float(np.median(t))
+
+    before = small_us()
+    res = ctx.autotune(sid, many, n, hits)
+    assert res.cfg.persistent == 0  # else this test says nothing
+    assert small_us() < 1.8 * before
+    want = gpu_trace(ctx, sid, W.incoherent_rays(4096, lo, hi, seed=39), cfg=native.launch_config(persistent=0))
+    ctx.trace(sid, few, 4096, hits)
+    assert np.array_equal(hits.to_numpy(np.uint32, 4 * 4096), want.view(np.uint32))
+    ctx.release(sid)
