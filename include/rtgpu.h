@@ -124,13 +124,15 @@ int rt_scene_upload(rt_context *ctx, uint32_t *scene_id, const rt_triangle *tris
                     const rt_sphere *spheres, uint32_t nsph, const rt_material *materials, uint32_t nmat,
                     const float *models, uint32_t nmodels, const rt_bvh_node *nodes, uint32_t nnodes,
                     const rt_build_options *opts);
+/* Waits for the work that reads the scene.  Up to 1 GiB of released scenes' memory stays with the context for the next
+ * uploads and for whatever else of it needs room; rt_destroy gives it back. */
 int rt_scene_release(rt_context *ctx, uint32_t scene_id);
 
 typedef struct rt_scene_info {
     uint32_t ntri, nsph, nmat, nprim;
     uint32_t width, leaf_size, nwide, wide_depth;
     uint32_t stack_bound, flags;
-    uint64_t device_bytes; /* resident bytes (wide nodes + leaf records + tables) */
+    uint64_t device_bytes; /* device memory it takes (nodes + leaf records + tables), blocks as allocated */
     float build_ms;        /* device time of the last build */
     float _pad;
 } rt_scene_info;
@@ -184,8 +186,10 @@ int rt_trace(rt_context *ctx, uint32_t scene_id, const rt_ray *rays, uint32_t n,
 /* How paths are scheduled.  By default rt_render renders bounce by bounce over width-4 trees with compressed nodes:
  * the primary segments are traced once per pixel, a shading kernel runs every sample's first bounce and queues
  * the paths that scatter, and one persistent launch carries every queued path to its end, with several lanes per path
- * for small images.  Over other trees, and in rt_render_batch, an image of fewer than 2^22 pixel-samples
- * instead carries every path to its end inside one persistent launch from the start.  The image is the same either way.
+ * for small images.  Over other trees, in rt_render_batch, while the stream is captured into a graph, and where the path
+ * storage (120 B a path) cannot be allocated, an image of fewer than 2^22 pixel-samples instead carries every path to its
+ * end inside one persistent launch from the start; with one sample a pixel that takes no storage.  The image is the same
+ * either way.
  * RT_RENDER_SPLIT_SAMPLES and RT_RENDER_NO_SPLIT describe the persistent launch and select it. */
 #define RT_RENDER_WAVEFRONT 16u          /* always bounce by bounce */
 #define RT_RENDER_PERSISTENT_PATHS 32u   /* always one persistent launch */

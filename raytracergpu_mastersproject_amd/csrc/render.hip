@@ -1519,11 +1519,32 @@ void launch_render(rt_context *ctx, const Scene &sc, const rt_params &p, uint32_
     RenderJob j = make_render_job(sc, p, width, height, spp, flags, accum);
     if (spp == 0) return;
     check_stack(sc, c);
-    const bool fits = !scratch || scratch_bytes >= wave_scratch_bytes((uint64_t)width * height);
-    if (bounce_by_bounce(ctx, sc, j, flags) && (fits || wave_schedule(width, height, spp, flags))) {
+    const uint64_t npix = (uint64_t)width * height;
+    const bool fits = !scratch || scratch_bytes >= wave_scratch_bytes(npix), must = wave_schedule(width, height, spp, flags);
+    bool wave = must || (fits && bounce_by_bounce(ctx, sc, j, flags));
+    std::unique_ptr<ScratchLease> paths;
+    if (wave && !must && !scratch) {
+        // An image that the persistent launch would do too takes no path storage where that may not be allocated: while
+        // its stream is captured, and when there is none.
+        hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
+        if (stream && hipStreamIsCapturing(stream, &cs) == hipSuccess && cs != hipStreamCaptureStatusNone) {
+            wave = false;
+        } else {
+            scratch_bytes = wave_scratch_bytes(npix * std::min<uint64_t>(spp, per_pass_limit(npix)));
+            try {
+                paths = std::make_unique<ScratchLease>(ctx->scratch, scratch_bytes, stream);
+                scratch = paths->ptr();
+            } catch (const Error &e) {
+                if (e.status != RT_ERR_NO_MEMORY) throw;
+                (void)hipGetLastError();
+                wave = false;
+            }
+        }
+    }
+    if (wave) {
         if (!fits)
             throw Error(RT_ERR_BUDGET, "one sample of a " + std::to_string(width) + "x" + std::to_string(height) +
-                                           " image needs " + std::to_string(wave_scratch_bytes((uint64_t)width * height)) +
+                                           " image needs " + std::to_string(wave_scratch_bytes(npix)) +
                                            " bytes of path storage; the scratch holds " + std::to_string(scratch_bytes));
         launch_render_wave(ctx, sc, j, segments, c, stream, scratch, scratch_bytes);
         return;
