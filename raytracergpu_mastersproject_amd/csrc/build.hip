@@ -18,6 +18,7 @@
 #include <thread>
 #include <vector>
 
+#include "box_levels.hpp"
 #include "rt_internal.hpp"
 
 namespace rtgpu {
@@ -490,29 +491,23 @@ __device__ inline Box box_union(const Box &a, const Box &b) {
 }
 __device__ inline Box node_box(const rt_bvh_node &n) { return Box{{n.minX, n.maxX, n.minY, n.maxY, n.minZ, n.maxZ}}; }
 
-// Level k of the table holds n >> k boxes (whole ones only) at offset(k), k >= 1.
-struct BoxTable {
+struct BoxTable {  // its levels: box_levels.hpp
     const rt_bvh_node *leaves;
     Box *boxes;
     uint32_t n;
-    __host__ __device__ static uint64_t boxes_before(uint32_t n, uint32_t k) {  // in levels 1..k-1
-        uint64_t s = 0;
-        for (uint32_t l = 1; l < k; ++l) s += n >> l;
-        return s;
-    }
 };
 
 // Levels level+1 .. level+8 from level `level` (0: the leaves).  A block takes 256 of its boxes.
 __global__ __launch_bounds__(kB) void k_box_table(BoxTable t, uint32_t level) {
     __shared__ Box sh[kB];
-    const uint32_t have = t.n >> level, i = blockIdx.x * kB + threadIdx.x;
+    const uint32_t have = box_count(t.n, level), i = blockIdx.x * kB + threadIdx.x;
     if (i < have) {
         if (level == 0) sh[threadIdx.x] = node_box(t.leaves[i]);
-        else sh[threadIdx.x] = t.boxes[BoxTable::boxes_before(t.n, level) + i];
+        else sh[threadIdx.x] = t.boxes[boxes_before(t.n, level) + i];
     }
-    uint64_t at = BoxTable::boxes_before(t.n, level + 1u);
+    uint64_t at = boxes_before(t.n, level + 1u);
     for (uint32_t k = 1; k <= 8u; ++k) {
-        const uint32_t count = t.n >> (level + k), j = blockIdx.x * (kB >> k) + threadIdx.x;
+        const uint32_t count = box_count(t.n, level + k), j = blockIdx.x * (kB >> k) + threadIdx.x;
         const bool mine = threadIdx.x < (kB >> k) && j < count;
         Box b;
         __syncthreads();
@@ -548,7 +543,7 @@ __global__ void k_refit(rt_bvh_node *nodes, const uint2 *range, BoxTable t) {
         }
         l >>= 1;
         r >>= 1;
-        at += level ? t.n >> level : 0u;
+        at += level ? box_count(t.n, level) : 0u;
         ++level;
     }
     const Box b = hl && hr ? box_union(left, right) : hl ? left : right;
@@ -576,7 +571,7 @@ uint64_t refit_temp_bytes(uint64_t n) { return round256(sizeof(Box) * n); }
 void refit(rt_bvh_node *nodes, const uint2 *range, uint32_t n, hipStream_t st, Temps &tmp) {
     const uint64_t mk = tmp.mark();
     BoxTable t{nodes + (n - 1), tmp.take<Box>(n), n};
-    for (uint32_t level = 0; (n >> level) > 1u; level += 8) k_box_table<<<grid_for(n >> level), kB, 0, st>>>(t, level);
+    for (uint32_t level = 0; box_count(n, level) > 1u; level += 8) k_box_table<<<grid_for(box_count(n, level)), kB, 0, st>>>(t, level);
     k_refit<<<grid_for(n - 1), kB, 0, st>>>(nodes, range, t);
     tmp.release(mk);
 }
