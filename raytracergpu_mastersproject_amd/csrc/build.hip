@@ -9,13 +9,10 @@
 // leaf slot (LeafRecord).  The reference's single-workgroup reduction and sort
 // are replaced by device-wide kernels.
 #include <algorithm>
-#include <atomic>
 #include <cmath>
 #include <cstddef>
 #include <cstring>
 #include <limits>
-#include <system_error>
-#include <thread>
 #include <vector>
 
 #include "box_levels.hpp"
@@ -1013,38 +1010,6 @@ void validate_nodes(const rt_bvh_node *nodes, uint32_t n, uint32_t ntri, uint32_
 }
 
 }  // namespace
-
-void HostStage::copy(int device, void *dst, const void *src, size_t bytes) {
-    const size_t chunks = (bytes + kChunk - 1) / kChunk;
-    std::atomic<size_t> next{0};
-    hipError_t status[kThreads] = {};
-    const auto work = [&](int id) {
-        hipError_t &e = status[id];
-        if ((e = hipSetDevice(device)) != hipSuccess) return;
-        for (int turn = 0;; turn ^= 1) {
-            const size_t c = next.fetch_add(1);
-            if (c >= chunks) return;
-            Buf &b = bufs_[id][turn];
-            if (!b.done && (e = hipEventCreateWithFlags(&b.done, hipEventDisableTiming)) != hipSuccess) return;
-            if (!b.host && (e = hipHostMalloc(&b.host, kChunk, hipHostMallocDefault)) != hipSuccess) return;
-            if (b.pending && (e = hipEventSynchronize(b.done)) != hipSuccess) return;
-            b.pending = false;
-            const size_t at = c * kChunk, len = std::min(kChunk, bytes - at);
-            std::memcpy(b.host, static_cast<const char *>(src) + at, len);
-            if ((e = hipMemcpyAsync(static_cast<char *>(dst) + at, b.host, len, hipMemcpyHostToDevice, nullptr)) != hipSuccess) return;
-            if ((e = hipEventRecord(b.done, nullptr)) != hipSuccess) return;
-            b.pending = true;
-        }
-    };
-    std::vector<std::thread> others;
-    try {
-        for (int id = 1; id < kThreads; ++id) others.emplace_back(work, id);
-    } catch (const std::system_error &) {  // fewer threads then: whoever runs takes the chunks
-    }
-    work(0);
-    for (std::thread &t : others) t.join();
-    for (hipError_t e : status) RT_HIP(e);
-}
 
 void build_scene(rt_context *ctx, Scene &sc, const rt_triangle *tris, uint32_t ntri, const rt_sphere *sph,
                  uint32_t nsph, const rt_material *mats, uint32_t nmat, const float *models, uint32_t nmodels,

@@ -4,6 +4,7 @@
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
+#include <atomic>
 #include <cstdint>
 #include <cstring>
 #include <map>
@@ -11,6 +12,7 @@
 #include <mutex>
 #include <stdexcept>
 #include <string>
+#include <thread>
 #include <vector>
 
 #include "../../include/rtgpu.h"
@@ -200,6 +202,39 @@ class HostStage {
     }
     void copy(int device, void *dst, const void *src, size_t bytes);
 };
+
+inline void HostStage::copy(int device, void *dst, const void *src, size_t bytes) {
+    const size_t chunks = (bytes + kChunk - 1) / kChunk;
+    std::atomic<size_t> next{0};
+    hipError_t status[kThreads] = {};
+    const auto work = [&](int id) {
+        hipError_t &e = status[id];
+        if ((e = hipSetDevice(device)) != hipSuccess) return;
+        for (int turn = 0;; turn ^= 1) {
+            const size_t c = next.fetch_add(1);
+            if (c >= chunks) return;
+            Buf &b = bufs_[id][turn];
+            if (!b.done && (e = hipEventCreateWithFlags(&b.done, hipEventDisableTiming)) != hipSuccess) return;
+            if (!b.host && (e = hipHostMalloc(&b.host, kChunk, hipHostMallocDefault)) != hipSuccess) return;
+            if (b.pending && (e = hipEventSynchronize(b.done)) != hipSuccess) return;
+            b.pending = false;
+            const size_t at = c * kChunk, len = std::min(kChunk, bytes - at);
+            std::memcpy(b.host, static_cast<const char *>(src) + at, len);
+            if ((e = hipMemcpyAsync(static_cast<char *>(dst) + at, b.host, len, hipMemcpyHostToDevice, nullptr)) != hipSuccess) return;
+            if ((e = hipEventRecord(b.done, nullptr)) != hipSuccess) return;
+            b.pending = true;
+        }
+    };
+    std::vector<std::thread> others;
+    try {
+        others.reserve(kThreads - 1);
+        for (int id = 1; id < kThreads; ++id) others.emplace_back(work, id);
+    } catch (const std::exception &) {  // fewer threads then: whoever runs takes the chunks
+    }
+    work(0);
+    for (std::thread &t : others) t.join();
+    for (hipError_t e : status) RT_HIP(e);
+}
 
 // A scene resident in HBM.
 struct Scene {

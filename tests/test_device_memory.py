@@ -16,6 +16,13 @@ using namespace rtgpu;
 static size_t limit = 1u << 30, used = 0;
 static int mallocs = 0, live_events = 0;
 static std::map<void *, size_t> blocks;
+static std::atomic<int> news_left{1 << 30};  // operator new fails when it has run out
+void *operator new(size_t n) {
+    if (news_left-- <= 0) throw std::bad_alloc();
+    return std::malloc(n ? n : 1);
+}
+void operator delete(void *p) noexcept { std::free(p); }
+void operator delete(void *p, size_t) noexcept { std::free(p); }
 extern "C" {
 hipError_t hipMalloc(void **p, size_t n) {
     ++mallocs;
@@ -40,6 +47,11 @@ hipError_t hipEventCreate(hipEvent_t *e) { ++live_events; *e = reinterpret_cast<
 hipError_t hipEventDestroy(hipEvent_t) { --live_events; return hipSuccess; }
 hipError_t hipEventQuery(hipEvent_t) { return hipSuccess; }
 hipError_t hipEventRecord(hipEvent_t, hipStream_t) { return hipSuccess; }
+hipError_t hipEventSynchronize(hipEvent_t) { return hipSuccess; }
+hipError_t hipSetDevice(int) { return hipSuccess; }
+hipError_t hipHostMalloc(void **p, size_t n, unsigned) { *p = std::malloc(n); return hipSuccess; }
+hipError_t hipHostFree(void *p) { std::free(p); return hipSuccess; }
+hipError_t hipMemcpyAsync(void *d, const void *s, size_t n, hipMemcpyKind, hipStream_t) { std::memcpy(d, s, n); return hipSuccess; }
 }
 #define CHECK(c) do { if (!(c)) { std::printf("line %d: %s\n", __LINE__, #c); return 1; } } while (0)
 int main() {
@@ -108,4 +120,20 @@ def test_events_of_a_refused_build_are_destroyed(tmp_path):
     } catch (const Error &) {
     }
     CHECK(live_events == 0);
+""")
+
+
+def test_staged_copy_goes_on_without_the_threads_it_cannot_start(tmp_path):
+    _run(tmp_path, """
+    HostStage stage;
+    const size_t n = 9 * MB + 5;
+    char *from = static_cast<char *>(std::malloc(n)), *to = static_cast<char *>(std::malloc(n));
+    for (int k = 0; k < 12; ++k) {  // memory for the first k allocations only
+        for (size_t i = 0; i < n; ++i) from[i] = (char)(i * 7 + i / 256 + k);
+        std::memset(to, 0, n);
+        news_left = k;
+        stage.copy(0, to, from, n);
+        news_left = 1 << 30;
+        CHECK(std::memcmp(from, to, n) == 0);
+    }
 """)
