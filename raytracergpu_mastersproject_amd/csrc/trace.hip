@@ -248,6 +248,11 @@ constexpr uint32_t kNoRay = ~0u;
 // and width 8's any hit too (1,052 -> 1,078).
 template <int W> constexpr bool kDefer = W == kQ4 || W == 4;
 
+// Work counters at most.  Width 2's kernel without the refinement has one (fixed here: as an argument it cost as much as 32): with 32,
+// launches from 2 M rays are slower than they were before (fp32 closest hits over 1 M triangles, 32 counters | one: 1 M rays 736 | 808 us,
+// 1.4 M 874 | 906, 2 M 1,090 | 1,005, 4 M 1,754 | 1,639, 12 M 4,568 | 3,738).
+template <int W, bool REFINE> constexpr uint32_t kLines = W == 2 && !REFINE ? 1u : kCounterLines;
+
 // REFINE: store each hit with t, u, v refined in double (store_refined) instead of the fp32 values.
 // LAST: the wave's last rays go on with teams of lanes (trace_last).
 // MARKED: only the rays that the launch before has marked (mark_ray).
@@ -277,7 +282,8 @@ __global__ __launch_bounds__(256, W == kQ4 ? 5 : 1) void k_trace_persistent(Trac
     }
     const uint32_t wpb = blockDim.x / 64u;
     const ChunkSchedule<uint32_t> sched(n, gridDim.x * wpb);
-    WorkLines lines(blockIdx.x * wpb + __builtin_amdgcn_readfirstlane(threadIdx.x / 64u), gridDim.x * wpb);
+    WorkLines lines(blockIdx.x * wpb + __builtin_amdgcn_readfirstlane(threadIdx.x / 64u), gridDim.x * wpb,
+                    kLines<W, REFINE>);
     Trav t;
     t.have = false;
     t.top = 0;
@@ -721,7 +727,10 @@ void launch_trace(rt_context *ctx, const Scene &sc, const rt_ray *rays, uint32_t
     // Persistent launches refine in the kernel, at each wave's refills: a separate pass reads every ray and hit again
     // (16.8 M any-hit rays 3,390 us with it, 3,295 without; 1 M on 1,024 triangles 106 and 100).  Width 8's any hit, with
     // its larger kernel, keeps the pass (4 M rays 1,093 us, 1,118 in the kernel).
-    const bool refine_in_kernel = refine && c.persistent && !(any && sc.width == 8);
+    // So do large any-hit launches of width 2 (12 M rays over 1 M triangles 4,382 us, 3,868 with the pass and the kernel without
+    // the refinement; 1.4 M 797 and 913).
+    const bool pass = any && (sc.width == 8 || (sc.width == 2 && n > 6144ull * (uint64_t)ctx->num_cus));
+    const bool refine_in_kernel = refine && c.persistent && !pass;
     TraceArgs a{view_of(sc), rays, hits, counts, n, c.refill, nullptr, c.leaf_weight, nullptr, team_limit(kLastTeam, sc.stack_bound)};
     uint32_t layout = sc.layout();
     if (counts) {  // the counts are those of the exact boxes
