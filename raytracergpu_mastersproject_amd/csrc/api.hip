@@ -210,7 +210,7 @@ int rt_render_batch(rt_context *ctx, const rt_render_job *jobs, uint32_t njobs, 
         const LaunchCfg c = resolve_cfg(ctx, ctx->scene(jobs[0].scene_id), cfg, false);
         hipStream_t st = static_cast<hipStream_t>(stream);
         std::map<uint32_t, std::vector<RenderJob>> by_layout;
-        std::vector<std::pair<const Scene *, RenderJob>> waves;  // images rendered bounce by bounce, as rt_render would
+        std::vector<std::pair<const Scene *, RenderJob>> waves;  // images rendered bounce by bounce (wave_schedule)
         std::vector<std::pair<uintptr_t, uintptr_t>> ranges;
         std::vector<std::pair<RenderJob *, uint32_t>> split;  // (job, samples per item)
         uint64_t split_bytes = 0;

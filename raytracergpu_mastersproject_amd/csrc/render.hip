@@ -13,7 +13,8 @@
 // queues the paths that scatter, those off dielectrics in a queue of their own;
 // k_wave_finish carries every queued path to its end in one persistent launch, the
 // dielectric queue first (those paths enter closed meshes and bounce longest), or k_path_team with several
-// lanes per path when the pass holds few; the samples are added to the image in order.  Path state lives in HBM between launches.
+// lanes per path when the pass holds few; k_path_redo ends the few paths that these leave over (kRedo); the samples are added to
+// the image in order.  Path state lives in HBM between launches.
 //
 // One persistent launch (fused small images, RT_RENDER_PERSISTENT_PATHS and the layout flags):
 // lanes take work items from 8x8 pixel tiles and run their samples to completion, advancing

@@ -301,9 +301,10 @@ struct RenderJob {
     uint32_t nwide, width, height, spp;
     Reach reach;
     uint32_t depth, random_state, flags, tiles_x;
-    uint32_t first_item, nitems, group;
+    uint32_t first_item, nitems;
+    uint32_t group;  // samples per split item (0 = whole pixels)
     uint32_t stack_bound;  // the scene's
-    uint32_t layout;  // of `nodes` (Scene::layout, or the width from a camera beyond Scene::reach.far_limit); group: samples per split item (0 = whole pixels)
+    uint32_t layout;  // of `nodes` (Scene::layout, or the width from a camera beyond Scene::reach.far_limit)
     float cam[12];  // pixel00, deltaU, deltaV, origin
 };
 // Split jobs give every (pixel, group of `group` consecutive samples) its own work item; the

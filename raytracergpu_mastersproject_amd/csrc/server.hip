@@ -5,8 +5,8 @@
 // allocation in one hipMalloc made at creation, so admission never calls the allocator).
 // Admitted requests advance in scheduling steps on two lanes, each a stream with up to
 // `pipeline` steps enqueued ahead of the device:
-//   - the big lane carries renders of at least kWaveMinSamples pixel-samples (rt_render's
-//     threshold for filling the device), the oldest alone, bounce by bounce as rt_render runs
+//   - the big lane carries renders of at least kWaveMinSamples pixel-samples, which fill the
+//     device, the oldest alone, bounce by bounce as rt_render runs
 //     it, in slices of the step's budget of device time (rates measured from earlier steps);
 //   - the small lane carries the other renders, together in one persistent launch
 //     (launch_render_jobs, split layout), whole where they fit the budget, plus one fused
@@ -344,7 +344,7 @@ bool enqueue_step(rt_server *s, bool big_lane) {
     // members are not held long by its last.  Ray queries ride along (slices of every admitted query).
     //
     // Big lane: the oldest device-filling render (at least kWaveMinSamples pixel-samples at
-    // admission, rt_render's own threshold) runs alone, bounce by bounce as rt_render would run
+    // admission) runs alone, bounce by bounce as rt_render runs
     // it (below), in slices of the budget.  Its last bounces run in one persistent launch that
     // holds the compute units to its end, so while small requests keep arriving (one admitted
     // within the last two step budgets) its slices are single passes whose finish launch yields

@@ -8,6 +8,8 @@
 //     lanes are refilled while long rays keep traversing.
 //   direct: one lane per ray (a launch-tuner candidate; the camera rays of renders).
 // A launch of few rays, and the last rays of each persistent wave, are traced by a team of lanes per ray (team.hpp).
+// Closest-hit launches over compressed nodes or by few lanes per ray leave marked the rays that need the exact nodes' order; a launch
+// behind them traces these (launch_marked, launch_team).
 // The batched variants run many scenes' ray batches in one launch.
 #include <algorithm>
 #include <cstdlib>

@@ -262,6 +262,9 @@ constexpr int kQ4 = 44;  // layout code of width 4 with compressed nodes (see no
 //   - When there is no other hit before E, their result is M.  When there is, the ray is traced
 //     again over the exact nodes in their order (kRedo).  That takes two hits a few roundings apart, at a corner
 //     that both triangles share: about one ray in 10^7 into a mesh, one in 10^6 aimed at its vertices.
+// It costs closest hits 4 to 10 % (4,096 rays / 120 k triangles 17.7 -> 19.2 us, 65,537 / 20 k 47 -> 53, 16.8 M / 4.2 M 3,505 -> 3,635;
+// 1080p x 16 frame 5,294 -> 5,558, 501x333x12 817 -> 892), as much on either side of the lines between routes: times given beside those
+// lines that were taken before are lower by as much.
 // ---------------------------------------------------------------------------
 constexpr uint32_t kRedo = 0xFFFFFFFEu;  // Trav::bslot
 
