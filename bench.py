@@ -20,6 +20,7 @@ from __future__ import annotations
 import argparse
 import json
 import os
+import re
 import sys
 import time
 from pathlib import Path
@@ -46,7 +47,7 @@ TRAFFIC_TABLE = ROOT / "profiles" / "trace_closest_rayquery_traffic.json"
 
 
 def load_traffic(launch_key):
-    """HBM bytes per launch of the headline traversal kernel at this launch configuration
+    """Bytes beyond L2 per launch of the headline traversal kernel at this launch configuration
     ("block,lds_stack,persistent,refill"), from the committed counter table; None when the table has no
     measurement of this configuration."""
     if launch_key is None or not TRAFFIC_TABLE.exists():
@@ -95,6 +96,22 @@ def _pmc_rows(path: Path, counter: str):
     return [(k, v) for _, k, v in rows]
 
 
+def _queries(rows):
+    """(traversal kernel, value) per ray query: a query's second launch, which walks again the rays that its first
+    one marked (k_trace_marked, or k_trace_persistent with MARKED, its last parameter), counts with the first."""
+    out = []
+    for k, v in rows:
+        if "::k_trace_" not in k:
+            continue
+        args = re.search(r"k_trace_persistent<([^>]*)>", k)
+        params = [] if args is None else [a.strip() for a in args.group(1).split(",")]
+        if out and ("::k_trace_marked" in k or (len(params) == 7 and params[6] == "true")):
+            out[-1] = (out[-1][0], out[-1][1] + v)
+        else:
+            out.append((k, v))
+    return out
+
+
 def traffic_table(fetch_csv: Path, write_csv: Path, configs, commands, out: Path = TRAFFIC_TABLE):
     """Builds the traffic table from a FETCH_SIZE run and a WRITE_SIZE run of --traffic-sweep.
     Each counter is scaled by what it reads for the copy of known size that leads the run."""
@@ -103,8 +120,7 @@ def traffic_table(fetch_csv: Path, write_csv: Path, configs, commands, out: Path
     cf = [v for k, v in fetch if k.startswith("__amd_rocclr_copyBuffer")][:5]
     cw = [v for k, v in write if k.startswith("__amd_rocclr_copyBuffer")][:5]
     f_scale, w_scale = copy_bytes / (np.mean(cf) * 1024), copy_bytes / (np.mean(cw) * 1024)
-    tf = [(k, v) for k, v in fetch if "::k_trace_" in k]
-    tw = [(k, v) for k, v in write if "::k_trace_" in k]
+    tf, tw = _queries(fetch), _queries(write)
     assert len(tf) == len(tw) == len(configs), (len(tf), len(tw), len(configs))
     table = {"counters": "FETCH_SIZE, WRITE_SIZE (KiB per dispatch)", "fetch_scale": f_scale, "write_scale": w_scale,
              "calibration": f"{len(cf)} device-to-device copies of {copy_bytes} bytes", "commands": commands,
@@ -730,12 +746,13 @@ def main():
     roofline = {"bound": "hbm", "achieved": None if achieved is None else round(achieved, 1), "peak": HBM_PEAK_GBS,
                 "unit": "GB/s", "frac": None if achieved is None else round(achieved / HBM_PEAK_GBS, 4),
                 "traffic": traffic, "kernel_ms": round(avg_kernel_ms, 4), "launch": launch_key,
-                "basis": "HBM bytes per launch measured by rocprofv3 (FETCH_SIZE x2 + WRITE_SIZE, copy-calibrated) "
-                         "for this launch configuration, over the traversal kernel's live average duration",
+                "basis": "bytes per launch beyond L2 measured by rocprofv3 (FETCH_SIZE x2 + WRITE_SIZE, "
+                         "copy-calibrated; what the memory-side cache serves is in them) for this launch "
+                         "configuration, over the traversal kernel's live average duration",
                 "algorithmic_gbs": round(algorithmic, 1),
                 "algorithmic_note": "32 B per AABB test + 36 B per triangle test + 48 B ray/hit, counted per ray by "
                                     "the kernel; node fetches are mostly served by L2 and the MALL, so this demand "
-                                    "rate exceeds what HBM moves"}
+                                    "rate exceeds what HBM could move"}
 
     cpu = parity = None
     if not args.no_cpu_baseline:
