@@ -401,9 +401,10 @@ __device__ __forceinline__ void node_step(Trav &t, const StackMem &m, const uint
 // ---------------------------------------------------------------------------
 // Compressed width-4 nodes (layout code kQ4; rt_device.hpp describes them).
 //
-// What bounds the per-lane traversal is the L1's address pipe: a 16-byte load takes one tag lookup per
-// lane, and a 128-byte node takes seven of them (measured on the 16.8 M-ray / 4.2 M-triangle query: 2.58e9
-// lookups, address unit busy 95 % of the launch).  A 64-byte node takes four, and moves half the bytes.
+// On exact nodes the L1's address pipe is the busiest unit of the per-lane traversal: a 16-byte load takes one
+// tag lookup per lane, and a 128-byte node takes seven of them (measured on the 16.8 M-ray / 4.2 M-triangle
+// query: 2.58e9 lookups, address unit busy 84 % of the launch, VALU issue 66 %).  A 64-byte node takes four,
+// and moves half the bytes.
 // Decoding costs less than it seems: the planes of four children lie in one word, so the near and far
 // planes of a ray are chosen per axis and not per child; a pair of children's planes becomes two half
 // floats with one byte permute, which a mixed-precision FMA reads directly.  Children are sorted as
@@ -417,8 +418,9 @@ __device__ __forceinline__ void node_step(Trav &t, const StackMem &m, const uint
 // boxes reach must not count, or results would depend on the node format: a hit is taken only if the ray enters
 // the leaf's exact box (leaf_entered, evaluated once per hit).
 //
-// Measured, exact -> compressed: 16.8 M rays / 4.2 M triangles 5.65 -> 3.68 ms (lookups 1.56e9, VALU
-// issue now 0.9 of the launch, HBM 19.2 GB = 5.2 TB/s, the rate of a large copy); 1080p x 16 spp frame 6.12 ->
+// Measured, exact -> compressed: 16.8 M rays / 4.2 M triangles 5.65 -> 3.68 ms (lookups 1.56e9, address unit
+// busy 62 %, VALU issue 95 % with 32 of 64 lanes active; 19.4 GB beyond L2 where exact nodes read 23.1, of which
+// the memory-side cache, which holds all 127 MB of nodes, serves an unknown part); 1080p x 16 spp frame 6.12 ->
 // 5.31 ms; 1.0 M any-hit rays / 1 M triangles 612 -> 556 us.
 // ---------------------------------------------------------------------------
 constexpr float kSlackQ = 0x1.4p-21f;  // 10 * 2^-24
